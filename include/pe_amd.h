@@ -286,13 +286,13 @@ int pe_world_set_axis(pe_world* w, int32_t axis);
  * the four timers of World (world.h:58-61).  enable = 1 records hipEvents around stages. */
 int pe_world_set_timing(pe_world* w, int32_t enable);
 int pe_world_get_stage_times(pe_world* w, double* ms /*4*/);
-/* Workgroups of the grid-wide Gauss-Seidel sweep (0 = the default: 4 to 16 by body count, about one
- * colour's pair per thread; clamped to the co-resident limit).  No counterpart in the reference; results
+/* Workgroups of the solve over the GPU (0 = the default: 8 to 256 by body count, about 16 pairs in contact
+ * per wave; clamped to the co-resident limit).  No counterpart in the reference; results
  * do not depend on it. */
 int pe_world_set_solver_blocks(pe_world* w, int32_t blocks);
-/* How the solver's colouring runs (0 = by body count: one workgroup's claims in LDS up to 3 000
- * bodies, rounds over the GPU beyond; 1 = one workgroup, at most 12 288 bodies; 2 = rounds).  Both
- * give the same colour classes.  No counterpart in the reference; results do not depend on it. */
+/* How the solver's colouring runs (0 = the default; 1 = one workgroup's claims, at most 12 288 bodies;
+ * 2 = over the GPU, unless a body is in more than 64 pairs in contact).  Both give the same colour
+ * classes.  No counterpart in the reference; results do not depend on it. */
 int pe_world_set_colouring(pe_world* w, int32_t mode);
 /* The per-body records the stage entry points take (layouts under "stage entry points" below),
  * as the world's last integrate stage wrote them: AABB records [n][8], collision records [n][20],

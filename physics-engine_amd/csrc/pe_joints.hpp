@@ -139,11 +139,10 @@ __device__ __forceinline__ void joint_setup(const BodyView& b, const JointDef& j
     }
 }
 
-// iterateSequentialImpulse of joint j on the bodies' temp velocities (solver records); each impulse
-// reads the angular velocities the ones before it left, as the reference reads them through
-// references to the bodies' members.
-__device__ __forceinline__ void joint_iterate(const BodyView& b, const JointDef& j, const JointRow& r) {
-    SolvBody A = load_solv(b, j.a), B = load_solv(b, j.b);
+// iterateSequentialImpulse of joint j on its bodies' temp velocities A.tv .. B.tw (never written for a
+// kinematic body); each impulse reads the angular velocities the ones before it left, as the reference
+// reads them through references to the bodies' members.
+__device__ __forceinline__ void joint_solve(const JointDef& j, const JointRow& r, SolvBody& A, SolvBody& B) {
     if (j.type == JT_BALL || j.type == JT_HINGE) {
         const f3 va = add(A.tv, cross(A.tw, r.ra));
         const f3 vb = add(B.tv, cross(B.tw, r.rb));
@@ -182,16 +181,6 @@ __device__ __forceinline__ void joint_iterate(const BodyView& b, const JointDef&
         const f3 rot = neg(mv(r.jmj_rot, sub(A.tw, B.tw)));
         apply_temp_angular(A.tw, A.kin, A.Iw, rot);
         apply_temp_angular(B.tw, B.kin, B.Iw, neg(rot));
-    }
-    if (!A.kin) {
-        float4* d = reinterpret_cast<float4*>(b.sbr(j.a));
-        d[0] = make_float4(A.tv.x, A.tv.y, A.tv.z, A.tw.x);
-        d[1].x = A.tw.y; d[1].y = A.tw.z;
-    }
-    if (!B.kin) {
-        float4* d = reinterpret_cast<float4*>(b.sbr(j.b));
-        d[0] = make_float4(B.tv.x, B.tv.y, B.tv.z, B.tw.x);
-        d[1].x = B.tw.y; d[1].y = B.tw.z;
     }
 }
 

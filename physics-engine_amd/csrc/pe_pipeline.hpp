@@ -683,76 +683,78 @@ __device__ __forceinline__ void iterate_pair(const BodyView& b, const PairStore&
     }
 }
 
-// iterate_pair split around the barrier before the pair's colour: gs_prefetch loads what no other
-// thread changes during the sweeps -- the pair's bodies, their world inverse inertias and its
-// first four rows (a pair's rows, accumulated impulses included, are only written by the thread
-// that solves it, every iteration the same thread) -- and gs_solve, after the barrier, loads the
-// bodies' temp velocities, which earlier colours changed, and solves the pair with the same
-// arithmetic in the same order.
-struct GsPair {
-    int p, ia, ib, n;
-    m33 Ia, Ib;
-    float rr[4][RW];
-};
-__device__ __forceinline__ void gs_prefetch(const BodyView& b, const PairStore& ps, int p, GsPair& G) {
-    G.p = p;
-    G.ia = ps.pa[p];
-    G.ib = ps.pb[p];
-    G.n = ps.npts[p];
-    const float* sa = b.sbr(G.ia);
-    const float* sb = b.sbr(G.ib);
-#pragma unroll
-    for (int k = 0; k < 9; k++) { G.Ia.m[k] = sa[SB_IW + k]; G.Ib.m[k] = sb[SB_IW + k]; }
-#pragma unroll
-    for (int u = 0; u < 4; u++)
-        if (u < G.n) ld_rec<RW / 4>(ps.rows + ((size_t)p * 8 + u) * RW, G.rr[u]);
+// ---- four lanes per pair
+// A row's update is a chain of about 190 instructions on one lane, and a colour's pass lasts as long as the
+// chains of its pairs' rows.  Spread over a quad of lanes -- lane c holds component c of both bodies'
+// velocities and of the row's vectors, the three directions' projections run side by side on the three
+// lanes, components cross the quad as DPP operands -- it is about 95, every operation the scalar row's
+// (iterate_row, apply_temp) on the same operands in the same order, so the results are the same bits.
+// Lane 3 repeats lane 2.
+template <int P0, int P1, int P2> __device__ __forceinline__ float quad_perm(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), P0 | P1 << 2 | P2 << 4 | P2 << 6, 0xf, 0xf, true));
 }
-__device__ __forceinline__ void gs_solve(const BodyView& b, const PairStore& ps, GsPair& G) {
-    const int p = G.p, n = G.n;
-    float* R = ps.rows;
-    const float4* qa = reinterpret_cast<const float4*>(b.sbr(G.ia));
-    const float4* qb = reinterpret_cast<const float4*>(b.sbr(G.ib));
-    const float4 a0 = qa[0], a1 = qa[1], b0 = qb[0], b1 = qb[1];
-    f3 tva{a0.x, a0.y, a0.z}, twa{a0.w, a1.x, a1.y}, tvb{b0.x, b0.y, b0.z}, twb{b0.w, b1.x, b1.y};
-    const float ima = a1.z, imb = b1.z;
-    const bool ka = a1.w != 0.0f, kb = b1.w != 0.0f;
-    for (int k0 = 0; k0 < n; k0 += 4) {
-        if (k0 > 0) {
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-                if (k0 + u < n) ld_rec<RW / 4>(R + ((size_t)p * 8 + k0 + u) * RW, G.rr[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            if (k0 + u < n) {
-                const float* o = G.rr[u];
-                Row r;
-                r.ra = f3{o[R_RA], o[R_RA + 1], o[R_RA + 2]};
-                r.rb = f3{o[R_RB], o[R_RB + 1], o[R_RB + 2]};
-                r.n = f3{o[R_N], o[R_N + 1], o[R_N + 2]};
-                r.t0 = f3{o[R_T0], o[R_T0 + 1], o[R_T0 + 2]};
-                r.t1 = f3{o[R_T1], o[R_T1 + 1], o[R_T1 + 2]};
-                r.rhs = o[R_RHS]; r.mn = o[R_MN]; r.mt0 = o[R_MT0]; r.mt1 = o[R_MT1]; r.mu = o[R_MU];
-                float ln = o[R_LN], lt0 = o[R_LT0], lt1 = o[R_LT1];
-                const f3 J = iterate_row(r, ln, lt0, lt1, tva, twa, tvb, twb);
-                if (!ka) apply_temp(tva, twa, ima, G.Ia, r.ra, J);
-                if (!kb) apply_temp(tvb, twb, imb, G.Ib, r.rb, neg(J));
-                G.rr[u][R_LN] = ln; G.rr[u][R_LT0] = lt0; G.rr[u][R_LT1] = lt1;
-                float4* dst = reinterpret_cast<float4*>(R + ((size_t)p * 8 + k0 + u) * RW) + 5;   // floats 20..23
-                *dst = make_float4(ln, lt0, lt1, 0.0f);
-            }
-        }
-    }
-    if (!ka) {
-        float4* d = reinterpret_cast<float4*>(b.sbr(G.ia));
-        d[0] = make_float4(tva.x, tva.y, tva.z, twa.x);
-        d[1].x = twa.y; d[1].y = twa.z;
-    }
-    if (!kb) {
-        float4* d = reinterpret_cast<float4*>(b.sbr(G.ib));
-        d[0] = make_float4(tvb.x, tvb.y, tvb.z, twb.x);
-        d[1].x = twb.y; d[1].y = twb.z;
-    }
+__device__ __forceinline__ float quad_x(float v) { return quad_perm<0, 0, 0>(v); }
+__device__ __forceinline__ float quad_y(float v) { return quad_perm<1, 1, 1>(v); }
+__device__ __forceinline__ float quad_z(float v) { return quad_perm<2, 2, 2>(v); }
+__device__ __forceinline__ float quad_next(float v) { return quad_perm<1, 2, 0>(v); }   // component c + 1
+__device__ __forceinline__ float quad_prev(float v) { return quad_perm<2, 0, 1>(v); }   // component c + 2
+// dot(a, v) with a's components in lane-invariant registers, v across the quad: a.x v.x + (a.y v.y + a.z v.z)
+__device__ __forceinline__ float quad_dot(float ax, float ay, float az, float v) {
+    return quad_x(v) * ax + (quad_y(v) * ay + quad_z(v) * az);
+}
+// Lane c's part of a body: temp velocities, row c of the world inverse inertia, the inverse mass.
+struct QuadBody {
+    float tv, tw, i0, i1, i2, im;
+    bool kin;
+};
+// Lane c's part of a solver row: r[c + 1], r[c + 2] of both arms, its own direction (lane 0 the normal, 1
+// and 2 the tangents) whole, component c of all three, the effective mass of its direction and the
+// impulse accumulated along it.
+struct QuadRow {
+    float ra1, ra2, rb1, rb2, dx, dy, dz, n, t0, t1, rhs, m, mu, acc;
+};
+__device__ __forceinline__ void quad_load_row(const float* o, int c, QuadRow& r) {
+    const int c1 = c == 2 ? 0 : c + 1, c2 = c == 0 ? 2 : c - 1;
+    r.ra1 = o[R_RA + c1]; r.ra2 = o[R_RA + c2];
+    r.rb1 = o[R_RB + c1]; r.rb2 = o[R_RB + c2];
+    r.dx = o[R_N + 3 * c]; r.dy = o[R_N + 3 * c + 1]; r.dz = o[R_N + 3 * c + 2];   // R_N, R_T0, R_T1 in turn
+    r.n = o[R_N + c]; r.t0 = o[R_T0 + c]; r.t1 = o[R_T1 + c];
+    r.rhs = o[R_RHS];
+    r.m = o[R_MN + c];
+    r.mu = o[R_MU];
+    r.acc = o[R_LN + c];
+}
+__device__ __forceinline__ void quad_load_body(const float* sb, int c, bool kin, QuadBody& q) {
+    q.i0 = sb[SB_IW + 3 * c]; q.i1 = sb[SB_IW + 3 * c + 1]; q.i2 = sb[SB_IW + 3 * c + 2];
+    q.im = sb[SB_IM];
+    q.kin = kin;
+}
+// RigidBody::applyTempImpulse (rigidbody.cpp:166-170), see apply_temp.
+__device__ __forceinline__ void quad_apply(QuadBody& q, float r1, float r2, float J) {
+    const float x = r1 * quad_prev(J) - r2 * quad_next(J);
+    const float tv = q.tv + J * q.im;
+    const float tw = q.tw + quad_dot(q.i0, q.i1, q.i2, x);
+    q.tv = q.kin ? q.tv : tv;
+    q.tw = q.kin ? q.tw : tw;
+}
+// FrictionContactConstraint::iterateSequentialImpulse (friction_contact_constraint.cpp:75-108) for one
+// row: iterate_row and both apply_temp.  first: this is lane 0 of its quad.
+__device__ __forceinline__ void quad_solve_row(QuadRow& r, bool first, QuadBody& A, QuadBody& B) {
+    const float ca = quad_next(A.tw) * r.ra2 - quad_prev(A.tw) * r.ra1;
+    const float cb = quad_next(B.tw) * r.rb2 - quad_prev(B.tw) * r.rb1;
+    const float vr = ((A.tv + ca) - B.tv) - cb;
+    // lane 0: the normal impulse's change, clamped; lanes 1, 2: the tangent impulses before the cone
+    const float v = (first ? r.rhs : r.acc) - quad_dot(r.dx, r.dy, r.dz, vr) * r.m;
+    const float dn = v > -r.acc ? v : -r.acc;
+    const float ln = r.acc + dn;
+    const float sq = v * v;
+    const float scale = r.mu * quad_x(ln) / sqrtf(quad_y(sq) + quad_z(sq));
+    const float t = scale < 1 ? v * scale : v;
+    const float delta = first ? dn : t - r.acc;
+    r.acc = first ? ln : t;
+    const float J = (quad_x(delta) * r.n + quad_y(delta) * r.t0) + quad_z(delta) * r.t1;
+    quad_apply(A, r.ra1, r.ra2, J);
+    quad_apply(B, r.rb1, r.rb2, -J);
 }
 
 // Solver state held in LDS for the Gauss-Seidel sweeps: per body (local index) one 64-byte record
@@ -835,15 +837,8 @@ __device__ __forceinline__ void iterate_pair_lds(const LdsSolve& L, int pl, floa
     }
 }
 
-// SequentialImpulseSolver::solve's syncTempVelocity (sequential_impulse_solver.cpp:71-80)
-__device__ __forceinline__ void sync_body(const BodyView& b, int i) {
-    if (b.iat(I_KIN, i)) return;
-    const float* s = b.sbr(i);
-    st3(b, F_V, i, f3{s[SB_TV], s[SB_TV + 1], s[SB_TV + 2]});
-    st3(b, F_W, i, f3{s[SB_TW], s[SB_TW + 1], s[SB_TW + 2]});
-}
-// The same for a world whose records hold its velocities (integrate_body<.., true>): into the
-// solver record's v, w.
+// SequentialImpulseSolver::solve's syncTempVelocity (sequential_impulse_solver.cpp:71-80) for a world whose
+// records hold its velocities (integrate_body<.., true>): into the solver record's v, w.
 __device__ __forceinline__ void sync_body_rec(const BodyView& b, int i) {
     if (b.iat(I_KIN, i)) return;
     float* s = b.sbr(i);
@@ -888,10 +883,22 @@ __host__ __device__ inline int prio(int p, int npts) {
 }
 }
 
+// Claims in LDS, or in global memory as device-scope atomics with a device-scope fence at each workgroup
+// barrier (the atomics pass the caches by).
 template <bool LDS>
 __device__ __forceinline__ int claim_get(int* claim, int i) {
     if (LDS) return claim[i];
     return __hip_atomic_load(&claim[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <bool LDS>
+__device__ __forceinline__ void claim_set(int* claim, int i, int v) {
+    if (LDS) claim[i] = v;
+    else __hip_atomic_store(&claim[i], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <bool LDS>
+__device__ __forceinline__ void claim_sync() {
+    if (!LDS) __threadfence();
+    __syncthreads();
 }
 
 // bufs: three lists of pair capacity; bufs[0] holds the nact active pairs on entry (pair store
@@ -908,7 +915,7 @@ __device__ int colour_pairs(const BodyView& b, const PairStore& ps, int* bufs[3]
     (void)wsum;
     int ia = 0, ncol = 0;
     if (tid == 0) cnt[0] = 0;
-    __syncthreads();
+    claim_sync<LDS>();
     while (nact > 0) {
         int* cand = bufs[ia];
         int* nxt = bufs[(ia + 1) % 3];
@@ -916,7 +923,7 @@ __device__ int colour_pairs(const BodyView& b, const PairStore& ps, int* bufs[3]
         int ncand = nact;
         const int col_begin = cnt[0];
         if (tid == 0) { cs[ncol] = col_begin; cnt[1] = 0; }
-        __syncthreads();
+        claim_sync<LDS>();
         while (ncand > 0) {
             for (int q = tid; q < ncand; q += B) {
                 const int p = cand[q];
@@ -926,7 +933,7 @@ __device__ int colour_pairs(const BodyView& b, const PairStore& ps, int* bufs[3]
                 if (!b.iat(I_KIN, c)) atomicMin(&claim[c - off], pr);
             }
             if (tid == 0) cnt[2] = 0;
-            __syncthreads();
+            claim_sync<LDS>();
             const int sub_begin = cnt[0];
             for (int base = 0; base < ncand; base += B) {
                 const int q = base + tid;
@@ -950,40 +957,40 @@ __device__ int colour_pairs(const BodyView& b, const PairStore& ps, int* bufs[3]
                 if (blk) def[ib] = p;
                 if (stay) nxt[is] = p;
             }
-            __syncthreads();
+            claim_sync<LDS>();
             const int sub_end = cnt[0], nstay = cnt[2];
             // clear this sub-round's claims (taken bodies stay taken)
             for (int q = tid; q < ncand; q += B) {
                 const int p = cand[q];
                 const int a = ps.pa[p], c = ps.pb[p];
-                if (!b.iat(I_KIN, a) && claim_get<LDS>(claim, a - off) != TAKEN) claim[a - off] = FREE;
-                if (!b.iat(I_KIN, c) && claim_get<LDS>(claim, c - off) != TAKEN) claim[c - off] = FREE;
+                if (!b.iat(I_KIN, a) && claim_get<LDS>(claim, a - off) != TAKEN) claim_set<LDS>(claim, a - off, FREE);
+                if (!b.iat(I_KIN, c) && claim_get<LDS>(claim, c - off) != TAKEN) claim_set<LDS>(claim, c - off, FREE);
             }
-            __syncthreads();
+            claim_sync<LDS>();
             for (int q = sub_begin + tid; q < sub_end; q += B) {
                 const int p = order[q];
                 const int a = ps.pa[p], c = ps.pb[p];
-                if (!b.iat(I_KIN, a)) claim[a - off] = TAKEN;
-                if (!b.iat(I_KIN, c)) claim[c - off] = TAKEN;
+                if (!b.iat(I_KIN, a)) claim_set<LDS>(claim, a - off, TAKEN);
+                if (!b.iat(I_KIN, c)) claim_set<LDS>(claim, c - off, TAKEN);
             }
-            __syncthreads();
+            claim_sync<LDS>();
             int* t = cand; cand = nxt; nxt = t;
             ncand = nstay;
         }
         const int col_end = cnt[0];
         for (int q = col_begin + tid; q < col_end; q += B) {
             const int p = order[q];
-            claim[ps.pa[p] - off] = FREE;
-            claim[ps.pb[p] - off] = FREE;
+            claim_set<LDS>(claim, ps.pa[p] - off, FREE);
+            claim_set<LDS>(claim, ps.pb[p] - off, FREE);
         }
         const int ndef = cnt[1];
-        __syncthreads();
+        claim_sync<LDS>();
         ia = (ia + 2) % 3;
         nact = ndef;
         ncol++;
     }
     if (tid == 0) cs[ncol] = cnt[0];
-    __syncthreads();
+    claim_sync<LDS>();
     return ncol;
 }
 

@@ -28,11 +28,11 @@ struct DevCounts {          // device-side counters of one step
     int32_t nshape;         // pairs of this narrowphase that involve a cylinder or a mesh ...
     int32_t nsat;           // ... of which these run the polyhedral separating-axis routine
     int32_t ncomp;          // ... and these involve a compound body
-    int32_t nact;           // pairs the colouring orders (contact points, not both bodies kinematic)
-    uint32_t jp_rem[3];     // colouring rounds: pairs left uncoloured, round r in slot r % 3 (a slot is
-                            // cleared two rounds before it is counted, one round after it is read)
+    int32_t nact;           // pairs the solve orders (contact points, not both bodies kinematic)
+    int32_t jp_ncol;        // colours the last sweep over the GPU counted
     uint32_t adj_total;     // colouring: adjacency entries
-    int32_t jp_rounds;      // colouring: rounds the last colouring took
+    int32_t jp_big;         // some body is in more pairs than the colouring over the GPU takes
+    int32_t jp_rounds;      // colouring over the GPU: the most times a thread tried its pairs
 };
 // Capacity errors, OR-ed into DevCounts::overflow by the step that hits them and kept until the
 // host reads and reports them: a result that lost pairs or contact points is never returned as a
@@ -40,6 +40,7 @@ struct DevCounts {          // device-side counters of one step
 constexpr int OVF_PAIRS = 1;         // the broadphase found more pairs than the pair capacity
 constexpr int OVF_CHUNKS = 4;        // the sweep had more candidates than its chunk capacity
 constexpr int OVF_CLIP = 8;          // a clipped polygon outgrew its buffer (contact points lost)
+constexpr int OVF_STALL = 16;        // the solver gave up a wait (not a capacity: a fault of this program)
 
 constexpr int SAP_CHUNK = 32;        // candidates per thread in the sweep
 static_assert(SAP_CHUNK <= 32, "a chunk's test outcomes are one 32-bit mask");

@@ -7,9 +7,9 @@
 //                      reference's (i, j) order, next axis
 //   k_narrow           thread / pair: shape dispatch + 8-slot contact cache + depth sort
 //   k_setup            thread / pair: solver rows (FrictionContactConstraint::initSequentialImpulse)
-//   k_colour           one 1024-thread workgroup: constraint-graph colouring (claims in LDS)
-//   k_gs_grid          cooperative launch over the whole GPU: Gauss-Seidel sweeps colour by
-//                      colour with a grid barrier between colours, then velocity sync
+//   k_jp_*             the constraint graph: per body its pairs
+//   k_solve_flow       cooperative launch over the whole GPU: colouring, then the Gauss-Seidel sweeps in
+//                      colour order as a data flow between the pairs, and the velocity sync
 #include "pe_common.hpp"
 #include "pe_device.hpp"
 #include "pe_prims.hpp"
@@ -32,9 +32,7 @@ using namespace pe;
 
 namespace {
 
-constexpr int MAX_COLORS = 1024;
-constexpr int SOLVE_THREADS = 1024;
-constexpr int CLAIM_LDS = 12288;     // bodies whose colouring claims fit in LDS (48 KiB)
+constexpr int CLAIM_MAX = 12288;     // bodies up to which a caller may ask for the colouring in one workgroup
 
 struct Dev {
     BodyView b;
@@ -43,17 +41,27 @@ struct Dev {
     int32_t* shape_list;    // [pcap] pairs handed from k_narrow to k_narrow_shapes (from the front)
                             // and to k_narrow_sat (from the back)
     int32_t* comp_list;     // [pcap] pairs with a compound body (worlds with compounds; else null)
-    // colouring by rounds: per-body degree offsets [n + 1] and fill cursors [n], adjacency [2 pcap],
-    // colour per pair [pcap], pairs per colour [pcap + 1]
-    uint32_t* jp_deg;
+    // the solve's constraint graph: per dynamic body its active pairs, jp_deg[i] entries from jp_off[i]
+    // on in jp_adj [2 pcap] (filled through the cursors jp_fill), per pair its colour and its place in
+    // the colour, pairs per colour [pcap + 1]
+    int32_t* jp_deg;
+    int32_t* jp_off;
     int32_t* jp_fill;
-    int2* jp_adj;        // per dynamic body, its active pairs: (pair, claim priority)
+    int2* jp_adj;        // (pair, claim priority)
     int32_t* jp_col;
+    int32_t* jp_idx;
     int32_t* jp_ccount;
+    int32_t* jp_hist;       // [FLOW_BINS][workgroups] pairs of each of the first colours per workgroup
+    int32_t* jp_items;      // [pcap + 1] sweep: first item of each colour (colours beyond those kept in LDS)
+    // the sweep (k_solve_flow): temp velocities with the number of updates made to them, and per place in
+    // the solve order its pair and its place in its bodies' sequences of updates
+    uint64_t* vel;          // [n][VELW]
+    int4* q_pair;           // [pcap] pair, bodies A and B (top bit: kinematic), rows
+    int4* q_seq;            // [pcap] A's updates before this pair's in an iteration, A's in an iteration; B's
     int32_t* order;         // [pcap]
     int32_t* act;           // [3*pcap] colouring work lists
     int32_t* color_start;   // [pcap+1]
-    int32_t* claim;         // [n] (global claims when n > CLAIM_LDS)
+    int32_t* claim;         // [n] claims of the colouring in one workgroup
     DevCounts* cnt;
     int pcap;
     float dt;
@@ -64,6 +72,8 @@ struct Dev {
     JointRow* jrows;
     const int32_t* jorder;   // [njoints] joint indices, colour by colour
     const int32_t* jcs;      // [njcol + 1] colour starts in jorder
+    const int2* jseq;        // [njoints] joints of body A (B) in earlier joint colours
+    const int32_t* jdeg;     // [n] joints of a dynamic body (null: no joints)
     int njoints, njcol;
     // sleeping, lifetimes, removals (World::updateObjectStatus) and collision reports
     StatusView st;
@@ -312,10 +322,83 @@ __global__ void k_narrow_finish(Dev d) {
 }
 
 // ------------------------------------------------------------------ stage 3: solver
-// SequentialImpulseSolver::setupSolver (sequential_impulse_solver.cpp:11-58), thread / pair.
+// Words of a body's temp velocities in d.vel: component c of the linear (c) and angular (4 + c) one, each
+// beside the number of updates made to the body in this solve (high half).  64 bytes per body.
+constexpr int VELW = 8;
+__device__ __forceinline__ uint64_t vel_word(float v, uint32_t seq) { return (uint64_t)seq << 32 | __float_as_uint(v); }
+
+// Clears the solve's per-body and per-colour counters and sets every body's velocity words.
+__global__ void k_solve_begin(Dev d) {
+    const int n = d.b.n;
+    const int gtid = blockIdx.x * blockDim.x + threadIdx.x, gsz = gridDim.x * blockDim.x;
+    for (int i = gtid; i < n; i += gsz) {
+        d.jp_deg[i] = 0;
+        d.jp_fill[i] = 0;
+        const float* sb = d.b.sbr(i);
+        ulonglong2* w = reinterpret_cast<ulonglong2*>(d.vel + (size_t)i * VELW);
+        w[0] = make_ulonglong2(vel_word(sb[SB_TV], 0), vel_word(sb[SB_TV + 1], 0));
+        w[1] = make_ulonglong2(vel_word(sb[SB_TV + 2], 0), 0);
+        w[2] = make_ulonglong2(vel_word(sb[SB_TW], 0), vel_word(sb[SB_TW + 1], 0));
+        w[3] = make_ulonglong2(vel_word(sb[SB_TW + 2], 0), 0);
+    }
+    for (int c = gtid; c < d.cnt->jp_ncol; c += gsz) d.jp_ccount[c] = 0;   // the colours the last solve counted
+    if (gtid == 0) {
+        d.cnt->nact = 0;
+        d.cnt->adj_total = 0;
+        d.cnt->jp_rounds = 0;
+        d.cnt->jp_big = 0;
+    }
+}
+
+// SequentialImpulseSolver::setupSolver (sequential_impulse_solver.cpp:11-58), thread / pair: the solver
+// rows, the list of the pairs to solve (contact points, not both bodies kinematic) and their dynamic
+// bodies' degrees.
 __global__ void k_setup(Dev d) {
     const int np = d.cnt->npairs;
-    for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < np; p += gridDim.x * blockDim.x) setup_pair(d.b, d.ps, p, d.dt);
+    const int gsz = gridDim.x * blockDim.x;
+    const int n_iter = (np + gsz - 1) / gsz;
+    for (int it = 0; it < n_iter; it++) {
+        const int p = it * gsz + blockIdx.x * blockDim.x + threadIdx.x;
+        bool act = false;
+        if (p < np && d.ps.npts[p] > 0) {
+            setup_pair(d.b, d.ps, p, d.dt);
+            const int a = d.ps.pa[p], c = d.ps.pb[p];
+            const bool ka = d.b.iat(I_KIN, a) != 0, kc = d.b.iat(I_KIN, c) != 0;
+            act = !(ka && kc);
+            if (act) {
+                d.jp_col[p] = -1;
+                if (!ka) atomicAdd(&d.jp_deg[a], 1);
+                if (!kc) atomicAdd(&d.jp_deg[c], 1);
+            }
+        }
+        const int slot = wave_append(act, &d.cnt->nact);
+        if (act) d.act[slot] = p;
+    }
+}
+// A body in more pairs than this is coloured around by claims (k_solve_flow): its pairs all take different
+// colours one after another, and every try would scan all of them.
+constexpr int JP_MAX_DEG = 64;
+// Each body's range of the adjacency lists (the ranges' order does not matter).
+__global__ void k_jp_alloc(Dev d) {
+    const int n = d.b.n;
+    const int gsz = gridDim.x * blockDim.x;
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int n_iter = (n + gsz - 1) / gsz;
+    for (int it = 0; it < n_iter; it++) {
+        const int i = it * gsz + blockIdx.x * blockDim.x + threadIdx.x;
+        const int deg = i < n ? d.jp_deg[i] : 0;
+        int incl = deg;
+#pragma unroll
+        for (int o = 1; o < WAVE; o <<= 1) {
+            const int y = __shfl_up(incl, o, WAVE);
+            if (lane >= o) incl += y;
+        }
+        int base = 0;
+        if (lane == WAVE - 1 && incl > 0) base = (int)atomicAdd(&d.cnt->adj_total, (uint32_t)incl);
+        base = __shfl(base, WAVE - 1, WAVE);
+        if (i < n) d.jp_off[i] = base + incl - deg;
+        if (__any(deg > JP_MAX_DEG) && lane == 0) d.cnt->jp_big = 1;
+    }
 }
 
 // BallJointConstraint / HingeJointConstraint / SliderJointConstraint::initSequentialImpulse, thread / joint
@@ -324,37 +407,6 @@ __global__ void k_joint_setup(Dev d) {
     for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < d.njoints; k += gridDim.x * blockDim.x)
         joint_setup(d.b, d.joints[k], d.jrows[k], d.dt);
 }
-
-// Constraint-graph colouring of the pairs with contact points, one workgroup (colour_pairs in
-// pe_pipeline.hpp): writes the solve order, colour starts and colour count.
-template <bool LDS_CLAIM>
-__global__ void __launch_bounds__(SOLVE_THREADS) k_colour(Dev d) {
-    extern __shared__ int s_claim[];
-    __shared__ int wsum[SOLVE_THREADS / WAVE + 1];
-    const BodyView& b = d.b;
-    const int np = d.cnt->npairs;
-    int* claim = LDS_CLAIM ? s_claim : d.claim;
-    for (int i = threadIdx.x; i < b.n; i += blockDim.x) claim[i] = colour::FREE;
-    int* act = d.act;
-    int nact = 0;
-    for (int base = 0; base < np; base += blockDim.x) {
-        const int p = base + threadIdx.x;
-        int flag = 0;
-        if (p < np && d.ps.npts[p] > 0) flag = !(b.iat(I_KIN, d.ps.pa[p]) && b.iat(I_KIN, d.ps.pb[p]));
-        int tot;
-        const int ex = block_exclusive_scan(flag, wsum, &tot);
-        if (flag) act[nact + ex] = p;
-        nact += tot;
-    }
-    __syncthreads();
-    int* bufs[3] = {act, act + d.pcap, act + 2 * (size_t)d.pcap};
-    const int ncol = colour_pairs<LDS_CLAIM>(b, d.ps, bufs, nact, d.order, d.color_start, claim, 0, 0, wsum);
-    if (threadIdx.x == 0) {
-        d.cnt->ncolors = ncol;
-        d.cnt->nordered = d.color_start[ncol];
-    }
-}
-
 
 // Sense-reversing barrier over all workgroups of a cooperative launch (every workgroup is
 // resident, so every wait ends).  The last arrival resets the count and bumps the generation.
@@ -379,67 +431,33 @@ __device__ __forceinline__ void grid_barrier(uint32_t* count, uint32_t* gen, uin
     __syncthreads();
 }
 
-// Constraint-graph colouring by rounds (Jones-Plassmann), the same colour classes as colour_pairs:
+// Constraint-graph colouring over the whole GPU (Jones-Plassmann), the same colour classes as colour_pairs:
 // colour_pairs builds each colour as the independent set its priority claims settle on, which is the
 // greedy independent set in priority order of the pairs left (the candidate of lowest priority always
 // holds its claims, and a pair joins exactly when no lower-priority neighbour joined); repeating that
 // colour after colour gives each pair the first colour no lower-priority neighbour (a pair sharing a
 // dynamic body) holds.  Here a pair takes that colour as soon as all its lower-priority neighbours
-// have theirs, in rounds over the whole GPU, and the colours read are final when seen, so the result
-// does not depend on timing.
-__global__ void k_jp_init(Dev d) {
-    const int n = d.b.n;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i <= n; i += gridDim.x * blockDim.x) {
-        d.jp_deg[i] = 0;
-        if (i < n) d.jp_fill[i] = 0;
-    }
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c <= d.pcap; c += gridDim.x * blockDim.x) d.jp_ccount[c] = 0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        d.cnt->nact = 0;
-        d.cnt->ncolors = 0;
-        d.cnt->jp_rem[0] = 0;
-        d.cnt->jp_rem[1] = 0;
-        d.cnt->jp_rem[2] = 0;
-    }
-}
-// The pairs to colour (contact points, not both bodies kinematic) and their dynamic bodies' degrees.
-__global__ void k_jp_active(Dev d) {
-    const int np = d.cnt->npairs;
-    const int n_iter = (np + (int)(gridDim.x * blockDim.x) - 1) / (int)(gridDim.x * blockDim.x);
-    for (int it = 0; it < n_iter; it++) {
-        const int p = (it * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
-        bool act = false;
-        int a = 0, c = 0;
-        bool ka = true, kc = true;
-        if (p < np && d.ps.npts[p] > 0) {
-            a = d.ps.pa[p];
-            c = d.ps.pb[p];
-            ka = d.b.iat(I_KIN, a) != 0;
-            kc = d.b.iat(I_KIN, c) != 0;
-            act = !(ka && kc);
-        }
-        const int slot = wave_append(act, &d.cnt->nact);
-        if (act) {
-            d.act[slot] = p;
-            d.jp_col[p] = -1;
-            if (!ka) atomicAdd(&d.jp_deg[a], 1u);
-            if (!kc) atomicAdd(&d.jp_deg[c], 1u);
-        }
-    }
-}
+// have theirs, and the colours read are final when seen, so the result does not depend on timing.
 __global__ void k_jp_fill(Dev d) {
     const int nact = d.cnt->nact;
     for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nact; k += gridDim.x * blockDim.x) {
         const int p = d.act[k];
         const int a = d.ps.pa[p], c = d.ps.pb[p];
         const int2 e = make_int2(p, colour::prio(p, d.ps.npts[p]));
-        if (!d.b.iat(I_KIN, a)) d.jp_adj[d.jp_deg[a] + atomicAdd(&d.jp_fill[a], 1)] = e;
-        if (!d.b.iat(I_KIN, c)) d.jp_adj[d.jp_deg[c] + atomicAdd(&d.jp_fill[c], 1)] = e;
+        if (!d.b.iat(I_KIN, a)) d.jp_adj[d.jp_off[a] + atomicAdd(&d.jp_fill[a], 1)] = e;
+        if (!d.b.iat(I_KIN, c)) d.jp_adj[d.jp_off[c] + atomicAdd(&d.jp_fill[c], 1)] = e;
     }
 }
-constexpr int JP_THREADS = 256;
 __device__ __forceinline__ int jp_col_load(const int32_t* col, int q) {
     return __hip_atomic_load(&col[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The first colour not in used: a pair has at most 2 (JP_MAX_DEG - 1) neighbours, so one below 128 is free.
+__device__ __forceinline__ int jp_first(const uint64_t (&used)[2]) {
+    return ~used[0] != 0ull ? __ffsll((unsigned long long)~used[0]) - 1 : 63 + __ffsll((unsigned long long)~used[1]);
+}
+__device__ __forceinline__ void jp_use(uint64_t (&used)[2], int c) {
+    if (c >= 0 && c < 64) used[0] |= 1ull << c;
+    else if (c >= 64) used[1] |= 1ull << (c & 63);
 }
 // Pair p's first-fit colour if every lower-priority neighbour is coloured, else -1.  The adjacency
 // entries and their colours are loaded eight at a time (independent loads in flight together: a
@@ -448,12 +466,11 @@ constexpr int JP_BATCH = 8;
 __device__ int jp_try(const Dev& d, int p) {
     const int pr = colour::prio(p, d.ps.npts[p]);
     const int body[2] = {d.ps.pa[p], d.ps.pb[p]};
-    uint64_t used = 0;
-    bool big = false;
+    uint64_t used[2] = {0, 0};
     for (int s = 0; s < 2; s++) {
         const int x = body[s];
         if (d.b.iat(I_KIN, x)) continue;
-        const int k0 = (int)d.jp_deg[x], k1 = (int)d.jp_deg[x + 1];
+        const int k0 = d.jp_off[x], k1 = k0 + d.jp_deg[x];
         for (int k = k0; k < k1; k += JP_BATCH) {
             int2 q[JP_BATCH];
             int cq[JP_BATCH];
@@ -468,176 +485,501 @@ __device__ int jp_try(const Dev& d, int p) {
 #pragma unroll
             for (int j = 0; j < JP_BATCH; j++) {
                 wait |= cq[j] == -1;
-                if (cq[j] >= 64) big = true;
-                else if (cq[j] >= 0) used |= 1ull << cq[j];
+                jp_use(used, cq[j]);
             }
             if (wait) return -1;
         }
     }
-    if (~used != 0ull) return __ffsll((unsigned long long)~used) - 1;
-    // 64 colours and more around this pair: the first colour no lower neighbour holds
-    (void)big;
-    for (int c = 64;; c++) {
-        bool taken = false;
-        for (int s = 0; s < 2 && !taken; s++) {
-            const int x = body[s];
-            if (d.b.iat(I_KIN, x)) continue;
-            for (int k = (int)d.jp_deg[x]; k < (int)d.jp_deg[x + 1] && !taken; k++) {
-                const int2 q = d.jp_adj[k];
-                if (q.x != p && q.y < pr && jp_col_load(d.jp_col, q.x) == c) taken = true;
+    return jp_first(used);
+}
+// The lower-priority neighbours of pair p to list[JP_KEEP]; their number, or -1 if they are more.
+constexpr int JP_KEEP = 32;
+__device__ int jp_lower(const Dev& d, int p, int* list) {
+    const int pr = colour::prio(p, d.ps.npts[p]);
+    const int body[2] = {d.ps.pa[p], d.ps.pb[p]};
+    int m = 0;
+    for (int s = 0; s < 2; s++) {
+        const int x = body[s];
+        if (d.b.iat(I_KIN, x)) continue;
+        const int k0 = d.jp_off[x], k1 = k0 + d.jp_deg[x];
+        for (int k = k0; k < k1; k += JP_BATCH) {
+            int2 q[JP_BATCH];
+#pragma unroll
+            for (int j = 0; j < JP_BATCH; j++) q[j] = k + j < k1 ? d.jp_adj[k + j] : make_int2(p, pr);
+#pragma unroll
+            for (int j = 0; j < JP_BATCH; j++) {
+                if (q[j].x == p || q[j].y >= pr) continue;
+                if (m == JP_KEEP) return -1;
+                list[m++] = q[j].x;
             }
         }
-        if (!taken) return c;
+    }
+    return m;
+}
+// Drops the coloured pairs of list[n] and enters their colours; the number left.
+__device__ __forceinline__ int jp_poll(const Dev& d, int* list, int n, uint64_t (&used)[2]) {
+    int m = 0;
+    for (int k = 0; k < n; k += JP_BATCH) {
+        int q[JP_BATCH], cq[JP_BATCH];
+#pragma unroll
+        for (int j = 0; j < JP_BATCH; j++) q[j] = k + j < n ? list[k + j] : -1;
+#pragma unroll
+        for (int j = 0; j < JP_BATCH; j++) cq[j] = q[j] >= 0 ? jp_col_load(d.jp_col, q[j]) : 0;
+#pragma unroll
+        for (int j = 0; j < JP_BATCH; j++) {
+            if (q[j] < 0) continue;
+            if (cq[j] < 0) list[m++] = q[j];   // at or before the entry read
+            else jp_use(used, cq[j]);
+        }
+    }
+    return m;
+}
+// Pairs of body x (not p) in a colour before c: p's place in x's sequence of updates.
+__device__ __forceinline__ int jp_rank(const Dev& d, int x, int p, int c) {
+    const int k0 = d.jp_off[x], k1 = k0 + d.jp_deg[x];
+    int r = 0;
+    for (int k = k0; k < k1; k += JP_BATCH) {
+        int q[JP_BATCH];
+#pragma unroll
+        for (int j = 0; j < JP_BATCH; j++) q[j] = k + j < k1 ? d.jp_adj[k + j].x : p;
+#pragma unroll
+        for (int j = 0; j < JP_BATCH; j++) r += q[j] != p && jp_col_load(d.jp_col, q[j]) < c;
+    }
+    return r;
+}
+
+// Colouring and Gauss-Seidel sweeps (SequentialImpulseSolver::solve, sequential_impulse_solver.cpp:60-81)
+// over the whole GPU in one cooperative launch (every workgroup resident, so every wait ends).
+//
+// The sweeps run as a data flow instead of colour by colour between grid barriers.  The colour order fixes
+// for every body the sequence of the pairs (then joints) that update it in an iteration, so a pair only
+// has to wait until its two bodies have had the updates before its own: each word of a body's temp
+// velocities carries the number of updates made (d.vel), a pair polls its bodies' words until they show
+// the number it expects, solves its rows and writes the words back with that number plus one.  The one pair
+// that expects a number is the only reader of that version and the next writer, so nothing else orders the
+// threads, and the words are relaxed device-scope atomics without fences.  Every body sees the updates
+// of the colour-by-colour sweep in the same order: the same bits.
+// What bounds it is the chain of dependent updates: iterations x colours x (the rows of a pair, 0.27 us each,
+// + about 0.9 us until the next pair of the body has seen the words: a store becomes visible to a polling
+// load in 0.5 to 0.67 us, on the same XCD or another).  Colour by colour, each pass also paid a grid
+// barrier (2 us at 32 workgroups, 4 to 7 at 256: atomics on one word) and waited for the slowest pair of the
+// colour.  10 000 boxes at rest (13 colours, 17 000 pairs, 36 000 points, 10 iterations): colouring 305 ->
+// 75 us, sweeps 850 -> 260 us.
+//
+// A wave works on items of 16 pairs of one colour, a quad of lanes per pair (quad_solve_row), or on 16
+// joints; it takes its items (wave, wave + waves, ...) in the order of iterations and colours.  The first
+// unfinished item in that order is therefore always at the head of its wave with everything it waits for
+// finished.  With an item per wave or less the rows stay in registers throughout.
+constexpr int FLOW_THREADS = 512;
+constexpr int FLOW_COLORS = 1024;       // colours whose starts every workgroup keeps in LDS
+constexpr int FLOW_BINS = 64;           // colours whose pairs every workgroup counts in LDS
+constexpr int FLOW_PAIRS = WAVE / 4;    // pairs per item
+constexpr int FLOW_JOINTS = 16;         // joints per wave at a time
+constexpr int FLOW_SPINS = 1 << 21;     // polls after which a wait is given up (seconds: a fault of this program)
+
+__device__ __forceinline__ uint64_t vel_load(const uint64_t* w) {
+    return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void vel_store(uint64_t* w, float v, uint32_t seq) {
+    __hip_atomic_store(w, vel_word(v, seq), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Pause between two polls of a wave that is not ready: by how many updates the farthest of its pairs still
+// waits for (polls of waves whose turn is far off only load the fabric: with short pauses throughout the
+// sweeps of 10 000 boxes at rest took 283 us, with these 260).
+__device__ __forceinline__ void flow_pause(bool waits, uint32_t dist) {
+    if (!__any(waits && dist > 1)) __builtin_amdgcn_s_sleep(1);
+    else if (!__any(waits && dist > 4)) __builtin_amdgcn_s_sleep(24);
+    else __builtin_amdgcn_s_sleep(100);
+}
+// A quad's pair.  wa, wb: the lane's words of the bodies' linear velocities (the angular ones 4 on).
+struct FlowPair {
+    int n, ia, ib;
+    int4 seq;
+    float* rows;
+    uint64_t *wa, *wb;
+    QuadBody A, B;
+};
+// Place q of the solve order (an empty pair beyond the colour's end).
+__device__ __forceinline__ void flow_load(const Dev& d, int q, bool valid, int c, FlowPair& f) {
+    int4 pr = make_int4(0, 1 << 31, 1 << 31, 0);
+    f.seq = make_int4(0, 0, 0, 0);
+    if (valid) {
+        pr = d.q_pair[q];
+        f.seq = d.q_seq[q];
+    }
+    f.n = pr.w;
+    f.ia = pr.y & 0x7fffffff;
+    f.ib = pr.z & 0x7fffffff;
+    f.rows = d.ps.rows + (size_t)pr.x * 8 * RW;
+    f.wa = d.vel + (size_t)f.ia * VELW + c;
+    f.wb = d.vel + (size_t)f.ib * VELW + c;
+    quad_load_body(d.b.sbr(f.ia), c, pr.y < 0, f.A);
+    quad_load_body(d.b.sbr(f.ib), c, pr.z < 0, f.B);
+}
+__device__ __forceinline__ void flow_rows(const FlowPair& f, int k0, int c, QuadRow (&r)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+        if (k0 + u < f.n) quad_load_row(f.rows + (size_t)(k0 + u) * RW, c, r[u]);
+}
+__device__ __forceinline__ void flow_store_acc(const FlowPair& f, int k0, int c, const QuadRow (&r)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+        if (k0 + u < f.n) f.rows[(size_t)(k0 + u) * RW + R_LN + c] = r[u].acc;
+}
+// Polls the lane's words of a body that is to have had e updates: whether it has, its velocity words into
+// q, and how many updates are missing.
+__device__ __forceinline__ void flow_take(QuadBody& q, uint64_t v, uint64_t w, uint32_t e, bool& ready, uint32_t& dist) {
+    const uint32_t s0 = (uint32_t)(v >> 32), s1 = (uint32_t)(w >> 32);
+    ready = s0 == e && s1 == e;
+    dist = max(dist, e - s0);
+    q.tv = __uint_as_float((uint32_t)v);
+    q.tw = __uint_as_float((uint32_t)w);
+}
+// Solves the pair's rows from r (its first four) and the row store (the rest, their impulses put back),
+// then hands the bodies on.  last_a (last_b): the update after which A (B) is solved, its velocities
+// then going to the body store (syncTempVelocity, sequential_impulse_solver.cpp:71-80).
+__device__ __forceinline__ void flow_solve(const Dev& d, FlowPair& f, int c, bool first, bool own, QuadRow (&r)[4], uint32_t ea,
+                                           uint32_t eb, uint32_t last_a, uint32_t last_b) {
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+        if (u < f.n) quad_solve_row(r[u], first, f.A, f.B);
+    for (int k = 4; k < f.n; k++) {
+        QuadRow x;
+        quad_load_row(f.rows + (size_t)k * RW, c, x);
+        quad_solve_row(x, first, f.A, f.B);
+        if (own) f.rows[(size_t)k * RW + R_LN + c] = x.acc;
+    }
+    auto hand_on = [&](const QuadBody& q, int i, uint64_t* w, uint32_t e, uint32_t last) {
+        if (q.kin) return;
+        vel_store(w, q.tv, e + 1);
+        vel_store(w + 4, q.tw, e + 1);
+        if (e + 1 == last) {
+            d.b.at(F_V + c, i) = q.tv;
+            d.b.at(F_W + c, i) = q.tw;
+            float* sb = d.b.sbr(i);
+            sb[SB_TV + c] = q.tv;
+            sb[SB_TW + c] = q.tw;
+        }
+    };
+    if (own) {
+        hand_on(f.A, f.ia, f.wa, ea, last_a);
+        hand_on(f.B, f.ib, f.wb, eb, last_b);
     }
 }
-// Rounds until every pair has its colour (each round colours at least the uncoloured pair of lowest
-// priority, so the loop ends), then the colour starts and the solve order, colour by colour.  First-fit
-// colours are dense (a pair of colour c has lower neighbours of every colour below c), so the colour
-// count is the first empty bin.  The colour counts go through LDS histograms, one global add per
-// workgroup and bin.  Launched cooperatively (all workgroups resident).
-constexpr int JP_BINS = 64;
-__global__ void __launch_bounds__(JP_THREADS) k_jp_colour(Dev d) {
-    __shared__ int s_any;
-    __shared__ int s_hist[JP_BINS], s_base[JP_BINS];
-    const int nact = d.cnt->nact;
-    const int gtid = blockIdx.x * blockDim.x + threadIdx.x, gsz = gridDim.x * blockDim.x;
-    // Round 0 takes every active pair, each later round the pairs the round before left uncoloured
-    // (lists alternating in act + pcap and act + 2 pcap; the count of round r's list in
-    // jp_rem[r % 3], cleared two rounds ahead, after every thread has read it).  Once at most
-    // JP_THREADS pairs are left, workgroup 0 finishes them alone, with workgroup barriers.
-    const int32_t* cur = d.act;
-    int ncur = nact;
-    int r = 0;
-    for (;; r++) {
-        int32_t* nxt = d.act + (size_t)(1 + (r & 1)) * d.pcap;
-        if (gtid == 0) d.cnt->jp_rem[(r + 2) % 3] = 0;
-        const int n_iter = (ncur + gsz - 1) / gsz;
-        for (int it = 0; it < n_iter; it++) {
-            const int k = it * gsz + gtid;
-            int p = -1, c = 0;
-            if (k < ncur) {
-                p = cur[k];
-                c = jp_try(d, p);
-                if (c >= 0) __hip_atomic_store(&d.jp_col[p], c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// The joints of lanes j0, j0 + nl, ... of jorder, over all iterations, a joint per lane at a time: each waits for
+// its bodies' contacts and earlier joints of the iteration.  False if given up.
+__device__ __forceinline__ bool flow_joints(const Dev& d, int j0, int nl) {
+    int at = j0, it = 0;
+    bool live = at < d.njoints && d.iterations > 0, fresh = true;
+    JointDef j{};
+    SolvBody S[2];
+    int body[2] = {0, 0}, k = 0;
+    uint32_t e[2] = {0, 0}, last[2] = {0, 0};
+    bool ready[2] = {false, false};
+    for (int spin = 0; __any(live); spin++) {
+        if (spin == FLOW_SPINS) return false;
+        if (live && fresh) {
+            fresh = false;
+            k = d.jorder[at];
+            j = d.joints[k];
+            const int2 seq = d.jseq[k];
+            body[0] = j.a;
+            body[1] = j.b;
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                S[s] = load_solv(d.b, body[s]);
+                S[s].tv = S[s].tw = f3{0.0f, 0.0f, 0.0f};   // a kinematic body's stay so
+                ready[s] = S[s].kin;
+                const int deg = d.jp_deg[body[s]], tot = deg + d.jdeg[body[s]];
+                e[s] = (uint32_t)(it * tot + deg + (s == 0 ? seq.x : seq.y));
+                last[s] = (uint32_t)(d.iterations * tot);
             }
-            const int slot = wave_append(p >= 0 && c < 0, (int*)&d.cnt->jp_rem[(r + 1) % 3]);
-            if (p >= 0 && c < 0) nxt[slot] = p;
         }
-        grid_barrier(&d.cnt->bar_count, &d.cnt->bar_gen, gridDim.x);
-        ncur = (int)__hip_atomic_load(&d.cnt->jp_rem[(r + 1) % 3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        cur = nxt;
-        if (ncur <= JP_THREADS) break;
+        uint32_t dist = 0;
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            if (!live || ready[s]) continue;
+            const uint64_t* w = d.vel + (size_t)body[s] * VELW;
+            uint64_t x[6];
+#pragma unroll
+            for (int m = 0; m < 6; m++) x[m] = vel_load(w + (m < 3 ? m : m + 1));
+            bool ok = true;
+#pragma unroll
+            for (int m = 0; m < 6; m++) ok = ok && (uint32_t)(x[m] >> 32) == e[s];
+            dist = max(dist, e[s] - (uint32_t)(x[0] >> 32));
+            ready[s] = ok;
+            auto val = [&](int m) { return __uint_as_float((uint32_t)x[m]); };
+            S[s].tv = f3{val(0), val(1), val(2)};
+            S[s].tw = f3{val(3), val(4), val(5)};
+        }
+        const bool go = live && ready[0] && ready[1];
+        if (go) {
+            joint_solve(j, d.jrows[k], S[0], S[1]);
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                if (S[s].kin) continue;
+                uint64_t* w = d.vel + (size_t)body[s] * VELW;
+                const float v[6] = {S[s].tv.x, S[s].tv.y, S[s].tv.z, S[s].tw.x, S[s].tw.y, S[s].tw.z};
+#pragma unroll
+                for (int m = 0; m < 6; m++) vel_store(w + (m < 3 ? m : m + 1), v[m], e[s] + 1);
+                if (e[s] + 1 == last[s]) {
+                    float* sb = d.b.sbr(body[s]);
+#pragma unroll
+                    for (int m = 0; m < 6; m++) {
+                        d.b.at((m < 3 ? F_V : F_W - 3) + m, body[s]) = v[m];
+                        sb[SB_TV + m] = v[m];   // SB_TW follows SB_TV
+                    }
+                }
+            }
+            fresh = true;
+            at += nl;
+            if (at >= d.njoints) {
+                at = j0;
+                live = ++it < d.iterations;
+            }
+        }
+        if (__any(go)) spin = 0;
+        else flow_pause(live, dist);
     }
-    r++;
-    if (blockIdx.x == 0) {
-        const int p = (int)threadIdx.x < ncur ? cur[threadIdx.x] : -1;
-        bool done = p < 0;
-        for (;; r++) {
-            if (threadIdx.x == 0) s_any = 0;
-            __syncthreads();
-            if (!done) {
-                const int c = jp_try(d, p);
+    return true;
+}
+
+// claims: the colouring runs in workgroup 0 (colour_pairs), as it does where a body is in more than
+// JP_MAX_DEG pairs.
+__global__ void __launch_bounds__(FLOW_THREADS) k_solve_flow(Dev d, int claims) {
+    __shared__ int s_cs[FLOW_COLORS + 1], s_is[FLOW_COLORS + 1], s_ncol;
+    __shared__ int s_hist[FLOW_BINS];
+    __shared__ int s_low[FLOW_THREADS][JP_KEEP + 1];   // rows of odd length: distinct banks
+    const int nact = d.cnt->nact;
+    const int tid = threadIdx.x, gtid = blockIdx.x * blockDim.x + tid, gsz = gridDim.x * blockDim.x;
+    if (tid < FLOW_BINS) s_hist[tid] = 0;
+    auto stalled = [&]() { atomicOr(&d.cnt->overflow, OVF_STALL); };
+    const bool coloured = claims || d.cnt->jp_big;   // the same for every workgroup
+    if (!coloured) {
+        // Every thread tries its pairs until all have their colours: the uncoloured pair of lowest priority
+        // gets its colour whenever it is tried, so the loops end.  With a pair per thread or less, a thread
+        // scans its bodies' lists once and keeps the lower-priority neighbours in LDS; a try then reads only
+        // the colours still missing, in flight together.
+        int tries = 0;
+        bool left = true;
+        if (nact <= gsz) {
+            const int p = gtid < nact ? d.act[gtid] : -1;
+            int* mine = s_low[tid];
+            int nlow = p >= 0 ? jp_lower(d, p, mine) : 0;   // neighbours whose colours are missing (-1: too many to keep)
+            uint64_t used[2] = {0, 0};   // colours the others hold
+            left = p >= 0;
+            for (; __any(left) && tries < FLOW_SPINS; tries++) {
+                if (!left) continue;
+                int c = -1;
+                if (nlow < 0) {
+                    c = jp_try(d, p);
+                } else {
+                    nlow = jp_poll(d, mine, nlow, used);
+                    if (nlow == 0) c = jp_first(used);
+                }
                 if (c >= 0) {
                     __hip_atomic_store(&d.jp_col[p], c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    done = true;
-                } else {
-                    s_any = 1;
+                    left = false;
                 }
             }
-            __syncthreads();
-            if (!s_any) break;
+        } else {
+            for (; __any(left) && tries < FLOW_SPINS; tries++) {
+                left = false;
+                for (int k = gtid; k < nact; k += gsz) {
+                    const int p = d.act[k];
+                    if (jp_col_load(d.jp_col, p) >= 0) continue;
+                    const int c = jp_try(d, p);
+                    if (c >= 0) __hip_atomic_store(&d.jp_col[p], c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    else left = true;
+                }
+            }
         }
-        if (threadIdx.x == 0) d.cnt->jp_rounds = ncur > 0 ? r + 1 : r;
-    }
-    grid_barrier(&d.cnt->bar_count, &d.cnt->bar_gen, gridDim.x);   // every colour is set
-    // pairs per colour: LDS bins per workgroup, one global add per workgroup and bin
-    for (int c = threadIdx.x; c < JP_BINS; c += blockDim.x) s_hist[c] = 0;
-    __syncthreads();
-    for (int k = gtid; k < nact; k += gsz) {
-        const int c = d.jp_col[d.act[k]];
-        if (c < JP_BINS) atomicAdd(&s_hist[c], 1);
-        else atomicAdd(&d.jp_ccount[c], 1);
-    }
-    __syncthreads();
-    for (int c = threadIdx.x; c < JP_BINS; c += blockDim.x)
-        if (s_hist[c]) atomicAdd(&d.jp_ccount[c], s_hist[c]);
-    grid_barrier(&d.cnt->bar_count, &d.cnt->bar_gen, gridDim.x);
-    if (gtid == 0) {
-        int run = 0, ncol = 0;
-        while (ncol <= d.pcap && d.jp_ccount[ncol] > 0) {
-            d.color_start[ncol] = run;
-            run += d.jp_ccount[ncol];
-            d.jp_ccount[ncol] = 0;
-            ncol++;
+        if (__any(left)) stalled();
+        if ((tid & (WAVE - 1)) == 0) atomicMax(&d.cnt->jp_rounds, tries);
+        // the pairs' places in their colours: among the workgroup's for the first colours, counted in LDS
+        // (an atomic on each colour's one counter serialises over the whole GPU)
+        __syncthreads();
+        for (int k = gtid; k < nact; k += gsz) {
+            const int p = d.act[k];
+            const int c = jp_col_load(d.jp_col, p);
+            if (c >= 0) d.jp_idx[p] = c < FLOW_BINS ? atomicAdd(&s_hist[c], 1) : atomicAdd(&d.jp_ccount[c], 1);
         }
-        d.color_start[ncol] = run;
-        d.cnt->ncolors = ncol;
-        d.cnt->nordered = run;
+        __syncthreads();
+        if (tid < FLOW_BINS) d.jp_hist[tid * gridDim.x + blockIdx.x] = s_hist[tid];
+    } else {
+        if (blockIdx.x == 0) {
+            __shared__ int wsum[FLOW_THREADS / WAVE + 1];
+            for (int i = tid; i < d.b.n; i += FLOW_THREADS) claim_set<false>(d.claim, i, colour::FREE);
+            claim_sync<false>();
+            int* bufs[3] = {d.act, d.act + d.pcap, d.act + 2 * (size_t)d.pcap};
+            const int nc = colour_pairs<false>(d.b, d.ps, bufs, nact, d.order, d.color_start, d.claim, 0, 0, wsum);
+            if (tid == 0) {
+                d.cnt->ncolors = nc;
+                d.cnt->nordered = d.color_start[nc];
+            }
+        }
+        grid_barrier(&d.cnt->bar_count, &d.cnt->bar_gen, gridDim.x);
+        const int ncol = d.cnt->ncolors, nord = d.cnt->nordered;
+        for (int q = gtid; q < nord; q += gsz) {
+            int lo = 0, hi = ncol;   // last colour starting at or before q
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (d.color_start[mid] <= q) lo = mid; else hi = mid;
+            }
+            const int p = d.order[q];
+            d.jp_col[p] = lo;
+            d.jp_idx[p] = q - d.color_start[lo];
+            if (q == d.color_start[lo]) d.jp_ccount[lo] = d.color_start[lo + 1] - q;
+        }
     }
-    grid_barrier(&d.cnt->bar_count, &d.cnt->bar_gen, gridDim.x);
-    // the solve order: each workgroup reserves its range of every colour once, then places its pairs
-    for (int c = threadIdx.x; c < JP_BINS; c += blockDim.x) {
-        s_base[c] = s_hist[c] ? atomicAdd(&d.jp_ccount[c], s_hist[c]) : 0;
-        s_hist[c] = 0;
+    grid_barrier(&d.cnt->bar_count, &d.cnt->bar_gen, gridDim.x);   // every colour is set and counted
+    // each colour's pairs, and for the colours counted per workgroup those of the workgroups before this one
+    if (!coloured) {
+        if (tid < FLOW_BINS) s_cs[tid] = 0;
+        __syncthreads();
+        for (int c = tid / WAVE; c < FLOW_BINS; c += FLOW_THREADS / WAVE) {
+            int all = 0, before = 0;
+            for (int g = tid & (WAVE - 1); g < (int)gridDim.x; g += WAVE) {
+                const int m = d.jp_hist[c * gridDim.x + g];
+                all += m;
+                before += g < (int)blockIdx.x ? m : 0;
+            }
+            for (int o = WAVE / 2; o > 0; o >>= 1) {
+                all += __shfl_xor(all, o, WAVE);
+                before += __shfl_xor(before, o, WAVE);
+            }
+            s_cs[c] = all;
+            s_hist[c] = before;
+            if (all == 0) break;   // the colours end at the first empty one at the latest
+        }
+    }
+    // Colour starts in the solve order and in the items.  First-fit colours are dense (a pair of colour c
+    // has lower neighbours of every colour below c), so the colours end at the first empty one.
+    for (int c = tid + (coloured ? 0 : FLOW_BINS); c < FLOW_COLORS; c += FLOW_THREADS) s_cs[c] = c <= d.pcap ? d.jp_ccount[c] : 0;
+    __syncthreads();
+    if (tid == 0) {
+        int run = 0, items = 0, c = 0;
+        for (; c < FLOW_COLORS && s_cs[c] > 0; c++) {
+            const int m = s_cs[c];
+            s_cs[c] = run;
+            s_is[c] = items;
+            run += m;
+            items += (m + FLOW_PAIRS - 1) / FLOW_PAIRS;
+        }
+        s_cs[c] = run;
+        s_is[c] = items;
+        s_ncol = c;
     }
     __syncthreads();
+    int ncol = s_ncol;
+    if (ncol == FLOW_COLORS) {   // the same for every workgroup: the starts beyond, through memory
+        if (gtid == 0) {
+            int run = s_cs[ncol], items = s_is[ncol], c = ncol;
+            for (; c <= d.pcap && d.jp_ccount[c] > 0; c++) {
+                const int m = d.jp_ccount[c];
+                d.color_start[c] = run;
+                d.jp_items[c] = items;
+                run += m;
+                items += (m + FLOW_PAIRS - 1) / FLOW_PAIRS;
+            }
+            d.color_start[c] = run;
+            d.jp_items[c] = items;
+            d.cnt->jp_ncol = c;
+        }
+        grid_barrier(&d.cnt->bar_count, &d.cnt->bar_gen, gridDim.x);
+        ncol = d.cnt->jp_ncol;
+    }
+    auto cs = [&](int c) { return c <= FLOW_COLORS ? s_cs[c] : d.color_start[c]; };
+    auto is = [&](int c) { return c <= FLOW_COLORS ? s_is[c] : d.jp_items[c]; };
+    if (blockIdx.x == 0) {
+        for (int c = tid; c <= ncol; c += FLOW_THREADS)
+            if (c <= FLOW_COLORS) d.color_start[c] = s_cs[c];
+        if (tid == 0) {
+            d.cnt->ncolors = ncol;
+            d.cnt->jp_ncol = ncol;
+            d.cnt->nordered = cs(ncol);
+        }
+    }
+    // the solve order, and each pair's place in its bodies' sequences of updates
+    const int32_t* list = coloured ? d.order : d.act;   // (the claims' lists are built in d.act)
     for (int k = gtid; k < nact; k += gsz) {
-        const int p = d.act[k];
+        const int p = list[k];
         const int c = d.jp_col[p];
-        const int at = c < JP_BINS ? s_base[c] + atomicAdd(&s_hist[c], 1) : atomicAdd(&d.jp_ccount[c], 1);
-        d.order[d.color_start[c] + at] = p;
+        if (c < 0) continue;   // only after a wait given up
+        const int q = cs(c) + d.jp_idx[p] + (!coloured && c < FLOW_BINS ? s_hist[c] : 0);
+        const int a = d.ps.pa[p], b = d.ps.pb[p];
+        const bool ka = d.b.iat(I_KIN, a) != 0, kb = d.b.iat(I_KIN, b) != 0;
+        d.order[q] = p;
+        d.q_pair[q] = make_int4(p, ka ? a | 1 << 31 : a, kb ? b | 1 << 31 : b, d.ps.npts[p]);
+        d.q_seq[q] = make_int4(ka ? 0 : jp_rank(d, a, p, c), ka ? 0 : d.jp_deg[a] + (d.jdeg ? d.jdeg[a] : 0),
+                               kb ? 0 : jp_rank(d, b, p, c), kb ? 0 : d.jp_deg[b] + (d.jdeg ? d.jdeg[b] : 0));
     }
-}
+    grid_barrier(&d.cnt->bar_count, &d.cnt->bar_gen, gridDim.x);   // the order is complete
 
-// Gauss-Seidel sweeps (SequentialImpulseSolver::solve, sequential_impulse_solver.cpp:60-81) in
-// colour order across the whole GPU: the pairs of one colour share no dynamic body, so they run
-// in parallel; a grid barrier separates colours.  Then syncTempVelocity.  Launched cooperatively
-// (all workgroups co-resident).
-constexpr int GS_THREADS = 256;
-
-__global__ void __launch_bounds__(GS_THREADS) k_gs_grid(Dev d) {
-    const int ncol = d.cnt->ncolors;
-    const int gtid = blockIdx.x * blockDim.x + threadIdx.x, gsz = gridDim.x * blockDim.x;
-    // A thread's first pair of each colour is loaded before the barrier ahead of it (gs_prefetch):
-    // only the bodies' temp velocities are read after the barrier.
-    GsPair G;
-    bool have = false;
-    auto fetch = [&](int c) {
-        const int q = d.color_start[c] + gtid;
-        have = q < d.color_start[c + 1];
-        if (have) gs_prefetch(d.b, d.ps, d.order[q], G);
-    };
-    if (ncol > 0) fetch(0);
-    // The last colours of at most GS_THREADS pairs each: every pair of such a colour falls to a thread
-    // of workgroup 0, so between two of them a workgroup barrier orders the updates (the grid barrier
-    // after the last one publishes them to the next iteration).
-    int ctail = ncol;
-    while (ctail > 0 && d.color_start[ctail] - d.color_start[ctail - 1] <= GS_THREADS) ctail--;
-    for (int it = 0; it < d.iterations; it++) {
-        for (int c = 0; c < ncol; c++) {
-            const int c0 = d.color_start[c], c1 = d.color_start[c + 1];
-            if (have) {
-                gs_solve(d.b, d.ps, G);
-                for (int q = c0 + gtid + gsz; q < c1; q += gsz) {
-                    gs_prefetch(d.b, d.ps, d.order[q], G);
-                    gs_solve(d.b, d.ps, G);
+    // consecutive items go to different workgroups, so a colour's pairs spread over the CUs; half of the
+    // waves take the joints, if there are any
+    const int wave = (tid / WAVE) * gridDim.x + blockIdx.x;
+    const int all_waves = gridDim.x * (FLOW_THREADS / WAVE), nwaves = d.njoints > 0 ? all_waves / 2 : all_waves;
+    const int lane = tid & (WAVE - 1);
+    if (wave >= nwaves) {
+        const int jw = wave - nwaves, nl = (all_waves - nwaves) * FLOW_JOINTS;
+        const int j0 = lane < FLOW_JOINTS ? jw * FLOW_JOINTS + lane : d.njoints;
+        if (!flow_joints(d, j0, nl)) stalled();
+        return;
+    }
+    const int quad = lane >> 2, c = (lane & 3) < 2 ? lane & 3 : 2;
+    const bool first = (lane & 3) == 0, own = (lane & 3) < 3;
+    const int nitems = is(ncol);
+    const bool resident = nitems <= nwaves;
+    // The wave goes through its places in the order: items wave, wave + nwaves, ... of every iteration, each
+    // solved once all its pairs are ready (solving the ready ones of a poll by themselves repeats the row
+    // chains, which cost as much as the wait: 380 us instead of 275 for 10 000 boxes at rest).
+    int item = wave, it = 0;
+    bool live = item < nitems && d.iterations > 0, fresh = true, ra = false, rb = false;
+    uint32_t ea = 0, eb = 0;
+    QuadRow r[4];
+    FlowPair f;
+    for (int spin = 0; __any(live); spin++) {
+        if (spin == FLOW_SPINS) { stalled(); return; }
+        if (live && fresh) {
+            if (it == 0 || !resident) {
+                int lo = 0, hi = ncol;   // last colour whose first item is at or before this one
+                while (hi - lo > 1) {
+                    const int mid = (lo + hi) >> 1;
+                    if (is(mid) <= item) lo = mid; else hi = mid;
                 }
+                const int q = cs(lo) + (item - is(lo)) * FLOW_PAIRS + quad;
+                flow_load(d, q, q < cs(lo + 1), c, f);
+                flow_rows(f, 0, c, r);
             }
-            if (c + 1 < ncol) fetch(c + 1);
-            else if (it + 1 < d.iterations) fetch(0);
-            if (c >= ctail && c + 1 < ncol) __syncthreads();
-            else grid_barrier(&d.cnt->bar_count, &d.cnt->bar_gen, gridDim.x);   // later colours read these velocities
+            fresh = false;
+            ra = f.A.kin;
+            rb = f.B.kin;
+            f.A.tv = f.A.tw = f.B.tv = f.B.tw = 0.0f;   // a kinematic body's stay so (rigidbody.cpp:72-80, 167)
+            ea = (uint32_t)(it * f.seq.y + f.seq.x);
+            eb = (uint32_t)(it * f.seq.w + f.seq.z);
         }
-        // the joints after the contacts, colour by colour (sequential_impulse_solver.cpp:66-68)
-        for (int c = 0; c < d.njcol; c++) {
-            for (int q = d.jcs[c] + gtid; q < d.jcs[c + 1]; q += gsz) {
-                const int k = d.jorder[q];
-                joint_iterate(d.b, d.joints[k], d.jrows[k]);
+        uint64_t a0 = 0, a1 = 0, b0 = 0, b1 = 0;
+        const bool pa = live && !ra, pb = live && !rb;
+        if (pa) { a0 = vel_load(f.wa); a1 = vel_load(f.wa + 4); }
+        if (pb) { b0 = vel_load(f.wb); b1 = vel_load(f.wb + 4); }
+        uint32_t dist = 0;
+        if (pa) flow_take(f.A, a0, a1, ea, ra, dist);
+        if (pb) flow_take(f.B, b0, b1, eb, rb, dist);
+        const bool go = !__any(live && !(ra && rb));
+        if (go) {
+            flow_solve(d, f, c, first, own, r, ea, eb, (uint32_t)(d.iterations * f.seq.y), (uint32_t)(d.iterations * f.seq.w));
+            fresh = true;
+            item += nwaves;
+            if (item >= nitems) {
+                item = wave;
+                live = ++it < d.iterations;
             }
-            grid_barrier(&d.cnt->bar_count, &d.cnt->bar_gen, gridDim.x);
+            if (own && (!resident || !live)) flow_store_acc(f, 0, c, r);
         }
+        if (go) spin = 0;
+        else flow_pause(!(ra && rb), dist);
     }
-    for (int i = gtid; i < d.b.n; i += gsz) sync_body(d.b, i);
 }
 
 // Contact points of this narrowphase: per-workgroup sums added to the counter k_narrow_finish
@@ -659,26 +1001,18 @@ __global__ void __launch_bounds__(256) k_count_points(Dev d) {
 }  // namespace
 
 // ====================================================================== host side
-// Workgroups of the cooperative Gauss-Seidel sweep: enough that a colour's pairs run about one
-// per thread, few enough that the grid barrier between colours stays cheap.  Measured at rest
-// (ms per step, 4 / 8 / 16 / 32 / 64 workgroups of 256): box rain of 1 000 bodies 0.45 / 0.47 / 0.49 /
-// 0.49, of 5 000 bodies 1.29 / 1.14 / 1.10 / 1.14, of 10 000 bodies (colouring rounds) - / 1.94 / 1.76 /
-// 1.72 / 1.82; 50k shape mix at step 280: 16 / 32 / 64 workgroups 7.29 / 7.06 / 7.08.
-static int default_gs_blocks(int n, int max_blocks) { return std::min(max_blocks, std::max(4, std::min(32, n / 300))); }
-// Bodies beyond which the colouring runs in rounds over the GPU rather than in one workgroup (box
-// rain at rest, ms per step with one workgroup / rounds: 1 000 bodies 0.42 / 0.46, 2 500 bodies
-// 0.67 / 0.69, 4 000 bodies 0.89 / 0.87, 6 000 bodies 1.26 / 1.14, 8 000 bodies 1.61 / 1.33).
-constexpr int COLOUR_ROUNDS_FROM = 3000;
+// Workgroups of the cooperative solve: enough waves for about an item each (a world at rest has up to
+// two pairs with contacts per body, 16 to an item), at most one workgroup per CU of the 256.
+static int default_flow_blocks(int n, int max_blocks) { return std::min(max_blocks, std::max(8, std::min(256, n / 80))); }
 
 struct pe_world {
     Dev d{};
     int n = 0, stride = 0;
     hipStream_t stream = nullptr;
     std::vector<void*> allocs;
-    int gs_blocks = 0;      // workgroups of the cooperative Gauss-Seidel kernel
-    int gs_max_blocks = 0;
-    int jp_blocks = 1;                       // workgroups of the cooperative colouring  // co-resident limit
-    int colouring = 0;                       // 0: by body count, 1: one workgroup's claims, 2: rounds
+    int flow_blocks = 0;    // workgroups of the cooperative solve
+    int flow_max_blocks = 0;                 // and the co-resident limit
+    int colouring = 0;                       // 0: by body count, 1: one workgroup's claims, 2: over the GPU
     bool timing = false;
     hipEvent_t ev[5] = {};
     hipEvent_t order_ev[2] = {};   // orders work on a caller's stream with the world's own stream
@@ -690,7 +1024,7 @@ struct pe_world {
     std::vector<uint64_t> ignore_keys;       // sorted ignore-pair keys
     std::vector<char> kinematic;             // per body (joint colouring)
     std::vector<char> finite_life, has_joint, removed;   // per body (joints and removals exclude each other)
-    void* joint_mem[4] = {};                 // device: definitions, rows, order, colour starts
+    void* joint_mem[6] = {};                 // device: definitions, rows, order, colour starts, sequence, degrees
     void* ignore_mem = nullptr;
     void* ray_mem = nullptr;                 // raycast inputs, ignore set and results
     size_t ray_bytes = 0;
@@ -739,22 +1073,14 @@ struct pe_world {
         return PE_OK;
     }
     int launch_solve() {
+        hipLaunchKernelGGL(k_solve_begin, dim3(grid(n, 256)), dim3(256), 0, stream, d);
         hipLaunchKernelGGL(k_setup, dim3(grid(d.pcap, 128)), dim3(128), 0, stream, d);
         if (d.njoints > 0) hipLaunchKernelGGL(k_joint_setup, dim3(grid(d.njoints, 64)), dim3(64), 0, stream, d);
-        if (colouring == 1 || (colouring == 0 && n <= COLOUR_ROUNDS_FROM)) {
-            // claims in one workgroup's LDS (at most CLAIM_LDS bodies)
-            hipLaunchKernelGGL(k_colour<true>, dim3(1), dim3(SOLVE_THREADS), n * sizeof(int), stream, d);
-        } else {
-            // colouring by rounds: the pairs and their bodies' adjacency, then the rounds (cooperative)
-            hipLaunchKernelGGL(k_jp_init, dim3(grid(std::max(n + 1, d.pcap + 1), 256)), dim3(256), 0, stream, d);
-            hipLaunchKernelGGL(k_jp_active, dim3(grid(d.pcap, 256)), dim3(256), 0, stream, d);
-            sap_scan(d.sap, d.jp_deg, n + 1, n + 1, nullptr, &d.cnt->adj_total, stream);
-            hipLaunchKernelGGL(k_jp_fill, dim3(grid(d.pcap, 256)), dim3(256), 0, stream, d);
-            void* jargs[] = {(void*)&d};
-            PE_HIP(hipLaunchCooperativeKernel((const void*)k_jp_colour, dim3(jp_blocks), dim3(JP_THREADS), jargs, 0, stream));
-        }
-        void* args[] = {(void*)&d};
-        PE_HIP(hipLaunchCooperativeKernel((const void*)k_gs_grid, dim3(gs_blocks), dim3(GS_THREADS), args, 0, stream));
+        hipLaunchKernelGGL(k_jp_alloc, dim3(grid(n, 256)), dim3(256), 0, stream, d);
+        hipLaunchKernelGGL(k_jp_fill, dim3(grid(d.pcap, 256)), dim3(256), 0, stream, d);
+        int claims = colouring == 1;
+        void* args[] = {(void*)&d, (void*)&claims};
+        PE_HIP(hipLaunchCooperativeKernel((const void*)k_solve_flow, dim3(flow_blocks), dim3(FLOW_THREADS), args, 0, stream));
         return PE_OK;
     }
     int step() {
@@ -794,10 +1120,11 @@ int report_overflow(pe_world* w, const DevCounts& c) {
     if (c.overflow & OVF_PAIRS) m += " more broadphase pairs than max_pairs (" + std::to_string(w->d.pcap) + ")";
     if (c.overflow & OVF_CHUNKS) m += " more sweep candidates than the sweep's chunk capacity";
     if (c.overflow & OVF_CLIP) m += " a clipped contact polygon outgrew its buffer";
+    if (c.overflow & OVF_STALL) m = "the solver gave up waiting for an update that never came";
     PE_HIP(hipMemsetAsync(&w->d.cnt->overflow, 0, sizeof(int32_t), w->stream));
     PE_HIP(hipStreamSynchronize(w->stream));
     pe_set_error(m);
-    return PE_ERR_CAPACITY;
+    return (c.overflow & OVF_STALL) ? PE_ERR_DEVICE : PE_ERR_CAPACITY;
 }
 }  // namespace
 
@@ -856,11 +1183,17 @@ int pe_world_create(const pe_scene_desc* sc, const pe_world_params* prm, int32_t
     rc |= w->alloc(&d.color_start, pcap + 1);
     rc |= w->alloc(&d.claim, n);
     rc |= w->alloc(&d.cnt, 1);
-    rc |= w->alloc(&d.jp_deg, (size_t)n + 1);
+    rc |= w->alloc(&d.jp_deg, n);
+    rc |= w->alloc(&d.jp_off, n);
     rc |= w->alloc(&d.jp_fill, n);
     rc |= w->alloc(&d.jp_adj, 2 * (size_t)pcap);
     rc |= w->alloc(&d.jp_col, pcap);
+    rc |= w->alloc(&d.jp_idx, pcap);
     rc |= w->alloc(&d.jp_ccount, (size_t)pcap + 1);
+    rc |= w->alloc(&d.jp_items, (size_t)pcap + 1);
+    rc |= w->alloc(&d.vel, (size_t)VELW * n);
+    rc |= w->alloc(&d.q_pair, pcap);
+    rc |= w->alloc(&d.q_seq, pcap);
     rc |= w->alloc(&d.st.flags, n);
     rc |= w->alloc(&d.st.sleep_time, n);
     rc |= w->alloc(&d.st.life, n);
@@ -944,22 +1277,13 @@ int pe_world_create(const pe_scene_desc* sc, const pe_world_params* prm, int32_t
     {
         int dev = 0, cus = 0, per_cu = 0;
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k_gs_grid, GS_THREADS, 0) != hipSuccess || per_cu < 1) {
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k_solve_flow, FLOW_THREADS, 0) != hipSuccess || per_cu < 1) {
             pe_set_error("cannot size the cooperative solver grid");
             return fail(PE_ERR_DEVICE);
         }
-        w->gs_max_blocks = cus * per_cu;
-        w->gs_blocks = default_gs_blocks(n, w->gs_max_blocks);
-        int jp_cu = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&jp_cu, (const void*)k_jp_colour, JP_THREADS, 0) != hipSuccess ||
-            jp_cu < 1) {
-            pe_set_error("cannot size the cooperative colouring grid");
-            return fail(PE_ERR_DEVICE);
-        }
-        // as many workgroups as the Gauss-Seidel sweep: each round ends in a grid barrier, and fewer,
-        // fuller workgroups measured faster (10k box rain at rest, ms per step with 16 / 32 / 64 / 128 /
-        // 256 workgroups: 1.22 / 1.19 / 1.20 / 1.22 / 1.31; 50k shape mix 5.90 / 5.84 / 5.86 / 5.91 / 5.98)
-        w->jp_blocks = std::max(1, std::min(cus * jp_cu, default_gs_blocks(n, cus * jp_cu)));
+        w->flow_max_blocks = cus * per_cu;
+        w->flow_blocks = default_flow_blocks(n, w->flow_max_blocks);
+        if (w->alloc(&d.jp_hist, (size_t)FLOW_BINS * w->flow_max_blocks) != PE_OK) return fail(PE_ERR_DEVICE);
     }
     if (hipStreamSynchronize(w->stream) != hipSuccess) { pe_set_error("init sync failed"); return fail(PE_ERR_DEVICE); }
     *out = w;
@@ -1012,17 +1336,25 @@ int pe_world_add_joints(pe_world* w, int32_t n, const pe_joint_desc* jd) {
         for (int x : {w->joints[k].a, w->joints[k].b})
             if (!w->kinematic[x]) body_cols[x].push_back(c);
     }
-    std::vector<int32_t> jorder, jcs;
+    std::vector<int32_t> jorder, jcs, jdeg(w->n, 0);
+    std::vector<int2> jseq(nj, make_int2(0, 0));   // a joint's place in the sequence of its bodies' joints
     for (int c = 0; c < ncol; c++) {
         jcs.push_back((int32_t)jorder.size());
-        for (int k = 0; k < nj; k++) if (col[k] == c) jorder.push_back(k);
+        for (int k = 0; k < nj; k++) {
+            if (col[k] != c) continue;
+            jorder.push_back(k);
+            const int a = w->joints[k].a, b = w->joints[k].b;
+            if (!w->kinematic[a]) jseq[k].x = jdeg[a]++;
+            if (!w->kinematic[b]) jseq[k].y = jdeg[b]++;
+        }
     }
     jcs.push_back((int32_t)jorder.size());
     PE_HIP(hipStreamSynchronize(w->stream));
     for (void*& p : w->joint_mem) if (p) { hipFree(p); p = nullptr; }
-    const size_t bytes[4] = {nj * sizeof(JointDef), nj * sizeof(JointRow), nj * sizeof(int32_t), jcs.size() * sizeof(int32_t)};
-    const void* src[4] = {w->joints.data(), nullptr, jorder.data(), jcs.data()};
-    for (int k = 0; k < 4; k++) {
+    const size_t bytes[6] = {nj * sizeof(JointDef), nj * sizeof(JointRow), nj * sizeof(int32_t), jcs.size() * sizeof(int32_t),
+                             nj * sizeof(int2), jdeg.size() * sizeof(int32_t)};
+    const void* src[6] = {w->joints.data(), nullptr, jorder.data(), jcs.data(), jseq.data(), jdeg.data()};
+    for (int k = 0; k < 6; k++) {
         PE_HIP(hipMalloc(&w->joint_mem[k], std::max<size_t>(bytes[k], 16)));
         if (src[k] && bytes[k]) PE_HIP(hipMemcpy(w->joint_mem[k], src[k], bytes[k], hipMemcpyHostToDevice));
     }
@@ -1030,6 +1362,8 @@ int pe_world_add_joints(pe_world* w, int32_t n, const pe_joint_desc* jd) {
     w->d.jrows = (JointRow*)w->joint_mem[1];
     w->d.jorder = (const int32_t*)w->joint_mem[2];
     w->d.jcs = (const int32_t*)w->joint_mem[3];
+    w->d.jseq = (const int2*)w->joint_mem[4];
+    w->d.jdeg = (const int32_t*)w->joint_mem[5];
     w->d.njoints = nj;
     w->d.njcol = ncol;
     return PE_OK;
@@ -1438,13 +1772,13 @@ int pe_world_get_stage_times(pe_world* w, double* ms) {
 int pe_world_set_solver_blocks(pe_world* w, int32_t blocks) {
     if (int rc = check_world(w)) return rc;
     if (blocks < 0) { pe_set_error("blocks must be >= 0"); return PE_ERR_INVALID; }
-    w->gs_blocks = blocks == 0 ? default_gs_blocks(w->n, w->gs_max_blocks) : std::min(blocks, w->gs_max_blocks);
+    w->flow_blocks = blocks == 0 ? default_flow_blocks(w->n, w->flow_max_blocks) : std::min(blocks, w->flow_max_blocks);
     return PE_OK;
 }
 
 int pe_world_set_colouring(pe_world* w, int32_t mode) {
     if (int rc = check_world(w)) return rc;
-    if (mode < 0 || mode > 2 || (mode == 1 && w->n > CLAIM_LDS)) {
+    if (mode < 0 || mode > 2 || (mode == 1 && w->n > CLAIM_MAX)) {
         pe_set_error("pe_world_set_colouring: mode 0, 1 (at most 12288 bodies) or 2");
         return PE_ERR_INVALID;
     }
@@ -1735,7 +2069,7 @@ int pe_stage_solve(pe_stage* s, int32_t n, const float* body, float* solver_body
     w->d.b.n = n;
     w->d.dt = dt;
     w->d.iterations = iterations;
-    w->gs_blocks = default_gs_blocks(n, w->gs_max_blocks);
+    w->flow_blocks = default_flow_blocks(n, w->flow_max_blocks);
     hipLaunchKernelGGL(k_stage_bodies, dim3(stage_grid(n, 256)), dim3(256), 0, w->stream, w->d, body, (int)n);
     hipLaunchKernelGGL(k_stage_solver_in, dim3(stage_grid(n, 256)), dim3(256), 0, w->stream, w->d, (const float*)solver_body, (int)n);
     hipLaunchKernelGGL(k_stage_pairs, dim3(stage_grid(npairs, 256)), dim3(256), 0, w->stream, w->d, pair_a, pair_b,

@@ -1,0 +1,89 @@
+"""The single world's solve over the GPU (colouring and data-flow sweeps) where its paths change: more
+items than waves and an item per wave, bodies whose pairs exceed what a thread keeps (32), what a workgroup
+counts in LDS (64 colours) and the colour starts kept there (1024), joints beside contacts.  Colour classes
+equal the oracle's; velocities and impulses are the oracle's colour-order solve's within the 1e-5 the
+other solver tests use (both sides round the same operations; the contact points differ by an ulp of
+atan2f at most)."""
+import numpy as np
+import pytest
+
+from helpers import impulse_error
+
+pytestmark = pytest.mark.gpu
+
+REL, ABS = 1e-5, 1e-6
+
+
+def _close(a, b):
+    a, b = np.asarray(a, np.float64), np.asarray(b, np.float64)
+    return np.all(np.abs(a - b) <= ABS + REL * np.abs(b))
+
+
+def plate_scene(spheres):
+    """A dynamic plate on the ground under `spheres` spheres, each resting on the plate alone: the plate is in
+    every contact but one, so its pairs all take different colours."""
+    from pe_amd.scenes import SHAPE_BOX, SHAPE_SPHERE, SceneBuilder
+    b = SceneBuilder()
+    side = int(np.ceil(np.sqrt(spheres)))
+    w = 0.5 * side + 1.0
+    b.add(SHAPE_BOX, (2 * w, 1.0, 2 * w), 1.0, (0.0, -0.5, 0.0), kin=1)
+    b.add(SHAPE_BOX, (w, 0.4, w), 50.0 * spheres, (0.0, 0.199, 0.0))
+    for k in range(spheres):
+        x, z = (k % side - side / 2 + 0.5) * 0.45, (k // side - side / 2 + 0.5) * 0.45
+        b.add(SHAPE_SPHERE, (0.2,), 10.0 + k % 7, (x, 0.598 - 0.0001 * (k % 3), z))
+    return b.scene(name=f"plate{spheres}")
+
+
+@pytest.mark.parametrize("spheres,blocks,mode", [(20, 0, 0), (80, 0, 0), (80, 1, 2), (80, 0, 1), (1100, 0, 2), (1100, 3, 2)])
+def test_one_body_in_many_pairs(spheres, blocks, mode):
+    import pe_amd
+    from pyoracle import OracleWorld
+    sc = plate_scene(spheres)
+    g, o = pe_amd.World(sc, max_pairs=40 * sc.n), OracleWorld(sc, 32)
+    g.set_solver_blocks(blocks)
+    g.set_colouring(mode)
+    print(f"[plate] {spheres} spheres, blocks {blocks}, colouring {mode}", flush=True)
+    for step in range(3):
+        for stage in ("integrate", "broadphase", "narrowphase", "solve"):
+            getattr(g, stage)()
+            getattr(o, stage)()
+        g.sync()
+        gp = g.pairs()
+        assert np.array_equal(gp, o.pairs())
+        order, cs = g.solve_order()
+        col = np.full(len(gp), -1)
+        for c in range(len(cs) - 1):
+            col[order[cs[c]:cs[c + 1]]] = c
+        assert np.array_equal(col, o.color_of()), f"colour classes step {step}"
+        assert len(cs) - 1 >= spheres
+        _, _, gv, gw = g.state()
+        _, _, ov, ow = o.state()
+        assert _close(gv, ov) and _close(gw, ow), f"velocities step {step}"
+        npts, _ = g.contacts()
+        err, _ = impulse_error(g.impulses(), o.impulses(), npts)
+        assert err <= REL, f"impulses step {step}: {err:.3e}"
+        o.set_state(*[np.asarray(x, np.float64) for x in g.state()])
+    g.close()
+
+
+@pytest.mark.parametrize("blocks", [1, 2, 7, 0])
+def test_results_do_not_depend_on_the_workgroups(blocks):
+    """A pile in contact, and joint chains whose ends strike the ground: the same bits with one workgroup
+    (many items per wave) as with the default's."""
+    import pe_amd
+    from pe_amd import scenes
+    for sc, steps in ((scenes.grid_world(700, seed=5, p_sphere=0.3), 90), (scenes.joint_chain_scene(30, 9, seed=3), 60)):
+        ref, w = pe_amd.World(sc), pe_amd.World(sc)
+        w.set_colouring(2)
+        w.set_solver_blocks(blocks)
+        ref.set_colouring(2)
+        ref.set_solver_blocks(16)
+        print(f"[workgroups] {sc.name}, blocks {blocks}", flush=True)
+        ref.step(steps)
+        w.step(steps)
+        w.sync()
+        for a, b in zip(w.state(), ref.state()):
+            assert np.array_equal(a.view(np.int32), b.view(np.int32))
+        assert np.array_equal(w.impulses(), ref.impulses())
+        ref.close()
+        w.close()
