@@ -7,6 +7,7 @@
 //                      reference's (i, j) order, next axis
 //   k_narrow           thread / pair: shape dispatch + 8-slot contact cache + depth sort
 //   k_setup            thread / pair: solver rows (FrictionContactConstraint::initSequentialImpulse)
+//   k_solve_small      worlds of up to 1024 bodies: colouring and sweeps in one workgroup, on LDS; else
 //   k_jp_*             the constraint graph: per body its pairs
 //   k_solve_flow       cooperative launch over the whole GPU: colouring, then the Gauss-Seidel sweeps in
 //                      colour order as a data flow between the pairs, and the velocity sync
@@ -351,9 +352,9 @@ __global__ void k_solve_begin(Dev d) {
 }
 
 // SequentialImpulseSolver::setupSolver (sequential_impulse_solver.cpp:11-58), thread / pair: the solver
-// rows, the list of the pairs to solve (contact points, not both bodies kinematic) and their dynamic
-// bodies' degrees.
-__global__ void k_setup(Dev d) {
+// rows, the list of the pairs to solve (contact points, not both bodies kinematic) and, for the colouring
+// over the GPU (GRAPH), their dynamic bodies' degrees.
+template <bool GRAPH> __global__ void k_setup(Dev d) {
     const int np = d.cnt->npairs;
     const int gsz = gridDim.x * blockDim.x;
     const int n_iter = (np + gsz - 1) / gsz;
@@ -365,7 +366,7 @@ __global__ void k_setup(Dev d) {
             const int a = d.ps.pa[p], c = d.ps.pb[p];
             const bool ka = d.b.iat(I_KIN, a) != 0, kc = d.b.iat(I_KIN, c) != 0;
             act = !(ka && kc);
-            if (act) {
+            if (GRAPH && act) {
                 d.jp_col[p] = -1;
                 if (!ka) atomicAdd(&d.jp_deg[a], 1);
                 if (!kc) atomicAdd(&d.jp_deg[c], 1);
@@ -982,6 +983,298 @@ __global__ void __launch_bounds__(FLOW_THREADS) k_solve_flow(Dev d, int claims) 
     }
 }
 
+// ---- the solve of a small world in one workgroup
+// Up to SMALL_BODIES bodies the solve runs in one workgroup of an ordinary launch: the bodies' temp velocities in
+// LDS, a workgroup barrier between colours (0.1 us) where the flow over the GPU pays 0.9 us for a store to
+// be seen on another CU, and none of the cooperative launch's queue switches (about 25 us a step).  Four
+// lanes per pair as there (quad_solve_row): a colour of up to SMALL_THREADS / 4 pairs is one pass as long as
+// its longest pair's row chains; a larger one takes several, which is where the flow becomes faster.
+constexpr int SMALL_THREADS = 512;
+constexpr int SMALL_LDS = 152 * 1024;
+constexpr int SMALL_COLORS = 128;   // colours counted in LDS (two 64-bit masks per body)
+constexpr int SMALL_ROW = RW + 1;   // a row's floats in LDS: an odd stride spreads the quads' rows over the banks
+
+// The same on the records in global memory, pairs on a thread each: where the pairs outgrow LDS or the masks.
+__device__ void small_global(const Dev& d, int nact, int* claim) {
+    __shared__ int wsum[SMALL_THREADS / WAVE + 1];
+    const int tid = threadIdx.x;
+    for (int i = tid; i < d.b.n; i += SMALL_THREADS) claim[i] = colour::FREE;
+    __syncthreads();
+    int* bufs[3] = {d.act, d.act + d.pcap, d.act + 2 * (size_t)d.pcap};
+    const int ncol = colour_pairs<true>(d.b, d.ps, bufs, nact, d.order, d.color_start, claim, 0, 0, wsum);
+    if (tid == 0) {
+        d.cnt->ncolors = ncol;
+        d.cnt->nordered = d.color_start[ncol];
+    }
+    for (int it = 0; it < d.iterations; it++) {
+        for (int c = 0; c < ncol; c++) {
+            for (int q = d.color_start[c] + tid; q < d.color_start[c + 1]; q += SMALL_THREADS) iterate_pair(d.b, d.ps, d.order[q]);
+            __syncthreads();
+        }
+        for (int c = 0; c < d.njcol; c++) {
+            for (int q = d.jcs[c] + tid; q < d.jcs[c + 1]; q += SMALL_THREADS) {
+                const int k = d.jorder[q];
+                const JointDef j = d.joints[k];
+                SolvBody A = load_solv(d.b, j.a), B = load_solv(d.b, j.b);
+                joint_solve(j, d.jrows[k], A, B);
+                for (int s = 0; s < 2; s++) {
+                    const SolvBody& S = s == 0 ? A : B;
+                    if (S.kin) continue;
+                    float* o = d.b.sbr(s == 0 ? j.a : j.b);
+                    o[SB_TV] = S.tv.x; o[SB_TV + 1] = S.tv.y; o[SB_TV + 2] = S.tv.z;
+                    o[SB_TW] = S.tw.x; o[SB_TW + 1] = S.tw.y; o[SB_TW + 2] = S.tw.z;
+                }
+            }
+            __syncthreads();
+        }
+    }
+    for (int i = tid; i < d.b.n; i += SMALL_THREADS) {
+        if (d.b.iat(I_KIN, i)) continue;
+        const float* o = d.b.sbr(i);
+        st3(d.b, F_V, i, f3{o[SB_TV], o[SB_TV + 1], o[SB_TV + 2]});
+        st3(d.b, F_W, i, f3{o[SB_TW], o[SB_TW + 1], o[SB_TW + 2]});
+    }
+}
+// The sweeps on LDS velocities vel ([n][8]: linear from 0, angular from 4) over the ordered pairs info (pair,
+// bodies A and B with the kinematic flag on top, rows | first row in rows << 4); ROWS_LDS: the rows are in
+// rows, else in the row store.
+template <bool ROWS_LDS>
+__device__ __forceinline__ void small_sweeps(const Dev& d, float* vel, const int4* info, float* rows, const int* cs, int ncol) {
+    const int tid = threadIdx.x;
+    const int quad = tid >> 2, c = (tid & 3) < 2 ? tid & 3 : 2;
+    const bool first = (tid & 3) == 0, own = (tid & 3) < 3;
+    QuadRow r[4];
+    QuadBody A, B;
+    int4 f = make_int4(0, 0, 0, 0);
+    bool have = false;
+    auto row = [&](int k) {
+        return ROWS_LDS ? rows + (size_t)((f.w >> 4) + k) * SMALL_ROW : d.ps.rows + ((size_t)f.x * 8 + k) * RW;
+    };
+    auto load4 = [&](int k0) {
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (k0 + u < (f.w & 15)) quad_load_row(row(k0 + u), c, r[u]);
+    };
+    auto solve4 = [&](int k0) {
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (k0 + u < (f.w & 15)) {
+                quad_solve_row(r[u], first, A, B);
+                if (own) row(k0 + u)[R_LN + c] = r[u].acc;
+            }
+    };
+    auto fetch = [&](int q, int end) {
+        have = q < end;
+        if (!have) return;
+        f = info[q];
+        quad_load_body(d.b.sbr(f.y & 0x7fffffff), c, f.y < 0, A);
+        quad_load_body(d.b.sbr(f.z & 0x7fffffff), c, f.z < 0, B);
+        load4(0);
+    };
+    auto solve = [&]() {
+        float* va = vel + (f.y & 0x7fffffff) * 8 + c;
+        float* vb = vel + (f.z & 0x7fffffff) * 8 + c;
+        A.tv = va[0]; A.tw = va[4];
+        B.tv = vb[0]; B.tw = vb[4];
+        solve4(0);
+        if ((f.w & 15) > 4) {
+            load4(4);
+            solve4(4);
+        }
+        if (own && !A.kin) { va[0] = A.tv; va[4] = A.tw; }
+        if (own && !B.kin) { vb[0] = B.tv; vb[4] = B.tw; }
+    };
+    if (ncol > 0) fetch(cs[0] + quad, cs[1]);
+    for (int it = 0; it < d.iterations; it++) {
+        for (int k = 0; k < ncol; k++) {
+            if (have) {
+                solve();
+                for (int q = cs[k] + quad + SMALL_THREADS / 4; q < cs[k + 1]; q += SMALL_THREADS / 4) {
+                    fetch(q, cs[k + 1]);
+                    solve();
+                }
+            }
+            const int nx = k + 1 < ncol ? k + 1 : 0;
+            fetch(cs[nx] + quad, cs[nx + 1]);   // all but the velocities, ahead of the barrier
+            __syncthreads();
+        }
+        // the joints after the contacts, colour by colour (sequential_impulse_solver.cpp:66-68)
+        for (int k = 0; k < d.njcol; k++) {
+            for (int q = d.jcs[k] + tid; q < d.jcs[k + 1]; q += SMALL_THREADS) {
+                const int id = d.jorder[q];
+                const JointDef j = d.joints[id];
+                SolvBody S[2] = {load_solv(d.b, j.a), load_solv(d.b, j.b)};
+#pragma unroll
+                for (int s = 0; s < 2; s++) {
+                    const float* v = vel + (s == 0 ? j.a : j.b) * 8;
+                    S[s].tv = f3{v[0], v[1], v[2]};
+                    S[s].tw = f3{v[4], v[5], v[6]};
+                }
+                joint_solve(j, d.jrows[id], S[0], S[1]);
+#pragma unroll
+                for (int s = 0; s < 2; s++) {
+                    if (S[s].kin) continue;
+                    float* v = vel + (s == 0 ? j.a : j.b) * 8;
+                    v[0] = S[s].tv.x; v[1] = S[s].tv.y; v[2] = S[s].tv.z;
+                    v[4] = S[s].tw.x; v[5] = S[s].tw.y; v[6] = S[s].tw.z;
+                }
+            }
+            __syncthreads();
+        }
+    }
+}
+__global__ void __launch_bounds__(SMALL_THREADS) k_solve_small(Dev d) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ int s_cnt[SMALL_COLORS], s_cs[SMALL_COLORS + 1], s_ncol, s_full, wsum[SMALL_THREADS / WAVE + 1];
+    const int tid = threadIdx.x, n = d.b.n;
+    const int nact = d.cnt->nact;
+    // LDS: velocities and ordered pairs; then the colouring's arrays, and over them the rows
+    float* vel = (float*)lds;
+    int4* info = (int4*)(lds + (size_t)n * 32);
+    unsigned char* rest = (unsigned char*)(info + nact);
+    uint64_t* mask = (uint64_t*)rest;                  // [n][2] colours of a body's coloured pairs
+    int* claim = (int*)(mask + 2 * (size_t)n);         // [2][n] claims of even and odd rounds
+    int* prio = claim + 2 * n;                         // per pair: claim priority,
+    uint32_t* ab = (uint32_t*)(prio + nact);           // bodies A | B << 16,
+    int* col = (int*)(ab + nact);                      // colour | place in the colour << 8 (-1: none yet)
+    bool small = (size_t)n * 32 + (size_t)nact * 28 + (size_t)n * 24 <= (size_t)SMALL_LDS;
+    if (small) {
+        if (tid < SMALL_COLORS) s_cnt[tid] = 0;
+        if (tid == 0) s_full = 0;
+        for (int i = tid; i < n; i += SMALL_THREADS) {
+            const float* s = d.b.sbr(i);
+            const float4 q0 = reinterpret_cast<const float4*>(s)[0], q1 = reinterpret_cast<const float4*>(s)[1];
+            float4* v = reinterpret_cast<float4*>(vel + (size_t)i * 8);   // tv 0..2, tw 3..5, im, kin in the record
+            v[0] = make_float4(q0.x, q0.y, q0.z, 0.0f);
+            v[1] = make_float4(q0.w, q1.x, q1.y, q1.w);   // [7]: the kinematic flag
+            mask[2 * i] = mask[2 * i + 1] = 0;
+            claim[i] = claim[n + i] = colour::FREE;
+        }
+        for (int k = tid; k < nact; k += SMALL_THREADS) {
+            const int p = d.act[k];
+            prio[k] = colour::prio(p, d.ps.npts[p]);
+            ab[k] = (uint32_t)d.ps.pa[p] | (uint32_t)d.ps.pb[p] << 16;
+            col[k] = -1;
+        }
+        __syncthreads();
+        // Rounds of claims: a pair that holds the lowest claim on its dynamic bodies among the uncoloured ones
+        // takes the first colour none of their coloured pairs has.  Those are exactly the neighbours of lower
+        // priority (one of higher priority cannot have held its claim before), so the classes are those of
+        // colour_pairs, all colours in the rounds of one (about 25 for box piles).
+        bool left = nact > 0;
+        for (int round = 0; __syncthreads_or(left && s_full == 0); round++) {
+            int* now = claim + (round & 1) * n;
+            int* next = claim + ((round + 1) & 1) * n;
+            for (int k = tid; k < nact; k += SMALL_THREADS) {
+                if (col[k] >= 0) continue;
+                const int a = ab[k] & 0xffff, b = ab[k] >> 16;
+                if (vel[8 * a + 7] == 0.0f) atomicMin(&now[a], prio[k]);
+                if (vel[8 * b + 7] == 0.0f) atomicMin(&now[b], prio[k]);
+            }
+            __syncthreads();
+            left = false;
+            for (int k = tid; k < nact; k += SMALL_THREADS) {
+                if (col[k] >= 0) continue;
+                const int a = ab[k] & 0xffff, b = ab[k] >> 16;
+                const bool ka = vel[8 * a + 7] != 0.0f, kb = vel[8 * b + 7] != 0.0f;
+                if (!ka) next[a] = colour::FREE;
+                if (!kb) next[b] = colour::FREE;
+                if (!((ka || now[a] == prio[k]) && (kb || now[b] == prio[k]))) {
+                    left = true;
+                    continue;
+                }
+                const uint64_t u0 = (ka ? 0 : mask[2 * a]) | (kb ? 0 : mask[2 * b]);
+                const uint64_t u1 = (ka ? 0 : mask[2 * a + 1]) | (kb ? 0 : mask[2 * b + 1]);
+                if (~u0 == 0 && ~u1 == 0) {
+                    s_full = 1;
+                    continue;
+                }
+                const int w = ~u0 != 0 ? 0 : 1, c = __ffsll((unsigned long long)~(w == 0 ? u0 : u1)) - 1;
+                if (!ka) mask[2 * a + w] |= 1ull << c;
+                if (!kb) mask[2 * b + w] |= 1ull << c;
+                col[k] = (64 * w + c) | atomicAdd(&s_cnt[64 * w + c], 1) << 8;
+            }
+        }
+        small = s_full == 0;
+        __syncthreads();
+    }
+    if (!small) {   // the same for every thread
+        small_global(d, nact, (int*)lds);
+        if (tid == 0) d.cnt->nact = 0;
+        return;
+    }
+    if (tid == 0) {
+        int run = 0, c = 0;
+        for (; c < SMALL_COLORS && s_cnt[c] > 0; c++) {
+            s_cs[c] = run;
+            run += s_cnt[c];
+        }
+        s_cs[c] = run;
+        s_ncol = c;
+    }
+    __syncthreads();
+    const int ncol = s_ncol;
+    for (int k = tid; k < nact; k += SMALL_THREADS) {
+        const int p = d.act[k], q = s_cs[col[k] & 0xff] + (col[k] >> 8);
+        const int a = ab[k] & 0xffff, b = ab[k] >> 16;
+        info[q] = make_int4(p, vel[8 * a + 7] != 0.0f ? a | 1 << 31 : a, vel[8 * b + 7] != 0.0f ? b | 1 << 31 : b, d.ps.npts[p]);
+        d.order[q] = p;
+    }
+    for (int c = tid; c <= ncol; c += SMALL_THREADS) d.color_start[c] = s_cs[c];
+    __syncthreads();
+    int nrows = 0;
+    for (int base = 0; base < nact; base += SMALL_THREADS) {
+        const int q = base + tid;
+        const int m = q < nact ? info[q].w : 0;
+        int tot;
+        const int ex = block_exclusive_scan(m, wsum, &tot);
+        if (q < nact) info[q].w = m | (nrows + ex) << 4;
+        nrows += tot;
+    }
+    __syncthreads();
+    float* rows = (float*)rest;
+    if ((size_t)n * 32 + (size_t)nact * 16 + (size_t)nrows * SMALL_ROW * 4 <= (size_t)SMALL_LDS) {
+        // a thread per float4 of a pair's rows (8 slots of 6)
+        for (int k = tid; k < nact * 48; k += SMALL_THREADS) {
+            const int q = k / 48, u = k % 48 / 6, part = k % 6;
+            const int4 f = info[q];
+            if (u >= (f.w & 15)) continue;
+            const float4 v = reinterpret_cast<const float4*>(d.ps.rows + ((size_t)f.x * 8 + u) * RW)[part];
+            float* o = rows + (size_t)((f.w >> 4) + u) * SMALL_ROW + 4 * part;
+            o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
+        }
+        __syncthreads();
+        small_sweeps<true>(d, vel, info, rows, s_cs, ncol);
+        for (int k = tid; k < nact * 8; k += SMALL_THREADS) {   // the accumulated impulses, for the getters
+            const int4 f = info[k >> 3];
+            if ((k & 7) >= (f.w & 15)) continue;
+            const float* o = rows + (size_t)((f.w >> 4) + (k & 7)) * SMALL_ROW + R_LN;
+            float* t = d.ps.rows + ((size_t)f.x * 8 + (k & 7)) * RW + R_LN;
+            t[0] = o[0]; t[1] = o[1]; t[2] = o[2];
+        }
+    } else {
+        small_sweeps<false>(d, vel, info, rows, s_cs, ncol);
+    }
+    __syncthreads();
+    // syncTempVelocity (sequential_impulse_solver.cpp:71-80)
+    for (int i = tid; i < n; i += SMALL_THREADS) {
+        const float* v = vel + (size_t)i * 8;
+        if (v[7] != 0.0f) continue;
+        float* s = d.b.sbr(i);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            d.b.at(F_V + k, i) = s[SB_TV + k] = v[k];
+            d.b.at(F_W + k, i) = s[SB_TW + k] = v[4 + k];
+        }
+    }
+    if (tid == 0) {
+        d.cnt->ncolors = ncol;
+        d.cnt->nordered = nact;
+        d.cnt->jp_rounds = 0;
+        d.cnt->nact = 0;   // counted from zero by the next step's set-up
+    }
+}
+
 // Contact points of this narrowphase: per-workgroup sums added to the counter k_narrow_finish
 // cleared; a pair whose clipper lost points (bit 1 of its swap word) raises OVF_CLIP.
 __global__ void __launch_bounds__(256) k_count_points(Dev d) {
@@ -1004,6 +1297,9 @@ __global__ void __launch_bounds__(256) k_count_points(Dev d) {
 // Workgroups of the cooperative solve: enough waves for about an item each (a world at rest has up to
 // two pairs with contacts per body, 16 to an item), at most one workgroup per CU of the 256.
 static int default_flow_blocks(int n, int max_blocks) { return std::min(max_blocks, std::max(8, std::min(256, n / 80))); }
+
+// Bodies up to which the solve runs in one workgroup (k_solve_small).
+constexpr int SMALL_BODIES = 1024;
 
 struct pe_world {
     Dev d{};
@@ -1073,8 +1369,14 @@ struct pe_world {
         return PE_OK;
     }
     int launch_solve() {
+        if (colouring == 0 && n <= SMALL_BODIES) {
+            hipLaunchKernelGGL(k_setup<false>, dim3(grid(d.pcap, 128)), dim3(128), 0, stream, d);
+            if (d.njoints > 0) hipLaunchKernelGGL(k_joint_setup, dim3(grid(d.njoints, 64)), dim3(64), 0, stream, d);
+            hipLaunchKernelGGL(k_solve_small, dim3(1), dim3(SMALL_THREADS), SMALL_LDS, stream, d);
+            return PE_OK;
+        }
         hipLaunchKernelGGL(k_solve_begin, dim3(grid(n, 256)), dim3(256), 0, stream, d);
-        hipLaunchKernelGGL(k_setup, dim3(grid(d.pcap, 128)), dim3(128), 0, stream, d);
+        hipLaunchKernelGGL(k_setup<true>, dim3(grid(d.pcap, 128)), dim3(128), 0, stream, d);
         if (d.njoints > 0) hipLaunchKernelGGL(k_joint_setup, dim3(grid(d.njoints, 64)), dim3(64), 0, stream, d);
         hipLaunchKernelGGL(k_jp_alloc, dim3(grid(n, 256)), dim3(256), 0, stream, d);
         hipLaunchKernelGGL(k_jp_fill, dim3(grid(d.pcap, 256)), dim3(256), 0, stream, d);
@@ -1279,6 +1581,10 @@ int pe_world_create(const pe_scene_desc* sc, const pe_world_params* prm, int32_t
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
             hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k_solve_flow, FLOW_THREADS, 0) != hipSuccess || per_cu < 1) {
             pe_set_error("cannot size the cooperative solver grid");
+            return fail(PE_ERR_DEVICE);
+        }
+        if (hipFuncSetAttribute((const void*)k_solve_small, hipFuncAttributeMaxDynamicSharedMemorySize, SMALL_LDS) != hipSuccess) {
+            pe_set_error("cannot size the small-world solver's LDS");
             return fail(PE_ERR_DEVICE);
         }
         w->flow_max_blocks = cus * per_cu;
@@ -1783,6 +2089,7 @@ int pe_world_set_colouring(pe_world* w, int32_t mode) {
         return PE_ERR_INVALID;
     }
     w->colouring = mode;
+    PE_HIP(hipMemsetAsync(&w->d.cnt->nact, 0, sizeof(int32_t), w->stream));   // as the one-workgroup solve leaves it
     return PE_OK;
 }
 
@@ -1874,6 +2181,7 @@ __global__ void k_stage_pairs(Dev d, const int32_t* __restrict__ pa, const int32
         d.cnt->nsat = 0;
         d.cnt->npoints = 0;
         d.cnt->overflow = 0;
+        d.cnt->nact = 0;
     }
     for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < np; p += gridDim.x * blockDim.x) {
         d.ps.pa[p] = pa[p];

@@ -1,6 +1,7 @@
-"""The single world's solve over the GPU (colouring and data-flow sweeps) where its paths change: more
+"""The single world's solve: over the GPU (colouring and data-flow sweeps) where its paths change: more
 items than waves and an item per wave, bodies whose pairs exceed what a thread keeps (32), what a workgroup
-counts in LDS (64 colours) and the colour starts kept there (1024), joints beside contacts.  Colour classes
+counts in LDS (64 colours) and the colour starts kept there (1024), joints beside contacts; in one
+workgroup (up to 1024 bodies) with its rows in LDS, in memory, and where pairs or colours outgrow it.  Colour classes
 equal the oracle's; velocities and impulses are the oracle's colour-order solve's within the 1e-5 the
 other solver tests use (both sides round the same operations; the contact points differ by an ulp of
 atan2f at most)."""
@@ -34,7 +35,7 @@ def plate_scene(spheres):
     return b.scene(name=f"plate{spheres}")
 
 
-@pytest.mark.parametrize("spheres,blocks,mode", [(20, 0, 0), (80, 0, 0), (80, 1, 2), (80, 0, 1), (1100, 0, 2), (1100, 3, 2)])
+@pytest.mark.parametrize("spheres,blocks,mode", [(20, 0, 0), (80, 0, 0), (80, 1, 2), (80, 0, 1), (150, 0, 0), (1100, 0, 2), (1100, 3, 2)])
 def test_one_body_in_many_pairs(spheres, blocks, mode):
     import pe_amd
     from pyoracle import OracleWorld
@@ -87,3 +88,48 @@ def test_results_do_not_depend_on_the_workgroups(blocks):
         assert np.array_equal(w.impulses(), ref.impulses())
         ref.close()
         w.close()
+
+
+def cluster_scene(n, size, seed=9):
+    """n overlapping spheres in a cube of edge `size`: many pairs in contact per body."""
+    from pe_amd.scenes import SHAPE_BOX, SHAPE_SPHERE, SceneBuilder
+    rng = np.random.default_rng(seed)
+    b = SceneBuilder()
+    b.add(SHAPE_BOX, (60.0, 1.0, 60.0), 1.0, (0.0, -0.5, 0.0), kin=1)
+    for x in rng.uniform(-0.5, 0.5, (n, 3)) * size + (0.0, 0.5 * size, 0.0):
+        b.add(SHAPE_SPHERE, (0.3,), 100.0, x)
+    return b.scene(name=f"cluster{n}")
+
+
+@pytest.mark.parametrize("name", ["pair", "mixed", "boxes", "limit", "chains", "joint_demo", "cluster"])
+def test_one_workgroup_equals_the_flow(name):
+    """The solve of a small world in one workgroup and over the GPU: the same bits, the same colour classes."""
+    import pe_amd
+    from pe_amd import scenes
+    sc, steps = {"pair": lambda: (scenes.grid_world(1, seed=2), 70),
+                 "mixed": lambda: (scenes.grid_world(700, seed=5), 90),
+                 "boxes": lambda: (scenes.grid_world(900, seed=6, p_sphere=0.0), 100),
+                 "limit": lambda: (scenes.grid_world(1023, seed=7, p_sphere=0.2), 80),
+                 "chains": lambda: (scenes.joint_chain_scene(30, 9, seed=3), 60),
+                 "joint_demo": lambda: (scenes.joint_demo_scene(), 60),
+                 "cluster": lambda: (cluster_scene(800, 3.2), 1)}[name]()
+    a, b = pe_amd.World(sc, max_pairs=200 * sc.n), pe_amd.World(sc, max_pairs=200 * sc.n)
+    b.set_colouring(2)
+    print(f"[one workgroup] {name}: {sc.n} bodies", flush=True)
+    for part in (steps, 2 if steps > 1 else 3):
+        a.step(part)
+        b.step(part)
+        a.sync()
+        b.sync()
+        for x, y in zip(a.state(), b.state()):
+            assert np.array_equal(x.view(np.int32), y.view(np.int32))
+        assert np.array_equal(a.impulses(), b.impulses())
+        (oa, ca), (ob, cb) = a.solve_order(), b.solve_order()
+        assert np.array_equal(ca, cb)
+        for k in range(len(ca) - 1):
+            assert np.array_equal(np.sort(oa[ca[k]:ca[k + 1]]), np.sort(ob[ca[k]:ca[k + 1]]))
+        print(f"[one workgroup] {name}: {a.counts()}", flush=True)
+        if name == "cluster" and part == steps:
+            assert len(oa) * 28 + sc.n * 56 > 152 * 1024   # beyond the LDS the kernel works in
+    a.close()
+    b.close()
