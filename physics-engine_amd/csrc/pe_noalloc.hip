@@ -17,41 +17,40 @@ using namespace pe;
 namespace {
 
 constexpr int NA_MAX_BODIES = PE_NOALLOC_MAX_BODIES;
-constexpr int NA_CHUNK_CAP = 1 << 20;   // sweep chunks: 32 Mi candidate tests
+constexpr int NA_CHUNK_CAP = 1 << 20;   // 32 Mi candidate tests
 
-// Byte offsets of the working arrays inside the scratch array (each 256-byte aligned).
+// Byte offsets of the working arrays inside the scratch array (each 256-byte aligned).  The units' owners, made
+// after the sort, take the place of the radix sort's other arrays.
 struct NoAllocLayout {
-    size_t keys, vals, keys2, vals2, skey, cand, hist, red, chunk, chunk_hit, scan_part, cnt, end;
+    size_t keys, keys2, vals2, hist, owner, vals, skey, srec, end_, first, red, blk, unit_hit, cnt, end;
     constexpr NoAllocLayout()
-        : keys(0), vals(0), keys2(0), vals2(0), skey(0), cand(0), hist(0), red(0), chunk(0), chunk_hit(0), scan_part(0),
-          cnt(0), end(0) {
+        : keys(0), keys2(0), vals2(0), hist(0), owner(0), vals(0), skey(0), srec(0), end_(0), first(0), red(0), blk(0),
+          unit_hit(0), cnt(0), end(0) {
         size_t o = 0;
         auto take = [&o](size_t bytes) { const size_t at = o; o += (bytes + 255) & ~(size_t)255; return at; };
+        const size_t units = (size_t)sap_units(NA_CHUNK_CAP, NA_MAX_BODIES);
         keys = take(4 * (size_t)NA_MAX_BODIES);
-        vals = take(4 * (size_t)NA_MAX_BODIES);
         keys2 = take(4 * (size_t)NA_MAX_BODIES);
         vals2 = take(4 * (size_t)NA_MAX_BODIES);
-        skey = take(4 * (size_t)NA_MAX_BODIES);
-        cand = take(4 * ((size_t)NA_MAX_BODIES + 1));
         hist = take(4 * 256 * (size_t)((NA_MAX_BODIES + RS_TILE - 1) / RS_TILE));
+        const size_t sort_end = o;
+        o = 0;
+        owner = take(4 * units);
+        if (o < sort_end) o = sort_end;
+        vals = take(4 * (size_t)NA_MAX_BODIES);
+        skey = take(4 * (size_t)NA_MAX_BODIES);
+        srec = take(32 * (size_t)NA_MAX_BODIES);
+        end_ = take(4 * (size_t)NA_MAX_BODIES);
+        first = take(4 * (size_t)NA_MAX_BODIES);
         red = take(8 * SAP_RED_VALUES * 256);
-        chunk = take(4 * (size_t)NA_CHUNK_CAP);
-        chunk_hit = take(4 * (size_t)NA_CHUNK_CAP);
-        scan_part = take(4 * (size_t)(((NA_CHUNK_CAP > NA_MAX_BODIES + 1 ? NA_CHUNK_CAP : NA_MAX_BODIES + 1) + SCAN_TILE - 1) /
-                                          SCAN_TILE + 1));
+        blk = take(sizeof(uint2) * (size_t)((NA_MAX_BODIES + SAP_BLOCK - 1) / SAP_BLOCK));
+        unit_hit = take(8 * units);
         cnt = take(sizeof(DevCounts));
         end = o;
     }
 };
 constexpr NoAllocLayout NA_LAYOUT{};
 static_assert(NA_LAYOUT.end <= PE_NOALLOC_SCRATCH_BYTES, "the working arrays fit the scratch array");
-
-// result[0] = pairs found, result[1] = next axis, result[2] = capacity-error bits (as pe_stage_broadphase)
-__global__ void k_noalloc_result(SapView s, int32_t* result) {
-    result[0] = (int32_t)s.cnt->nchunk_pairs;
-    result[1] = s.cnt->axis;
-    result[2] = s.cnt->overflow;
-}
 
 }  // namespace
 
@@ -110,22 +109,24 @@ extern "C" int pe_stage_broadphase_noalloc(int32_t n, const float* aabb, int32_t
     s.keys2 = reinterpret_cast<uint32_t*>(base + NA_LAYOUT.keys2);
     s.vals2 = reinterpret_cast<uint32_t*>(base + NA_LAYOUT.vals2);
     s.skey = reinterpret_cast<float*>(base + NA_LAYOUT.skey);
-    s.cand = reinterpret_cast<uint32_t*>(base + NA_LAYOUT.cand);
+    s.end = reinterpret_cast<uint32_t*>(base + NA_LAYOUT.end_);
+    s.first = reinterpret_cast<uint32_t*>(base + NA_LAYOUT.first);
     s.hist = reinterpret_cast<uint32_t*>(base + NA_LAYOUT.hist);
     s.red = reinterpret_cast<double*>(base + NA_LAYOUT.red);
-    s.chunk = reinterpret_cast<uint32_t*>(base + NA_LAYOUT.chunk);
-    s.chunk_hit = reinterpret_cast<uint32_t*>(base + NA_LAYOUT.chunk_hit);
-    s.scan_part = reinterpret_cast<uint32_t*>(base + NA_LAYOUT.scan_part);
+    s.srec = reinterpret_cast<float*>(base + NA_LAYOUT.srec);
+    s.blk = reinterpret_cast<uint2*>(base + NA_LAYOUT.blk);
+    s.owner = reinterpret_cast<uint32_t*>(base + NA_LAYOUT.owner);
+    s.unit_hit = reinterpret_cast<uint64_t*>(base + NA_LAYOUT.unit_hit);
     s.cnt = reinterpret_cast<DevCounts*>(base + NA_LAYOUT.cnt);
     s.pa = pair_a;
     s.pb = pair_b;
     s.pcap = cap;
     s.chunk_cap = NA_CHUNK_CAP;
+    s.axis_in = axis;
+    s.result = result;
     hipStream_t st = (hipStream_t)stream;
-    // the counters the sweep accumulates into start from zero, whatever the last call left
-    hipLaunchKernelGGL(k_sap_begin, dim3(1), dim3(1), 0, st, s, (int)axis);
     if (n >= 2) sap_launch(s, st);
-    hipLaunchKernelGGL(k_noalloc_result, dim3(1), dim3(1), 0, st, s, result);
+    else hipLaunchKernelGGL(k_sap_none, dim3(1), dim3(1), 0, st, s);
     PE_HIP(hipGetLastError());
     return PE_OK;
 }

@@ -1,11 +1,15 @@
 // Sweep-and-prune broadphase over n AABBs on the whole GPU (BroadPhaseSweepAndPrune::
 // calcCollisionPairs, broad_phase_sweep_and_prune.cpp:6-41), shared by the single-world pipeline
 // (its body store) and the stage entry points (a caller's AABB records):
-//   k_sap_keys + radix   stable LSD sort of (aabb_min[axis] + 0, index), 4 passes of 8 bits
-//   k_sap_ranges/cand    per sorted body, the candidate run j > i with min_j <= max_i
-//   k_sap_chunks         load-balanced sweep over all candidates, two passes (count, emit), so
-//                        pairs come out in the reference's (i, j) sweep order
-//   k_sap_axis_*         next axis = argmax variance of AABB centres (FP64, fixed blocks)
+//   k_sap_rank           up to SAP_RANK_MAX bodies: stable sort of (aabb_min[axis] + 0, index) by counting,
+//                        or k_sap_keys + radix, a stable LSD sort in 4 passes of 8 bits; both leave the
+//                        AABB records in sorted order; beside them the next axis's partial sums
+//   k_sap_runs           SAP_BLOCK sorted bodies per workgroup: their candidate runs (j > i with min_j <=
+//                        max_i), cut into units of 64 candidates
+//   k_sap_test           a wave per unit tests its candidates, a lane each (up to SAP_FUSED_MAX bodies
+//                        k_sap_runs does so itself)
+//   k_sap_emit           the pairs that passed, in the reference's (i, j) sweep order; the next axis =
+//                        argmax variance of AABB centres (FP64, fixed blocks)
 #pragma once
 #include "pe_common.hpp"
 #include "pe_prims.hpp"
@@ -17,12 +21,13 @@ struct DevCounts {          // device-side counters of one step
     int32_t prev_npairs;    // pairs of the previous narrowphase (contact slots that survive)
     int32_t axis;           // SAP axis for the next sort
     int32_t overflow;       // sticky capacity-error bits (OVF_*), cleared when the host reports them
-    uint32_t ncand;         // total sweep candidates
     uint32_t nchunk_pairs;  // pairs counted by the sweep (unclamped)
     int32_t ncolors;
     int32_t nordered;       // pairs in the solve order
     int32_t npoints;        // contact points of the last narrowphase
-    uint32_t nchunks;       // live sweep chunks
+    uint32_t nunits;        // units of candidates handed out to the workgroups of the sweep
+    uint32_t pad;
+    uint64_t ncand;         // sweep candidates
     uint32_t bar_count;     // grid barrier: arrivals (0 between barriers)
     uint32_t bar_gen;       // grid barrier: generation
     int32_t nshape;         // pairs of this narrowphase that involve a cylinder or a mesh ...
@@ -42,8 +47,12 @@ constexpr int OVF_CHUNKS = 4;        // the sweep had more candidates than its c
 constexpr int OVF_CLIP = 8;          // a clipped polygon outgrew its buffer (contact points lost)
 constexpr int OVF_STALL = 16;        // the solver gave up a wait (not a capacity: a fault of this program)
 
-constexpr int SAP_CHUNK = 32;        // candidates per thread in the sweep
-static_assert(SAP_CHUNK <= 32, "a chunk's test outcomes are one 32-bit mask");
+constexpr int SAP_BLOCK = 16;        // sorted bodies per workgroup of the sweep
+constexpr int SAP_THREADS = 256;     // its threads (16 lanes search the run of each body)
+constexpr int SAP_UNIT = 64;         // candidates per unit
+constexpr int SAP_CHUNK = 32;        // the workspace is sized in chunks of this many candidates
+// Units for at most `chunks` chunks of candidates over n bodies' runs.
+__host__ __device__ constexpr int64_t sap_units(int64_t chunks, int64_t n) { return chunks * SAP_CHUNK / SAP_UNIT + n + 1; }
 constexpr int SAP_RED_THREADS = 256;
 constexpr int SAP_RED_VALUES = 7;   // axis reduction: centre sums (3), squared sums (3), bodies
 
@@ -62,27 +71,31 @@ struct SapView {
     uint32_t* keys2;
     uint32_t* vals2;
     float* skey;            // [n] sorted keys as floats
-    float* srec;            // [n][8] the AABB records in sorted order (or null: read through vals)
-    uint32_t* cand;         // [n + 1] candidate counts -> offsets
-    uint32_t* chunk;        // [chunk_cap] pairs per chunk -> offsets
-    uint32_t* chunk_hit;    // [chunk_cap] per chunk, bit k: its candidate k is a pair
-    uint32_t* scan_part;    // [scan_parts(n, chunk_cap)] tile totals of the grid-wide scans
+    float* srec;            // [n][8] the AABB records in sorted order
+    uint32_t* end;          // [n] per sorted body: the end of its run
+    uint32_t* first;        // [n] and its first unit
+    uint2* blk;             // [sap_blocks(n)] per SAP_BLOCK sorted bodies: units, pairs
+    uint32_t* owner;        // [sap_units(chunk_cap, n)] per unit its sorted body
+    uint64_t* unit_hit;     // [sap_units(chunk_cap, n)] per unit, bit k: its candidate k is a pair
     uint32_t* hist;         // [256 * radix_blocks(n)] radix histograms
     double* red;            // [6 * red_blocks(n)] axis reduction partials
     DevCounts* cnt;
     int32_t* pa;            // [pcap] pair output: body A, body B (sorted position order)
     int32_t* pb;
     int pcap;
-    int chunk_cap;
+    int chunk_cap;          // at most this many times SAP_CHUNK candidates
+    int axis_in;            // the sort axis (-1: the one in cnt, left by the last sweep)
+    int32_t* result;        // [3] or null: pairs found, next axis, capacity-error bits
     const uint64_t* ignore; // [nignore] sorted keys (lo << 32 | hi) of body pairs that never collide
     int nignore;
+    __device__ __forceinline__ int ax() const { return axis_in >= 0 ? axis_in : cnt->axis; }
     __device__ __forceinline__ float mn(int k, int i) const { return amin[(size_t)k * fs + (size_t)i * bs]; }
     __device__ __forceinline__ float mx(int k, int i) const { return amax[(size_t)k * fs + (size_t)i * bs]; }
 };
 
 __host__ inline int sap_radix_blocks(int n) { return (n + RS_TILE - 1) / RS_TILE; }
 __host__ inline int sap_red_blocks(int n) { return n < 1 ? 1 : (n + SAP_RED_THREADS - 1) / SAP_RED_THREADS < 256 ? (n + SAP_RED_THREADS - 1) / SAP_RED_THREADS : 256; }
-__host__ inline int sap_scan_parts(int n, int chunk_cap) { return ((chunk_cap > n + 1 ? chunk_cap : n + 1) + SCAN_TILE - 1) / SCAN_TILE + 1; }
+__host__ inline int sap_blocks(int n) { return (n + SAP_BLOCK - 1) / SAP_BLOCK; }
 
 // BroadPhaseBase::validateCollisionPair (broad_phase_base.cpp:5-19) on two AABB records: the
 // ignore-collision flags, both kinematic, then closed-interval overlap on x, y, z.  Ignore-id pairs
@@ -114,12 +127,8 @@ __device__ __forceinline__ void sap_ld_rec(const float* src, float (&dst)[8]) {
     dst[0] = a.x; dst[1] = a.y; dst[2] = a.z; dst[3] = a.w;
     dst[4] = b.x; dst[5] = b.y; dst[6] = b.z; dst[7] = b.w;
 }
-// The record of the body at sorted position q: from the sorted copy (contiguous loads along a run
-// of candidates) when there is one.
-__device__ __forceinline__ void sap_ld_sorted(const SapView& s, int q, float (&dst)[8]) {
-    if (s.srec) sap_ld_rec(s.srec + (size_t)q * 8, dst);
-    else sap_ld_rec(s.rec + (size_t)s.vals[q] * 8, dst);
-}
+// The record of the body at sorted position q (contiguous loads along a run of candidates).
+__device__ __forceinline__ void sap_ld_sorted(const SapView& s, int q, float (&dst)[8]) { sap_ld_rec(s.srec + (size_t)q * 8, dst); }
 // sap_pair_allowed for the bodies at sorted positions qa and qb (their indices are loaded only
 // for the ignore-pair search).
 __device__ __forceinline__ bool sap_pair_allowed_sorted(const SapView& s, const float (&A)[8], const float (&B)[8],
@@ -129,135 +138,28 @@ __device__ __forceinline__ bool sap_pair_allowed_sorted(const SapView& s, const 
     return sap_pair_allowed(s, A, B, (int)s.vals[qa], (int)s.vals[qb]);
 }
 
-// Sets the axis of this sweep and clears the overflow bits a previous stage call left (the
-// single-world pipeline keeps both in its counters and does not launch this).
-static __global__ void k_sap_begin(SapView s, int axis) {
-    s.cnt->axis = axis;
+// A sweep over fewer than two bodies through a stage entry point: no pairs, the axis stays.
+static __global__ void k_sap_none(SapView s) {
+    s.cnt->axis = s.axis_in;
     s.cnt->overflow = 0;
     s.cnt->npairs = 0;
     s.cnt->nchunk_pairs = 0;
+    s.result[0] = 0;
+    s.result[1] = s.axis_in;
+    s.result[2] = 0;
 }
-
-static __global__ void k_sap_keys(SapView s) {
-    const int ax = s.cnt->axis;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < s.n; i += gridDim.x * blockDim.x) {
-        s.keys[i] = float_key(s.mn(ax, i) + 0.0f);
-        s.vals[i] = (uint32_t)i;
-    }
+// Clears what the sweep counts (a given axis: a stage entry point, whose last call's errors are dropped).
+__device__ __forceinline__ void sap_begin(const SapView& s) {
+    s.cnt->nunits = 0;
+    s.cnt->ncand = 0;
+    if (s.axis_in >= 0) s.cnt->overflow = 0;
 }
-
-// After the sort: sorted float keys and, per sorted position s, the number of candidates
-// j > s with key_j <= max_i (the reference's sweep breaks at the first key_j > max_i).
-static __global__ void k_sap_ranges(SapView s) {
-    const int ax = s.cnt->axis;
-    for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < s.n; q += gridDim.x * blockDim.x) {
-        const int i = (int)s.vals[q];
-        s.skey[q] = s.mn(ax, i) + 0.0f;
-        if (s.srec) {
-            const float4* src = reinterpret_cast<const float4*>(s.rec + (size_t)i * 8);
-            float4* dst = reinterpret_cast<float4*>(s.srec + (size_t)q * 8);
-            dst[0] = src[0];
-            dst[1] = src[1];
-        }
-    }
-}
-static __global__ void k_sap_cand(SapView s) {
-    const int n = s.n;
-    const int ax = s.cnt->axis;
-    for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x) {
-        const int i = (int)s.vals[q];
-        const float m = s.mx(ax, i);
-        int lo = q + 1, hi = n;  // first position in [q+1, n) with skey > m
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (s.skey[mid] > m) hi = mid; else lo = mid + 1;
-        }
-        s.cand[q] = (uint32_t)(lo - q - 1);
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) s.cand[n] = 0;
-}
-
-// Locates candidate t: sorted position q with cand[q] <= t < cand[q+1] (cand holds offsets).
-__device__ __forceinline__ int sap_find(const uint32_t* off, int n, uint32_t t) {
-    int lo = 0, hi = n;  // last q with off[q] <= t
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (off[mid] <= t) lo = mid; else hi = mid;
-    }
-    return lo;
-}
-
-template <bool EMIT>
-static __global__ void k_sap_chunks(SapView s) {
-    const int n = s.n;
-    const uint32_t S = s.cnt->ncand;
-    const uint32_t nchunks = min((S + SAP_CHUNK - 1) / SAP_CHUNK, (uint32_t)s.chunk_cap);
-    for (uint32_t c = blockIdx.x * blockDim.x + threadIdx.x; c < nchunks; c += gridDim.x * blockDim.x) {
-        uint32_t t = c * SAP_CHUNK;
-        const uint32_t tend = min(S, t + SAP_CHUNK);
-        int q = sap_find(s.cand, n, t);
-        while (s.cand[q + 1] <= t) q++;
-        if (EMIT) {
-            // the counting pass left the outcome of each of the chunk's tests in chunk_hit[c]
-            uint32_t out = s.chunk[c];
-            uint32_t hit = s.chunk_hit[c];
-            const uint32_t t0 = t;
-            int cur = q;
-            uint32_t cb = s.cand[cur], nb = s.cand[cur + 1];
-            while (hit) {
-                const uint32_t tt = t0 + (uint32_t)(__ffs(hit) - 1);
-                hit &= hit - 1;
-                while (nb <= tt) {
-                    cur++;
-                    cb = nb;
-                    nb = s.cand[cur + 1];
-                }
-                if ((int)out < s.pcap) {
-                    s.pa[out] = (int)s.vals[cur];
-                    s.pb[out] = (int)s.vals[cur + 1 + (int)(tt - cb)];
-                }
-                out++;
-            }
-        } else {
-            uint32_t cntv = 0, hit = 0;
-            const uint32_t t0 = t;
-            int cur = q;
-            // the run's first candidate and the next run's, in registers: a candidate's record is then
-            // addressed without a load of the offsets (only a change of run reads them)
-            uint32_t cb = s.cand[cur], nb = s.cand[cur + 1];
-            float A[8], B[8];
-            sap_ld_sorted(s, cur, A);   // the run body's record stays in registers
-            for (; t < tend; t++) {
-                while (nb <= t) {
-                    cur++;
-                    cb = nb;
-                    nb = s.cand[cur + 1];
-                    sap_ld_sorted(s, cur, A);
-                }
-                const int qj = cur + 1 + (int)(t - cb);
-                sap_ld_sorted(s, qj, B);
-                if (sap_pair_allowed_sorted(s, A, B, cur, qj)) {
-                    cntv++;
-                    hit |= 1u << (t - t0);
-                }
-            }
-            s.chunk[c] = cntv;
-            s.chunk_hit[c] = hit;
-        }
-    }
-}
-
-// Number of live sweep chunks, for the chunk scan.
-static __global__ void k_sap_nchunks(SapView s) {
-    const uint32_t want = (s.cnt->ncand + SAP_CHUNK - 1) / SAP_CHUNK;
-    s.cnt->nchunks = min(want, (uint32_t)s.chunk_cap);
-    if (want > (uint32_t)s.chunk_cap) s.cnt->overflow |= OVF_CHUNKS;
-}
-
-static __global__ void k_sap_finish(SapView s) {
-    const uint32_t total = s.cnt->nchunk_pairs;
-    if (total > (uint32_t)s.pcap) s.cnt->overflow |= OVF_PAIRS;
-    s.cnt->npairs = total > (uint32_t)s.pcap ? s.pcap : (int32_t)total;
+__device__ __forceinline__ void sap_sorted(const SapView& s, uint32_t q, int i, float key) {
+    s.skey[q] = key;
+    const float4* src = reinterpret_cast<const float4*>(s.rec + (size_t)i * 8);
+    float4* dst = reinterpret_cast<float4*>(s.srec + (size_t)q * 8);
+    dst[0] = src[0];
+    dst[1] = src[1];
 }
 
 // Next SAP axis (broad_phase_sweep_and_prune.cpp:37-40): variance of AABB centres, reduced in
@@ -265,81 +167,325 @@ static __global__ void k_sap_finish(SapView s) {
 // A body whose AABB is empty (min > max) has left the world (World::removeRigidBody, an ended
 // lifetime): it sorts last with an infinite key, has no candidates and is not in the variance; with
 // fewer than two bodies left the axis stays (the reference's sweep returns early).
-static __global__ void __launch_bounds__(SAP_RED_THREADS) k_sap_axis_partial(SapView s) {
-    __shared__ double sh[SAP_RED_VALUES][SAP_RED_THREADS];
-    double acc[SAP_RED_VALUES] = {0, 0, 0, 0, 0, 0, 0};
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < s.n; i += gridDim.x * blockDim.x) {
-        if (!(s.mn(0, i) <= s.mx(0, i))) continue;
+// The partial sums of block b of nb (SAP_RED_THREADS threads of the workgroup work).
+__device__ __forceinline__ void sap_axis_partial(const SapView& s, int b, int nb, double (&sh)[SAP_RED_VALUES][SAP_RED_THREADS]) {
+    const int t = threadIdx.x;
+    if (t < SAP_RED_THREADS) {
+        double acc[SAP_RED_VALUES] = {0, 0, 0, 0, 0, 0, 0};
+        for (int i = b * SAP_RED_THREADS + t; i < s.n; i += nb * SAP_RED_THREADS) {
+            if (!(s.mn(0, i) <= s.mx(0, i))) continue;
 #pragma unroll
-        for (int k = 0; k < 3; k++) {
-            const float c = (s.mn(k, i) + s.mx(k, i)) * 0.5f;
-            acc[k] += (double)c;
-            acc[3 + k] += (double)(c * c);
+            for (int k = 0; k < 3; k++) {
+                const float c = (s.mn(k, i) + s.mx(k, i)) * 0.5f;
+                acc[k] += (double)c;
+                acc[3 + k] += (double)(c * c);
+            }
+            acc[6] += 1.0;
         }
-        acc[6] += 1.0;
-    }
 #pragma unroll
-    for (int k = 0; k < SAP_RED_VALUES; k++) sh[k][threadIdx.x] = acc[k];
+        for (int k = 0; k < SAP_RED_VALUES; k++) sh[k][t] = acc[k];
+    }
     __syncthreads();
     for (int o = SAP_RED_THREADS / 2; o > 0; o >>= 1) {
-        if (threadIdx.x < o)
+        if (t < o)
 #pragma unroll
-            for (int k = 0; k < SAP_RED_VALUES; k++) sh[k][threadIdx.x] += sh[k][threadIdx.x + o];
+            for (int k = 0; k < SAP_RED_VALUES; k++) sh[k][t] += sh[k][t + o];
         __syncthreads();
     }
-    if (threadIdx.x == 0)
-#pragma unroll
-        for (int k = 0; k < SAP_RED_VALUES; k++) s.red[k * gridDim.x + blockIdx.x] = sh[k][0];
+    if (t < SAP_RED_VALUES) s.red[t * nb + b] = sh[t][0];
 }
-static __global__ void k_sap_axis_final(SapView s, int nblocks) {
-    if (threadIdx.x != 0) return;
-    double t[SAP_RED_VALUES] = {0, 0, 0, 0, 0, 0, 0};
-    for (int b = 0; b < nblocks; b++)
-        for (int k = 0; k < SAP_RED_VALUES; k++) t[k] += s.red[k * nblocks + b];
-    if (t[6] < 2.0) return;
+// The axis from the nb partial sums, by one wave (lane k adds up value k, in block order); returned by
+// every lane (-1: it stays).
+__device__ __forceinline__ int sap_axis_final(const SapView& s, int nb) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    double t = 0;
+    if (lane < SAP_RED_VALUES) {
+        const double* r = s.red + lane * nb;
+        int b = 0;
+        for (; b + 8 <= nb; b += 8) {   // eight loads in flight, added in order
+            double x[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) x[j] = r[b + j];
+#pragma unroll
+            for (int j = 0; j < 8; j++) t += x[j];
+        }
+        for (; b < nb; b++) t += r[b];
+    }
+    const double cnt = __shfl(t, 6, WAVE);
     double v[3];
-    for (int k = 0; k < 3; k++) v[k] = t[3 + k] - t[k] * t[k] / t[6];
+    for (int k = 0; k < 3; k++) {
+        const double m = __shfl(t, k, WAVE), q = __shfl(t, 3 + k, WAVE);
+        v[k] = q - m * m / cnt;
+    }
+    if (cnt < 2.0) return -1;
     int axis = 0;
     if (v[1] > v[0]) axis = 1;
     if (v[2] > v[axis]) axis = 2;
-    s.cnt->axis = axis;
+    return axis;
 }
 
-// Grid-wide exclusive scan of n elements (of *count when count is given; at most cap).
-inline void sap_scan(const SapView& s, uint32_t* data, int cap, int n, const uint32_t* count, uint32_t* total, hipStream_t st) {
-    const int nb = (cap + SCAN_TILE - 1) / SCAN_TILE < 1 ? 1 : (cap + SCAN_TILE - 1) / SCAN_TILE;
-    hipLaunchKernelGGL(k_scan_tiles, dim3(nb), dim3(1024), 0, st, data, n, count, s.scan_part);
-    hipLaunchKernelGGL(k_scan_u32, dim3(1), dim3(1024), 0, st, s.scan_part, nb, total);
-    hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(1024), 0, st, data, n, count, s.scan_part);
+// Stable sort by counting: a body's sorted position is the number of bodies with a smaller key, or an equal
+// one and a lower index.  SAP_RANK_BODIES bodies per workgroup, a lane each, the other keys split over its
+// waves: n^2 / 64 wave steps of about two instructions, spread over the whole GPU -- 10 000 bodies 9 us, in
+// one launch, where the radix sort's twelve take about 60 (each costs 4.5 us in a stream whatever it does).
+// Beyond SAP_RANK_MAX the square overtakes it.  The workgroups from nrank on make the axis's partial sums.
+constexpr int SAP_RANK_MAX = 16384;
+constexpr int SAP_RANK_BODIES = WAVE, SAP_RANK_THREADS = 512, SAP_RANK_TILE = 2048;
+static __global__ void __launch_bounds__(SAP_RANK_THREADS) k_sap_rank(SapView s, int nrank) {
+    __shared__ double sh[SAP_RED_VALUES][SAP_RED_THREADS];
+    if ((int)blockIdx.x >= nrank) {
+        sap_axis_partial(s, blockIdx.x - nrank, gridDim.x - nrank, sh);
+        return;
+    }
+    __shared__ __align__(16) uint32_t tile[SAP_RANK_TILE];
+    __shared__ int part[SAP_RANK_THREADS / WAVE][WAVE];
+    const int ax = s.ax(), n = s.n;
+    const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+    const int i0 = blockIdx.x * SAP_RANK_BODIES, i = i0 + lane;
+    if (blockIdx.x == 0 && threadIdx.x == 0) sap_begin(s);
+    const float key = i < n ? s.mn(ax, i) + 0.0f : 0.0f;
+    const uint32_t ki = float_key(key);
+    int count = 0;
+    for (int base = 0; base < n; base += SAP_RANK_TILE) {
+        const int m = min(SAP_RANK_TILE, n - base);
+        __syncthreads();
+        for (int j = threadIdx.x; j < m; j += SAP_RANK_THREADS) tile[j] = float_key(s.mn(ax, base + j) + 0.0f);
+        __syncthreads();
+        const int per = ((m + SAP_RANK_THREADS / WAVE - 1) / (SAP_RANK_THREADS / WAVE) + 3) & ~3;
+        const int j0 = min(m, w * per), j1 = min(m, j0 + per);
+        // before the workgroup's own bodies an equal key counts, after them it does not
+        const int own0 = min(max(i0 - base, j0), j1), own1 = min(max(i0 + SAP_RANK_BODIES - base, j0), j1);
+        auto run = [&](int a, int b, bool equal) {
+            int j = a;
+            for (; j < b && (j & 3); j++) count += equal ? tile[j] <= ki : tile[j] < ki;
+#pragma unroll 4
+            for (; j + 4 <= b; j += 4) {
+                const uint4 k = *reinterpret_cast<const uint4*>(&tile[j]);
+                if (equal) count += (k.x <= ki) + (k.y <= ki) + (k.z <= ki) + (k.w <= ki);
+                else count += (k.x < ki) + (k.y < ki) + (k.z < ki) + (k.w < ki);
+            }
+            for (; j < b; j++) count += equal ? tile[j] <= ki : tile[j] < ki;
+        };
+        run(j0, own0, true);
+        for (int j = own0; j < own1; j++) count += tile[j] < ki || (tile[j] == ki && base + j < i);
+        run(own1, j1, false);
+    }
+    part[w][lane] = count;
+    __syncthreads();
+    if (w != 0 || i >= n) return;
+    uint32_t q = 0;
+#pragma unroll
+    for (int k = 0; k < SAP_RANK_THREADS / WAVE; k++) q += (uint32_t)part[k][lane];
+    s.vals[q] = (uint32_t)i;
+    sap_sorted(s, q, i, key);
+}
+
+// The radix sort's keys; the workgroups from nkeys on make the axis's partial sums.
+static __global__ void __launch_bounds__(SAP_RED_THREADS) k_sap_keys(SapView s, int nkeys) {
+    __shared__ double sh[SAP_RED_VALUES][SAP_RED_THREADS];
+    if ((int)blockIdx.x >= nkeys) {
+        sap_axis_partial(s, blockIdx.x - nkeys, gridDim.x - nkeys, sh);
+        return;
+    }
+    const int ax = s.ax();
+    if (blockIdx.x == 0 && threadIdx.x == 0) sap_begin(s);
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < s.n; i += nkeys * blockDim.x) {
+        s.keys[i] = float_key(s.mn(ax, i) + 0.0f);
+        s.vals[i] = (uint32_t)i;
+    }
+}
+// After the radix sort: the sorted float keys and records.
+static __global__ void k_sap_gather(SapView s) {
+    const int ax = s.ax();
+    for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < s.n; q += gridDim.x * blockDim.x) {
+        const int i = (int)s.vals[q];
+        sap_sorted(s, q, i, s.mn(ax, i) + 0.0f);
+    }
+}
+
+// First sorted position in [lo, hi) whose key is above m, hi if none: the binary search, four of its levels a
+// step on 16 lanes (lane l of a group has node l of the levels' tree in heap order), so a run's end costs
+// a quarter of the dependent loads.  The same for the 16 lanes.
+__device__ __forceinline__ int sap_search(const float* skey, int lo, int hi, float m) {
+    const int l = threadIdx.x & 15;
+    while (__any(lo < hi)) {
+        int a = lo, b = hi;
+        const int depth = 31 - __clz(l | 1);
+        for (int k = depth - 1; k >= 0; k--) {
+            const int mid = (a + b) >> 1;
+            if (a < b) {
+                if ((l >> k) & 1) a = mid + 1; else b = mid;
+            }
+        }
+        const bool above = l > 0 && a < b && skey[(a + b) >> 1] > m;
+        const uint32_t g = (uint32_t)(__ballot(above) >> (threadIdx.x & 48)) & 0xffffu;
+        for (int k = 0, node = 1; k < 4; k++) {
+            if (lo >= hi) break;
+            const int mid = (lo + hi) >> 1;
+            if ((g >> node) & 1) { hi = mid; node = 2 * node; } else { lo = mid + 1; node = 2 * node + 1; }
+        }
+    }
+    return lo;
+}
+// Tests unit k of sorted body q (its run ends before `end`), a lane per candidate -- neighbouring lanes read
+// neighbouring records -- and leaves the outcomes in unit_hit[u]; the number of pairs.
+__device__ __forceinline__ int sap_test_unit(const SapView& s, uint32_t u, int q, int k, int end) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int j = q + 1 + k * SAP_UNIT + lane;
+    bool ok = false;
+    if (j < end) {
+        float A[8], B[8];
+        sap_ld_sorted(s, q, A);
+        sap_ld_sorted(s, j, B);
+        ok = sap_pair_allowed_sorted(s, A, B, q, j);
+    }
+    const uint64_t hit = __ballot(ok);
+    if (lane == 0) s.unit_hit[u] = hit;
+    return (int)__popcll(hit);
+}
+// The candidate runs of SAP_BLOCK sorted bodies (the reference's sweep breaks at the first key above a body's
+// maximum) and their units, numbered from a common counter.  FUSED: the workgroup tests them itself, which
+// saves a launch while the longest run (of a ground: every body) stays short; else k_sap_test spreads
+// all units over the GPU (10 000 boxes at rest: with every workgroup testing its own, the ground's run alone
+// took 40 us).
+constexpr int SAP_FUSED_MAX = 2048;
+template <bool FUSED>
+static __global__ void __launch_bounds__(SAP_THREADS) k_sap_runs(SapView s) {
+    __shared__ uint32_t s_len[SAP_BLOCK], s_unit[SAP_BLOCK + 1], s_base;
+    __shared__ int s_pairs;
+    const int n = s.n, q0 = blockIdx.x * SAP_BLOCK, nq = min(SAP_BLOCK, n - q0);
+    const int tid = threadIdx.x, r = tid >> 4, q = q0 + r;
+    const float m = r < nq ? s.srec[(size_t)q * 8 + 4 + s.ax()] : 0.0f;
+    const int end = sap_search(s.skey, r < nq ? q + 1 : n, n, m);
+    if ((tid & 15) == 0) s_len[r] = r < nq ? (uint32_t)(end - q - 1) : 0u;
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t run = 0, cand = 0;
+        for (int k = 0; k < SAP_BLOCK; k++) {
+            s_unit[k] = run;
+            run += (s_len[k] + SAP_UNIT - 1) / SAP_UNIT;
+            cand += s_len[k];
+        }
+        s_unit[SAP_BLOCK] = run;
+        s_base = atomicAdd(&s.cnt->nunits, run);
+        atomicAdd((unsigned long long*)&s.cnt->ncand, (unsigned long long)cand);
+        s_pairs = 0;
+    }
+    __syncthreads();
+    // the units beyond the workspace are dropped (an error that k_sap_emit reports)
+    const uint32_t slots = (uint32_t)sap_units(s.chunk_cap, n), base = s_base;
+    const uint32_t units = base >= slots ? 0u : min(s_unit[SAP_BLOCK], slots - base);
+    if (r < nq) {
+        if ((tid & 15) == 0) {
+            s.end[q] = (uint32_t)end;
+            s.first[q] = base + s_unit[r];
+        }
+        if (!FUSED)
+            for (uint32_t u = s_unit[r] + (tid & 15); u < s_unit[r + 1] && u < units; u += 16) s.owner[base + u] = (uint32_t)q;
+    }
+    if (FUSED) {
+        int pairs = 0, o = 0;   // o: the run of the wave's unit
+        for (uint32_t u = tid / WAVE; u < units; u += SAP_THREADS / WAVE) {
+            while (s_unit[o + 1] <= u) o++;
+            pairs += sap_test_unit(s, base + u, q0 + o, (int)(u - s_unit[o]), q0 + o + 1 + (int)s_len[o]);
+        }
+        if ((tid & (WAVE - 1)) == 0 && pairs) atomicAdd(&s_pairs, pairs);
+        __syncthreads();
+    }
+    if (tid == 0) s.blk[blockIdx.x] = make_uint2(units, (uint32_t)s_pairs);
+}
+static __global__ void __launch_bounds__(256) k_sap_test(SapView s) {
+    const uint32_t units = min(s.cnt->nunits, (uint32_t)sap_units(s.chunk_cap, s.n));
+    const uint32_t wave = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE, nw = gridDim.x * (blockDim.x / WAVE);
+    for (uint32_t u = wave; u < units; u += nw) {
+        const int q = (int)s.owner[u];
+        const int pairs = sap_test_unit(s, u, q, (int)(u - s.first[q]), (int)s.end[q]);
+        if ((threadIdx.x & (WAVE - 1)) == 0 && pairs) atomicAdd(&s.blk[q / SAP_BLOCK].y, (uint32_t)pairs);
+    }
+}
+
+// The pairs of a workgroup's bodies after those of the workgroups before it; the last workgroup knows all of
+// them and sets the counts and the next axis from its nred partial sums.
+static __global__ void __launch_bounds__(SAP_THREADS) k_sap_emit(SapView s, int nred) {
+    __shared__ uint32_t s_unit[SAP_BLOCK];
+    __shared__ int wsum[SAP_THREADS / WAVE + 1];
+    const int tid = threadIdx.x, q0 = blockIdx.x * SAP_BLOCK, nq = min(SAP_BLOCK, s.n - q0);
+    const uint2 me = s.blk[blockIdx.x];
+    const uint32_t base = s.first[q0];
+    int before = 0;
+    for (int b = tid; b < (int)blockIdx.x; b += SAP_THREADS) before += (int)s.blk[b].y;
+    if (tid < nq) s_unit[tid] = s.first[q0 + tid] - base;
+    int carry;
+    block_exclusive_scan(before, wsum, &carry);
+    if (blockIdx.x + 1 == gridDim.x && tid < WAVE) {
+        const int axis = sap_axis_final(s, nred);
+        if (tid == 0) {
+            const uint32_t total = (uint32_t)carry + me.y;
+            int32_t ovf = 0;
+            if (s.cnt->ncand > (uint64_t)s.chunk_cap * SAP_CHUNK) ovf |= OVF_CHUNKS;
+            if (total > (uint32_t)s.pcap) ovf |= OVF_PAIRS;
+            ovf |= s.cnt->overflow;
+            s.cnt->overflow = ovf;
+            s.cnt->nchunk_pairs = total;
+            s.cnt->npairs = total > (uint32_t)s.pcap ? s.pcap : (int32_t)total;
+            if (axis >= 0) s.cnt->axis = axis;
+            else if (s.axis_in >= 0) s.cnt->axis = s.axis_in;
+            if (s.result) {
+                s.result[0] = (int32_t)total;
+                s.result[1] = s.cnt->axis;
+                s.result[2] = ovf;
+            }
+        }
+    }
+    if (me.y == 0) return;
+    for (uint32_t u0 = 0; u0 < me.x; u0 += SAP_THREADS) {
+        const uint32_t u = u0 + tid;
+        uint64_t hit = u < me.x ? s.unit_hit[base + u] : 0ull;
+        int tot;
+        uint32_t out = (uint32_t)(carry + block_exclusive_scan((int)__popcll(hit), wsum, &tot));
+        carry += tot;
+        if (hit == 0) continue;
+        int r = 0;   // the last of the runs that start at or before this unit (empty runs share their starts)
+#pragma unroll
+        for (int k = 1; k < SAP_BLOCK; k++) r = k < nq && s_unit[k] <= u ? k : r;
+        const int a = (int)s.vals[q0 + r], j0 = q0 + r + 1 + (int)(u - s_unit[r]) * SAP_UNIT;
+        for (; hit; hit &= hit - 1, out++) {
+            if ((int)out >= s.pcap) break;
+            s.pa[out] = a;
+            s.pb[out] = (int)s.vals[j0 + __ffsll((unsigned long long)hit) - 1];
+        }
+    }
 }
 
 // The whole sweep on stream st (no host synchronisation): pairs to s.pa / s.pb, their count and
-// the next axis to s.cnt.  n >= 1.
+// the next axis to s.cnt (and s.result).  n >= 1.
 inline void sap_launch(const SapView& s, hipStream_t st) {
     const int n = s.n;
-    auto grid = [](int work, int block) { const int g = (work + block - 1) / block; return g < 1 ? 1 : (g > 4096 ? 4096 : g); };
-    const int rsb = sap_radix_blocks(n);
-    hipLaunchKernelGGL(k_sap_keys, dim3(grid(n, 256)), dim3(256), 0, st, s);
-    uint32_t *ki = s.keys, *vi = s.vals, *ko = s.keys2, *vo = s.vals2;
-    for (int pass = 0; pass < 4; pass++) {
-        hipLaunchKernelGGL(k_radix_hist, dim3(rsb), dim3(RS_THREADS), 0, st, ki, n, pass * 8, s.hist, rsb);
-        hipLaunchKernelGGL(k_scan_u32, dim3(1), dim3(1024), 0, st, s.hist, 256 * rsb, (uint32_t*)nullptr);
-        hipLaunchKernelGGL(k_radix_scatter, dim3(rsb), dim3(RS_THREADS), 0, st, ki, vi, ko, vo, n, pass * 8, s.hist, rsb);
-        uint32_t* t = ki; ki = ko; ko = t;
-        t = vi; vi = vo; vo = t;
+    const int nred = sap_red_blocks(n);
+    if (n <= SAP_RANK_MAX) {
+        const int nrank = (n + SAP_RANK_BODIES - 1) / SAP_RANK_BODIES;
+        hipLaunchKernelGGL(k_sap_rank, dim3(nrank + nred), dim3(SAP_RANK_THREADS), 0, st, s, nrank);
+    } else {
+        const int rsb = sap_radix_blocks(n), nk = (n + 255) / 256 > 4096 ? 4096 : (n + 255) / 256;
+        hipLaunchKernelGGL(k_sap_keys, dim3(nk + nred), dim3(SAP_RED_THREADS), 0, st, s, nk);
+        uint32_t *ki = s.keys, *vi = s.vals, *ko = s.keys2, *vo = s.vals2;
+        for (int pass = 0; pass < 4; pass++) {
+            hipLaunchKernelGGL(k_radix_hist, dim3(rsb), dim3(RS_THREADS), 0, st, ki, n, pass * 8, s.hist, rsb);
+            hipLaunchKernelGGL(k_scan_u32, dim3(1), dim3(1024), 0, st, s.hist, 256 * rsb, (uint32_t*)nullptr);
+            hipLaunchKernelGGL(k_radix_scatter, dim3(rsb), dim3(RS_THREADS), 0, st, ki, vi, ko, vo, n, pass * 8, s.hist, rsb);
+            uint32_t* t = ki; ki = ko; ko = t;
+            t = vi; vi = vo; vo = t;
+        }
+        // after 4 passes the sorted data is back in keys / vals
+        hipLaunchKernelGGL(k_sap_gather, dim3(nk), dim3(256), 0, st, s);
     }
-    // after 4 passes the sorted data is back in keys / vals
-    hipLaunchKernelGGL(k_sap_ranges, dim3(grid(n, 256)), dim3(256), 0, st, s);
-    hipLaunchKernelGGL(k_sap_cand, dim3(grid(n, 256)), dim3(256), 0, st, s);
-    sap_scan(s, s.cand, n + 1, n + 1, nullptr, &s.cnt->ncand, st);
-    hipLaunchKernelGGL(k_sap_nchunks, dim3(1), dim3(1), 0, st, s);
-    hipLaunchKernelGGL(k_sap_chunks<false>, dim3(2048), dim3(256), 0, st, s);
-    sap_scan(s, s.chunk, s.chunk_cap, 0, &s.cnt->nchunks, &s.cnt->nchunk_pairs, st);
-    hipLaunchKernelGGL(k_sap_chunks<true>, dim3(2048), dim3(256), 0, st, s);
-    hipLaunchKernelGGL(k_sap_finish, dim3(1), dim3(1), 0, st, s);
-    const int rb = sap_red_blocks(n);
-    hipLaunchKernelGGL(k_sap_axis_partial, dim3(rb), dim3(SAP_RED_THREADS), 0, st, s);
-    hipLaunchKernelGGL(k_sap_axis_final, dim3(1), dim3(64), 0, st, s, rb);
+    if (n <= SAP_FUSED_MAX) {
+        hipLaunchKernelGGL(k_sap_runs<true>, dim3(sap_blocks(n)), dim3(SAP_THREADS), 0, st, s);
+    } else {
+        hipLaunchKernelGGL(k_sap_runs<false>, dim3(sap_blocks(n)), dim3(SAP_THREADS), 0, st, s);
+        hipLaunchKernelGGL(k_sap_test, dim3(2048), dim3(256), 0, st, s);
+    }
+    hipLaunchKernelGGL(k_sap_emit, dim3(sap_blocks(n)), dim3(SAP_THREADS), 0, st, s, nred);
 }
 
 }  // namespace pe

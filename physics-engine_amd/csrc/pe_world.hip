@@ -7,7 +7,7 @@
 //                      reference's (i, j) order, next axis
 //   k_narrow           thread / pair: shape dispatch + 8-slot contact cache + depth sort
 //   k_setup            thread / pair: solver rows (FrictionContactConstraint::initSequentialImpulse)
-//   k_solve_small      worlds of up to 1024 bodies: colouring and sweeps in one workgroup, on LDS; else
+//   k_solve_small      worlds of up to 600 bodies: colouring and sweeps in one workgroup, on LDS; else
 //   k_jp_*             the constraint graph: per body its pairs
 //   k_solve_flow       cooperative launch over the whole GPU: colouring, then the Gauss-Seidel sweeps in
 //                      colour order as a data flow between the pairs, and the velocity sync
@@ -1298,8 +1298,10 @@ __global__ void __launch_bounds__(256) k_count_points(Dev d) {
 // two pairs with contacts per body, 16 to an item), at most one workgroup per CU of the 256.
 static int default_flow_blocks(int n, int max_blocks) { return std::min(max_blocks, std::max(8, std::min(256, n / 80))); }
 
-// Bodies up to which the solve runs in one workgroup (k_solve_small).
-constexpr int SMALL_BODIES = 1024;
+// Bodies up to which the solve runs in one workgroup (k_solve_small).  At rest, us per step in one workgroup /
+// over the GPU: boxes 250 bodies 248 / 322, 500 370 / 376, 750 440 / 396, 1 000 560 / 440; boxes and
+// spheres 250 230 / 290, 500 325 / 366, 750 390 / 372, 1 000 474 / 413.
+constexpr int SMALL_BODIES = 600;
 
 struct pe_world {
     Dev d{};
@@ -1522,18 +1524,20 @@ int pe_world_create(const pe_scene_desc* sc, const pe_world_params* prm, int32_t
     rc |= w->alloc(&sp.vals2, n);
     rc |= w->alloc(&sp.skey, n);
     rc |= w->alloc(&sp.srec, (size_t)8 * n);
-    rc |= w->alloc(&sp.cand, n + 1);
+    rc |= w->alloc(&sp.end, n);
+    rc |= w->alloc(&sp.first, n);
+    rc |= w->alloc(&sp.blk, sap_blocks(n));
+    sp.axis_in = -1;
     rc |= w->alloc(&sp.hist, 256 * (size_t)sap_radix_blocks(n));
     rc |= w->alloc(&sp.red, SAP_RED_VALUES * (size_t)sap_red_blocks(n));
     // sweep chunks: the candidates (bodies overlapping on the sweep axis) are at most n (n - 1) / 2,
     // and a pile that lands while the axis is still the fall direction comes close to that (the
-    // reference's sweep too: the axis is chosen after the sweep); 8 bytes per 32 candidates, so the
-    // bound itself is allocated, up to 2^31 candidates (the counters are 32-bit)
+    // reference's sweep too: the axis is chosen after the sweep); 12 bytes per 64 candidates, so the
+    // bound itself is allocated, up to 2^31 candidates
     const int64_t max_cand = std::min<int64_t>((int64_t)n * (n - 1) / 2, (int64_t)1 << 31);
     sp.chunk_cap = (int)std::max<int64_t>(max_cand / SAP_CHUNK + 1, 1024);
-    rc |= w->alloc(&sp.chunk, sp.chunk_cap);
-    rc |= w->alloc(&sp.chunk_hit, sp.chunk_cap);
-    rc |= w->alloc(&sp.scan_part, sap_scan_parts(n, sp.chunk_cap));
+    rc |= w->alloc(&sp.owner, sap_units(sp.chunk_cap, n));
+    rc |= w->alloc(&sp.unit_hit, sap_units(sp.chunk_cap, n));
     if (rc != PE_OK) return fail(PE_ERR_DEVICE);
 
     // host staging of the body store (FP32) and of the scene's meshes
@@ -2226,20 +2230,16 @@ __global__ void k_stage_impulses_out(Dev d, int np, float* __restrict__ imp) {
                 imp[((size_t)p * 8 + k) * 3 + q] = k < m ? d.ps.rows[((size_t)p * 8 + k) * RW + R_LN + q] : 0.0f;
     }
 }
-// result[0] = pairs the sweep found (more than the capacity when it overflowed), result[1] = the
-// next axis, result[2] = capacity-error bits.
-__global__ void k_stage_sap_result(SapView s, int32_t* result) {
-    result[0] = (int32_t)s.cnt->nchunk_pairs;
-    result[1] = s.cnt->axis;
-    result[2] = s.cnt->overflow;
-}
 __global__ void k_stage_result(Dev d, int32_t* result, int which) {
     result[0] = which == 0 ? d.cnt->overflow : d.cnt->ncolors;
     if (which == 1) result[1] = d.cnt->overflow;
 }
 
 // A sweep over a caller's AABB records ([n][8]) with the given working memory and pair outputs.
-SapView sap_over_records(const SapView& work, int n, const float* aabb, int32_t* pa, int32_t* pb, int cap) {
+// result[0] = pairs found (more than the capacity when it overflowed), result[1] = the next axis, result[2] =
+// capacity-error bits.
+SapView sap_over_records(const SapView& work, int n, const float* aabb, int axis, int32_t* pa, int32_t* pb, int cap,
+                         int32_t* result) {
     SapView s = work;
     s.n = n;
     s.amin = aabb;
@@ -2250,6 +2250,8 @@ SapView sap_over_records(const SapView& work, int n, const float* aabb, int32_t*
     s.pa = pa;
     s.pb = pb;
     s.pcap = cap;
+    s.axis_in = axis;
+    s.result = result;
     return s;
 }
 
@@ -2326,10 +2328,9 @@ int pe_stage_broadphase(pe_stage* s, int32_t n, const float* aabb, int32_t axis,
     }
     pe_clear_stale_error();
     hipStream_t st = (hipStream_t)stream;
-    const SapView v = sap_over_records(s->w->d.sap, n, aabb, pair_a, pair_b, cap);
-    hipLaunchKernelGGL(k_sap_begin, dim3(1), dim3(1), 0, st, v, (int)axis);
+    const SapView v = sap_over_records(s->w->d.sap, n, aabb, axis, pair_a, pair_b, cap, result);
     if (n >= 2) sap_launch(v, st);   // fewer than 2 bodies: no pairs, the axis stays (broad_phase_sweep_and_prune.cpp:8)
-    hipLaunchKernelGGL(k_stage_sap_result, dim3(1), dim3(1), 0, st, v, result);
+    else hipLaunchKernelGGL(k_sap_none, dim3(1), dim3(1), 0, st, v);
     PE_HIP(hipGetLastError());
     return PE_OK;
 }

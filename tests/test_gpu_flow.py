@@ -1,7 +1,7 @@
 """The single world's solve: over the GPU (colouring and data-flow sweeps) where its paths change: more
 items than waves and an item per wave, bodies whose pairs exceed what a thread keeps (32), what a workgroup
 counts in LDS (64 colours) and the colour starts kept there (1024), joints beside contacts; in one
-workgroup (up to 1024 bodies) with its rows in LDS, in memory, and where pairs or colours outgrow it.  Colour classes
+workgroup (up to 600 bodies) with its rows in LDS, in memory, and where pairs or colours outgrow it.  Colour classes
 equal the oracle's; velocities and impulses are the oracle's colour-order solve's within the 1e-5 the
 other solver tests use (both sides round the same operations; the contact points differ by an ulp of
 atan2f at most)."""
@@ -107,12 +107,12 @@ def test_one_workgroup_equals_the_flow(name):
     import pe_amd
     from pe_amd import scenes
     sc, steps = {"pair": lambda: (scenes.grid_world(1, seed=2), 70),
-                 "mixed": lambda: (scenes.grid_world(700, seed=5), 90),
-                 "boxes": lambda: (scenes.grid_world(900, seed=6, p_sphere=0.0), 100),
-                 "limit": lambda: (scenes.grid_world(1023, seed=7, p_sphere=0.2), 80),
+                 "mixed": lambda: (scenes.grid_world(350, seed=5), 90),
+                 "boxes": lambda: (scenes.grid_world(560, seed=6, p_sphere=0.0), 100),
+                 "limit": lambda: (scenes.grid_world(599, seed=7, p_sphere=0.2), 80),
                  "chains": lambda: (scenes.joint_chain_scene(30, 9, seed=3), 60),
                  "joint_demo": lambda: (scenes.joint_demo_scene(), 60),
-                 "cluster": lambda: (cluster_scene(800, 3.2), 1)}[name]()
+                 "cluster": lambda: (cluster_scene(590, 2.6), 1)}[name]()
     a, b = pe_amd.World(sc, max_pairs=200 * sc.n), pe_amd.World(sc, max_pairs=200 * sc.n)
     b.set_colouring(2)
     print(f"[one workgroup] {name}: {sc.n} bodies", flush=True)
