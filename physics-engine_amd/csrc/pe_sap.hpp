@@ -36,6 +36,9 @@ struct DevCounts {          // device-side counters of one step
     int32_t nact;           // pairs the solve orders (contact points, not both bodies kinematic)
     int32_t jp_ncol;        // colours the last sweep over the GPU counted
     uint32_t adj_total;     // colouring: adjacency entries
+    uint32_t fl_arrive;     // solve over the GPU: workgroups that have started,
+    uint32_t fl_state;      // whether all have in time (FLOW_*),
+    uint32_t fl_exit;       // and workgroups that left when not
     int32_t jp_big;         // some body is in more pairs than the colouring over the GPU takes
     int32_t jp_rounds;      // colouring over the GPU: the most times a thread tried its pairs
 };

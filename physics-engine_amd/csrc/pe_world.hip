@@ -348,6 +348,9 @@ __global__ void k_solve_begin(Dev d) {
         d.cnt->adj_total = 0;
         d.cnt->jp_rounds = 0;
         d.cnt->jp_big = 0;
+        d.cnt->fl_arrive = 0;
+        d.cnt->fl_state = 0;
+        d.cnt->fl_exit = 0;
     }
 }
 
@@ -409,8 +412,7 @@ __global__ void k_joint_setup(Dev d) {
         joint_setup(d.b, d.joints[k], d.jrows[k], d.dt);
 }
 
-// Sense-reversing barrier over all workgroups of a cooperative launch (every workgroup is
-// resident, so every wait ends).  The last arrival resets the count and bumps the generation.
+// Sense-reversing barrier over all workgroups of a launch that are on the GPU together (every wait ends).  The last arrival resets the count and bumps the generation.
 // It also orders memory across the grid: the workgroup's writes before the barrier are visible to
 // every workgroup after it.  One thread per workgroup fences (a release fence before arriving, an
 // acquire fence after the wait: the workgroup barriers around them carry the ordering to its other
@@ -550,7 +552,7 @@ __device__ __forceinline__ int jp_rank(const Dev& d, int x, int p, int c) {
 }
 
 // Colouring and Gauss-Seidel sweeps (SequentialImpulseSolver::solve, sequential_impulse_solver.cpp:60-81)
-// over the whole GPU in one cooperative launch (every workgroup resident, so every wait ends).
+// over the whole GPU in one launch whose workgroups run at the same time (flow_together), so every wait ends.
 //
 // The sweeps run as a data flow instead of colour by colour between grid barriers.  The colour order fixes
 // for every body the sequence of the pairs (then joints) that update it in an iteration, so a pair only
@@ -745,14 +747,100 @@ __device__ __forceinline__ bool flow_joints(const Dev& d, int j0, int nl) {
     return true;
 }
 
+// The whole solve by one workgroup of FLOW_THREADS on the records in global memory, a pair per thread, the claims in
+// LDS or (n bodies, any n) in memory: where a small world's pairs or colours outgrow its workgroup's
+// LDS, and where the workgroups of k_solve_flow could not all be had at once.
+template <bool LDS_CLAIM>
+__device__ void solve_alone(const Dev& d, int nact, int* claim) {
+    __shared__ int wsum[FLOW_THREADS / WAVE + 1];
+    const int tid = threadIdx.x;
+    for (int i = tid; i < d.b.n; i += FLOW_THREADS) claim_set<LDS_CLAIM>(claim, i, colour::FREE);
+    claim_sync<LDS_CLAIM>();
+    int* bufs[3] = {d.act, d.act + d.pcap, d.act + 2 * (size_t)d.pcap};
+    const int ncol = colour_pairs<LDS_CLAIM>(d.b, d.ps, bufs, nact, d.order, d.color_start, claim, 0, 0, wsum);
+    if (tid == 0) {
+        d.cnt->ncolors = ncol;
+        d.cnt->nordered = d.color_start[ncol];
+        d.cnt->jp_rounds = 0;
+    }
+    for (int it = 0; it < d.iterations; it++) {
+        for (int c = 0; c < ncol; c++) {
+            for (int q = d.color_start[c] + tid; q < d.color_start[c + 1]; q += FLOW_THREADS) iterate_pair(d.b, d.ps, d.order[q]);
+            __syncthreads();
+        }
+        // the joints after the contacts, colour by colour (sequential_impulse_solver.cpp:66-68)
+        for (int c = 0; c < d.njcol; c++) {
+            for (int q = d.jcs[c] + tid; q < d.jcs[c + 1]; q += FLOW_THREADS) {
+                const int k = d.jorder[q];
+                const JointDef j = d.joints[k];
+                SolvBody A = load_solv(d.b, j.a), B = load_solv(d.b, j.b);
+                joint_solve(j, d.jrows[k], A, B);
+                for (int s = 0; s < 2; s++) {
+                    const SolvBody& S = s == 0 ? A : B;
+                    if (S.kin) continue;
+                    float* o = d.b.sbr(s == 0 ? j.a : j.b);
+                    o[SB_TV] = S.tv.x; o[SB_TV + 1] = S.tv.y; o[SB_TV + 2] = S.tv.z;
+                    o[SB_TW] = S.tw.x; o[SB_TW + 1] = S.tw.y; o[SB_TW + 2] = S.tw.z;
+                }
+            }
+            __syncthreads();
+        }
+    }
+    for (int i = tid; i < d.b.n; i += FLOW_THREADS) {
+        if (d.b.iat(I_KIN, i)) continue;
+        const float* o = d.b.sbr(i);
+        st3(d.b, F_V, i, f3{o[SB_TV], o[SB_TV + 1], o[SB_TV + 2]});
+        st3(d.b, F_W, i, f3{o[SB_TW], o[SB_TW + 1], o[SB_TW + 2]});
+    }
+}
+
+// Whether all workgroups of the launch are on the GPU at once, which their waits on each other need.  The launch is
+// an ordinary one (a cooperative one changes queues: 28 us a step, and with several worlds' streams up to
+// 170), its grid no more than the GPU holds; but other launches may hold the GPU at the time.  The
+// last workgroup to start says so to the others; one that has waited `patience` (ticks of 10 ns) calls the
+// launch off instead, and whichever comes first holds for all.  Called off, the workgroups leave
+// as they come, nothing done, and the last of them, now alone, solves by itself.
+constexpr uint32_t FLOW_GO = 1, FLOW_OFF = 2;
+__device__ __forceinline__ bool flow_together(const Dev& d, uint64_t patience, int* alone) {
+    __shared__ uint32_t s_state;
+    if (threadIdx.x == 0) {
+        DevCounts* c = d.cnt;
+        uint32_t st = 0;
+        if (__hip_atomic_fetch_add(&c->fl_arrive, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
+            uint32_t none = 0;
+            __hip_atomic_compare_exchange_strong(&c->fl_state, &none, FLOW_GO, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+        }
+        const uint64_t t0 = wall_clock64();
+        while ((st = __hip_atomic_load(&c->fl_state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0) {
+            if (wall_clock64() - t0 >= patience) {
+                uint32_t none = 0;
+                __hip_atomic_compare_exchange_strong(&c->fl_state, &none, FLOW_OFF, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT);
+            } else {
+                __builtin_amdgcn_s_sleep(1);
+            }
+        }
+        s_state = st;
+        if (st == FLOW_OFF)
+            *alone = __hip_atomic_fetch_add(&c->fl_exit, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    }
+    __syncthreads();
+    return s_state == FLOW_GO;
+}
+
 // claims: the colouring runs in workgroup 0 (colour_pairs), as it does where a body is in more than
 // JP_MAX_DEG pairs.
-__global__ void __launch_bounds__(FLOW_THREADS) k_solve_flow(Dev d, int claims) {
+__global__ void __launch_bounds__(FLOW_THREADS) k_solve_flow(Dev d, int claims, uint64_t patience) {
     __shared__ int s_cs[FLOW_COLORS + 1], s_is[FLOW_COLORS + 1], s_ncol;
     __shared__ int s_hist[FLOW_BINS];
     __shared__ int s_low[FLOW_THREADS][JP_KEEP + 1];   // rows of odd length: distinct banks
     const int nact = d.cnt->nact;
     const int tid = threadIdx.x, gtid = blockIdx.x * blockDim.x + tid, gsz = gridDim.x * blockDim.x;
+    if (!flow_together(d, patience, &s_ncol)) {
+        if (s_ncol) solve_alone<false>(d, nact, d.claim);
+        return;
+    }
     if (tid < FLOW_BINS) s_hist[tid] = 0;
     auto stalled = [&]() { atomicOr(&d.cnt->overflow, OVF_STALL); };
     const bool coloured = claims || d.cnt->jp_big;   // the same for every workgroup
@@ -989,52 +1077,11 @@ __global__ void __launch_bounds__(FLOW_THREADS) k_solve_flow(Dev d, int claims) 
 // be seen on another CU, and none of the cooperative launch's queue switches (about 25 us a step).  Four
 // lanes per pair as there (quad_solve_row): a colour of up to SMALL_THREADS / 4 pairs is one pass as long as
 // its longest pair's row chains; a larger one takes several, which is where the flow becomes faster.
-constexpr int SMALL_THREADS = 512;
+constexpr int SMALL_THREADS = FLOW_THREADS;
 constexpr int SMALL_LDS = 152 * 1024;
 constexpr int SMALL_COLORS = 128;   // colours counted in LDS (two 64-bit masks per body)
 constexpr int SMALL_ROW = RW + 1;   // a row's floats in LDS: an odd stride spreads the quads' rows over the banks
 
-// The same on the records in global memory, pairs on a thread each: where the pairs outgrow LDS or the masks.
-__device__ void small_global(const Dev& d, int nact, int* claim) {
-    __shared__ int wsum[SMALL_THREADS / WAVE + 1];
-    const int tid = threadIdx.x;
-    for (int i = tid; i < d.b.n; i += SMALL_THREADS) claim[i] = colour::FREE;
-    __syncthreads();
-    int* bufs[3] = {d.act, d.act + d.pcap, d.act + 2 * (size_t)d.pcap};
-    const int ncol = colour_pairs<true>(d.b, d.ps, bufs, nact, d.order, d.color_start, claim, 0, 0, wsum);
-    if (tid == 0) {
-        d.cnt->ncolors = ncol;
-        d.cnt->nordered = d.color_start[ncol];
-    }
-    for (int it = 0; it < d.iterations; it++) {
-        for (int c = 0; c < ncol; c++) {
-            for (int q = d.color_start[c] + tid; q < d.color_start[c + 1]; q += SMALL_THREADS) iterate_pair(d.b, d.ps, d.order[q]);
-            __syncthreads();
-        }
-        for (int c = 0; c < d.njcol; c++) {
-            for (int q = d.jcs[c] + tid; q < d.jcs[c + 1]; q += SMALL_THREADS) {
-                const int k = d.jorder[q];
-                const JointDef j = d.joints[k];
-                SolvBody A = load_solv(d.b, j.a), B = load_solv(d.b, j.b);
-                joint_solve(j, d.jrows[k], A, B);
-                for (int s = 0; s < 2; s++) {
-                    const SolvBody& S = s == 0 ? A : B;
-                    if (S.kin) continue;
-                    float* o = d.b.sbr(s == 0 ? j.a : j.b);
-                    o[SB_TV] = S.tv.x; o[SB_TV + 1] = S.tv.y; o[SB_TV + 2] = S.tv.z;
-                    o[SB_TW] = S.tw.x; o[SB_TW + 1] = S.tw.y; o[SB_TW + 2] = S.tw.z;
-                }
-            }
-            __syncthreads();
-        }
-    }
-    for (int i = tid; i < d.b.n; i += SMALL_THREADS) {
-        if (d.b.iat(I_KIN, i)) continue;
-        const float* o = d.b.sbr(i);
-        st3(d.b, F_V, i, f3{o[SB_TV], o[SB_TV + 1], o[SB_TV + 2]});
-        st3(d.b, F_W, i, f3{o[SB_TW], o[SB_TW + 1], o[SB_TW + 2]});
-    }
-}
 // The sweeps on LDS velocities vel ([n][8]: linear from 0, angular from 4) over the ordered pairs info (pair,
 // bodies A and B with the kinematic flag on top, rows | first row in rows << 4); ROWS_LDS: the rows are in
 // rows, else in the row store.
@@ -1199,7 +1246,7 @@ __global__ void __launch_bounds__(SMALL_THREADS) k_solve_small(Dev d) {
         __syncthreads();
     }
     if (!small) {   // the same for every thread
-        small_global(d, nact, (int*)lds);
+        solve_alone<true>(d, nact, (int*)lds);
         if (tid == 0) d.cnt->nact = 0;
         return;
     }
@@ -1298,6 +1345,34 @@ __global__ void __launch_bounds__(256) k_count_points(Dev d) {
 // two pairs with contacts per body, 16 to an item), at most one workgroup per CU of the 256.
 static int default_flow_blocks(int n, int max_blocks) { return std::min(max_blocks, std::max(8, std::min(256, n / 80))); }
 
+struct pe_world;
+namespace {
+// Turns at k_solve_flow between this process's worlds on one GPU.  As long as all of them fit on it at once
+// nothing is done; else each launch waits for the one before it (on another stream), so that two of them
+// never share the GPU with neither complete.
+struct FlowTurns {
+    std::mutex m;
+    int blocks = 0;              // workgroups of all live worlds
+    hipEvent_t last = nullptr;   // after the last launch (kept for the process)
+    hipStream_t stream = nullptr;
+};
+FlowTurns& flow_turns() {
+    static FlowTurns t[64];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+    return t[dev];
+}
+struct FlowTurn {
+    explicit FlowTurn(pe_world& w);
+    int done();
+    pe_world& w;
+    FlowTurns& t;
+    std::unique_lock<std::mutex> lock;
+    bool crowded;
+    hipError_t err = hipSuccess;
+};
+}  // namespace
+
 // Bodies up to which the solve runs in one workgroup (k_solve_small).  At rest, us per step in one workgroup /
 // over the GPU: boxes 250 bodies 248 / 322, 500 370 / 376, 750 440 / 396, 1 000 560 / 440; boxes and
 // spheres 250 230 / 290, 500 325 / 366, 750 390 / 372, 1 000 474 / 413.
@@ -1308,8 +1383,16 @@ struct pe_world {
     int n = 0, stride = 0;
     hipStream_t stream = nullptr;
     std::vector<void*> allocs;
-    int flow_blocks = 0;    // workgroups of the cooperative solve
-    int flow_max_blocks = 0;                 // and the co-resident limit
+    int flow_blocks = 0;    // workgroups of the solve over the GPU
+    int flow_max_blocks = 0;                 // and how many of them the GPU holds at once
+    uint64_t flow_patience = 5000000;        // 50 ms
+    int flow_counted = 0;                    // workgroups entered in flow_turns()
+    void count_flow(int blocks) {
+        FlowTurns& t = flow_turns();
+        std::lock_guard<std::mutex> g(t.m);
+        t.blocks += blocks - flow_counted;
+        flow_counted = blocks;
+    }
     int colouring = 0;                       // 0: by body count, 1: one workgroup's claims, 2: over the GPU
     bool timing = false;
     hipEvent_t ev[5] = {};
@@ -1329,6 +1412,7 @@ struct pe_world {
 
     ~pe_world() {
         if (stream) hipStreamSynchronize(stream);
+        count_flow(0);
         for (void* p : allocs) hipFree(p);
         for (void* p : joint_mem) if (p) hipFree(p);
         if (ignore_mem) hipFree(ignore_mem);
@@ -1383,9 +1467,9 @@ struct pe_world {
         hipLaunchKernelGGL(k_jp_alloc, dim3(grid(n, 256)), dim3(256), 0, stream, d);
         hipLaunchKernelGGL(k_jp_fill, dim3(grid(d.pcap, 256)), dim3(256), 0, stream, d);
         int claims = colouring == 1;
-        void* args[] = {(void*)&d, (void*)&claims};
-        PE_HIP(hipLaunchCooperativeKernel((const void*)k_solve_flow, dim3(flow_blocks), dim3(FLOW_THREADS), args, 0, stream));
-        return PE_OK;
+        FlowTurn turn(*this);
+        hipLaunchKernelGGL(k_solve_flow, dim3(flow_blocks), dim3(FLOW_THREADS), 0, stream, d, claims, flow_patience);
+        return turn.done();
     }
     int step() {
         pe_clear_stale_error();
@@ -1412,6 +1496,26 @@ struct pe_world {
 };
 
 namespace {
+FlowTurn::FlowTurn(pe_world& w_) : w(w_), t(flow_turns()), lock(t.m), crowded(t.blocks > w_.flow_max_blocks) {
+    if (crowded) {   // a stream under capture takes no part: what it waits for then is not this launch's time
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        crowded = hipStreamIsCapturing(w.stream, &st) != hipSuccess || st == hipStreamCaptureStatusNone;
+    }
+    if (!crowded) {
+        lock.unlock();
+        return;
+    }
+    if (!t.last) err = hipEventCreateWithFlags(&t.last, hipEventDisableTiming);
+    else if (t.stream != w.stream) err = hipStreamWaitEvent(w.stream, t.last, 0);
+}
+int FlowTurn::done() {
+    if (crowded && err == hipSuccess) {
+        err = hipEventRecord(t.last, w.stream);
+        t.stream = w.stream;
+    }
+    PE_HIP(err);
+    return PE_OK;
+}
 int check_world(pe_world* w) {
     if (!w) { pe_set_error("null world"); return PE_ERR_INVALID; }
     return PE_OK;
@@ -1593,6 +1697,7 @@ int pe_world_create(const pe_scene_desc* sc, const pe_world_params* prm, int32_t
         }
         w->flow_max_blocks = cus * per_cu;
         w->flow_blocks = default_flow_blocks(n, w->flow_max_blocks);
+        w->count_flow(n > SMALL_BODIES ? w->flow_blocks : 0);
         if (w->alloc(&d.jp_hist, (size_t)FLOW_BINS * w->flow_max_blocks) != PE_OK) return fail(PE_ERR_DEVICE);
     }
     if (hipStreamSynchronize(w->stream) != hipSuccess) { pe_set_error("init sync failed"); return fail(PE_ERR_DEVICE); }
@@ -2083,6 +2188,7 @@ int pe_world_set_solver_blocks(pe_world* w, int32_t blocks) {
     if (int rc = check_world(w)) return rc;
     if (blocks < 0) { pe_set_error("blocks must be >= 0"); return PE_ERR_INVALID; }
     w->flow_blocks = blocks == 0 ? default_flow_blocks(w->n, w->flow_max_blocks) : std::min(blocks, w->flow_max_blocks);
+    w->count_flow(w->n > SMALL_BODIES || w->colouring != 0 ? w->flow_blocks : 0);
     return PE_OK;
 }
 
@@ -2093,7 +2199,15 @@ int pe_world_set_colouring(pe_world* w, int32_t mode) {
         return PE_ERR_INVALID;
     }
     w->colouring = mode;
+    w->count_flow(w->n > SMALL_BODIES || mode != 0 ? w->flow_blocks : 0);
     PE_HIP(hipMemsetAsync(&w->d.cnt->nact, 0, sizeof(int32_t), w->stream));   // as the one-workgroup solve leaves it
+    return PE_OK;
+}
+
+// For the tests: how long (ticks of 10 ns) the workgroups of the solve over the GPU wait for each other to start.
+int pe_internal_set_flow_patience(pe_world* w, int64_t ticks) {
+    if (int rc = check_world(w)) return rc;
+    w->flow_patience = (uint64_t)std::max<int64_t>(ticks, 0);
     return PE_OK;
 }
 

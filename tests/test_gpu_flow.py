@@ -133,3 +133,53 @@ def test_one_workgroup_equals_the_flow(name):
             assert len(oa) * 28 + sc.n * 56 > 152 * 1024   # beyond the LDS the kernel works in
     a.close()
     b.close()
+
+
+def test_launch_called_off_solves_the_same():
+    """Workgroups that do not wait for each other call the solve over the GPU off, and the last of them solves
+    alone (any world whose workgroups could not be had at once): the same bits, also with more workgroups
+    than the GPU holds beside other worlds' and with joints."""
+    import ctypes
+    import pe_amd
+    from pe_amd import scenes
+    from pe_amd._lib import check, lib
+    for sc, steps in ((scenes.grid_world(900, seed=5, p_sphere=0.3), 90), (scenes.joint_chain_scene(80, 9, seed=3), 60)):
+        a, b = pe_amd.World(sc), pe_amd.World(sc)
+        b.set_solver_blocks(200)
+        check(lib().pe_internal_set_flow_patience(b.h, ctypes.c_int64(0)))
+        print(f"[called off] {sc.name}", flush=True)
+        a.step(steps)
+        b.step(steps)
+        b.sync()
+        for x, y in zip(a.state(), b.state()):
+            assert np.array_equal(x.view(np.int32), y.view(np.int32))
+        assert np.array_equal(a.impulses(), b.impulses())
+        a.close()
+        b.close()
+
+
+def test_worlds_on_their_own_streams_and_threads():
+    """More worlds than the GPU holds solves over it at once, stepped from several threads on their own streams:
+    each as it is alone."""
+    import threading
+    import pe_amd
+    from pe_amd import scenes
+    sc = scenes.grid_world(900, seed=15, p_sphere=0.3)
+    ref = pe_amd.World(sc)
+    ref.step(80)
+    want = ref.state()
+    ws = [pe_amd.World(sc) for _ in range(6)]
+    for w in ws:
+        w.set_solver_blocks(256)
+    print("[threads] 6 worlds", flush=True)
+    ts = [threading.Thread(target=lambda w=w: [w.step(20) for _ in range(4)]) for w in ws]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for w in ws:
+        w.sync()
+        for x, y in zip(w.state(), want):
+            assert np.array_equal(x.view(np.int32), y.view(np.int32))
+        w.close()
+    ref.close()
