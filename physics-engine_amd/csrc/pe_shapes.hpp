@@ -257,6 +257,50 @@ PE_HD void project_verts(const float4* v, int nv, const Pose& t, f3 axis, float&
     mn += off; mx += off;
     pmn = xf_apply(t, lmn); pmx = xf_apply(t, lmx);
 }
+// project without its witness points: the interval alone.
+PE_HD void project_interval(const Poly& S, const Pose& t, f3 axis, float& mn, float& mx) {
+    const f3 la = mtv(t.R, axis);
+    const float off = dot(t.p, axis);
+    if (S.kind == PK_BOX) {
+        const f3 ext{la.x > 0 ? S.h.x : -S.h.x, la.y > 0 ? S.h.y : -S.h.y, la.z > 0 ? S.h.z : -S.h.z};
+        const float he = dot(ext, la);
+        mn = off - he; mx = off + he;
+    } else if (S.kind == PK_CYL) {
+        const float rad = S.h.x, hh = S.h.y;
+        float el;
+        if (fabsf(la.x - 0.0f) < EPS && fabsf(la.z - 0.0f) < EPS) {
+            el = hh;
+        } else if (fabsf(la.y - 0.0f) < EPS) {
+            el = rad;
+        } else {
+            const float r = sqrtf(la.x * la.x + la.z * la.z);
+            el = dot(f3{rad * la.x / r, hh * (la.y > 0 ? 1.0f : -1.0f), rad * la.z / r}, la);
+        }
+        mn = off - el; mx = off + el;
+    } else {
+        mn = REAL_MAX; mx = REAL_MIN;
+        const int nv = S.kind == PK_MESH ? S.nv : 3;
+        for (int i = 0; i < nv; i++) {
+            const float x = dot(S.kind == PK_MESH ? ld4(S.v[i]) : S.t[i], la);
+            const bool lt = x < mn;
+            mn = lt ? x : mn;
+            mx = !lt && x > mx ? x : mx;
+        }
+        mn += off; mx += off;
+    }
+}
+PE_HD void project_verts_interval(const float4* v, int nv, const Pose& t, f3 axis, float& mn, float& mx) {
+    const f3 la = mtv(t.R, axis);
+    const float off = dot(t.p, axis);
+    mn = REAL_MAX; mx = REAL_MIN;
+    for (int i = 0; i < nv; i++) {
+        const float x = dot(ld4(v[i]), la);
+        const bool lt = x < mn;
+        mn = lt ? x : mn;
+        mx = !lt && x > mx ? x : mx;
+    }
+    mn += off; mx += off;
+}
 // Shape::localIsInside -- box_shape.cpp:45-49, cylinder_shape.cpp:45-48, convex_mesh_shape.cpp:152-158
 PE_HD bool inside(const Poly& S, f3 q) {
     if (S.kind == PK_BOX) return fabsf(q.x) <= S.h.x && fabsf(q.y) <= S.h.y && fabsf(q.z) <= S.h.z;
@@ -397,6 +441,17 @@ PE_HD bool test_axis_with(PA&& projA, PB&& projB, f3 ax, float& depth, f3& wa, f
     else { depth = d1; wa = pmna; wb = pmxb; }
     return true;
 }
+// testSepAxis's separation and depth alone.
+template <class PA, class PB>
+PE_HD bool test_depth_with(PA&& projA, PB&& projB, f3 ax, float& depth) {
+    float min0, max0, min1, max1;
+    projA(ax, min0, max0);
+    projB(ax, min1, max1);
+    if (max0 < min1 || max1 < min0) return false;
+    const float d0 = max0 - min1, d1 = max1 - min0;
+    depth = d0 < d1 ? d0 : d1;
+    return true;
+}
 // Orders a wave's LDS stores before its later LDS loads of other lanes' words (a wave's LDS
 // instructions execute in order; this keeps the compiler from moving them across).
 __device__ __forceinline__ void wave_lds_sync() {
@@ -408,6 +463,15 @@ __device__ __forceinline__ void wave_lds_sync() {
 // projections of the separating-axis test: every axis projects every vertex of both shapes, and
 // LDS serves a wave's same-address loads faster than the vector memory path.
 constexpr int MESH_LDS_VERTS = 64;
+__device__ __forceinline__ float4* mesh_lds_row(int which) {   // 0: the wave's copy of A, 1: of B
+    __shared__ float4 s_vtx[4][2][MESH_LDS_VERTS];
+    return s_vtx[(threadIdx.x / WAVE) % 4][which];
+}
+__device__ __forceinline__ void mesh_to_lds(const Poly& P, float4* row) {
+    wave_lds_sync();
+    for (int i = (int)(threadIdx.x & (WAVE - 1)); i < P.nv; i += WAVE) row[i] = P.v[i];
+    wave_lds_sync();
+}
 // The same for the world directions of both shapes' edges (up to EDGE_LDS_DIRS each), the operands
 // every edge-pair axis reads: computed once per pair instead of once per axis.
 constexpr int EDGE_LDS_DIRS = 128;
@@ -423,6 +487,10 @@ PE_HD bool on_line(f3 v0, f3 v1, f3 v2) {
 // returns at the first), and the axis kept is the first in scan order of the least depth among
 // those the scan would accept (an edge axis only below the face depth and with both witness
 // points on their edges), which is the one the sequential scan ends with.
+// Most axes decide nothing but "not separated, deeper than the best", so each is tested for its depth
+// alone (a mesh vertex costs about 10 instructions instead of 20, a cylinder no square-root-free
+// corner cases less but no point transforms) and the witness points are made only for an axis below the
+// best so far and, once, for the one kept.
 template <int G>
 // keep_a (a wave only): the wave's LDS already holds A's vertex copy, staged by its previous call
 // with the same A (the triangles of one concave pair), so it is not staged again.
@@ -435,20 +503,14 @@ __device__ __noinline__ void convex_convex(Cache& c, const PairCtx& x, const Pol
     bool pt_on_a = false;
     const int nfa = n_faces(A), nfb = n_faces(B);
     // with a wave: the vertices of a convex mesh A or B staged in LDS (same values, same order)
-    __shared__ float4 s_vtx[G == 1 ? 1 : 4][2][G == 1 ? 1 : MESH_LDS_VERTS];
-    float4* va = s_vtx[G == 1 ? 0 : (threadIdx.x / WAVE) % 4][0];
-    float4* vb = s_vtx[G == 1 ? 0 : (threadIdx.x / WAVE) % 4][1];
     const bool sa = G > 1 && A.kind == PK_MESH && A.nv <= MESH_LDS_VERTS;
     const bool sb = G > 1 && B.kind == PK_MESH && B.nv <= MESH_LDS_VERTS;
-    if (G > 1 && ((sa && !keep_a) || sb)) {
-        wave_lds_sync();
-        if (sa && !keep_a) for (int i = L::rank(); i < A.nv; i += G) va[i] = A.v[i];
-        if (sb) for (int i = L::rank(); i < B.nv; i += G) vb[i] = B.v[i];
-        wave_lds_sync();
-    }
+    float4* va = G > 1 ? mesh_lds_row(0) : nullptr;
+    float4* vb = G > 1 ? mesh_lds_row(1) : nullptr;
+    if (sa && !keep_a) mesh_to_lds(A, va);
+    if (sb) mesh_to_lds(B, vb);
     // testSepAxis, with a mesh's vertices from the wave's LDS copy when there is one
-    auto test_axis = [&](const Poly& A, const Poly& B, const Pose& ta, const Pose& tb, f3 ax, float& depth, f3& wa,
-                         f3& wb) {
+    auto test_axis = [&](f3 ax, float& depth, f3& wa, f3& wb) {
         return test_axis_with(
             [&](f3 a, float& mn, float& mx, f3& pn, f3& px) {
                 if (sa) project_verts(va, A.nv, ta, a, mn, mx, pn, px);
@@ -460,28 +522,39 @@ __device__ __noinline__ void convex_convex(Cache& c, const PairCtx& x, const Pol
             },
             ax, depth, wa, wb);
     };
+    auto test_depth = [&](f3 ax, float& depth) {
+        return test_depth_with(
+            [&](f3 a, float& mn, float& mx) {
+                if (sa) project_verts_interval(va, A.nv, ta, a, mn, mx);
+                else project_interval(A, ta, a, mn, mx);
+            },
+            [&](f3 a, float& mn, float& mx) {
+                if (sb) project_verts_interval(vb, B.nv, tb, a, mn, mx);
+                else project_interval(B, tb, a, mn, mx);
+            },
+            ax, depth);
+    };
     {
         float bd = REAL_MAX;
         int bi = 0x7fffffff;
-        f3 bn{0, 0, 0}, bpt{0, 0, 0};
         bool separated = false;
+        auto face_axis = [&](int i) {
+            const f3 n = i >= nfa ? mv(tb.R, face_normal(B, i - nfa)) : mv(ta.R, face_normal(A, i));
+            return dot(dc, n) < 0 ? mul(n, -1.0f) : n;
+        };
         for (int i = L::rank(); i < nfa + nfb; i += G) {
-            const bool on_b = i >= nfa;
-            f3 n = on_b ? mv(tb.R, face_normal(B, i - nfa)) : mv(ta.R, face_normal(A, i));
-            if (dot(dc, n) < 0) n = mul(n, -1.0f);
             float d;
-            f3 wa, wb;
-            if (!test_axis(A, B, ta, tb, n, d, wa, wb)) { separated = true; break; }
-            if (d < bd) { bd = d; bi = i; bn = n; bpt = on_b ? add(wa, mul(n, d)) : wb; }
+            if (!test_depth(face_axis(i), d)) { separated = true; break; }
+            if (d < bd) { bd = d; bi = i; }
         }
         if (L::any(separated)) return;
         L::argmin(bd, bi);
         if (bi != 0x7fffffff) {
-            const int src = bi & (G - 1);
-            dmin = bd;
-            sep = L::bcast(bn, src);
-            dmin_pt = L::bcast(bpt, src);
+            sep = face_axis(bi);
+            f3 wa, wb;
+            test_axis(sep, dmin, wa, wb);
             pt_on_a = bi >= nfa;
+            dmin_pt = pt_on_a ? add(wa, mul(sep, dmin)) : wb;
         }
     }
     if ((pt_on_a && inside(B, xf_inv(tb, dmin_pt))) || (!pt_on_a && inside(A, xf_inv(ta, dmin_pt))))
@@ -492,7 +565,6 @@ __device__ __noinline__ void convex_convex(Cache& c, const PairCtx& x, const Pol
     if (nea > 0 && neb > 0) {
         float bd = dmin;
         int bi = 0x7fffffff;
-        f3 bsep{0, 0, 0}, bwea{0, 0, 0}, bweb{0, 0, 0}, bwpa{0, 0, 0}, bwpb{0, 0, 0};
         bool separated = false;
         const int ne = nea * neb;
         // with a wave: B's world edge directions (the inner loop's operand), computed once into LDS
@@ -521,43 +593,40 @@ __device__ __noinline__ void convex_convex(Cache& c, const PairCtx& x, const Pol
             }
             wave_lds_sync();
         }
+        auto dir_a = [&](int e) {
+            if (sea) return ld4(adir[e]);
+            f3 p0, p1;
+            edge_of(A, e, p0, p1);
+            return mv(ta.R, normalized(sub(p0, p1)));
+        };
+        auto dir_b = [&](int e) {
+            if (se) return ld4(edir[e]);
+            f3 p0, p1;
+            edge_of(B, e, p0, p1);
+            return mv(tb.R, normalized(sub(p0, p1)));
+        };
         int t = L::rank();
         int e0 = t / neb, e1 = t - e0 * neb;
         int cur0 = -1;
-        f3 a0, a1, we0;
+        f3 we0{0, 0, 0};
         for (; t < ne; t += G) {
             if (e0 != cur0) {
-                if (sea) {
-                    we0 = ld4(adir[e0]);
-                } else {
-                    edge_of(A, e0, a0, a1);
-                    we0 = mv(ta.R, normalized(sub(a0, a1)));
-                }
+                we0 = dir_a(e0);
                 cur0 = e0;
             }
-            f3 we1;
-            if (se) {
-                we1 = ld4(edir[e1]);
-            } else {
-                f3 b0, b1;
-                edge_of(B, e1, b0, b1);
-                we1 = mv(tb.R, normalized(sub(b0, b1)));
-            }
-            f3 cr = cross(we0, we1);
+            f3 cr = cross(we0, dir_b(e1));
             if (!(fabsf(norm(cr) - 0.0f) < EPS)) {
                 cr = normalized(cr);
                 if (dot(dc, cr) < 0) cr = mul(cr, -1.0f);
                 float dist;
-                f3 wa, wb;
-                if (!test_axis(A, B, ta, tb, cr, dist, wa, wb)) { separated = true; break; }
+                if (!test_depth(cr, dist)) { separated = true; break; }
                 if (dist < bd) {
-                    if (sea) edge_of(A, e0, a0, a1);
-                }
-                if (dist < bd && on_line(a0, a1, xf_inv(ta, wa))) {
-                    f3 b0, b1;
-                    edge_of(B, e1, b0, b1);
-                    if (on_line(b0, b1, xf_inv(tb, wb))) {
-                        bd = dist; bi = t; bsep = cr; bwea = we0; bweb = we1; bwpa = wa; bwpb = wb;
+                    f3 wa, wb, p0, p1;
+                    test_axis(cr, dist, wa, wb);
+                    edge_of(A, e0, p0, p1);
+                    if (on_line(p0, p1, xf_inv(ta, wa))) {
+                        edge_of(B, e1, p0, p1);
+                        if (on_line(p0, p1, xf_inv(tb, wb))) { bd = dist; bi = t; }
                     }
                 }
             }
@@ -567,15 +636,13 @@ __device__ __noinline__ void convex_convex(Cache& c, const PairCtx& x, const Pol
         if (L::any(separated)) return;
         L::argmin(bd, bi);
         if (bi != 0x7fffffff) {
-            const int src = bi & (G - 1);
-            dmin = bd;
             ea = bi / neb;
             eb = bi - ea * neb;
-            sep = L::bcast(bsep, src);
-            wea = L::bcast(bwea, src);
-            web = L::bcast(bweb, src);
-            wpa = L::bcast(bwpa, src);
-            wpb = L::bcast(bwpb, src);
+            wea = dir_a(ea);
+            web = dir_b(eb);
+            sep = normalized(cross(wea, web));
+            if (dot(dc, sep) < 0) sep = mul(sep, -1.0f);
+            test_axis(sep, dmin, wpa, wpb);
         }
     }
     if (ea >= 0 && eb >= 0) {
@@ -1265,8 +1332,7 @@ __device__ __noinline__ void concave_poly(Cache& c, const PairCtx& x, const Mesh
         bb = add(bb, rel.p);
     }
     const Poly M = poly_mesh(&ms, mesh);
-    bool staged = false;   // a wave copies A's vertices to LDS once per pair (convex_convex's keep_a)
-    bvh_visit<G>(ms, mesh, aa, bb, [&](int f) {
+    auto triangle = [&](int f) {
         Poly T;
         T.kind = PK_TRI;
         T.ms = &ms;
@@ -1274,9 +1340,39 @@ __device__ __noinline__ void concave_poly(Cache& c, const PairCtx& x, const Mesh
         T.t[1] = face_vertex(M, f, 1);
         T.t[2] = face_vertex(M, f, 2);
         T.tn = face_normal(M, f);
-        convex_convex<G>(c, x, A, T, pa, pm, ref_scale, staged);
-        staged = G > 1;
-    });
+        return T;
+    };
+    if constexpr (G == 1) {
+        bvh_visit(ms, mesh, aa, bb, [&](int f) { convex_convex<1>(c, x, A, triangle(f), pa, pm, ref_scale); });
+    } else {
+        // Most triangles of the leaves are separated from the polyhedron, and the convex routine gives no point
+        // for one that any of its face axes separates: each lane first tests a triangle of its own along the
+        // triangle's normal and, for a box, along the box's, and the wave runs the routine only for the
+        // triangles left, in the walk's order (a whole-wave test per triangle used 7 of its lanes for a box).
+        const bool sa = A.kind == PK_MESH && A.nv <= MESH_LDS_VERTS;
+        float4* va = mesh_lds_row(0);
+        if (sa) mesh_to_lds(A, va);
+        const f3 dc = sub(pa.p, pm.p);
+        bvh_faces_wave(ms, mesh, aa, bb,
+            [&](int f) {
+                const Poly T = triangle(f);
+                const int na = A.kind == PK_BOX ? 6 : 0;
+                for (int i = -1; i < na; i++) {
+                    f3 n = i < 0 ? mv(pm.R, T.tn) : mv(pa.R, face_normal(A, i));
+                    if (dot(dc, n) < 0) n = mul(n, -1.0f);
+                    float d;
+                    const bool meet = test_depth_with(
+                        [&](f3 a, float& mn, float& mx) {
+                            if (sa) project_verts_interval(va, A.nv, pa, a, mn, mx);
+                            else project_interval(A, pa, a, mn, mx);
+                        },
+                        [&](f3 a, float& mn, float& mx) { project_interval(T, pm, a, mn, mx); }, n, d);
+                    if (!meet) return 0u;
+                }
+                return 1u;
+            },
+            [&](int f, int) { convex_convex<G>(c, x, A, triangle(f), pa, pm, ref_scale, sa); });
+    }
 }
 
 }  // namespace pe
