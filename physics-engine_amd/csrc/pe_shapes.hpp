@@ -891,7 +891,8 @@ __device__ __forceinline__ int* bvh_stack_row() {
 // that misses the box is never pushed.  Children are tested and pushed left then right, so the
 // nodes that pass are popped, and the faces visited, in the same order as by the walk below.
 __device__ __forceinline__ int4* bvh_wave_stack_row() {
-    __shared__ int4 s_st[4][BVH_STACK];   // a row per wave (every lane writes the same value)
+    __shared__ int4 s_st[4][WAVE];   // a row per wave: a stack (every lane writes the same value) or a lane's entry each
+    static_assert(BVH_STACK <= WAVE, "the stack fits the row");
     return s_st[(threadIdx.x / WAVE) % 4];
 }
 template <class F>
@@ -952,6 +953,77 @@ __device__ inline void bvh_visit(const MeshSet& ms, int mesh, f3 aa, f3 bb, F&& 
     }
 }
 
+// A wave's face list in LDS: the faces a walk found, in its order.
+constexpr int FACE_REC = 128;
+__device__ __forceinline__ int* face_rec_row() {
+    __shared__ int s_rec[4][FACE_REC];
+    return s_rec[(threadIdx.x / WAVE) % 4];
+}
+// The walk level by level: the nodes still to open, in the order the depth-first walk would pop them, one per lane;
+// each round every lane reads its node's children and puts those that meet the box in its place, the right
+// one first.  A box that meets a few leaves of a tree of thousands of faces takes a round of dependent
+// loads per level (13 for a 64 x 64 heightfield) instead of one per node popped (about 50: 100 000 of the
+// 120 000 cycles a box-heightfield pair took).  The faces of the leaves go to rec in the walk's order;
+// returns their number, or -1 when the nodes outgrow the wave's lanes or the faces rec (then the walk above
+// is taken).  Every node on the way down meets the box when its child does, so both visit the same leaves.
+__device__ inline int bvh_gather_wave(const MeshSet& ms, int mesh, f3 aa, f3 bb, int* rec) {
+    const int32_t* mr = ms.rec + MRW * mesh;
+    if (mr[MR_NB] == 0) return 0;
+    const float4* node = ms.arena + mr[MR_NODE];
+    const int2* leaf = reinterpret_cast<const int2*>(ms.arena + mr[MR_LEAF]);
+    int4* st = bvh_wave_stack_row();
+    const int lane = (int)(threadIdx.x & (WAVE - 1));
+    auto hit = [&](float4 lo, float4 hi) {
+        return !(lo.x > bb.x || lo.y > bb.y || lo.z > bb.z) && !(hi.x < aa.x || hi.y < aa.y || hi.z < aa.z);
+    };
+    // a lane's node: faces (0: an inner node), first face, children
+    int4 e = make_int4(0, 0, -1, -1);
+    bool have = false;
+    {
+        const float4 lo = node[0], hi = node[1];
+        const int2 lf = leaf[0];
+        have = lane == 0 && hit(lo, hi);
+        e = make_int4(lf.x, lf.y, __float_as_int(lo.w), __float_as_int(hi.w));
+    }
+    while (__any(have && e.x <= 0)) {
+        int4 c0 = e, c1 = e;   // what takes the node's place: c0, then c1
+        bool h0 = have, h1 = false;
+        if (have && e.x <= 0) {
+            float4 llo{}, lhi{}, rlo{}, rhi{};
+            int2 llf{}, rlf{};
+            if (e.z >= 0) { llo = node[2 * e.z]; lhi = node[2 * e.z + 1]; llf = leaf[e.z]; }
+            if (e.w >= 0) { rlo = node[2 * e.w]; rhi = node[2 * e.w + 1]; rlf = leaf[e.w]; }
+            h0 = e.w >= 0 && hit(rlo, rhi);
+            h1 = e.z >= 0 && hit(llo, lhi);
+            c0 = make_int4(rlf.x, rlf.y, __float_as_int(rlo.w), __float_as_int(rhi.w));
+            c1 = make_int4(llf.x, llf.y, __float_as_int(llo.w), __float_as_int(lhi.w));
+        }
+        const uint64_t m0 = __ballot(h0), m1 = __ballot(h1);
+        const int total = (int)(__popcll(m0) + __popcll(m1));
+        if (total > WAVE) return -1;
+        const int at = (int)(__popcll(m0 & lanemask_lt()) + __popcll(m1 & lanemask_lt()));
+        wave_lds_sync();
+        if (h0) st[at] = c0;
+        if (h1) st[at + (h0 ? 1 : 0)] = c1;
+        wave_lds_sync();
+        have = lane < total;
+        if (have) e = st[lane];
+        else e = make_int4(0, 0, -1, -1);
+    }
+    int incl = have ? e.x : 0;
+#pragma unroll
+    for (int o = 1; o < WAVE; o <<= 1) {
+        const int y = __shfl_up(incl, o, WAVE);
+        if (lane >= o) incl += y;
+    }
+    const int n = __shfl(incl, WAVE - 1, WAVE);
+    if (n > FACE_REC) return -1;
+    wave_lds_sync();
+    if (have)
+        for (int i = 0; i < e.x; i++) rec[incl - e.x + i] = e.y + i;
+    wave_lds_sync();
+    return n;
+}
 // The faces bvh_visit<WAVE> finds, tested by a wave's lanes in batches of WAVE and added in the
 // walk's order.  test(f), on the lane that holds face f, returns the bit mask of f's items (the
 // routine's own units: triangles of a fan, segments, edges) that give contact points; commit(f, i)
@@ -959,19 +1031,10 @@ __device__ inline void bvh_visit(const MeshSet& ms, int mesh, f3 aa, f3 bb, F&& 
 // item by item in ascending order -- the order in which a sequential walk adds the points, so the
 // contact cache ends as it would.  Most faces yield no point, so the tests (most of the work) run
 // in parallel and only the hits are computed again, serially, to be added.
-// With rec, the walk's faces are also kept in rec (a wave's LDS row: every lane writes the same
-// value) while there are at most FACE_REC of them, and *nrec is their count: a second walk over the
-// same box then runs over the list (faces_list_wave) instead of the tree.
-constexpr int FACE_REC = 128;
-__device__ __forceinline__ int* face_rec_row() {
-    __shared__ int s_rec[4][FACE_REC];
-    return s_rec[(threadIdx.x / WAVE) % 4];
-}
 template <class Test, class Commit>
-__device__ inline void bvh_faces_wave(const MeshSet& ms, int mesh, f3 aa, f3 bb, Test&& test, Commit&& commit,
-                                      int* rec = nullptr, int* nrec = nullptr) {
+__device__ inline void bvh_walk_wave(const MeshSet& ms, int mesh, f3 aa, f3 bb, Test&& test, Commit&& commit) {
     const int r = (int)(threadIdx.x & (WAVE - 1));
-    int mine = -1, cnt = 0, all = 0;
+    int mine = -1, cnt = 0;
     auto flush = [&]() {
         const uint32_t m = r < cnt ? test(mine) : 0u;
         uint64_t hit = __ballot(m != 0u);
@@ -989,15 +1052,12 @@ __device__ inline void bvh_faces_wave(const MeshSet& ms, int mesh, f3 aa, f3 bb,
         cnt = 0;
     };
     bvh_visit<WAVE>(ms, mesh, aa, bb, [&](int f) {
-        if (rec && all < FACE_REC) rec[all] = f;
-        all++;
         if (r == cnt) mine = f;
         if (++cnt == WAVE) flush();
     });
     if (cnt > 0) flush();
-    if (nrec) *nrec = all;
 }
-// The same tests and commits over faces already found: rec[0 .. n), in order.
+// The same over faces already found: rec[0 .. n), in order.
 template <class Test, class Commit>
 __device__ inline void faces_list_wave(const int* rec, int n, Test&& test, Commit&& commit) {
     const int r = (int)(threadIdx.x & (WAVE - 1));
@@ -1018,6 +1078,17 @@ __device__ inline void faces_list_wave(const int* rec, int n, Test&& test, Commi
             }
         }
     }
+}
+
+// The faces of the leaves that meet the box, by either walk; returns their number in the wave's face list, -1 if
+// they are not there.
+template <class Test, class Commit>
+__device__ inline int bvh_faces_wave(const MeshSet& ms, int mesh, f3 aa, f3 bb, Test&& test, Commit&& commit) {
+    int* rec = face_rec_row();
+    const int n = bvh_gather_wave(ms, mesh, aa, bb, rec);
+    if (n >= 0) faces_list_wave(rec, n, test, commit);
+    else bvh_walk_wave(ms, mesh, aa, bb, test, commit);
+    return n;
 }
 
 // ------------------------------------------------------------------ cylinder-mesh
@@ -1170,16 +1241,14 @@ __device__ __noinline__ void cylinder_mesh(Cache& c, const PairCtx& x, const Mes
     } else {
         // the second walk is over the same box: it visits the faces the first one found, in the same
         // order, so it runs over their list when the first walk could keep it
-        int* rec = face_rec_row();
-        int nrec = 0;
-        bvh_faces_wave(ms, mesh, q.aa, q.bb,
+        const int nrec = bvh_faces_wave(ms, mesh, q.aa, q.bb,
             [&](int f) {
                 const CylFace F = cyl_face_frame(M, f, q.ax);
                 uint32_t m = 0;
                 for (int i = 0; i < cyl_face_items(F); i++) m |= (cyl_face_hit(M, f, F, q, i) ? 1u : 0u) << i;
                 return m;
             },
-            [&](int f, int i) { cyl_face_add(c, x, M, f, cyl_face_frame(M, f, q.ax), q, i, pm); }, rec, &nrec);
+            [&](int f, int i) { cyl_face_add(c, x, M, f, cyl_face_frame(M, f, q.ax), q, i, pm); });
         auto edge_test = [&](int f) {
             const int nf = face_len(M, f);
             uint32_t m = 0;
@@ -1191,8 +1260,8 @@ __device__ __noinline__ void cylinder_mesh(Cache& c, const PairCtx& x, const Mes
             return m;
         };
         auto edge_commit = [&](int f, int i) { cyl_edge_add(c, x, M, f, i, q, pm); };
-        if (nrec <= FACE_REC) faces_list_wave(rec, nrec, edge_test, edge_commit);
-        else bvh_faces_wave(ms, mesh, q.aa, q.bb, edge_test, edge_commit);
+        if (nrec >= 0) faces_list_wave(face_rec_row(), nrec, edge_test, edge_commit);
+        else bvh_walk_wave(ms, mesh, q.aa, q.bb, edge_test, edge_commit);
     }
 }
 
