@@ -373,6 +373,73 @@ struct Grp {
     static __device__ __forceinline__ f3 bcast(f3 v, int src) { return G == 1 ? v : f3{__shfl(v.x, src), __shfl(v.y, src), __shfl(v.z, src)}; }
 };
 
+// Orders a wave's LDS stores before its later LDS loads of other lanes' words (a wave's LDS
+// instructions execute in order; this keeps the compiler from moving them across).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// add_point with a wave on one cache in LDS: lane i (of each eight) looks at slot i, the one chosen writes itself.
+// Called by all lanes with the same values.
+__device__ __forceinline__ float oct_min(float v) {   // over each eight lanes
+    auto dpp = [](float x, auto ctrl) {
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), decltype(ctrl)::value, 0xf, 0xf, true));
+    };
+    const float a = dpp(v, std::integral_constant<int, 0xb1>{});      // lanes 1 0 3 2
+    v = a < v ? a : v;
+    const float b = dpp(v, std::integral_constant<int, 0x4e>{});      // lanes 2 3 0 1
+    v = b < v ? b : v;
+    const float h = dpp(v, std::integral_constant<int, 0x141>{});     // the eight lanes mirrored
+    return h < v ? h : v;
+}
+__device__ __forceinline__ void add_point_wave(Cache& c, const PairCtx& x, f3 world_normal, f3 world_pos, float depth) {
+    f3 pa = world_pos, pb = world_pos, n = world_normal, point = world_pos;
+    if (x.swap) {
+        n = neg(n);
+        pb = add(world_pos, mul(world_normal, depth));
+        point = pb;
+    } else {
+        pa = add(world_pos, mul(world_normal, depth));
+    }
+    const f3 la = xf_inv(x.A, pa);
+    const f3 lb = xf_inv(x.B, pb);
+    const int lane = (int)(threadIdx.x & (WAVE - 1)), i = lane & 7;
+    wave_lds_sync();
+    const bool valid = c.wx[i] < REAL_MAX + 0.1f;
+    const float d = c.d[i];
+    const f3 dd{c.bx[i] - lb.x, c.by[i] - lb.y, c.bz[i] - lb.z};
+    const float dist = dot(dd, dd);
+    const float inf = __builtin_inff();
+    const bool close = valid && dist < x.same_th2;
+    const float least = oct_min(close ? dist : inf);
+    const uint32_t near = (uint32_t)__ballot(close && dist == least) & 0xffu;   // the first of the nearest
+    uint32_t slot;
+    if (near) {
+        const float dn = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(d), __ffs(near) - 1));
+        slot = depth < dn ? near : 0u;
+    } else {
+        slot = ~(uint32_t)__ballot(valid) & 0xffu;   // the first free slot, else the first of the farthest
+        if (!slot) {
+            const float most = -oct_min(d > REAL_MIN ? -d : inf);
+            slot = (uint32_t)__ballot(d > REAL_MIN && d == most) & 0xffu;
+        }
+    }
+    if (slot && lane == __ffs(slot) - 1) {
+        c.wx[i] = point.x; c.wy[i] = point.y; c.wz[i] = point.z;
+        c.nx[i] = n.x; c.ny[i] = n.y; c.nz[i] = n.z;
+        c.ax[i] = la.x; c.ay[i] = la.y; c.az[i] = la.z;
+        c.bx[i] = lb.x; c.by[i] = lb.y; c.bz[i] = lb.z;
+        c.d[i] = depth;
+    }
+    wave_lds_sync();
+}
+template <int G>
+__device__ __forceinline__ void add_pt(Cache& c, const PairCtx& x, f3 n, f3 p, float depth) {
+    if (G == 1) add_point(c, x, n, p, depth);
+    else add_point_wave(c, x, n, p, depth);
+}
+
 // clipHullAgainstHull + clipFaceAgainstHull (:63-170)
 template <int G>
 __device__ __noinline__ void clip_hull_hull(Cache& c, const PairCtx& x, f3 sep, const Poly& A, const Poly& B,
@@ -424,7 +491,7 @@ __device__ __noinline__ void clip_hull_hull(Cache& c, const PairCtx& x, f3 sep, 
     for (int i = 0; i < n; i++) {
         const f3 vtx = pin[i];
         const float depth = dot(ln, sub(xf_inv(ta, vtx), pv));
-        if (depth <= max_dist && depth >= min_dist) add_point(c, x, sep, sub(vtx, mul(sep, 0.0f)), depth + 0.0f * 2);
+        if (depth <= max_dist && depth >= min_dist) add_pt<G>(c, x, sep, sub(vtx, mul(sep, 0.0f)), depth + 0.0f * 2);
     }
 }
 // testSepAxis (:216-243)
@@ -451,13 +518,6 @@ PE_HD bool test_depth_with(PA&& projA, PB&& projB, f3 ax, float& depth) {
     const float d0 = max0 - min1, d1 = max1 - min0;
     depth = d0 < d1 ? d0 : d1;
     return true;
-}
-// Orders a wave's LDS stores before its later LDS loads of other lanes' words (a wave's LDS
-// instructions execute in order; this keeps the compiler from moving them across).
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 // A wave's copies of two convex meshes' vertices in LDS (up to MESH_LDS_VERTS each), for the
 // projections of the separating-axis test: every axis projects every vertex of both shapes, and
@@ -558,7 +618,7 @@ __device__ __noinline__ void convex_convex(Cache& c, const PairCtx& x, const Pol
         }
     }
     if ((pt_on_a && inside(B, xf_inv(tb, dmin_pt))) || (!pt_on_a && inside(A, xf_inv(ta, dmin_pt))))
-        add_point(c, x, sep, sub(dmin_pt, mul(sep, 0.0f)), -dmin + 0.0f * 2);
+        add_pt<G>(c, x, sep, sub(dmin_pt, mul(sep, 0.0f)), -dmin + 0.0f * 2);
     int ea = -1, eb = -1;
     f3 wea{0, 0, 0}, web{0, 0, 0}, wpa{0, 0, 0}, wpb{0, 0, 0};
     const int nea = n_edges(A), neb = n_edges(B);
@@ -678,7 +738,7 @@ __device__ __noinline__ void convex_convex(Cache& c, const PairCtx& x, const Pol
             pv = mul(pv, 1.0f / nl);
             if (dot(pv, dc) < 0) pv = mul(pv, -1.0f);
             const f3 pob = add(wpb, ob);
-            add_point(c, x, pv, sub(pob, mul(pv, 0.0f)), -nl + 0.0f * 2);
+            add_pt<G>(c, x, pv, sub(pob, mul(pv, 0.0f)), -nl + 0.0f * 2);
         }
     }
     if (dot(dc, sep) < 0) sep = neg(sep);
@@ -734,8 +794,18 @@ PE_HD void point_on_box(Cache& c, const PairCtx& x, f3 pc, int face, f3 he, cons
     const f3 pw = xf_apply(to, p);
     add_point(c, x, nw, sub(pw, mul(nw, 0.0f)), pen + 2 * 0.0f);
 }
+// Contact points a face's item gives: up to two with one normal.
+struct FacePoints {
+    f3 n, p0, p1;
+    float d0, d1;
+    int count;
+};
+PE_HD void add_points(Cache& c, const PairCtx& x, const FacePoints& o) {
+    if (o.count > 0) add_point(c, x, o.n, o.p0, o.d0);
+    if (o.count > 1) add_point(c, x, o.n, o.p1, o.d1);
+}
 // addContactPointOnCylinder (:116-139)
-PE_HD void point_on_cyl(Cache& c, const PairCtx& x, f3 p, f3 pc, f3 ax, float rad, float h, const Pose& to) {
+PE_HD FacePoints cyl_point(f3 p, f3 pc, f3 ax, float rad, float h, const Pose& to) {
     const f3 r = sub(p, pc);
     const float dy = dot(r, ax);
     const float dxz = sqrtf(dot(r, r) - dy * dy);
@@ -746,7 +816,12 @@ PE_HD void point_on_cyl(Cache& c, const PairCtx& x, f3 p, f3 pc, f3 ax, float ra
     else { dist = d_top; n = dy < 0 ? ax : neg(ax); }
     n = mv(to.R, n);
     const f3 pw = xf_apply(to, p);
-    add_point(c, x, n, sub(pw, mul(n, 0.0f)), -dist + 2 * 0.0f);
+    FacePoints o{};
+    o.n = n;
+    o.p0 = sub(pw, mul(n, 0.0f));
+    o.d0 = -dist + 2 * 0.0f;
+    o.count = 1;
+    return o;
 }
 // findClosestBoxFace (:141-157)
 PE_HD int closest_box_face(f3 he, f3 q) {
@@ -864,7 +939,7 @@ __device__ __noinline__ void box_cylinder(Cache& c, const PairCtx& x, const Pose
                 float tmin, tmax;
                 if (seg_cyl(ec, ed, eh, pc, ax, h, rad, EPS, tmin, tmax)) {
                     const f3 pmid = add(ec, mul(ed, (tmin + tmax) / 2));
-                    point_on_cyl(c, x, pmid, pc, ax, rad, h, pb);
+                    add_points(c, x, cyl_point(pmid, pc, ax, rad, h, pb));
                 }
             }
         }
@@ -1024,70 +1099,87 @@ __device__ inline int bvh_gather_wave(const MeshSet& ms, int mesh, f3 aa, f3 bb,
     wave_lds_sync();
     return n;
 }
-// The faces bvh_visit<WAVE> finds, tested by a wave's lanes in batches of WAVE and added in the
-// walk's order.  test(f), on the lane that holds face f, returns the bit mask of f's items (the
-// routine's own units: triangles of a fan, segments, edges) that give contact points; commit(f, i)
-// then runs on every lane with the same values for each such item, face by face in walk order and
-// item by item in ascending order -- the order in which a sequential walk adds the points, so the
-// contact cache ends as it would.  Most faces yield no point, so the tests (most of the work) run
-// in parallel and only the hits are computed again, serially, to be added.
-template <class Test, class Commit>
-__device__ inline void bvh_walk_wave(const MeshSet& ms, int mesh, f3 aa, f3 bb, Test&& test, Commit&& commit) {
+__device__ __forceinline__ float lane_value(float v, int src) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
+}
+__device__ __forceinline__ f3 lane_value(f3 v, int src) { return f3{lane_value(v.x, src), lane_value(v.y, src), lane_value(v.z, src)}; }
+// What a lane's faces give, added in the walk's order.  test(f), on the lane that holds face f, returns the bit
+// mask of f's items (the routine's own units: triangles of a fan, segments, edges) that give contact points;
+// the items that do are numbered in order, face by face and item by item -- the order in which a
+// sequential walk adds the points, so the contact cache ends as it would -- and add(hits, list) gets up to 64
+// of them at a time, list[k] = (face, item) in the wave's LDS.
+template <class Test, class Add>
+__device__ inline void face_hits_wave(int f, bool have, Test&& test, Add&& add) {
+    uint32_t m = have ? test(f) : 0u;
+    if (__ballot(m != 0u) == 0) return;
+    const int lane = (int)(threadIdx.x & (WAVE - 1));
+    int incl = __popc(m);
+#pragma unroll
+    for (int o = 1; o < WAVE; o <<= 1) {
+        const int y = __shfl_up(incl, o, WAVE);
+        if (lane >= o) incl += y;
+    }
+    const int total = __shfl(incl, WAVE - 1, WAVE);
+    int at = incl - __popc(m);
+    __shared__ int2 s_hits[4][WAVE];
+    int2* list = s_hits[(threadIdx.x / WAVE) % 4];
+    for (int k0 = 0; k0 < total; k0 += WAVE) {
+        wave_lds_sync();
+        while (m && at < k0 + WAVE) {
+            list[at - k0] = int2{f, __ffs(m) - 1};
+            m &= m - 1;
+            at++;
+        }
+        wave_lds_sync();
+        add(total - k0 < WAVE ? total - k0 : WAVE, (const int2*)list);
+    }
+}
+// The adder for items whose points a lane can make by itself, point(f, i) -> FacePoints: each lane makes one hit's
+// points, all of them at once, and the wave adds them in turn.
+template <class Point>
+__device__ __forceinline__ auto add_hits(Cache& c, const PairCtx& x, Point&& point) {
+    return [&c, &x, point](int hits, const int2* list) {
+        const int lane = (int)(threadIdx.x & (WAVE - 1));
+        FacePoints q{};
+        if (lane < hits) q = point(list[lane].x, list[lane].y);
+        for (int k = 0; k < hits; k++) {
+            const int m = __builtin_amdgcn_readlane(q.count, k);
+            if (m == 0) continue;
+            const f3 n = lane_value(q.n, k);
+            add_point_wave(c, x, n, lane_value(q.p0, k), lane_value(q.d0, k));
+            if (m > 1) add_point_wave(c, x, n, lane_value(q.p1, k), lane_value(q.d1, k));
+        }
+    };
+}
+// The faces bvh_visit<WAVE> finds, 64 at a time.
+template <class Test, class Add>
+__device__ inline void bvh_walk_wave(const MeshSet& ms, int mesh, f3 aa, f3 bb, Test&& test, Add&& add) {
     const int r = (int)(threadIdx.x & (WAVE - 1));
     int mine = -1, cnt = 0;
-    auto flush = [&]() {
-        const uint32_t m = r < cnt ? test(mine) : 0u;
-        uint64_t hit = __ballot(m != 0u);
-        while (hit) {
-            const int src = __ffsll((unsigned long long)hit) - 1;
-            hit &= hit - 1;
-            const int f = __shfl(mine, src);
-            uint32_t mk = (uint32_t)__shfl((int)m, src);
-            while (mk) {
-                const int i = __ffs(mk) - 1;
-                mk &= mk - 1;
-                commit(f, i);
-            }
-        }
-        cnt = 0;
-    };
     bvh_visit<WAVE>(ms, mesh, aa, bb, [&](int f) {
         if (r == cnt) mine = f;
-        if (++cnt == WAVE) flush();
+        if (++cnt == WAVE) {
+            face_hits_wave(mine, true, test, add);
+            cnt = 0;
+        }
     });
-    if (cnt > 0) flush();
+    if (cnt > 0) face_hits_wave(mine, r < cnt, test, add);
 }
 // The same over faces already found: rec[0 .. n), in order.
-template <class Test, class Commit>
-__device__ inline void faces_list_wave(const int* rec, int n, Test&& test, Commit&& commit) {
+template <class Test, class Add>
+__device__ inline void faces_list_wave(const int* rec, int n, Test&& test, Add&& add) {
     const int r = (int)(threadIdx.x & (WAVE - 1));
-    for (int base = 0; base < n; base += WAVE) {
-        const int cnt = n - base < WAVE ? n - base : WAVE;
-        const int mine = r < cnt ? rec[base + r] : -1;
-        const uint32_t m = r < cnt ? test(mine) : 0u;
-        uint64_t hit = __ballot(m != 0u);
-        while (hit) {
-            const int src = __ffsll((unsigned long long)hit) - 1;
-            hit &= hit - 1;
-            const int f = __shfl(mine, src);
-            uint32_t mk = (uint32_t)__shfl((int)m, src);
-            while (mk) {
-                const int i = __ffs(mk) - 1;
-                mk &= mk - 1;
-                commit(f, i);
-            }
-        }
-    }
+    for (int base = 0; base < n; base += WAVE) face_hits_wave(base + r < n ? rec[base + r] : -1, base + r < n, test, add);
 }
 
 // The faces of the leaves that meet the box, by either walk; returns their number in the wave's face list, -1 if
 // they are not there.
-template <class Test, class Commit>
-__device__ inline int bvh_faces_wave(const MeshSet& ms, int mesh, f3 aa, f3 bb, Test&& test, Commit&& commit) {
+template <class Test, class Add>
+__device__ inline int bvh_faces_wave(const MeshSet& ms, int mesh, f3 aa, f3 bb, Test&& test, Add&& add) {
     int* rec = face_rec_row();
     const int n = bvh_gather_wave(ms, mesh, aa, bb, rec);
-    if (n >= 0) faces_list_wave(rec, n, test, commit);
-    else bvh_walk_wave(ms, mesh, aa, bb, test, commit);
+    if (n >= 0) faces_list_wave(rec, n, test, add);
+    else bvh_walk_wave(ms, mesh, aa, bb, test, add);
     return n;
 }
 
@@ -1188,19 +1280,23 @@ PE_HD bool cyl_face_hit(const Poly& M, int f, const CylFace& F, const CylInMesh&
     cyl_face_seg(F, q, i, ps, sd, l);
     return seg_face(M, f, ps, sd, l, t1, t2, d1, d2);
 }
-PE_HD void cyl_face_add(Cache& c, const PairCtx& x, const Poly& M, int f, const CylFace& F, const CylInMesh& q,
-                        int i, const Pose& pm) {
+PE_HD FacePoints cyl_face_points(const Poly& M, int f, const CylFace& F, const CylInMesh& q, int i, const Pose& pm) {
     f3 ps, sd;
     float l, t1, t2, d1, d2;
+    FacePoints o{};
     cyl_face_seg(F, q, i, ps, sd, l);
     if (seg_face(M, f, ps, sd, l, t1, t2, d1, d2)) {
         const f3 fn = face_normal(M, f);
         const f3 p1 = xf_apply(pm, sub(add(ps, mul(sd, t1)), mul(fn, d1)));
         const f3 p2 = xf_apply(pm, sub(add(ps, mul(sd, t2)), mul(fn, d2)));
-        const f3 n = mv(pm.R, fn);
-        add_point(c, x, n, sub(p1, mul(n, 0.0f)), d1 + 0.0f * 2);
-        add_point(c, x, n, sub(p2, mul(n, 0.0f)), d2 + 0.0f * 2);
+        o.n = mv(pm.R, fn);
+        o.p0 = sub(p1, mul(o.n, 0.0f));
+        o.d0 = d1 + 0.0f * 2;
+        o.p1 = sub(p2, mul(o.n, 0.0f));
+        o.d1 = d2 + 0.0f * 2;
+        o.count = 2;
     }
+    return o;
 }
 // Second walk, face f: item i is the face's edge from vertex i to vertex i + 1.
 PE_HD bool cyl_edge_seg(const Poly& M, int f, int i, const CylInMesh& q, f3& ss, f3& sd, float& t1, float& t2) {
@@ -1212,15 +1308,14 @@ PE_HD bool cyl_edge_seg(const Poly& M, int f, int i, const CylInMesh& q, f3& ss,
     sd = divs(sub(v2, v1), l * 2);
     return seg_cyl(ss, sd, l, q.pc, q.ax, q.h, q.rad, 0.0f, t1, t2);
 }
-PE_HD void cyl_edge_add(Cache& c, const PairCtx& x, const Poly& M, int f, int i, const CylInMesh& q, const Pose& pm) {
+PE_HD FacePoints cyl_edge_points(const Poly& M, int f, int i, const CylInMesh& q, const Pose& pm) {
     f3 ss, sd;
     float t1, t2;
-    if (cyl_edge_seg(M, f, i, q, ss, sd, t1, t2)) {
-        const f3 p1 = add(ss, mul(sd, t1));
-        const f3 p2 = add(ss, mul(sd, t2));
-        const f3 pmid = divs(add(p1, p2), 2.0f);
-        point_on_cyl(c, x, pmid, q.pc, q.ax, q.rad, q.h, pm);
-    }
+    if (!cyl_edge_seg(M, f, i, q, ss, sd, t1, t2)) return FacePoints{};
+    const f3 p1 = add(ss, mul(sd, t1));
+    const f3 p2 = add(ss, mul(sd, t2));
+    const f3 pmid = divs(add(p1, p2), 2.0f);
+    return cyl_point(pmid, q.pc, q.ax, q.rad, q.h, pm);
 }
 // The whole routine for the mesh of a convex or concave body (pm: mesh body pose): G = 1 on one
 // lane; G = WAVE on a wave's lanes, the faces of each walk split over them (bvh_faces_wave).
@@ -1232,11 +1327,11 @@ __device__ __noinline__ void cylinder_mesh(Cache& c, const PairCtx& x, const Mes
     if (G == 1) {
         bvh_visit(ms, mesh, q.aa, q.bb, [&](int f) {
             const CylFace F = cyl_face_frame(M, f, q.ax);
-            for (int i = 0; i < cyl_face_items(F); i++) cyl_face_add(c, x, M, f, F, q, i, pm);
+            for (int i = 0; i < cyl_face_items(F); i++) add_points(c, x, cyl_face_points(M, f, F, q, i, pm));
         });
         bvh_visit(ms, mesh, q.aa, q.bb, [&](int f) {
             const int nf = face_len(M, f);
-            for (int i = 0; i < nf; i++) cyl_edge_add(c, x, M, f, i, q, pm);
+            for (int i = 0; i < nf; i++) add_points(c, x, cyl_edge_points(M, f, i, q, pm));
         });
     } else {
         // the second walk is over the same box: it visits the faces the first one found, in the same
@@ -1248,7 +1343,7 @@ __device__ __noinline__ void cylinder_mesh(Cache& c, const PairCtx& x, const Mes
                 for (int i = 0; i < cyl_face_items(F); i++) m |= (cyl_face_hit(M, f, F, q, i) ? 1u : 0u) << i;
                 return m;
             },
-            [&](int f, int i) { cyl_face_add(c, x, M, f, cyl_face_frame(M, f, q.ax), q, i, pm); });
+            add_hits(c, x, [&](int f, int i) { return cyl_face_points(M, f, cyl_face_frame(M, f, q.ax), q, i, pm); }));
         auto edge_test = [&](int f) {
             const int nf = face_len(M, f);
             uint32_t m = 0;
@@ -1259,9 +1354,9 @@ __device__ __noinline__ void cylinder_mesh(Cache& c, const PairCtx& x, const Mes
             }
             return m;
         };
-        auto edge_commit = [&](int f, int i) { cyl_edge_add(c, x, M, f, i, q, pm); };
-        if (nrec >= 0) faces_list_wave(face_rec_row(), nrec, edge_test, edge_commit);
-        else bvh_walk_wave(ms, mesh, q.aa, q.bb, edge_test, edge_commit);
+        auto edge_add = add_hits(c, x, [&](int f, int i) { return cyl_edge_points(M, f, i, q, pm); });
+        if (nrec >= 0) faces_list_wave(face_rec_row(), nrec, edge_test, edge_add);
+        else bvh_walk_wave(ms, mesh, q.aa, q.bb, edge_test, edge_add);
     }
 }
 
@@ -1341,14 +1436,18 @@ PE_HD bool sphere_fan_tri(const Poly& M, int f, int i, f3 cc, float rad, f3& p, 
     depth = 0;
     return sphere_tri(cc, rad, vt, p, n, depth);
 }
-PE_HD void sphere_fan_add(Cache& c, const PairCtx& x, const Poly& M, int f, int i, f3 cc, float rad, const Pose& pm) {
+PE_HD FacePoints sphere_fan_points(const Poly& M, int f, int i, f3 cc, float rad, const Pose& pm) {
     f3 p, n;
     float depth;
+    FacePoints o{};
     if (sphere_fan_tri(M, f, i, cc, rad, p, n, depth)) {
-        n = mv(pm.R, n);
+        o.n = mv(pm.R, n);
         p = xf_apply(pm, p);
-        add_point(c, x, n, sub(p, mul(n, 0.0f)), depth + 2 * 0.0f);
+        o.p0 = sub(p, mul(o.n, 0.0f));
+        o.d0 = depth + 2 * 0.0f;
+        o.count = 1;
     }
+    return o;
 }
 template <int G = 1>
 __device__ __noinline__ void sphere_mesh(Cache& c, const PairCtx& x, const MeshSet& ms, int mesh, const Pose& pm,
@@ -1359,7 +1458,7 @@ __device__ __noinline__ void sphere_mesh(Cache& c, const PairCtx& x, const MeshS
     if (G == 1) {
         bvh_visit(ms, mesh, aa, bb, [&](int f) {
             const int nf = face_len(M, f);
-            for (int i = 0; i < nf - 2; i++) sphere_fan_add(c, x, M, f, i, cc, rad, pm);
+            for (int i = 0; i < nf - 2; i++) add_points(c, x, sphere_fan_points(M, f, i, cc, rad, pm));
         });
     } else {
         bvh_faces_wave(ms, mesh, aa, bb,
@@ -1373,7 +1472,7 @@ __device__ __noinline__ void sphere_mesh(Cache& c, const PairCtx& x, const MeshS
                 }
                 return m;
             },
-            [&](int f, int i) { sphere_fan_add(c, x, M, f, i, cc, rad, pm); });
+            add_hits(c, x, [&](int f, int i) { return sphere_fan_points(M, f, i, cc, rad, pm); }));
     }
 }
 
@@ -1440,7 +1539,9 @@ __device__ __noinline__ void concave_poly(Cache& c, const PairCtx& x, const Mesh
                 }
                 return 1u;
             },
-            [&](int f, int) { convex_convex<G>(c, x, A, triangle(f), pa, pm, ref_scale, sa); });
+            [&](int hits, const int2* list) {
+                for (int k = 0; k < hits; k++) convex_convex<G>(c, x, A, triangle(list[k].x), pa, pm, ref_scale, sa);
+            });
     }
 }
 

@@ -184,3 +184,30 @@ def test_mesh_walks_longer_than_a_wave_match_oracle():
     for t in ((1, 4), (2, 4), (0, 3), (1, 3), (2, 3)):
         assert t in seen
 
+
+
+@pytest.mark.parametrize("shape,args,y", [(1, (1.0,), 0.2), (1, (0.3,), 0.2), (2, (0.8, 0.8), 0.1), (2, (0.4, 1.5), 0.0)])
+def test_more_contact_points_than_lanes_match_oracle(shape, args, y):
+    """A body sunk into a fine mesh gives more contact points (per face up to three edges and a section) than the
+    wave makes at a time, and far more than a contact cache's eight: which of them stay, and replaced by which,
+    is the sequential order's result."""
+    import pe_amd
+    from pe_amd import scenes
+    from pyoracle import OracleWorld
+    rng = np.random.default_rng(5)
+    b = scenes.SceneBuilder()
+    b.add(scenes.SHAPE_CONCAVE, (), 1.0, (0.0, 0.0, 0.0), kin=1,
+          mesh=b.add_mesh(scenes.heightfield_mesh(rng, 48, 48, (4.0, 4.0), 0.08)))
+    kind = scenes.SHAPE_SPHERE if shape == 1 else scenes.SHAPE_CYLINDER
+    b.add(kind, args, 500.0, (0.03, y, 0.02))
+    sc = b.scene(name="sunk")
+    g, o = pe_amd.World(sc), OracleWorld(sc, 32)
+    for step in range(4):
+        g.integrate(); o.integrate()
+        g.broadphase(); o.broadphase()
+        g.narrowphase(); o.narrowphase()
+        gn, gpts = g.contacts()
+        on, _, opts = o.contacts()
+        assert np.array_equal(gn, on) and on.sum() > 1, f"step {step}: {gn} {on}"
+        vm = np.arange(8)[None, :] < on[:, None]
+        assert _close(gpts[vm], opts[vm]), f"step {step}"
