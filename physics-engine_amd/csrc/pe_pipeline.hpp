@@ -493,8 +493,23 @@ static __device__ __forceinline__ void narrow_pair(const BodyView& b, const Pair
         c.d[k] = p < prev_np ? dprev[k] : REAL_MAX;
     }
     c.trunc = 0;
-    const CollBody A = load_coll(b, ia), B = load_coll(b, ib);
-    PairCtx x;
+    // what the routines take by reference is in LDS too where a wave shares it
+    struct WaveArgs {
+        CollBody A, B;
+        PairCtx x;
+        MeshSet ms;
+        Poly pa, pb;
+    };
+    __shared__ char s_args[G == 1 ? 1 : 4][G == 1 ? 16 : sizeof(WaveArgs)] __attribute__((aligned(16)));
+    CollBody A_reg, B_reg;
+    PairCtx x_reg;
+    WaveArgs* wa = reinterpret_cast<WaveArgs*>(s_args[G == 1 ? 0 : (threadIdx.x / WAVE) % 4]);
+    CollBody& A = G == 1 ? A_reg : wa->A;
+    CollBody& B = G == 1 ? B_reg : wa->B;
+    PairCtx& x = G == 1 ? x_reg : wa->x;
+    A = load_coll(b, ia);
+    B = load_coll(b, ib);
+    if (G > 1) wa->ms = b.ms;
     x.A = A.P;
     x.B = B.P;
     x.swap = false;
@@ -503,23 +518,26 @@ static __device__ __forceinline__ void narrow_pair(const BodyView& b, const Pair
         const float th = (sa < sb ? sa : sb) * 0.02f;
         x.same_th2 = th * th;
     }
-    const int ta = A.type, tb = B.type;
+    const int ta = uni<G>(A.type), tb = uni<G>(B.type);
     bool swapped = false;
     if (COMPOUND) {
         swapped = narrow_compound(b.ms, c, x, A, B, (x.A.scale + x.B.scale) * 0.05f);
     } else if (G > 1) {
         const float ref_scale = (x.A.scale + x.B.scale) * 0.05f;
         if (ta == SHAPE_SPHERE || tb == SHAPE_SPHERE || (ta == SHAPE_CYLINDER) != (tb == SHAPE_CYLINDER)) {
-            narrow_shapes<G>(b.ms, c, x, A, B);   // a sphere or a cylinder with a mesh
+            narrow_shapes<G>(wa->ms, c, x, A, B);   // a sphere or a cylinder with a mesh
         } else if (ta == SHAPE_CONCAVE || tb == SHAPE_CONCAVE) {
             // concave_convex_collision_algorithm.cpp: the convex body is A (narrow_shapes)
             const CollBody& mb = ta == SHAPE_CONCAVE ? A : B;
             const CollBody& ob = ta == SHAPE_CONCAVE ? B : A;
             x.swap = ta == SHAPE_CONCAVE;
-            concave_poly<G>(c, x, b.ms, __float_as_int(mb.sp[0]), mb.P, body_poly(b.ms, ob), ob.P, ref_scale);
+            wa->pa = body_poly(b.ms, ob);
+            concave_poly<G>(c, x, wa->ms, __float_as_int(mb.sp[0]), mb.P, wa->pa, ob.P, ref_scale);
             x.swap = false;
         } else {
-            convex_convex<G>(c, x, body_poly(b.ms, A), body_poly(b.ms, B), A.P, B.P, ref_scale);
+            wa->pa = body_poly(b.ms, A);
+            wa->pb = body_poly(b.ms, B);
+            convex_convex<G>(c, x, wa->pa, wa->pb, A.P, B.P, ref_scale);
         }
     } else if (ta == SHAPE_BOX && tb == SHAPE_BOX) box_box(c, x, A.P, B.P, A.sp, B.sp);
     else if (ta == SHAPE_BOX && tb == SHAPE_SPHERE) box_sphere(c, x, true, A.P, B.P, A.sp, B.sp[0]);

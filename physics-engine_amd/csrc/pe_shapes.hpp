@@ -31,7 +31,7 @@ struct Poly {
     int kind;
     f3 h;               // box: half extents; cylinder: (radius, half height, 0)
     float r2, hgt;      // cylinder: 2 radius, height (the mesh scale)
-    const MeshSet* ms;  // cylinder unit tables / mesh arena
+    const float* cyl;   // cylinder: the unit tables
     const float4* v;    // mesh: vertices, face normals, faces, face indices, edges
     const float4* fn;
     const int2* face;
@@ -42,7 +42,7 @@ struct Poly {
 };
 
 PE_HD f3 cyl_ring(const Poly& P, bool top, int i) {
-    const float* u = P.ms->cyl + (top ? 0 : 40);
+    const float* u = P.cyl + (top ? 0 : 40);
     return f3{u[i] * P.r2, top ? 0.5f * P.hgt : -0.5f * P.hgt, u[20 + i] * P.r2};
 }
 PE_HD int n_faces(const Poly& P) { return P.kind == PK_BOX ? 6 : P.kind == PK_CYL ? 42 : P.kind == PK_MESH ? P.nf : 1; }
@@ -51,7 +51,7 @@ PE_HD f3 face_normal(const Poly& P, int f) {
     if (P.kind == PK_BOX) return f3{(float)BOX_N[f][0], (float)BOX_N[f][1], (float)BOX_N[f][2]};
     if (P.kind == PK_CYL) {
         if (f < 2) return f3{0.0f, f == 0 ? 1.0f : -1.0f, 0.0f};
-        const float* n = P.ms->cyl + 80 + 3 * (f - 2);
+        const float* n = P.cyl + 80 + 3 * (f - 2);
         return f3{n[0], n[1], n[2]};
     }
     if (P.kind == PK_MESH) return ld4(P.fn[f]);
@@ -102,11 +102,28 @@ PE_HD void edge_of(const Poly& P, int e, f3& a, f3& b) {
     }
 }
 
+// A box's and a cylinder's edges by direction: edges of one class have the same direction bit for bit, up to its
+// sign (and the signs of zeros).  A box's twelve edges have three directions; of a cylinder's 80 those of a cap
+// ring are point-symmetric (edge k + 10 is edge k reversed), so they have ten each and the 40 of the
+// side one each, 60 in all.  Every edge of a mesh is a class.
+PE_HD int n_edge_classes(const Poly& P) { return P.kind == PK_BOX ? 3 : P.kind == PK_CYL ? 60 : n_edges(P); }
+PE_HD bool edge_class_mixed(const Poly& P, int u) { return P.kind == PK_CYL && u < 20; }   // has both signs
+// Member m of class u (ascending), -1 past the last; rev: against the direction of the first.
+PE_HD int edge_of_class(const Poly& P, int u, int m, bool& rev) {
+    rev = false;
+    if (P.kind == PK_BOX) return m < 4 ? 4 * u + m : -1;
+    if (P.kind == PK_CYL && u < 20) {
+        rev = m == 1;
+        return m < 2 ? (u < 10 ? u : u + 10) + 10 * m : -1;
+    }
+    return m > 0 ? -1 : P.kind == PK_CYL ? 20 + u : u;
+}
+
 PE_HD Poly poly_box(const float size[3]) {
     Poly P;
     P.kind = PK_BOX;
     P.h = f3{size[0] / 2.0f, size[1] / 2.0f, size[2] / 2.0f};
-    P.ms = nullptr;
+    P.cyl = nullptr;
     return P;
 }
 PE_HD Poly poly_cyl(const MeshSet* ms, float r, float h) {
@@ -115,13 +132,12 @@ PE_HD Poly poly_cyl(const MeshSet* ms, float r, float h) {
     P.h = f3{r, h * 0.5f, 0.0f};
     P.r2 = r * 2.0f;
     P.hgt = h;
-    P.ms = ms;
+    P.cyl = ms->cyl;
     return P;
 }
 PE_HD Poly poly_mesh(const MeshSet* ms, int mesh) {
     Poly P;
     P.kind = PK_MESH;
-    P.ms = ms;
     const int32_t* r = ms->rec + MRW * mesh;
     const float4* A = ms->arena;
     P.v = A + r[MR_V]; P.fn = A + r[MR_FN];
@@ -301,17 +317,6 @@ PE_HD void project_verts_interval(const float4* v, int nv, const Pose& t, f3 axi
     }
     mn += off; mx += off;
 }
-// Shape::localIsInside -- box_shape.cpp:45-49, cylinder_shape.cpp:45-48, convex_mesh_shape.cpp:152-158
-PE_HD bool inside(const Poly& S, f3 q) {
-    if (S.kind == PK_BOX) return fabsf(q.x) <= S.h.x && fabsf(q.y) <= S.h.y && fabsf(q.z) <= S.h.z;
-    if (S.kind == PK_CYL)
-        return q.y >= -S.hgt * 0.5f && q.y <= S.hgt * 0.5f && q.x * q.x + q.z * q.z <= S.h.x * S.h.x;
-    const int nf = n_faces(S);
-    for (int f = 0; f < nf; f++)
-        if (dot(face_normal(S, f), sub(q, face_vertex(S, f, 0))) >= 0) return false;
-    return true;
-}
-
 // ------------------------------------------------------------------ convex SAT + clipping
 // convex_convex_collision_algorithm.cpp
 constexpr int CLIP_CAP = 2 * MAX_FACE_VERTS;   // clipped polygon capacity (a 20-gon cap clipped by 20 planes needs 40)
@@ -344,6 +349,28 @@ PE_HD int clip_face(const f3* in, int nin, f3* out, f3 pn, float pe, int& trunc)
         ds = de;
     }
     return no;
+}
+// What a whole wave was given, as values the compiler knows to be the same on all lanes: they are held in scalar
+// registers, and a branch on a shape's kind is a branch.  The routines below are called with references;
+// without the copies every use of an argument was a load of every lane from its own scratch
+// memory (1.8 KB a lane, more than the caches hold for the waves in flight) and each kind's code a masked block:
+// an edge axis that came down to its witness points took 40 000 cycles.  G = 1: the argument itself.
+template <class T>
+__device__ __forceinline__ T wave_uniform(const T& v) {
+    static_assert(std::is_trivially_copyable<T>::value && sizeof(T) % 4 == 0, "copied as words");
+    int w[sizeof(T) / 4];
+    T r;
+    __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+    for (size_t k = 0; k < sizeof(T) / 4; k++) w[k] = __builtin_amdgcn_readfirstlane(w[k]);
+    __builtin_memcpy(&r, w, sizeof(T));
+    return r;
+}
+template <int G, class T> using Uni = typename std::conditional<G == 1, const T&, const T>::type;
+template <int G, class T>
+__device__ __forceinline__ Uni<G, T> uni(const T& v) {
+    if constexpr (G == 1) return v;
+    else return wave_uniform(v);
 }
 // Lanes that work on one pair together: G = 1 is a thread alone; G = 64 is a whole wave, all
 // of whose lanes hold the same pair, run the same control flow on the same values, and split
@@ -380,6 +407,10 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
+__device__ __forceinline__ float lane_value(float v, int src) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
+}
+__device__ __forceinline__ f3 lane_value(f3 v, int src) { return f3{lane_value(v.x, src), lane_value(v.y, src), lane_value(v.z, src)}; }
 // add_point with a wave on one cache in LDS: lane i (of each eight) looks at slot i, the one chosen writes itself.
 // Called by all lanes with the same values.
 __device__ __forceinline__ float oct_min(float v) {   // over each eight lanes
@@ -440,11 +471,18 @@ __device__ __forceinline__ void add_pt(Cache& c, const PairCtx& x, f3 n, f3 p, f
     else add_point_wave(c, x, n, p, depth);
 }
 
-// clipHullAgainstHull + clipFaceAgainstHull (:63-170)
+// clipHullAgainstHull + clipFaceAgainstHull (:63-170).  With a wave the reference face's planes are made a lane
+// each, and lane k holds the polygon's vertex k: a plane's cut is one step of all lanes, its new polygon
+// numbered by ballots in the order clip_face gives it (a cap clipped by a cap is 20 planes by 20 and more
+// vertices one after the other).
 template <int G>
-__device__ __noinline__ void clip_hull_hull(Cache& c, const PairCtx& x, f3 sep, const Poly& A, const Poly& B,
-                                            const Pose& ta, const Pose& tb, float min_dist, float max_dist) {
+__device__ __noinline__ void clip_hull_hull(Cache& c, const PairCtx& x_, f3 sep_, const Poly& A_, const Poly& B_,
+                                            const Pose& ta_, const Pose& tb_, float min_dist, float max_dist) {
     using L = Grp<G>;
+    Uni<G, PairCtx> x = uni<G>(x_);
+    Uni<G, Poly> A = uni<G>(A_), B = uni<G>(B_);
+    Uni<G, Pose> ta = uni<G>(ta_), tb = uni<G>(tb_);
+    Uni<G, f3> sep = uni<G>(sep_);
     // B's face most along sep (first of the largest), A's face most against it (first of the
     // least): as argmin of (-d, f) and (d, f)
     float bd = REAL_MAX;
@@ -465,34 +503,98 @@ __device__ __noinline__ void clip_hull_hull(Cache& c, const PairCtx& x, f3 sep, 
     }
     L::argmin(ad, ca);
     if (ca == 0x7fffffff) return;
-    // polygon buffers: a lane's own (scratch) when it works alone; one copy per wave in LDS when the
-    // wave's lanes work together (every lane writes the same value to the same word)
-    f3 pbuf0[G == 1 ? CLIP_CAP : 1], pbuf1[G == 1 ? CLIP_CAP : 1];
-    __shared__ f3 s_clip[G == 1 ? 1 : 4][2][CLIP_CAP];
-    f3* buf0 = G == 1 ? pbuf0 : s_clip[(threadIdx.x / WAVE) % 4][0];
-    f3* buf1 = G == 1 ? pbuf1 : s_clip[(threadIdx.x / WAVE) % 4][1];
-    int n = face_len(B, cb);
-    for (int k = 0; k < n; k++) buf0[k] = xf_apply(tb, face_vertex(B, cb, k));
-    const int nva = face_len(A, ca);
-    const f3 wn = mv(ta.R, face_normal(A, ca));
-    f3* pin = buf0;
-    f3* pout = buf1;
-    for (int e0 = 0; e0 < nva; e0++) {
-        const f3 a = face_vertex(A, ca, e0), b = face_vertex(A, ca, (e0 + 1) % nva);
-        const f3 ew = mv(ta.R, sub(a, b));
-        const f3 pn = neg(cross(ew, wn));
-        const f3 wa = xf_apply(ta, a);
-        const float pe = -dot(wa, pn);
-        n = clip_face(pin, n, pout, pn, pe, c.trunc);
-        f3* t = pin; pin = pout; pout = t;
+    if constexpr (G == 1) {
+        f3 buf0[CLIP_CAP], buf1[CLIP_CAP];
+        int n = face_len(B, cb);
+        for (int k = 0; k < n; k++) buf0[k] = xf_apply(tb, face_vertex(B, cb, k));
+        const int nva = face_len(A, ca);
+        const f3 wn = mv(ta.R, face_normal(A, ca));
+        f3* pin = buf0;
+        f3* pout = buf1;
+        for (int e0 = 0; e0 < nva; e0++) {
+            const f3 a = face_vertex(A, ca, e0), b = face_vertex(A, ca, (e0 + 1) % nva);
+            const f3 ew = mv(ta.R, sub(a, b));
+            const f3 pn = neg(cross(ew, wn));
+            const f3 wa = xf_apply(ta, a);
+            const float pe = -dot(wa, pn);
+            n = clip_face(pin, n, pout, pn, pe, c.trunc);
+            f3* t = pin; pin = pout; pout = t;
+        }
+        const f3 pv = face_vertex(A, ca, 0);
+        const f3 ln = face_normal(A, ca);
+        for (int i = 0; i < n; i++) {
+            const f3 vtx = pin[i];
+            const float depth = dot(ln, sub(xf_inv(ta, vtx), pv));
+            if (depth <= max_dist && depth >= min_dist) add_point(c, x, sep, sub(vtx, mul(sep, 0.0f)), depth + 0.0f * 2);
+        }
+    } else {
+        static_assert(CLIP_CAP <= WAVE, "a lane per vertex");
+        __shared__ f3 s_clip[4][CLIP_CAP];
+        f3* poly = s_clip[(threadIdx.x / WAVE) % 4];
+        const int lane = (int)(threadIdx.x & (WAVE - 1));
+        cb = __builtin_amdgcn_readfirstlane(cb);
+        ca = __builtin_amdgcn_readfirstlane(ca);
+        int n = __builtin_amdgcn_readfirstlane(face_len(B, cb));
+        const int nva = __builtin_amdgcn_readfirstlane(face_len(A, ca));
+        const f3 ln = face_normal(A, ca);
+        f3 v{0, 0, 0}, pn{0, 0, 0};
+        float pe = 0;
+        if (lane < n) v = xf_apply(tb, face_vertex(B, cb, lane));
+        if (lane < nva) {
+            const f3 a = face_vertex(A, ca, lane), b = face_vertex(A, ca, (lane + 1) % nva);
+            const f3 ew = mv(ta.R, sub(a, b));
+            pn = neg(cross(ew, mv(ta.R, ln)));
+            pe = -dot(xf_apply(ta, a), pn);
+        }
+        for (int e0 = 0; e0 < nva; e0++) {
+            if (n < 2) { n = 0; break; }
+            const f3 q = lane_value(pn, e0);
+            const float de = dot(q, v) + lane_value(pe, e0);
+            const int prev = lane == 0 ? n - 1 : lane - 1;
+            const f3 first{__shfl(v.x, prev), __shfl(v.y, prev), __shfl(v.z, prev)};
+            const float ds = __shfl(de, prev);
+            const bool in = lane < n;
+            const bool out_s = in && ds < 0, out_e = in && de < 0;
+            const bool one = out_s || out_e, two = !out_s && out_e;
+            const uint64_t m1 = __ballot(one), m2 = __ballot(two);
+            if (m1 == __ballot(in && out_s && out_e) && m2 == 0) {   // nothing cut
+                if (m1 != __ballot(in)) { n = 0; break; }
+                continue;
+            }
+            const int at = (int)(__popcll(m1 & lanemask_lt()) + __popcll(m2 & lanemask_lt()));
+            const int total = (int)(__popcll(m1) + __popcll(m2));
+            wave_lds_sync();
+            if (one) {
+                const f3 cut = add(first, mul(sub(v, first), ds * 1.0f / (ds - de)));
+                if (at < CLIP_CAP) poly[at] = out_s && out_e ? v : cut;
+                if (two && at + 1 < CLIP_CAP) poly[at + 1] = v;
+            }
+            wave_lds_sync();
+            if (total > CLIP_CAP) c.trunc = 1;
+            n = total < CLIP_CAP ? total : CLIP_CAP;
+            v = lane < n ? poly[lane] : f3{0, 0, 0};
+        }
+        const f3 pv = face_vertex(A, ca, 0);
+        const float depth = dot(ln, sub(xf_inv(ta, v), pv));
+        uint64_t keep = __ballot(lane < n && depth <= max_dist && depth >= min_dist);
+        while (keep) {
+            const int k = __ffsll((unsigned long long)keep) - 1;
+            keep &= keep - 1;
+            add_point_wave(c, x, sep, sub(lane_value(v, k), mul(sep, 0.0f)), lane_value(depth, k) + 0.0f * 2);
+        }
     }
-    const f3 pv = face_vertex(A, ca, 0);
-    const f3 ln = face_normal(A, ca);
-    for (int i = 0; i < n; i++) {
-        const f3 vtx = pin[i];
-        const float depth = dot(ln, sub(xf_inv(ta, vtx), pv));
-        if (depth <= max_dist && depth >= min_dist) add_pt<G>(c, x, sep, sub(vtx, mul(sep, 0.0f)), depth + 0.0f * 2);
-    }
+}
+// Shape::localIsInside -- box_shape.cpp:45-49, cylinder_shape.cpp:45-48, convex_mesh_shape.cpp:152-158; a mesh's faces
+// over the lanes.
+template <int G>
+__device__ __forceinline__ bool inside(const Poly& S, f3 q) {
+    if (S.kind == PK_BOX) return fabsf(q.x) <= S.h.x && fabsf(q.y) <= S.h.y && fabsf(q.z) <= S.h.z;
+    if (S.kind == PK_CYL)
+        return q.y >= -S.hgt * 0.5f && q.y <= S.hgt * 0.5f && q.x * q.x + q.z * q.z <= S.h.x * S.h.x;
+    const int nf = n_faces(S);
+    bool out = false;
+    for (int f = Grp<G>::rank(); f < nf && !out; f += G) out = dot(face_normal(S, f), sub(q, face_vertex(S, f, 0))) >= 0;
+    return !Grp<G>::any(out);
 }
 // testSepAxis (:216-243)
 // projA(ax, mn, mx, pmn, pmx) and projB: Shape::project of the two shapes.
@@ -535,10 +637,26 @@ __device__ __forceinline__ void mesh_to_lds(const Poly& P, float4* row) {
 // The same for the world directions of both shapes' edges (up to EDGE_LDS_DIRS each), the operands
 // every edge-pair axis reads: computed once per pair instead of once per axis.
 constexpr int EDGE_LDS_DIRS = 128;
+// Edge axes are tested per pair of edge classes: the 6400 axes of two cylinders are 3600 different ones, a box's
+// with a mesh of n edges 3 n of 12 n.  An axis kept still has to have its witness points on its edges, so
+// its first edges that do are looked for among the classes'.
 // isOnLine (:245-249)
 PE_HD bool on_line(f3 v0, f3 v1, f3 v2) {
     const f3 n = cross(sub(v1, v0), sub(v2, v0));
     return dot(n, n) < EPS;
+}
+// The first edge of class u with local point q on its line, of want's direction only unless want is 0 (1: the
+// class's first edge's, -1: the reverse); -1: none.
+PE_HD int first_on_line(const Poly& P, int u, f3 q, int want) {
+    for (int m = 0;; m++) {
+        bool rev;
+        const int e = edge_of_class(P, u, m, rev);
+        if (e < 0) return -1;
+        if (want != 0 && rev != (want < 0)) continue;
+        f3 p0, p1;
+        edge_of(P, e, p0, p1);
+        if (on_line(p0, p1, q)) return e;
+    }
 }
 // findSeparatingAxis (:251-402) + ConvexConvexCollisionAlgorithm::getClosestPoints (:408-432).
 // The deep-point contact is added before the edge axes are tested and stays even when an edge
@@ -554,9 +672,12 @@ PE_HD bool on_line(f3 v0, f3 v1, f3 v2) {
 template <int G>
 // keep_a (a wave only): the wave's LDS already holds A's vertex copy, staged by its previous call
 // with the same A (the triangles of one concave pair), so it is not staged again.
-__device__ __noinline__ void convex_convex(Cache& c, const PairCtx& x, const Poly& A, const Poly& B, const Pose& ta,
-                                           const Pose& tb, float ref_scale, bool keep_a = false) {
+__device__ __noinline__ void convex_convex(Cache& c, const PairCtx& x_, const Poly& A_, const Poly& B_, const Pose& ta_,
+                                           const Pose& tb_, float ref_scale, bool keep_a = false) {
     using L = Grp<G>;
+    Uni<G, PairCtx> x = uni<G>(x_);
+    Uni<G, Poly> A = uni<G>(A_), B = uni<G>(B_);
+    Uni<G, Pose> ta = uni<G>(ta_), tb = uni<G>(tb_);
     const f3 dc = sub(ta.p, tb.p);
     float dmin = REAL_MAX;
     f3 dmin_pt{0, 0, 0}, sep{0, 0, 0};
@@ -617,7 +738,7 @@ __device__ __noinline__ void convex_convex(Cache& c, const PairCtx& x, const Pol
             dmin_pt = pt_on_a ? add(wa, mul(sep, dmin)) : wb;
         }
     }
-    if ((pt_on_a && inside(B, xf_inv(tb, dmin_pt))) || (!pt_on_a && inside(A, xf_inv(ta, dmin_pt))))
+    if (pt_on_a ? inside<G>(B, xf_inv(tb, dmin_pt)) : inside<G>(A, xf_inv(ta, dmin_pt)))
         add_pt<G>(c, x, sep, sub(dmin_pt, mul(sep, 0.0f)), -dmin + 0.0f * 2);
     int ea = -1, eb = -1;
     f3 wea{0, 0, 0}, web{0, 0, 0}, wpa{0, 0, 0}, wpb{0, 0, 0};
@@ -626,80 +747,87 @@ __device__ __noinline__ void convex_convex(Cache& c, const PairCtx& x, const Pol
         float bd = dmin;
         int bi = 0x7fffffff;
         bool separated = false;
-        const int ne = nea * neb;
-        // with a wave: B's world edge directions (the inner loop's operand), computed once into LDS
+        const int nca = n_edge_classes(A), ncb = n_edge_classes(B);
+        const int ne = nca * ncb;
+        auto dir_of = [](const Poly& P, const Pose& tp, int e) {
+            f3 p0, p1;
+            edge_of(P, e, p0, p1);
+            return mv(tp.R, normalized(sub(p0, p1)));
+        };
+        auto dir_of_class = [&](const Poly& P, const Pose& tp, int u) {
+            bool rev;
+            return dir_of(P, tp, edge_of_class(P, u, 0, rev));
+        };
+        // with a wave: the classes' world directions, computed once into LDS
         __shared__ float4 s_edir[G == 1 ? 1 : 4][2][G == 1 ? 1 : EDGE_LDS_DIRS];
         float4* adir = s_edir[G == 1 ? 0 : (threadIdx.x / WAVE) % 4][0];
         float4* edir = s_edir[G == 1 ? 0 : (threadIdx.x / WAVE) % 4][1];
-        const bool sea = G > 1 && nea <= EDGE_LDS_DIRS;
-        const bool se = G > 1 && neb <= EDGE_LDS_DIRS;
+        const bool sea = G > 1 && nca <= EDGE_LDS_DIRS;
+        const bool se = G > 1 && ncb <= EDGE_LDS_DIRS;
         if (G > 1 && (sea || se)) {
             wave_lds_sync();
             if (sea) {
-                for (int e = L::rank(); e < nea; e += G) {
-                    f3 p0, p1;
-                    edge_of(A, e, p0, p1);
-                    const f3 d = mv(ta.R, normalized(sub(p0, p1)));
+                for (int e = L::rank(); e < nca; e += G) {
+                    const f3 d = dir_of_class(A, ta, e);
                     adir[e] = make_float4(d.x, d.y, d.z, 0.0f);
                 }
             }
             if (se) {
-                for (int e = L::rank(); e < neb; e += G) {
-                    f3 b0, b1;
-                    edge_of(B, e, b0, b1);
-                    const f3 d = mv(tb.R, normalized(sub(b0, b1)));
+                for (int e = L::rank(); e < ncb; e += G) {
+                    const f3 d = dir_of_class(B, tb, e);
                     edir[e] = make_float4(d.x, d.y, d.z, 0.0f);
                 }
             }
             wave_lds_sync();
         }
-        auto dir_a = [&](int e) {
-            if (sea) return ld4(adir[e]);
-            f3 p0, p1;
-            edge_of(A, e, p0, p1);
-            return mv(ta.R, normalized(sub(p0, p1)));
-        };
-        auto dir_b = [&](int e) {
-            if (se) return ld4(edir[e]);
-            f3 p0, p1;
-            edge_of(B, e, p0, p1);
-            return mv(tb.R, normalized(sub(p0, p1)));
-        };
         int t = L::rank();
-        int e0 = t / neb, e1 = t - e0 * neb;
+        int e0 = t / ncb, e1 = t - e0 * ncb;
         int cur0 = -1;
         f3 we0{0, 0, 0};
         for (; t < ne; t += G) {
             if (e0 != cur0) {
-                we0 = dir_a(e0);
+                we0 = sea ? ld4(adir[e0]) : dir_of_class(A, ta, e0);
                 cur0 = e0;
             }
-            f3 cr = cross(we0, dir_b(e1));
+            f3 cr = cross(we0, se ? ld4(edir[e1]) : dir_of_class(B, tb, e1));
             if (!(fabsf(norm(cr) - 0.0f) < EPS)) {
                 cr = normalized(cr);
-                if (dot(dc, cr) < 0) cr = mul(cr, -1.0f);
-                float dist;
-                if (!test_depth(cr, dist)) { separated = true; break; }
-                if (dist < bd) {
-                    f3 wa, wb, p0, p1;
-                    test_axis(cr, dist, wa, wb);
-                    edge_of(A, e0, p0, p1);
-                    if (on_line(p0, p1, xf_inv(ta, wa))) {
-                        edge_of(B, e1, p0, p1);
-                        if (on_line(p0, p1, xf_inv(tb, wb))) { bd = dist; bi = t; }
+                const float side = dot(dc, cr);
+                if (side < 0) cr = mul(cr, -1.0f);
+                // an axis is turned along dc, so its edges' signs do not matter unless it is square to dc:
+                // then it stays as its edges gave it, and a class of both signs has it both ways
+                const bool square = !(side < 0) && !(side > 0);
+                const bool both = square && (edge_class_mixed(A, e0) || edge_class_mixed(B, e1));
+                for (int way = 1; way >= (both ? -1 : 1) && !separated; way -= 2) {
+                    if (way < 0) cr = mul(cr, -1.0f);
+                    float dist;
+                    if (!test_depth(cr, dist)) { separated = true; break; }
+                    if (dist < bd || (dist == bd && bi != 0x7fffffff)) {
+                        f3 wa, wb;
+                        test_axis(cr, dist, wa, wb);
+                        wa = xf_inv(ta, wa);
+                        wb = xf_inv(tb, wb);
+                        for (int sg = 1; sg >= (both ? -1 : 1); sg -= 2) {
+                            const int fa = first_on_line(A, e0, wa, both ? sg : 0);
+                            const int fb = fa < 0 ? -1 : first_on_line(B, e1, wb, both ? sg * way : 0);
+                            if (fb < 0) continue;
+                            const int q = fa * neb + fb;
+                            if (dist < bd || q < bi) { bd = dist; bi = q; }
+                        }
                     }
                 }
+                if (separated) break;
             }
             e1 += G;
-            while (e1 >= neb) { e1 -= neb; e0++; }
+            while (e1 >= ncb) { e1 -= ncb; e0++; }
         }
         if (L::any(separated)) return;
         L::argmin(bd, bi);
         if (bi != 0x7fffffff) {
             ea = bi / neb;
             eb = bi - ea * neb;
-            wea = dir_a(ea);
-            web = dir_b(eb);
+            wea = dir_of(A, ta, ea);
+            web = dir_of(B, tb, eb);
             sep = normalized(cross(wea, web));
             if (dot(dc, sep) < 0) sep = mul(sep, -1.0f);
             test_axis(sep, dmin, wpa, wpb);
@@ -742,7 +870,7 @@ __device__ __noinline__ void convex_convex(Cache& c, const PairCtx& x, const Pol
         }
     }
     if (dot(dc, sep) < 0) sep = neg(sep);
-    clip_hull_hull<G>(c, x, sep, A, B, ta, tb, -ref_scale, 0.0f);
+    clip_hull_hull<G>(c, x_, sep, A_, B_, ta_, tb_, -ref_scale, 0.0f);
 }
 
 // ------------------------------------------------------------------ sphere-cylinder
@@ -1099,10 +1227,6 @@ __device__ inline int bvh_gather_wave(const MeshSet& ms, int mesh, f3 aa, f3 bb,
     wave_lds_sync();
     return n;
 }
-__device__ __forceinline__ float lane_value(float v, int src) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
-}
-__device__ __forceinline__ f3 lane_value(f3 v, int src) { return f3{lane_value(v.x, src), lane_value(v.y, src), lane_value(v.z, src)}; }
 // What a lane's faces give, added in the walk's order.  test(f), on the lane that holds face f, returns the bit
 // mask of f's items (the routine's own units: triangles of a fan, segments, edges) that give contact points;
 // the items that do are numbered in order, face by face and item by item -- the order in which a
@@ -1320,8 +1444,13 @@ PE_HD FacePoints cyl_edge_points(const Poly& M, int f, int i, const CylInMesh& q
 // The whole routine for the mesh of a convex or concave body (pm: mesh body pose): G = 1 on one
 // lane; G = WAVE on a wave's lanes, the faces of each walk split over them (bvh_faces_wave).
 template <int G = 1>
-__device__ __noinline__ void cylinder_mesh(Cache& c, const PairCtx& x, const MeshSet& ms, int mesh, const Pose& pm,
-                                           const Pose& pcy, float rad, float height) {
+__device__ __noinline__ void cylinder_mesh(Cache& c, const PairCtx& x_, const MeshSet& ms_, int mesh_, const Pose& pm_,
+                                           const Pose& pcy_, float rad_, float height_) {
+    Uni<G, PairCtx> x = uni<G>(x_);
+    Uni<G, MeshSet> ms = uni<G>(ms_);
+    Uni<G, Pose> pm = uni<G>(pm_), pcy = uni<G>(pcy_);
+    Uni<G, int> mesh = uni<G>(mesh_);
+    Uni<G, float> rad = uni<G>(rad_), height = uni<G>(height_);
     const Poly M = poly_mesh(&ms, mesh);
     const CylInMesh q = cyl_in_mesh(pm, pcy, rad, height);
     if (G == 1) {
@@ -1450,8 +1579,13 @@ PE_HD FacePoints sphere_fan_points(const Poly& M, int f, int i, f3 cc, float rad
     return o;
 }
 template <int G = 1>
-__device__ __noinline__ void sphere_mesh(Cache& c, const PairCtx& x, const MeshSet& ms, int mesh, const Pose& pm,
-                                         const Pose& psph, float rad) {
+__device__ __noinline__ void sphere_mesh(Cache& c, const PairCtx& x_, const MeshSet& ms_, int mesh_, const Pose& pm_,
+                                         const Pose& psph_, float rad_) {
+    Uni<G, PairCtx> x = uni<G>(x_);
+    Uni<G, MeshSet> ms = uni<G>(ms_);
+    Uni<G, Pose> pm = uni<G>(pm_), psph = uni<G>(psph_);
+    Uni<G, int> mesh = uni<G>(mesh_);
+    Uni<G, float> rad = uni<G>(rad_);
     const Poly M = poly_mesh(&ms, mesh);
     const f3 cc = xf_inv(pm, psph.p);
     const f3 aa = sub(cc, f3{rad, rad, rad}), bb = add(cc, f3{rad, rad, rad});
@@ -1481,8 +1615,12 @@ __device__ __noinline__ void sphere_mesh(Cache& c, const PairCtx& x, const MeshS
 // each triangle of a BVH leaf overlapping the polyhedron's box (in the mesh frame) is a one-face
 // shape without unique edges, run through the convex routine with the polyhedron as A.
 template <int G>
-__device__ __noinline__ void concave_poly(Cache& c, const PairCtx& x, const MeshSet& ms, int mesh, const Pose& pm,
-                                          const Poly& A, const Pose& pa, float ref_scale) {
+__device__ __noinline__ void concave_poly(Cache& c, const PairCtx& x_, const MeshSet& ms_, int mesh_, const Pose& pm_,
+                                          const Poly& A_, const Pose& pa_, float ref_scale) {
+    Uni<G, MeshSet> ms = uni<G>(ms_);
+    Uni<G, Pose> pm = uni<G>(pm_), pa = uni<G>(pa_);
+    Uni<G, Poly> A = uni<G>(A_);
+    Uni<G, int> mesh = uni<G>(mesh_);
     const Pose rel = pose_mul(pose_inv(pm), pa);
     f3 aa, bb;
     if (A.kind == PK_BOX) {
@@ -1501,9 +1639,8 @@ __device__ __noinline__ void concave_poly(Cache& c, const PairCtx& x, const Mesh
     }
     const Poly M = poly_mesh(&ms, mesh);
     auto triangle = [&](int f) {
-        Poly T;
+        Poly T{};
         T.kind = PK_TRI;
-        T.ms = &ms;
         T.t[0] = face_vertex(M, f, 0);
         T.t[1] = face_vertex(M, f, 1);
         T.t[2] = face_vertex(M, f, 2);
@@ -1511,7 +1648,7 @@ __device__ __noinline__ void concave_poly(Cache& c, const PairCtx& x, const Mesh
         return T;
     };
     if constexpr (G == 1) {
-        bvh_visit(ms, mesh, aa, bb, [&](int f) { convex_convex<1>(c, x, A, triangle(f), pa, pm, ref_scale); });
+        bvh_visit(ms, mesh, aa, bb, [&](int f) { convex_convex<1>(c, x_, A_, triangle(f), pa_, pm_, ref_scale); });
     } else {
         // Most triangles of the leaves are separated from the polyhedron, and the convex routine gives no point
         // for one that any of its face axes separates: each lane first tests a triangle of its own along the
@@ -1540,7 +1677,12 @@ __device__ __noinline__ void concave_poly(Cache& c, const PairCtx& x, const Mesh
                 return 1u;
             },
             [&](int hits, const int2* list) {
-                for (int k = 0; k < hits; k++) convex_convex<G>(c, x, A, triangle(list[k].x), pa, pm, ref_scale, sa);
+                __shared__ Poly s_tri[4];   // (an argument by reference: not in scratch memory)
+                Poly& T = s_tri[(threadIdx.x / WAVE) % 4];
+                for (int k = 0; k < hits; k++) {
+                    T = triangle(list[k].x);
+                    convex_convex<G>(c, x_, A_, T, pa_, pm_, ref_scale, sa);
+                }
             });
     }
 }

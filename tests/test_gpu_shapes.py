@@ -211,3 +211,51 @@ def test_more_contact_points_than_lanes_match_oracle(shape, args, y):
         assert np.array_equal(gn, on) and on.sum() > 1, f"step {step}: {gn} {on}"
         vm = np.arange(8)[None, :] < on[:, None]
         assert _close(gpts[vm], opts[vm]), f"step {step}"
+
+
+@pytest.mark.parametrize("kinds", [(2, 2), (0, 2), (2, 3), (0, 3), (2, 4), (3, 3)])
+@pytest.mark.parametrize("turn", [0, 1, 2])
+def test_aligned_bodies_whose_edge_axes_tie_match_oracle(kinds, turn):
+    """Aligned shapes: many edge axes share a direction and a depth, and many are square to the line between the
+    centres, where an axis keeps the sign its own edges give it.  The first such axis in the order of the edges is
+    the one a sequential scan ends with."""
+    import pe_amd
+    from pe_amd import scenes
+    from pyoracle import OracleWorld
+    rng = np.random.default_rng(3)
+    turns = [np.eye(3), np.array([[0.0, -1.0, 0.0], [1.0, 0.0, 0.0], [0.0, 0.0, 1.0]]),
+             np.array([[1.0, 0.0, 0.0], [0.0, 0.0, -1.0], [0.0, 1.0, 0.0]])]
+    cube = np.array([[x, y, z] for x in (-0.5, 0.5) for y in (-0.5, 0.5) for z in (-0.5, 0.5)])
+    b = scenes.SceneBuilder()
+    hull = b.add_mesh(scenes.hull_mesh(cube))
+    field = b.add_mesh(scenes.heightfield_mesh(rng, 8, 8, (3.0, 3.0), 0.0))
+    for col, (dx, dz) in enumerate([(0.0, 0.0), (0.25, 0.0), (0.0, -0.125), (0.5, 0.5)]):
+        for k, kind in enumerate(kinds[::-1]):
+            at = (8.0 * col + k * dx, 0.98 * k if kinds[1] != 4 else 0.49 * k, k * dz)
+            R = turns[turn] if k else np.eye(3)
+            if kind == 0:
+                b.add(scenes.SHAPE_BOX, (1.0, 1.0, 1.0), 1000.0, at, R, kin=1 - k)
+            elif kind == 2:
+                b.add(scenes.SHAPE_CYLINDER, (0.5, 1.0), 785.0, at, R, kin=1 - k)
+            elif kind == 3:
+                b.add(scenes.SHAPE_CONVEX, (), 1000.0, at, R, kin=1 - k, mesh=hull)
+            else:
+                b.add(scenes.SHAPE_CONCAVE, (), 1.0, at, kin=1, mesh=field)
+    sc = b.scene(name="aligned")
+    g, o = pe_amd.World(sc), OracleWorld(sc, 32)
+    touched = 0
+    for step in range(6):
+        g.integrate(); o.integrate()
+        g.broadphase(); o.broadphase()
+        assert np.array_equal(g.pairs(), o.pairs()), f"pair order step {step}"
+        g.narrowphase(); o.narrowphase()
+        gn, gpts = g.contacts()
+        on, _, opts = o.contacts()
+        assert np.array_equal(gn, on), f"step {step}: {gn} {on}"
+        touched += int(on.sum())
+        vm = np.arange(8)[None, :] < on[:, None]
+        assert _close(gpts[vm], opts[vm]), f"contact points step {step}"
+        g.solve(); o.solve()
+        g.sync()
+        o.set_state(*[np.asarray(x, np.float64) for x in g.state()])
+    assert touched > 0
