@@ -63,6 +63,11 @@ PE_HD int face_len(const Poly& P, int f) {
     if (P.kind == PK_MESH) return P.face[f].y;
     return 3;
 }
+// Vertex k of a triangle: by selects, an index would keep the whole Poly in memory.
+PE_HD f3 tri_vertex(const Poly& P, int k) {
+    const f3 a = P.t[0], b = P.t[1], c = P.t[2];
+    return f3{k == 0 ? a.x : k == 1 ? b.x : c.x, k == 0 ? a.y : k == 1 ? b.y : c.y, k == 0 ? a.z : k == 1 ? b.z : c.z};
+}
 // k-th vertex of face f
 PE_HD f3 face_vertex(const Poly& P, int f, int k) {
     if (P.kind == PK_BOX) {
@@ -80,7 +85,7 @@ PE_HD f3 face_vertex(const Poly& P, int f, int k) {
         return k == 0 ? cyl_ring(P, true, j) : cyl_ring(P, false, k == 1 ? (j + 19) % 20 : j);
     }
     if (P.kind == PK_MESH) return ld4(P.v[P.fi[P.face[f].x + k]]);
-    return P.t[k];
+    return tri_vertex(P, k);
 }
 PE_HD void edge_of(const Poly& P, int e, f3& a, f3& b) {
     if (P.kind == PK_BOX) {
@@ -249,7 +254,7 @@ PE_HD void project(const Poly& S, const Pose& t, f3 axis, float& mn, float& mx, 
         f3 lmn{0, 0, 0}, lmx{0, 0, 0};
         const int nv = S.kind == PK_MESH ? S.nv : 3;
         for (int i = 0; i < nv; i++) {
-            const f3 q = S.kind == PK_MESH ? ld4(S.v[i]) : S.t[i];
+            const f3 q = S.kind == PK_MESH ? ld4(S.v[i]) : tri_vertex(S, i);
             const float x = dot(q, la);
             if (x < mn) { mn = x; lmn = q; }
             else if (x > mx) { mx = x; lmx = q; }
@@ -297,7 +302,7 @@ PE_HD void project_interval(const Poly& S, const Pose& t, f3 axis, float& mn, fl
         mn = REAL_MAX; mx = REAL_MIN;
         const int nv = S.kind == PK_MESH ? S.nv : 3;
         for (int i = 0; i < nv; i++) {
-            const float x = dot(S.kind == PK_MESH ? ld4(S.v[i]) : S.t[i], la);
+            const float x = dot(S.kind == PK_MESH ? ld4(S.v[i]) : tri_vertex(S, i), la);
             const bool lt = x < mn;
             mn = lt ? x : mn;
             mx = !lt && x > mx ? x : mx;
@@ -353,7 +358,7 @@ PE_HD int clip_face(const f3* in, int nin, f3* out, f3 pn, float pe, int& trunc)
 // What a whole wave was given, as values the compiler knows to be the same on all lanes: they are held in scalar
 // registers, and a branch on a shape's kind is a branch.  The routines below are called with references;
 // without the copies every use of an argument was a load of every lane from its own scratch
-// memory (1.8 KB a lane, more than the caches hold for the waves in flight) and each kind's code a masked block:
+// memory (1.8 KB a lane, 0.7 now, more than the caches hold for the waves in flight) and each kind's code a masked block:
 // an edge axis that came down to its witness points took 40 000 cycles.  G = 1: the argument itself.
 template <class T>
 __device__ __forceinline__ T wave_uniform(const T& v) {
