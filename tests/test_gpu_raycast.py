@@ -80,3 +80,42 @@ def test_raycast_matches_oracle(name):
     print(f"[raycast] {name}: {hits} hits ({mesh} on meshes), {partial} queries ended early with a partial "
           f"result, of {len(rays)}", flush=True)
     g.close()
+
+
+@pytest.mark.parametrize("count", [1023, 1024, 1027])
+@pytest.mark.parametrize("basis", ["turned", "scaled"])
+def test_many_rays_sharing_a_pass_match_oracle(count, basis):
+    """From 1024 rays on several share a workgroup, and boxes a ray passes well clear of are left out by a bound:
+    grazing rays, rays along the axes, directions of other lengths than 1, starts far off and bases that
+    are no rotations (where the bound does not hold and is not used) give the oracle's results."""
+    import pe_amd
+    from pyoracle import OracleWorld
+    sc = small_rain(90, seed=11)
+    rng = np.random.default_rng(count)
+    g, o = pe_amd.World(sc), OracleWorld(sc, 32)
+    pos, rot, v, w = (np.array(x, np.float32) for x in g.state())
+    if basis == "scaled":
+        rot[::2] = rot[::2] * np.float32(1.7)
+        rot[1::4] = rot[1::4] * np.float32(0.4)
+    g.set_state(pos, rot, v, w)
+    o.set_state(*[x.astype(np.float64) for x in (pos, rot, v, w)])
+    body = rng.integers(0, sc.n, count)
+    far = rng.choice([0.0, 3.0, 60.0], count)[:, None]
+    at = pos[body] + rng.uniform(-0.8, 0.8, (count, 3))      # past, along and through the faces and corners
+    d = rng.normal(size=(count, 3))
+    axis = rng.random(count) < 0.3
+    d[axis] = np.eye(3)[rng.integers(0, 3, axis.sum())] * rng.choice([-1.0, 1.0], axis.sum())[:, None]
+    d /= np.linalg.norm(d, axis=1)[:, None]
+    st = (at - far * d).astype(np.float32)
+    d = (d * rng.choice([1.0, 1.0, 0.05, 0.5, 4.0], count)[:, None]).astype(np.float32)
+    ln = rng.uniform(0.5, 300.0, count).astype(np.float32)
+    print(f"[raycast] {count} rays at once, {basis}", flush=True)
+    gh, gb, gd, gp, gn = g.raycast(st, d, ln)
+    hits = 0
+    for k in range(count):
+        oh, ob, od, op, on = o.raycast(st[k].astype(np.float64), d[k].astype(np.float64), float(ln[k]))
+        assert bool(gh[k]) == oh and int(gb[k]) == ob and gd[k] == np.float32(od), f"ray {k}"
+        assert np.array_equal(gp[k], op.astype(np.float32)) and np.array_equal(gn[k], on.astype(np.float32)), f"ray {k}"
+        hits += oh
+    assert hits > count // 4
+    g.close()
