@@ -2,14 +2,14 @@
 //
 // Per step, on one HIP stream, no host synchronisation:
 //   k_integrate        World::updateObjectStatus + applyExternalForce    (thread / body)
-//   k_sap_*            sweep-and-prune broadphase over the body store (pe_sap.hpp): stable
-//                      radix sort on aabb_min[axis], candidate runs, load-balanced sweep in the
+//   k_sap_*            sweep-and-prune broadphase over the body store (pe_sap.hpp): stable sort
+//                      on aabb_min[axis], candidate runs, load-balanced sweep in the
 //                      reference's (i, j) order, next axis
 //   k_narrow           thread / pair: shape dispatch + 8-slot contact cache + depth sort
 //   k_setup            thread / pair: solver rows (FrictionContactConstraint::initSequentialImpulse)
 //   k_solve_small      worlds of up to 600 bodies: colouring and sweeps in one workgroup, on LDS; else
 //   k_jp_*             the constraint graph: per body its pairs
-//   k_solve_flow       cooperative launch over the whole GPU: colouring, then the Gauss-Seidel sweeps in
+//   k_solve_flow       one launch over the whole GPU: colouring, then the Gauss-Seidel sweeps in
 //                      colour order as a data flow between the pairs, and the velocity sync
 #include "pe_common.hpp"
 #include "pe_device.hpp"
@@ -1415,7 +1415,7 @@ __global__ void __launch_bounds__(256) k_count_points(Dev d) {
 }  // namespace
 
 // ====================================================================== host side
-// Workgroups of the cooperative solve: enough waves for about an item each (a world at rest has up to
+// Workgroups of the solve over the GPU: enough waves for about an item each (a world at rest has up to
 // two pairs with contacts per body, 16 to an item), at most one workgroup per CU of the 256.
 static int default_flow_blocks(int n, int max_blocks) { return std::min(max_blocks, std::max(8, std::min(256, n / 80))); }
 
@@ -1762,7 +1762,7 @@ int pe_world_create(const pe_scene_desc* sc, const pe_world_params* prm, int32_t
         int dev = 0, cus = 0, per_cu = 0;
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
             hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k_solve_flow, FLOW_THREADS, 0) != hipSuccess || per_cu < 1) {
-            pe_set_error("cannot size the cooperative solver grid");
+            pe_set_error("cannot size the solver grid");
             return fail(PE_ERR_DEVICE);
         }
         if (hipFuncSetAttribute((const void*)k_solve_small, hipFuncAttributeMaxDynamicSharedMemorySize, SMALL_LDS) != hipSuccess) {
