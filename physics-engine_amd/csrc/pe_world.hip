@@ -348,6 +348,7 @@ __global__ void k_events(Dev d) {
 __global__ void __launch_bounds__(128) k_narrow(Dev d) {
     const int np = d.cnt->npairs;
     const int prev = d.cnt->prev_npairs;
+    if (blockIdx.x == 0 && threadIdx.x == 0) d.cnt->npoints = 0;   // summed by k_count_points
     for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < np; p += gridDim.x * blockDim.x) {
         const bool simple = pair_is_simple(d.b, d.ps, p);
         const bool comp = !simple && (d.b.iat(I_TYPE, d.ps.pa[p]) == SHAPE_COMPOUND ||
@@ -387,13 +388,6 @@ __global__ void __launch_bounds__(64) k_narrow_compound(Dev d) {
     const int prev = d.cnt->prev_npairs;
     for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < nc; q += gridDim.x * blockDim.x)
         narrow_pair<true, 1, true>(d.b, d.ps, d.comp_list[q], prev);
-}
-__global__ void k_narrow_finish(Dev d) {
-    d.cnt->prev_npairs = d.cnt->npairs;
-    d.cnt->nshape = 0;
-    d.cnt->nsat = 0;
-    d.cnt->ncomp = 0;
-    d.cnt->npoints = 0;   // summed by k_count_points next
 }
 
 // ------------------------------------------------------------------ stage 3: solver
@@ -1396,8 +1390,9 @@ __global__ void __launch_bounds__(SMALL_THREADS) k_solve_small(Dev d) {
     }
 }
 
-// Contact points of this narrowphase: per-workgroup sums added to the counter k_narrow_finish
-// cleared; a pair whose clipper lost points (bit 1 of its swap word) raises OVF_CLIP.
+// Ends a narrowphase: its contact points, per-workgroup sums added to the counter k_narrow cleared; a pair whose
+// clipper lost points (bit 1 of its swap word) raises OVF_CLIP; the pairs become the previous step's and the
+// lists are empty again (no workgroup here reads either; a launch of its own for that was 4.5 us a step).
 __global__ void __launch_bounds__(256) k_count_points(Dev d) {
     __shared__ int wsum[256 / WAVE + 1];
     const int np = d.cnt->npairs;
@@ -1409,6 +1404,12 @@ __global__ void __launch_bounds__(256) k_count_points(Dev d) {
     int tot;
     block_exclusive_scan(acc, wsum, &tot);
     if (threadIdx.x == 0 && tot) atomicAdd(&d.cnt->npoints, tot);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        d.cnt->prev_npairs = np;
+        d.cnt->nshape = 0;
+        d.cnt->nsat = 0;
+        d.cnt->ncomp = 0;
+    }
     if (lost) atomicOr(&d.cnt->overflow, OVF_CLIP);
 }
 
@@ -1522,7 +1523,6 @@ struct pe_world {
             hipLaunchKernelGGL(k_narrow_sat, dim3(std::min(grid(d.pcap, 4), 4096)), dim3(256), 0, stream, d);
         }
         if (d.comp_list) hipLaunchKernelGGL(k_narrow_compound, dim3(grid(d.pcap, 64)), dim3(64), 0, stream, d);
-        hipLaunchKernelGGL(k_narrow_finish, dim3(1), dim3(1), 0, stream, d);
         hipLaunchKernelGGL(k_count_points, dim3(grid(d.pcap, 1024)), dim3(256), 0, stream, d);
         if (d.status_on) hipLaunchKernelGGL(k_neighbours, dim3(grid(d.pcap, 256)), dim3(256), 0, stream, d);
         if (d.report_on) hipLaunchKernelGGL(k_events, dim3(grid(d.pcap, 256)), dim3(256), 0, stream, d);
