@@ -102,8 +102,8 @@ __global__ void k_integrate_status(Dev d) {
         integrate_body<true>(d.b, i, d.dt, d.g, &st);
 }
 
-// DefaultRaycastSolver::performRaycast (default_raycast_solver.cpp:11-86), one workgroup per RAYS rays
-// over the world's bodies.  Skipped: removed bodies, ignore-collision bodies, the call's ignore
+// DefaultRaycastSolver::performRaycast (default_raycast_solver.cpp:11-86), one workgroup per ray or RAYS_MAX
+// of them over the world's bodies.  Skipped: removed bodies, ignore-collision bodies, the call's ignore
 // set (sorted).  The reference walks the bodies in order and ends the query, reporting no hit, at the
 // first mesh body whose AABB the unbounded ray misses, its result keeping the best hit of the bodies
 // before it; so the first pass finds that body (the lowest such index), the second takes the nearest
@@ -113,10 +113,13 @@ __global__ void k_integrate_status(Dev d) {
 // are far off.  So a body is read once for several rays, and a box is only tested (some 150 instructions, a dozen
 // divisions) for a ray that ray_may_hit_box lets through.  4096 rays against 10 000 boxes: 470 -> 247 us (the
 // tests left gathered in LDS and done 64 at a time: 314, by their second reads and the LDS they take from the waves).
+// MESH: the world has meshes.  Their walks take a stack row per thread (bvh_stack_row), so a workgroup has no more
+// threads than there are rows; and the one thread that holds a terrain would walk it for each of its workgroup's rays
+// in turn, so it has one ray.
 constexpr int RAY_IN = 7;    // start (3), direction (3), length
 constexpr int RAY_OUT = 12;  // hit, body (int bits), distance, point (3), normal (3), pad
-constexpr int RAY_THREADS = 256;
 constexpr int RAYS_MAX = 4;
+constexpr int ray_threads(bool mesh) { return mesh ? BVH_ROWS : 256; }
 // Rays from which on a workgroup takes RAYS_MAX of them: with fewer a workgroup each fills the GPU better.
 constexpr int RAYS_SHARED = 1024;
 // Whether ray_box could report a hit of the ray, for a ray whose direction is no shorter than 0.5 (dir2 its squared
@@ -136,8 +139,11 @@ __device__ __forceinline__ bool nearly_orthonormal(const m33& R) {
     return fabsf(dot(a, a) - 1.0f) < e && fabsf(dot(b, b) - 1.0f) < e && fabsf(dot(c, c) - 1.0f) < e && fabsf(dot(a, b)) < e &&
            fabsf(dot(a, c)) < e && fabsf(dot(b, c)) < e;
 }
-__global__ void __launch_bounds__(RAY_THREADS) k_raycast(Dev d, const float* rays, int nrays, int per_group,
-                                                         const int32_t* ignore, int nignore, float* out) {
+template <bool MESH>
+__global__ void __launch_bounds__(ray_threads(MESH)) k_raycast(Dev d, const float* rays, int nrays, int per_group,
+                                                               const int32_t* ignore, int nignore, float* out) {
+    constexpr int RAY_THREADS = ray_threads(MESH);
+    static_assert(!MESH || RAY_THREADS <= BVH_ROWS, "a stack row per thread");
     __shared__ float s_ray[RAYS_MAX][8];                     // start, direction, length, squared length of direction
     __shared__ int s_abort[RAYS_MAX];
     __shared__ uint64_t s_best[RAYS_MAX][RAY_THREADS];
@@ -166,7 +172,7 @@ __global__ void __launch_bounds__(RAY_THREADS) k_raycast(Dev d, const float* ray
         }
         return lo < nignore && ignore[lo] == i;
     };
-    {
+    if (MESH) {
         uint32_t open = (1u << nr) - 1u;   // rays whose query no body of this thread has ended yet
         for (int i = tid; i < n && open; i += RAY_THREADS) {
             if (d.b.iat(I_TYPE, i) < SHAPE_CONVEX || skipped(i)) continue;
@@ -213,8 +219,10 @@ __global__ void __launch_bounds__(RAY_THREADS) k_raycast(Dev d, const float* ray
             if (type == SHAPE_BOX) ret = ray_box(start, dir, len, sp, R, o, t, hp, hn);
             else if (type == SHAPE_SPHERE) ret = ray_sphere(start, dir, len, sp[0], o, t, hp, hn);
             else if (type == SHAPE_CYLINDER) ret = ray_cylinder(start, dir, len, sp[0], sp[1], R, o, t, hp, hn);
-            else if (type != SHAPE_COMPOUND) ret = ray_mesh(d.b.ms, __float_as_int(sp[0]), start, dir, len, R, o, t, hp, hn);
-            else {
+            else if (type != SHAPE_COMPOUND) {
+                ret = false;
+                if constexpr (MESH) ret = ray_mesh(d.b.ms, __float_as_int(sp[0]), start, dir, len, R, o, t, hp, hn);
+            } else {
                 // each child in turn writes the same outputs, its hit or-ed in: the last child's distance and
                 // point decide (default_raycast_solver.cpp:50-78)
                 ret = false;
@@ -227,7 +235,7 @@ __global__ void __launch_bounds__(RAY_THREADS) k_raycast(Dev d, const float* ray
                     if (ct == SHAPE_BOX) ret |= ray_box(start, dir, len, csp, Rc, pc, t, hp, hn);
                     else if (ct == SHAPE_SPHERE) ret |= ray_sphere(start, dir, len, csp[0], pc, t, hp, hn);
                     else if (ct == SHAPE_CYLINDER) ret |= ray_cylinder(start, dir, len, csp[0], csp[1], Rc, pc, t, hp, hn);
-                    else ret |= ray_mesh(d.b.ms, __float_as_int(csp[0]), start, dir, len, Rc, pc, t, hp, hn);
+                    else if constexpr (MESH) ret |= ray_mesh(d.b.ms, __float_as_int(csp[0]), start, dir, len, Rc, pc, t, hp, hn);
                 }
             }
             if (ret && t <= len && t < REAL_MAX) {
@@ -1475,6 +1483,7 @@ struct pe_world {
     double stage_ms[4] = {0, 0, 0, 0};
     int n_dynamic = 0;
     bool has_shapes = false;   // any cylinder / convex / concave body
+    bool has_mesh = false;     // any convex / concave mesh (a compound's children too)
     DevMeshes meshes;
     std::vector<JointDef> joints;            // host copies of the joint definitions
     std::vector<uint64_t> ignore_keys;       // sorted ignore-pair keys
@@ -1725,6 +1734,7 @@ int pe_world_create(const pe_scene_desc* sc, const pe_world_params* prm, int32_t
     if (int rc2 = stage_bodies(sc, hf, hi, S, 0, hm)) return fail(rc2);
     if (int rc2 = w->meshes.upload(hm, w->stream)) return fail(rc2);
     d.b.ms = w->meshes.view();
+    w->has_mesh = hm.count() > 0;
     int ndyn = 0;
     bool has_compound = false;
     w->kinematic.resize(n);
@@ -1924,9 +1934,10 @@ int pe_world_raycast(pe_world* w, int32_t nrays, const float* rays, int32_t nign
     float* d_out = (float*)(base + ((in_b + 255) & ~(size_t)255) + ((ig_b + 255) & ~(size_t)255));
     PE_HIP(hipMemcpyAsync(d_rays, rays, in_b, hipMemcpyHostToDevice, w->stream));
     if (!ig.empty()) PE_HIP(hipMemcpyAsync(d_ig, ig.data(), ig.size() * 4, hipMemcpyHostToDevice, w->stream));
-    const int per_group = nrays >= RAYS_SHARED ? RAYS_MAX : 1;
-    hipLaunchKernelGGL(k_raycast, dim3((nrays + per_group - 1) / per_group), dim3(RAY_THREADS), 0, w->stream, w->d,
-                       (const float*)d_rays, nrays, per_group, (const int32_t*)d_ig, (int)ig.size(), d_out);
+    const int per_group = nrays >= RAYS_SHARED && !w->has_mesh ? RAYS_MAX : 1;
+    hipLaunchKernelGGL(w->has_mesh ? k_raycast<true> : k_raycast<false>, dim3((nrays + per_group - 1) / per_group),
+                       dim3(ray_threads(w->has_mesh)), 0, w->stream, w->d, (const float*)d_rays, nrays, per_group,
+                       (const int32_t*)d_ig, (int)ig.size(), d_out);
     PE_HIP(hipGetLastError());
     std::vector<float> res((size_t)nrays * RAY_OUT);
     PE_HIP(hipMemcpyAsync(res.data(), d_out, out_b, hipMemcpyDeviceToHost, w->stream));

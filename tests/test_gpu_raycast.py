@@ -119,3 +119,43 @@ def test_many_rays_sharing_a_pass_match_oracle(count, basis):
         hits += oh
     assert hits > count // 4
     g.close()
+
+
+@pytest.mark.parametrize("count", [1, 300, 1027])
+def test_rays_through_many_meshes_match_oracle(count):
+    """260 concentric hulls of several trees' sizes among boxes and spheres, every ray through the boxes of all
+    of them: each thread of a workgroup walks a mesh at the same time (a stack row each), over
+    every place a body can have in it."""
+    import pe_amd
+    from pe_amd import scenes
+    from pe_amd.scenes import SHAPE_BOX, SHAPE_CONVEX, SHAPE_SPHERE, SceneBuilder
+    from pyoracle import OracleWorld
+    rng = np.random.default_rng(31)
+    b = SceneBuilder()
+    ids = [b.add_mesh(scenes.gaussian_hull(rng, int(k), r)) for k, r in ((8, 2.0), (20, 1.0), (60, 1.5), (200, 1.2), (400, 1.8))]
+    rots = scenes.quat_to_matrix(scenes.random_quaternions(rng, 300))
+    for k in range(300):
+        if k % 15 == 0:
+            b.add(SHAPE_BOX, rng.uniform(0.2, 1.0, 3), 1.0, rng.uniform(-2.0, 2.0, 3), rot=rots[k], kin=1)
+        elif k % 15 == 1:
+            b.add(SHAPE_SPHERE, (0.3,), 1.0, rng.uniform(-2.0, 2.0, 3), kin=1)
+        else:
+            b.add(SHAPE_CONVEX, (), 1.0, rng.uniform(-0.05, 0.05, 3), rot=rots[k], kin=1, mesh=ids[int(rng.integers(0, len(ids)))])
+    sc = b.scene(name="nested")
+    g, o = pe_amd.World(sc), OracleWorld(sc, 32)
+    g.integrate()   # (all kinematic: this makes their AABBs)
+    o.integrate()
+    way = rng.normal(size=(count, 3))
+    way /= np.linalg.norm(way, axis=1)[:, None]
+    st = (rng.uniform(-0.1, 0.1, (count, 3)) - 6.0 * way).astype(np.float32)
+    d, ln = way.astype(np.float32), rng.uniform(3.0, 9.0, count).astype(np.float32)
+    print(f"[raycast] {count} rays through {sc.n} bodies", flush=True)
+    gh, gb, gd, gp, gn = g.raycast(st, d, ln)
+    mesh = 0
+    for k in range(count):
+        oh, ob, od, op, on = o.raycast(st[k].astype(np.float64), d[k].astype(np.float64), float(ln[k]))
+        assert bool(gh[k]) == oh and int(gb[k]) == ob and gd[k] == np.float32(od), f"ray {k}"
+        assert np.array_equal(gp[k], op.astype(np.float32)) and np.array_equal(gn[k], on.astype(np.float32)), f"ray {k}"
+        mesh += oh and sc.shape_type[ob] == SHAPE_CONVEX
+    assert mesh > count // 4
+    g.close()
