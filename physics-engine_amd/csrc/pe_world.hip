@@ -120,6 +120,7 @@ constexpr int RAY_IN = 7;    // start (3), direction (3), length
 constexpr int RAY_OUT = 12;  // hit, body (int bits), distance, point (3), normal (3), pad
 constexpr int RAYS_MAX = 4;
 constexpr int ray_threads(bool mesh) { return mesh ? BVH_ROWS : 256; }
+constexpr int ray_share(bool mesh) { return mesh ? 1 : RAYS_MAX; }
 // Rays from which on a workgroup takes RAYS_MAX of them: with fewer a workgroup each fills the GPU better.
 constexpr int RAYS_SHARED = 1024;
 // Whether ray_box could report a hit of the ray, for a ray whose direction is no shorter than 0.5 (dir2 its squared
@@ -144,22 +145,27 @@ __global__ void __launch_bounds__(ray_threads(MESH)) k_raycast(Dev d, const floa
                                                                const int32_t* ignore, int nignore, float* out) {
     constexpr int RAY_THREADS = ray_threads(MESH);
     static_assert(!MESH || RAY_THREADS <= BVH_ROWS, "a stack row per thread");
-    __shared__ float s_ray[RAYS_MAX][8];                     // start, direction, length, squared length of direction
-    __shared__ int s_abort[RAYS_MAX];
-    __shared__ uint64_t s_best[RAYS_MAX][RAY_THREADS];
-    __shared__ float s_hit[RAYS_MAX][7][RAY_THREADS];        // of a thread's best: distance, point, normal
+    constexpr int RAYS = ray_share(MESH);
+    __shared__ float s_ray[RAYS][8];                         // start, direction, length, squared length of direction
+    __shared__ int s_abort[RAYS];
+    // a thread's best of each ray: key, and distance, point, normal (of one ray in registers)
+    __shared__ uint64_t s_best[RAYS][RAYS > 1 ? RAY_THREADS : 1];
+    __shared__ float s_hit[RAYS][7][RAYS > 1 ? RAY_THREADS : 1];
+    uint64_t best = ~0ull;
+    float hit[7];
     const int tid = threadIdx.x;
     const int ray0 = blockIdx.x * per_group;
     const int nr = nrays - ray0 < per_group ? nrays - ray0 : per_group;
-    if (tid < RAYS_MAX) s_abort[tid] = 0x7fffffff;
+    if (tid < RAYS) s_abort[tid] = 0x7fffffff;
     if (tid < nr) {
         const float* r = rays + (size_t)(ray0 + tid) * RAY_IN;
 #pragma unroll
         for (int k = 0; k < RAY_IN; k++) s_ray[tid][k] = r[k];
         s_ray[tid][7] = dot(f3{r[3], r[4], r[5]}, f3{r[3], r[4], r[5]});
     }
+    if constexpr (RAYS > 1)
 #pragma unroll
-    for (int k = 0; k < RAYS_MAX; k++) s_best[k][tid] = ~0ull;
+        for (int k = 0; k < RAYS; k++) s_best[k][tid] = ~0ull;
     __syncthreads();
     const int n = d.b.n;
     auto skipped = [&](int i) {
@@ -202,7 +208,7 @@ __global__ void __launch_bounds__(ray_threads(MESH)) k_raycast(Dev d, const floa
         if (type == SHAPE_BOX && nearly_orthonormal(R)) {
             const float rad = 0.5f * sqrtf(sp[0] * sp[0] + sp[1] * sp[1] + sp[2] * sp[2]);
 #pragma unroll
-            for (int k = 0; k < RAYS_MAX; k++) {
+            for (int k = 0; k < RAYS; k++) {
                 const float* r = s_ray[k];
                 if (k < nr && r[7] >= 0.25f && !ray_may_hit_box(f3{r[0], r[1], r[2]}, f3{r[3], r[4], r[5]}, r[7], o, rad))
                     rest &= ~(1u << k);
@@ -240,11 +246,17 @@ __global__ void __launch_bounds__(ray_threads(MESH)) k_raycast(Dev d, const floa
             }
             if (ret && t <= len && t < REAL_MAX) {
                 const uint64_t key = ((uint64_t)float_key(t + 0.0f) << 32) | (uint32_t)i;
-                if (key < s_best[q][tid]) {
-                    s_best[q][tid] = key;
-                    const float h[7] = {t, hp.x, hp.y, hp.z, hn.x, hn.y, hn.z};
+                const float h[7] = {t, hp.x, hp.y, hp.z, hn.x, hn.y, hn.z};
+                if constexpr (RAYS > 1) {
+                    if (key < s_best[q][tid]) {
+                        s_best[q][tid] = key;
 #pragma unroll
-                    for (int k = 0; k < 7; k++) s_hit[q][k][tid] = h[k];
+                        for (int k = 0; k < 7; k++) s_hit[q][k][tid] = h[k];
+                    }
+                } else if (key < best) {
+                    best = key;
+#pragma unroll
+                    for (int k = 0; k < 7; k++) hit[k] = h[k];
                 }
             }
         }
@@ -252,28 +264,39 @@ __global__ void __launch_bounds__(ray_threads(MESH)) k_raycast(Dev d, const floa
     __syncthreads();
     // a wave per ray: the least key, and what the thread that found it kept
     const int lane = tid & (WAVE - 1);
-    for (int q = tid / WAVE; q < nr; q += RAY_THREADS / WAVE) {
-        uint64_t win = ~0ull;
-        int at = 0;
-        for (int k = lane; k < RAY_THREADS; k += WAVE)
-            if (s_best[q][k] < win) { win = s_best[q][k]; at = k; }
+    auto least = [](uint64_t& win, int& at) {
 #pragma unroll
         for (int m = 1; m < WAVE; m <<= 1) {
             const uint64_t w = (uint64_t)__shfl_xor((unsigned long long)win, m, WAVE);
             const int a = __shfl_xor(at, m, WAVE);
             if (w < win) { win = w; at = a; }
         }
-        if (lane != 0) continue;
-        float* o = out + (size_t)(ray0 + q) * RAY_OUT;
-        if (win == ~0ull) {
-            const float e[RAY_OUT] = {0.0f, __int_as_float(-1), REAL_MAX, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-            st_rec<RAY_OUT / 4>(o, e);
-        } else {
-            float e[RAY_OUT] = {s_abort[q] == 0x7fffffff ? 1.0f : 0.0f, __int_as_float((int)(uint32_t)win)};
+    };
+    auto result = [&](int q, uint64_t win, auto&& kept) {
+        float e[RAY_OUT] = {0.0f, __int_as_float(-1), REAL_MAX};
+        if (win != ~0ull) {
+            e[0] = s_abort[q] == 0x7fffffff ? 1.0f : 0.0f;
+            e[1] = __int_as_float((int)(uint32_t)win);
 #pragma unroll
-            for (int k = 0; k < 7; k++) e[2 + k] = s_hit[q][k][at];
-            st_rec<RAY_OUT / 4>(o, e);
+            for (int k = 0; k < 7; k++) e[2 + k] = kept(k);
         }
+        st_rec<RAY_OUT / 4>(out + (size_t)(ray0 + q) * RAY_OUT, e);
+    };
+    if constexpr (RAYS > 1) {
+        for (int q = tid / WAVE; q < nr; q += RAY_THREADS / WAVE) {
+            uint64_t win = ~0ull;
+            int at = 0;
+            for (int k = lane; k < RAY_THREADS; k += WAVE)
+                if (s_best[q][k] < win) { win = s_best[q][k]; at = k; }
+            least(win, at);
+            if (lane == 0) result(q, win, [&](int k) { return s_hit[q][k][at]; });
+        }
+    } else {
+        static_assert(RAYS > 1 || RAY_THREADS == WAVE, "one wave");
+        uint64_t win = best;
+        int at = lane;
+        least(win, at);
+        if (win == ~0ull ? lane == 0 : lane == at) result(0, win, [&](int k) { return hit[k]; });
     }
 }
 
@@ -1934,7 +1957,7 @@ int pe_world_raycast(pe_world* w, int32_t nrays, const float* rays, int32_t nign
     float* d_out = (float*)(base + ((in_b + 255) & ~(size_t)255) + ((ig_b + 255) & ~(size_t)255));
     PE_HIP(hipMemcpyAsync(d_rays, rays, in_b, hipMemcpyHostToDevice, w->stream));
     if (!ig.empty()) PE_HIP(hipMemcpyAsync(d_ig, ig.data(), ig.size() * 4, hipMemcpyHostToDevice, w->stream));
-    const int per_group = nrays >= RAYS_SHARED && !w->has_mesh ? RAYS_MAX : 1;
+    const int per_group = nrays >= RAYS_SHARED ? ray_share(w->has_mesh) : 1;
     hipLaunchKernelGGL(w->has_mesh ? k_raycast<true> : k_raycast<false>, dim3((nrays + per_group - 1) / per_group),
                        dim3(ray_threads(w->has_mesh)), 0, w->stream, w->d, (const float*)d_rays, nrays, per_group,
                        (const int32_t*)d_ig, (int)ig.size(), d_out);
