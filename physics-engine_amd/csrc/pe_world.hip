@@ -481,7 +481,9 @@ template <bool GRAPH> __global__ void k_setup(Dev d) {
 // A body in more pairs than this is coloured around by claims (k_solve_flow): its pairs all take different
 // colours one after another, and every try would scan all of them.
 constexpr int JP_MAX_DEG = 64;
-// Each body's range of the adjacency lists (the ranges' order does not matter).
+// Each body's range of the adjacency lists (the ranges' order does not matter); and syncTempVelocity
+// (sequential_impulse_solver.cpp:71-80) of the bodies that no pair or joint updates (the others' comes with their last
+// update): a removed body's temp velocities are not made anew from those the caller has set since.
 __global__ void k_jp_alloc(Dev d) {
     const int n = d.b.n;
     const int gsz = gridDim.x * blockDim.x;
@@ -499,7 +501,17 @@ __global__ void k_jp_alloc(Dev d) {
         int base = 0;
         if (lane == WAVE - 1 && incl > 0) base = (int)atomicAdd(&d.cnt->adj_total, (uint32_t)incl);
         base = __shfl(base, WAVE - 1, WAVE);
-        if (i < n) d.jp_off[i] = base + incl - deg;
+        if (i < n) {
+            d.jp_off[i] = base + incl - deg;
+            if ((deg + (d.jdeg ? d.jdeg[i] : 0) == 0 || d.iterations <= 0) && !d.b.iat(I_KIN, i)) {
+                const float* t = d.b.sbr(i);
+#pragma unroll
+                for (int k = 0; k < 3; k++) {
+                    d.b.at(F_V + k, i) = t[SB_TV + k];
+                    d.b.at(F_W + k, i) = t[SB_TW + k];
+                }
+            }
+        }
         if (__any(deg > JP_MAX_DEG) && lane == 0) d.cnt->jp_big = 1;
     }
 }

@@ -183,3 +183,41 @@ def test_worlds_on_their_own_streams_and_threads():
             assert np.array_equal(x.view(np.int32), y.view(np.int32))
         w.close()
     ref.close()
+
+
+def test_velocities_nothing_updates_are_solved_alike():
+    """A removed body, which no contact updates, has the solver's velocities after a solve on every path, also where
+    the caller has set others since (the solver's are those of its last step): in one workgroup, over the GPU, and
+    with the launch called off."""
+    import ctypes
+    import pe_amd
+    from pe_amd import scenes
+    from pe_amd._lib import check, lib
+    sc = scenes.grid_world(150, seed=8, p_sphere=0.3)
+    gone = 5
+    print("[untouched] 151 bodies", flush=True)
+    states = []
+    for mode, patience in ((0, None), (2, None), (2, 0)):
+        w = pe_amd.World(sc)
+        w.set_colouring(mode)
+        if patience is not None:
+            check(lib().pe_internal_set_flow_patience(w.h, ctypes.c_int64(patience)))
+        w.step(60)
+        w.remove_body(gone)
+        w.step(1)
+        before = w.state()
+        assert w.counts()["points"] > 0
+        set_v = np.full((sc.n, 3), 3.25, np.float32)
+        out = []
+        for call in (w.solve, lambda: w.step(1)):
+            w.set_state(v=set_v, w=set_v)
+            call()
+            w.sync()
+            out.append(w.state())
+            assert np.array_equal(out[-1][2][gone], before[2][gone]) and np.array_equal(out[-1][3][gone], before[3][gone])
+        states.append(out)
+        w.close()
+    for other in states[1:]:
+        for a, b in zip(states[0], other):
+            for x, y in zip(a, b):
+                assert np.array_equal(x.view(np.int32), y.view(np.int32))
