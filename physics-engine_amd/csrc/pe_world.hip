@@ -1466,19 +1466,17 @@ static int default_flow_blocks(int n, int max_blocks) { return std::min(max_bloc
 struct pe_world;
 namespace {
 // Turns at k_solve_flow between this process's worlds on one GPU.  As long as all of them fit on it at once
-// nothing is done; else each launch waits for the one before it (on another stream), so that two of them
-// never share the GPU with neither complete.
+// nothing is done; else each launch waits for the one before it, so that two of them never share the GPU with
+// neither complete.
 struct FlowTurns {
     std::mutex m;
     int blocks = 0;              // workgroups of all live worlds
     hipEvent_t last = nullptr;   // after the last launch (kept for the process)
-    hipStream_t stream = nullptr;
 };
-FlowTurns& flow_turns() {
+// Those of a world's own device, whichever is current when it is changed or destroyed.
+FlowTurns& flow_turns(int device) {
     static FlowTurns t[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    return t[dev];
+    return t[device >= 0 && device < 64 ? device : 0];
 }
 struct FlowTurn {
     explicit FlowTurn(pe_world& w);
@@ -1504,9 +1502,10 @@ struct pe_world {
     int flow_blocks = 0;    // workgroups of the solve over the GPU
     int flow_max_blocks = 0;                 // and how many of them the GPU holds at once
     uint64_t flow_patience = 5000000;        // 50 ms
-    int flow_counted = 0;                    // workgroups entered in flow_turns()
+    int device = 0;
+    int flow_counted = 0;                    // workgroups entered in flow_turns(device)
     void count_flow(int blocks) {
-        FlowTurns& t = flow_turns();
+        FlowTurns& t = flow_turns(device);
         std::lock_guard<std::mutex> g(t.m);
         t.blocks += blocks - flow_counted;
         flow_counted = blocks;
@@ -1614,7 +1613,7 @@ struct pe_world {
 };
 
 namespace {
-FlowTurn::FlowTurn(pe_world& w_) : w(w_), t(flow_turns()), lock(t.m), crowded(t.blocks > w_.flow_max_blocks) {
+FlowTurn::FlowTurn(pe_world& w_) : w(w_), t(flow_turns(w_.device)), lock(t.m), crowded(t.blocks > w_.flow_max_blocks) {
     if (crowded) {   // a stream under capture takes no part: what it waits for then is not this launch's time
         hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
         crowded = hipStreamIsCapturing(w.stream, &st) != hipSuccess || st == hipStreamCaptureStatusNone;
@@ -1624,13 +1623,10 @@ FlowTurn::FlowTurn(pe_world& w_) : w(w_), t(flow_turns()), lock(t.m), crowded(t.
         return;
     }
     if (!t.last) err = hipEventCreateWithFlags(&t.last, hipEventDisableTiming);
-    else if (t.stream != w.stream) err = hipStreamWaitEvent(w.stream, t.last, 0);
+    else err = hipStreamWaitEvent(w.stream, t.last, 0);
 }
 int FlowTurn::done() {
-    if (crowded && err == hipSuccess) {
-        err = hipEventRecord(t.last, w.stream);
-        t.stream = w.stream;
-    }
+    if (crowded && err == hipSuccess) err = hipEventRecord(t.last, w.stream);
     PE_HIP(err);
     return PE_OK;
 }
@@ -1814,6 +1810,7 @@ int pe_world_create(const pe_scene_desc* sc, const pe_world_params* prm, int32_t
             pe_set_error("cannot size the small-world solver's LDS");
             return fail(PE_ERR_DEVICE);
         }
+        w->device = dev;
         w->flow_max_blocks = cus * per_cu;
         w->flow_blocks = default_flow_blocks(n, w->flow_max_blocks);
         w->count_flow(n > SMALL_BODIES ? w->flow_blocks : 0);
