@@ -925,7 +925,7 @@ __device__ __forceinline__ void claim_sync() {
 // The lists are compacted with atomics, so the order inside a colour varies from run to run;
 // the colour classes do not, and neither does any result (pairs of a colour are independent).
 template <bool LDS>
-__device__ int colour_pairs(const BodyView& b, const PairStore& ps, int* bufs[3], int nact, int* order, int* cs,
+__device__ __forceinline__ int colour_pairs(const BodyView& b, const PairStore& ps, int* bufs[3], int nact, int* order, int* cs,
                             int* claim, int off, int pbase, int* wsum) {
     using namespace colour;
     __shared__ int cnt[3];   // winners (order), deferred, staying candidates

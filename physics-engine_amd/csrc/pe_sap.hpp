@@ -39,7 +39,10 @@ struct DevCounts {          // device-side counters of one step
     uint32_t fl_arrive;     // solve over the GPU: workgroups that have started,
     uint32_t fl_state;      // whether all have in time (FLOW_*),
     uint32_t fl_exit;       // and workgroups that left when not
-    int32_t jp_big;         // some body is in more pairs than the colouring over the GPU takes
+    int32_t jp_heavy;       // bodies in more than JP_HEAVY pairs,
+    int32_t jp_maxdeg;      // the most pairs one of them is in,
+    uint32_t jp_words;      // words of their colour sets,
+    int32_t jp_fall;        // and whether those are more than there are
     int32_t jp_rounds;      // colouring over the GPU: the most times a thread tried its pairs
 };
 // Capacity errors, OR-ed into DevCounts::overflow by the step that hits them and kept until the

@@ -51,6 +51,8 @@ struct Dev {
     int2* jp_adj;        // (pair, claim priority)
     int32_t* jp_col;
     int32_t* jp_idx;
+    uint64_t* jp_set;       // [pcap] heavy bodies: the set of colours their pairs have, body i's from jp_set_at[i] on
+    int32_t* jp_set_at;
     int32_t* jp_ccount;
     int32_t* jp_hist;       // [FLOW_BINS][workgroups] pairs of each of the first colours per workgroup
     int32_t* jp_items;      // [pcap + 1] sweep: first item of each colour (colours beyond those kept in LDS)
@@ -446,7 +448,10 @@ __global__ void k_solve_begin(Dev d) {
         d.cnt->nact = 0;
         d.cnt->adj_total = 0;
         d.cnt->jp_rounds = 0;
-        d.cnt->jp_big = 0;
+        d.cnt->jp_heavy = 0;
+        d.cnt->jp_maxdeg = 0;
+        d.cnt->jp_words = 0;
+        d.cnt->jp_fall = 0;
         d.cnt->fl_arrive = 0;
         d.cnt->fl_state = 0;
         d.cnt->fl_exit = 0;
@@ -478,12 +483,12 @@ template <bool GRAPH> __global__ void k_setup(Dev d) {
         if (act) d.act[slot] = p;
     }
 }
-// A body in more pairs than this is coloured around by claims (k_solve_flow): its pairs all take different
-// colours one after another, and every try would scan all of them.
-constexpr int JP_MAX_DEG = 64;
+// A body in more pairs than this is heavy: its pairs, which take different colours one after another, do not look at each
+// other but at the set of their colours (jp_colour_heavy).
+constexpr int JP_HEAVY = 32;
 // Each body's range of the adjacency lists (the ranges' order does not matter); and syncTempVelocity
-// (sequential_impulse_solver.cpp:71-80) of the bodies that no pair or joint updates (the others' comes with their last
-// update): a removed body's temp velocities are not made anew from those the caller has set since.
+// (sequential_impulse_solver.cpp:71-80) of the removed bodies: the others' comes with their last update or, where
+// there is none, changes nothing, but a removed body's temp velocities are not made anew from those the caller sets.
 __global__ void k_jp_alloc(Dev d) {
     const int n = d.b.n;
     const int gsz = gridDim.x * blockDim.x;
@@ -503,7 +508,7 @@ __global__ void k_jp_alloc(Dev d) {
         base = __shfl(base, WAVE - 1, WAVE);
         if (i < n) {
             d.jp_off[i] = base + incl - deg;
-            if ((deg + (d.jdeg ? d.jdeg[i] : 0) == 0 || d.iterations <= 0) && !d.b.iat(I_KIN, i)) {
+            if (d.status_on && (d.st.flags[i] & ST_REMOVED) && !d.b.iat(I_KIN, i)) {
                 const float* t = d.b.sbr(i);
 #pragma unroll
                 for (int k = 0; k < 3; k++) {
@@ -512,7 +517,15 @@ __global__ void k_jp_alloc(Dev d) {
                 }
             }
         }
-        if (__any(deg > JP_MAX_DEG) && lane == 0) d.cnt->jp_big = 1;
+        const uint64_t heavy = __ballot(deg > JP_HEAVY);
+        if (heavy) {
+            int most = deg;
+            for (int o = WAVE / 2; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, WAVE));
+            if (lane == 0) {
+                atomicAdd(&d.cnt->jp_heavy, (int)__popcll(heavy));
+                atomicMax(&d.cnt->jp_maxdeg, most);
+            }
+        }
     }
 }
 
@@ -565,19 +578,20 @@ __global__ void k_jp_fill(Dev d) {
 __device__ __forceinline__ int jp_col_load(const int32_t* col, int q) {
     return __hip_atomic_load(&col[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// The first colour not in used: a pair has at most 2 (JP_MAX_DEG - 1) neighbours, so one below 128 is free.
+// The first colour not in used: a pair of no heavy body has at most 2 (JP_HEAVY - 1) neighbours, so one below 128 is
+// free, and colours above that do not matter to it.
 __device__ __forceinline__ int jp_first(const uint64_t (&used)[2]) {
     return ~used[0] != 0ull ? __ffsll((unsigned long long)~used[0]) - 1 : 63 + __ffsll((unsigned long long)~used[1]);
 }
 __device__ __forceinline__ void jp_use(uint64_t (&used)[2], int c) {
     if (c >= 0 && c < 64) used[0] |= 1ull << c;
-    else if (c >= 64) used[1] |= 1ull << (c & 63);
+    else if (c >= 64 && c < 128) used[1] |= 1ull << (c & 63);
 }
-// Pair p's first-fit colour if every lower-priority neighbour is coloured, else -1.  The adjacency
+// Pair p's (of no heavy body) first-fit colour if every lower-priority neighbour is coloured, else -1.  The adjacency
 // entries and their colours are loaded eight at a time (independent loads in flight together: a
 // neighbour scan is a chain of L2 round trips otherwise).
 constexpr int JP_BATCH = 8;
-__device__ int jp_try(const Dev& d, int p) {
+__device__ __forceinline__ int jp_try(const Dev& d, int p) {
     const int pr = colour::prio(p, d.ps.npts[p]);
     const int body[2] = {d.ps.pa[p], d.ps.pb[p]};
     uint64_t used[2] = {0, 0};
@@ -606,9 +620,10 @@ __device__ int jp_try(const Dev& d, int p) {
     }
     return jp_first(used);
 }
-// The lower-priority neighbours of pair p to list[JP_KEEP]; their number, or -1 if they are more.
+// The lower-priority neighbours of pair p at its bodies that are not heavy to list[JP_KEEP]; their number, or -1 if they are
+// more.
 constexpr int JP_KEEP = 32;
-__device__ int jp_lower(const Dev& d, int p, int* list) {
+__device__ __forceinline__ int jp_lower(const Dev& d, int p, int* list) {
     const int pr = colour::prio(p, d.ps.npts[p]);
     const int body[2] = {d.ps.pa[p], d.ps.pb[p]};
     int m = 0;
@@ -616,6 +631,7 @@ __device__ int jp_lower(const Dev& d, int p, int* list) {
         const int x = body[s];
         if (d.b.iat(I_KIN, x)) continue;
         const int k0 = d.jp_off[x], k1 = k0 + d.jp_deg[x];
+        if (k1 - k0 > JP_HEAVY) continue;
         for (int k = k0; k < k1; k += JP_BATCH) {
             int2 q[JP_BATCH];
 #pragma unroll
@@ -648,10 +664,16 @@ __device__ __forceinline__ int jp_poll(const Dev& d, int* list, int n, uint64_t 
     }
     return m;
 }
-// Pairs of body x (not p) in a colour before c: p's place in x's sequence of updates.
-__device__ __forceinline__ int jp_rank(const Dev& d, int x, int p, int c) {
+// Pairs of body x (not p) in a colour before c: p's place in x's sequence of updates.  sets: heavy bodies have the sets of
+// their colours.
+__device__ __forceinline__ int jp_rank(const Dev& d, int x, int p, int c, bool sets) {
     const int k0 = d.jp_off[x], k1 = k0 + d.jp_deg[x];
     int r = 0;
+    if (sets && k1 - k0 > JP_HEAVY) {
+        const uint64_t* set = d.jp_set + d.jp_set_at[x];
+        for (int w = 0; w < c >> 6; w++) r += (int)__popcll(set[w]);
+        return r + (int)__popcll(set[c >> 6] & ((1ull << (c & 63)) - 1ull));
+    }
     for (int k = k0; k < k1; k += JP_BATCH) {
         int q[JP_BATCH];
 #pragma unroll
@@ -660,6 +682,185 @@ __device__ __forceinline__ int jp_rank(const Dev& d, int x, int p, int c) {
         for (int j = 0; j < JP_BATCH; j++) r += q[j] != p && jp_col_load(d.jp_col, q[j]) < c;
     }
     return r;
+}
+
+// ---- worlds with heavy bodies
+// A heavy body's pairs are coloured in the order of their priorities, and their colours differ: so the pair with r
+// of them before it is next when the set of their colours, which each adds its own to, has r members, and
+// it then has those colours at hand.  A try reads that set (a word per 64 pairs) where a scan of the body's pairs reads
+// all of them, twice.  2 500 bodies of which 40 / 150 / 500 lie on one plate: 0.72 / 2.2 / 6.9 ms a step, most of it
+// the sweeps' 40 / 140 / 460 colours (with scans 0.89 ms for 40; every pair by claims in one workgroup 5.5 / 20.0).
+struct JpHeavy {
+    uint64_t* set;   // the body's set (null: it is not heavy)
+    int words, rank;
+    int lo;          // leading words seen full: they stay so
+};
+// Words of the set of a body with deg pairs: a colour is at most the number of the pair's other neighbours.
+__device__ __forceinline__ int jp_set_words(int deg, int maxdeg) { return (deg + maxdeg) / 64 + 1; }
+// Hands out the sets, empty.
+__device__ __forceinline__ void jp_set_alloc(const Dev& d, int gtid, int gsz) {
+    for (int i = gtid; i < d.b.n; i += gsz) {
+        if (d.jp_deg[i] <= JP_HEAVY) continue;
+        const int m = jp_set_words(d.jp_deg[i], d.cnt->jp_maxdeg);
+        const uint32_t at = atomicAdd(&d.cnt->jp_words, (uint32_t)m);
+        if ((uint64_t)at + m > (uint64_t)d.pcap) {
+            d.cnt->jp_fall = 1;
+            return;
+        }
+        d.jp_set_at[i] = (int)at;
+        for (int w = 0; w < m; w++) d.jp_set[at + w] = 0;
+    }
+}
+__device__ __forceinline__ uint64_t jp_set_load(const uint64_t* w) {
+    return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool jp_is_heavy(const Dev& d, int x) { return !d.b.iat(I_KIN, x) && d.jp_deg[x] > JP_HEAVY; }
+// The set of body x and pair p's place among its pairs (rank < 0: counted here).
+__device__ __forceinline__ JpHeavy jp_heavy(const Dev& d, int x, int p, int rank) {
+    JpHeavy h{nullptr, 0, 0, 0};
+    if (!jp_is_heavy(d, x)) return h;
+    h.set = d.jp_set + d.jp_set_at[x];
+    h.words = jp_set_words(d.jp_deg[x], d.cnt->jp_maxdeg);
+    h.rank = rank;
+    if (rank >= 0) return h;
+    const int pr = colour::prio(p, d.ps.npts[p]);
+    h.rank = 0;
+    const int k0 = d.jp_off[x], k1 = k0 + d.jp_deg[x];
+    for (int k = k0; k < k1; k += 2 * JP_BATCH) {
+        int q[2 * JP_BATCH];
+#pragma unroll
+        for (int j = 0; j < 2 * JP_BATCH; j++) q[j] = k + j < k1 ? d.jp_adj[k + j].y : pr;
+#pragma unroll
+        for (int j = 0; j < 2 * JP_BATCH; j++) h.rank += q[j] < pr;
+    }
+    return h;
+}
+// How many pairs of a heavy body are still to be coloured before this one.
+__device__ __forceinline__ int jp_heavy_missing(const Dev& d, JpHeavy& h) {
+    if (!h.set) return 0;
+    // with one heavy body a colour is at most its pair's place and what a body that is not heavy adds
+    const int hi = d.cnt->jp_heavy == 1 ? min(h.words, (h.rank + JP_HEAVY) / 64 + 1) : h.words;
+    int sum = 64 * h.lo;
+    bool lead = true;
+    for (int w = h.lo; w < hi; w += 4) {
+        uint64_t v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = w + u < hi ? jp_set_load(h.set + w + u) : 0ull;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            sum += (int)__popcll(v[u]);
+            lead = lead && ~v[u] == 0ull;
+            h.lo += lead;
+        }
+    }
+    return h.rank - sum;
+}
+// The first colour in neither set nor among list[n], which is entered in the sets; -1: none (not reached).
+__device__ __forceinline__ int jp_heavy_take(const JpHeavy& a, const JpHeavy& b, const int* list, int n) {
+    const int words = !a.set ? b.words : !b.set ? a.words : min(a.words, b.words);
+    for (int w = max(a.lo, b.lo); w < words; w++) {
+        uint64_t used = 0;
+        if (a.set) used |= jp_set_load(a.set + w);
+        if (b.set) used |= jp_set_load(b.set + w);
+        for (int k = 0; k < n; k++)
+            if (list[k] >> 6 == w) used |= 1ull << (list[k] & 63);
+        if (~used == 0ull) continue;
+        const int bit = __ffsll((unsigned long long)~used) - 1;
+        if (a.set) __hip_atomic_fetch_or(a.set + w, 1ull << bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (b.set) __hip_atomic_fetch_or(b.set + w, 1ull << bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return 64 * w + bit;
+    }
+    return -1;
+}
+// Puts the colours that are there in the place of the pairs in list whose bits are set in miss; the bits left.
+__device__ __forceinline__ uint32_t jp_poll_keep(const Dev& d, int* list, uint32_t miss) {
+    for (uint32_t todo = miss; todo;) {
+        int at[4], c[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            at[u] = todo ? __ffs(todo) - 1 : -1;
+            todo &= todo - 1;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) c[u] = at[u] >= 0 ? jp_col_load(d.jp_col, list[at[u]]) : -1;
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (c[u] >= 0) {
+                list[at[u]] = c[u];
+                miss &= ~(1u << at[u]);
+            }
+    }
+    return miss;
+}
+// Colours every pair, as the loops of k_solve_flow do where no body is heavy; mine: the thread's JP_KEEP words of LDS.
+// The number of tries, negated where pairs of this thread were given up.
+__device__ __forceinline__ int jp_colour_heavy(const Dev& d, int nact, int gtid, int gsz, int* mine, int spins) {
+    int tries = 0;
+    bool left = true;
+    if (nact <= gsz) {
+        const int p = gtid < nact ? d.act[gtid] : -1;
+        JpHeavy a{nullptr, 0, 0, 0}, b = a;
+        int n = 0;
+        if (p >= 0) {
+            a = jp_heavy(d, d.ps.pa[p], p, -1);
+            b = jp_heavy(d, d.ps.pb[p], p, -1);
+            n = jp_lower(d, p, mine);
+        }
+        const bool heavy = a.set || b.set;
+        uint32_t miss = heavy ? (uint32_t)((1ull << n) - 1ull) : 0u;   // (then n < JP_HEAVY)
+        uint64_t used[2] = {0, 0};
+        left = p >= 0;
+        int skip = 0;   // rounds until the next look: a pair whose turn is far off only loads the fabric
+        while (__any(left) && tries < spins) {
+            const bool look = left && skip == 0;
+            if (left && skip > 0) skip--;
+            if (look) {
+                int c = -1;
+                if (heavy) {
+                    if (miss) miss = jp_poll_keep(d, mine, miss);
+                    const int before = max(jp_heavy_missing(d, a), jp_heavy_missing(d, b));
+                    if (before == 0 && miss == 0) c = jp_heavy_take(a, b, mine, n);
+                    skip = before > 4 ? min(before >> 2, 1024) : 0;
+                } else if (n < 0) {
+                    c = jp_try(d, p);
+                } else {
+                    n = jp_poll(d, mine, n, used);
+                    if (n == 0) c = jp_first(used);
+                }
+                if (c >= 0) {
+                    __hip_atomic_store(&d.jp_col[p], c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    left = false;
+                }
+            }
+            if (__any(look)) tries++;
+            else __builtin_amdgcn_s_sleep(16);
+        }
+    } else {
+        // several pairs per thread: their places wait in q_seq, which is only made after the colouring
+        for (int k = gtid; k < nact; k += gsz) {
+            const int p = d.act[k];
+            d.q_seq[k] = make_int4(jp_heavy(d, d.ps.pa[p], p, -1).rank, jp_heavy(d, d.ps.pb[p], p, -1).rank, 0, 0);
+        }
+        for (; __any(left) && tries < spins; tries++) {
+            left = false;
+            for (int k = gtid; k < nact; k += gsz) {
+                const int p = d.act[k];
+                if (jp_col_load(d.jp_col, p) >= 0) continue;
+                const int4 r = d.q_seq[k];
+                JpHeavy a = jp_heavy(d, d.ps.pa[p], p, r.x), b = jp_heavy(d, d.ps.pb[p], p, r.y);
+                int c = -1;
+                if (!a.set && !b.set) {
+                    c = jp_try(d, p);
+                } else if (jp_heavy_missing(d, a) == 0 && jp_heavy_missing(d, b) == 0) {
+                    const int n = jp_lower(d, p, mine);
+                    if (jp_poll_keep(d, mine, (uint32_t)((1ull << n) - 1ull)) == 0) c = jp_heavy_take(a, b, mine, n);
+                }
+                if (c >= 0) __hip_atomic_store(&d.jp_col[p], c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                else left = true;
+            }
+        }
+    }
+    return left ? -tries : tries;
 }
 
 // Colouring and Gauss-Seidel sweeps (SequentialImpulseSolver::solve, sequential_impulse_solver.cpp:60-81)
@@ -862,7 +1063,7 @@ __device__ __forceinline__ bool flow_joints(const Dev& d, int j0, int nl) {
 // LDS or (n bodies, any n) in memory: where a small world's pairs or colours outgrow its workgroup's
 // LDS, and where the workgroups of k_solve_flow could not all be had at once.
 template <bool LDS_CLAIM>
-__device__ void solve_alone(const Dev& d, int nact, int* claim) {
+__device__ __forceinline__ void solve_alone(const Dev& d, int nact, int* claim) {
     __shared__ int wsum[FLOW_THREADS / WAVE + 1];
     const int tid = threadIdx.x;
     for (int i = tid; i < d.b.n; i += FLOW_THREADS) claim_set<LDS_CLAIM>(claim, i, colour::FREE);
@@ -940,8 +1141,7 @@ __device__ __forceinline__ bool flow_together(const Dev& d, uint64_t patience, i
     return s_state == FLOW_GO;
 }
 
-// claims: the colouring runs in workgroup 0 (colour_pairs), as it does where a body is in more than
-// JP_MAX_DEG pairs.
+// claims: the colouring runs in workgroup 0 (colour_pairs), as it does where the heavy bodies' sets outgrow their memory.
 __global__ void __launch_bounds__(FLOW_THREADS) k_solve_flow(Dev d, int claims, uint64_t patience) {
     __shared__ int s_cs[FLOW_COLORS + 1], s_is[FLOW_COLORS + 1], s_ncol;
     __shared__ int s_hist[FLOW_BINS];
@@ -954,7 +1154,14 @@ __global__ void __launch_bounds__(FLOW_THREADS) k_solve_flow(Dev d, int claims, 
     }
     if (tid < FLOW_BINS) s_hist[tid] = 0;
     auto stalled = [&]() { atomicOr(&d.cnt->overflow, OVF_STALL); };
-    const bool coloured = claims || d.cnt->jp_big;   // the same for every workgroup
+    // the same for every workgroup: heavy bodies have their sets; the colouring is done by claims
+    bool sets = !claims && d.cnt->jp_heavy > 0, coloured = claims;
+    if (sets) {
+        jp_set_alloc(d, gtid, gsz);
+        grid_barrier(&d.cnt->bar_count, &d.cnt->bar_gen, gridDim.x);
+        coloured = d.cnt->jp_fall != 0;
+        sets = !coloured;
+    }
     if (!coloured) {
         // Every thread tries its pairs until all have their colours: the uncoloured pair of lowest priority
         // gets its colour whenever it is tried, so the loops end.  With a pair per thread or less, a thread
@@ -962,7 +1169,11 @@ __global__ void __launch_bounds__(FLOW_THREADS) k_solve_flow(Dev d, int claims, 
         // the colours still missing, in flight together.
         int tries = 0;
         bool left = true;
-        if (nact <= gsz) {
+        if (sets) {
+            tries = jp_colour_heavy(d, nact, gtid, gsz, s_low[tid], FLOW_SPINS);
+            left = tries < 0;
+            tries = abs(tries);
+        } else if (nact <= gsz) {
             const int p = gtid < nact ? d.act[gtid] : -1;
             int* mine = s_low[tid];
             int nlow = p >= 0 ? jp_lower(d, p, mine) : 0;   // neighbours whose colours are missing (-1: too many to keep)
@@ -1111,8 +1322,8 @@ __global__ void __launch_bounds__(FLOW_THREADS) k_solve_flow(Dev d, int claims, 
         const bool ka = d.b.iat(I_KIN, a) != 0, kb = d.b.iat(I_KIN, b) != 0;
         d.order[q] = p;
         d.q_pair[q] = make_int4(p, ka ? a | 1 << 31 : a, kb ? b | 1 << 31 : b, d.ps.npts[p]);
-        d.q_seq[q] = make_int4(ka ? 0 : jp_rank(d, a, p, c), ka ? 0 : d.jp_deg[a] + (d.jdeg ? d.jdeg[a] : 0),
-                               kb ? 0 : jp_rank(d, b, p, c), kb ? 0 : d.jp_deg[b] + (d.jdeg ? d.jdeg[b] : 0));
+        d.q_seq[q] = make_int4(ka ? 0 : jp_rank(d, a, p, c, sets), ka ? 0 : d.jp_deg[a] + (d.jdeg ? d.jdeg[a] : 0),
+                               kb ? 0 : jp_rank(d, b, p, c, sets), kb ? 0 : d.jp_deg[b] + (d.jdeg ? d.jdeg[b] : 0));
     }
     grid_barrier(&d.cnt->bar_count, &d.cnt->bar_gen, gridDim.x);   // the order is complete
 
@@ -1711,6 +1922,8 @@ int pe_world_create(const pe_scene_desc* sc, const pe_world_params* prm, int32_t
     rc |= w->alloc(&d.jp_adj, 2 * (size_t)pcap);
     rc |= w->alloc(&d.jp_col, pcap);
     rc |= w->alloc(&d.jp_idx, pcap);
+    rc |= w->alloc(&d.jp_set, pcap);
+    rc |= w->alloc(&d.jp_set_at, n);
     rc |= w->alloc(&d.jp_ccount, (size_t)pcap + 1);
     rc |= w->alloc(&d.jp_items, (size_t)pcap + 1);
     rc |= w->alloc(&d.vel, (size_t)VELW * n);

@@ -135,6 +135,52 @@ def test_one_workgroup_equals_the_flow(name):
     b.close()
 
 
+def heavy_scene(name):
+    """Bodies in more than 32 pairs in contact beside each other: two plates on each other under spheres; a cluster
+    whose bodies are all heavy; a plate in so many pairs that, beside the cluster, the colour sets outgrow
+    their memory (max_pairs is the number of pairs)."""
+    from pe_amd import scenes
+    from pe_amd.scenes import SHAPE_BOX
+    far = lambda sc, x: (sc.position.__iadd__(np.array([x, 0.0, 0.0])), sc)[1]
+    if name == "plates":
+        a, b = plate_scene(70), plate_scene(200)
+        b.shape_param[1, :3] = (11.0, 0.4, 30.0)       # reaches over the smaller plate's spheres and plate
+        return scenes.concat([a, far(b, 9.0)], "plates")
+    if name == "cluster":
+        return cluster_scene(300, 1.2)
+    return scenes.concat([plate_scene(2000), far(cluster_scene(140, 0.9), 200.0)], "hub")
+
+
+@pytest.mark.parametrize("name,blocks", [("plates", 0), ("plates", 1), ("cluster", 0), ("cluster", 3), ("hub", 0), ("hub", 2)])
+def test_heavy_bodies_are_coloured_alike(name, blocks):
+    """Pairs of bodies in many pairs, coloured over the GPU by the sets of their colours (a pair per thread and several,
+    both bodies heavy, sets that do not fit), and by claims in one workgroup: the same classes, the same bits."""
+    import pe_amd
+    sc = heavy_scene(name)
+    probe = pe_amd.World(sc, max_pairs=400 * sc.n)
+    probe.step(1)
+    cap = len(probe.pairs()) if name == "hub" else 400 * sc.n
+    probe.close()
+    a, b = pe_amd.World(sc, max_pairs=cap), pe_amd.World(sc, max_pairs=cap)
+    a.set_colouring(2)
+    a.set_solver_blocks(blocks)
+    b.set_colouring(1)
+    print(f"[heavy] {name}: {sc.n} bodies, {cap} pairs at most, blocks {blocks}", flush=True)
+    for step in range(1 if name == "hub" else 3):
+        a.step(1)
+        b.step(1)
+        (oa, ca), (ob, cb) = a.solve_order(), b.solve_order()
+        assert np.array_equal(ca, cb) and len(ca) > 33
+        for k in range(len(ca) - 1):
+            assert np.array_equal(np.sort(oa[ca[k]:ca[k + 1]]), np.sort(ob[ca[k]:ca[k + 1]]))
+        for x, y in zip(a.state(), b.state()):
+            assert np.array_equal(x.view(np.int32), y.view(np.int32))
+        assert np.array_equal(a.impulses(), b.impulses())
+        print(f"[heavy] {name}: {a.counts()}", flush=True)
+    a.close()
+    b.close()
+
+
 def test_launch_called_off_solves_the_same():
     """Workgroups that do not wait for each other call the solve over the GPU off, and the last of them solves
     alone (any world whose workgroups could not be had at once): the same bits, also with more workgroups
