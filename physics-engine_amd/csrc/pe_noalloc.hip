@@ -43,7 +43,7 @@ struct NoAllocLayout {
         end_ = take(4 * (size_t)NA_MAX_BODIES);
         first = take(4 * (size_t)NA_MAX_BODIES);
         red = take(8 * SAP_RED_VALUES * 256);
-        blk = take(sizeof(uint2) * (size_t)((NA_MAX_BODIES + SAP_BLOCK - 1) / SAP_BLOCK));
+        blk = take(sizeof(uint4) * (size_t)sap_blocks(NA_MAX_BODIES));
         unit_hit = take(8 * units);
         cnt = take(sizeof(DevCounts));
         end = o;
@@ -114,7 +114,7 @@ extern "C" int pe_stage_broadphase_noalloc(int32_t n, const float* aabb, int32_t
     s.hist = reinterpret_cast<uint32_t*>(base + NA_LAYOUT.hist);
     s.red = reinterpret_cast<double*>(base + NA_LAYOUT.red);
     s.srec = reinterpret_cast<float*>(base + NA_LAYOUT.srec);
-    s.blk = reinterpret_cast<uint2*>(base + NA_LAYOUT.blk);
+    s.blk = reinterpret_cast<uint4*>(base + NA_LAYOUT.blk);
     s.owner = reinterpret_cast<uint32_t*>(base + NA_LAYOUT.owner);
     s.unit_hit = reinterpret_cast<uint64_t*>(base + NA_LAYOUT.unit_hit);
     s.cnt = reinterpret_cast<DevCounts*>(base + NA_LAYOUT.cnt);

@@ -4,8 +4,8 @@
 //   k_sap_rank           up to SAP_RANK_MAX bodies: stable sort of (aabb_min[axis] + 0, index) by counting,
 //                        or k_sap_keys + radix, a stable LSD sort in 4 passes of 8 bits; both leave the
 //                        AABB records in sorted order; beside them the next axis's partial sums
-//   k_sap_runs           SAP_BLOCK sorted bodies per workgroup: their candidate runs (j > i with min_j <=
-//                        max_i), cut into units of 64 candidates
+//   k_sap_runs           16 or 64 sorted bodies per workgroup (a block): their candidate runs (j > i with
+//                        min_j <= max_i), cut into units of 64 candidates
 //   k_sap_test           a wave per unit tests its candidates, a lane each (up to SAP_FUSED_MAX bodies
 //                        k_sap_runs does so itself)
 //   k_sap_emit           the pairs that passed, in the reference's (i, j) sweep order; the next axis =
@@ -26,8 +26,6 @@ struct DevCounts {          // device-side counters of one step
     int32_t nordered;       // pairs in the solve order
     int32_t npoints;        // contact points of the last narrowphase
     uint32_t nunits;        // units of candidates handed out to the workgroups of the sweep
-    uint32_t pad;
-    uint64_t ncand;         // sweep candidates
     uint32_t bar_count;     // grid barrier: arrivals (0 between barriers)
     uint32_t bar_gen;       // grid barrier: generation
     int32_t nshape;         // pairs of this narrowphase that involve a cylinder or a mesh ...
@@ -53,8 +51,12 @@ constexpr int OVF_CHUNKS = 4;        // the sweep had more candidates than its c
 constexpr int OVF_CLIP = 8;          // a clipped polygon outgrew its buffer (contact points lost)
 constexpr int OVF_STALL = 16;        // the solver gave up a wait (not a capacity: a fault of this program)
 
-constexpr int SAP_BLOCK = 16;        // sorted bodies per workgroup of the sweep
-constexpr int SAP_THREADS = 256;     // its threads (16 lanes search the run of each body)
+// Sorted bodies per workgroup of the sweep: few where its workgroups also test their candidates (FUSED); else more, since
+// each takes its units' numbers from one counter, 12 ns after the other (50 000 bodies in blocks of 16: 78 us of
+// that, in blocks of 64: 16), and sums up the pairs of those before it.  16 lanes search a run.
+constexpr int sap_block(bool fused) { return fused ? 16 : 64; }
+constexpr int sap_threads(bool fused) { return 16 * sap_block(fused); }
+constexpr int SAP_EMIT_THREADS = 256;
 constexpr int SAP_UNIT = 64;         // candidates per unit
 constexpr int SAP_CHUNK = 32;        // the workspace is sized in chunks of this many candidates
 // Units for at most `chunks` chunks of candidates over n bodies' runs.
@@ -80,7 +82,7 @@ struct SapView {
     float* srec;            // [n][8] the AABB records in sorted order
     uint32_t* end;          // [n] per sorted body: the end of its run
     uint32_t* first;        // [n] and its first unit
-    uint2* blk;             // [sap_blocks(n)] per SAP_BLOCK sorted bodies: units, pairs
+    uint4* blk;             // [sap_blocks(n)] per block: units, pairs, candidates (low and high half)
     uint32_t* owner;        // [sap_units(chunk_cap, n)] per unit its sorted body
     uint64_t* unit_hit;     // [sap_units(chunk_cap, n)] per unit, bit k: its candidate k is a pair
     uint32_t* hist;         // [256 * radix_blocks(n)] radix histograms
@@ -101,7 +103,7 @@ struct SapView {
 
 __host__ inline int sap_radix_blocks(int n) { return (n + RS_TILE - 1) / RS_TILE; }
 __host__ inline int sap_red_blocks(int n) { return n < 1 ? 1 : (n + SAP_RED_THREADS - 1) / SAP_RED_THREADS < 256 ? (n + SAP_RED_THREADS - 1) / SAP_RED_THREADS : 256; }
-__host__ inline int sap_blocks(int n) { return (n + SAP_BLOCK - 1) / SAP_BLOCK; }
+__host__ __device__ constexpr int sap_blocks(int n, bool fused = true) { return (n + sap_block(fused) - 1) / sap_block(fused); }
 
 // BroadPhaseBase::validateCollisionPair (broad_phase_base.cpp:5-19) on two AABB records: the
 // ignore-collision flags, both kinematic, then closed-interval overlap on x, y, z.  Ignore-id pairs
@@ -157,7 +159,6 @@ static __global__ void k_sap_none(SapView s) {
 // Clears what the sweep counts (a given axis: a stage entry point, whose last call's errors are dropped).
 __device__ __forceinline__ void sap_begin(const SapView& s) {
     s.cnt->nunits = 0;
-    s.cnt->ncand = 0;
     if (s.axis_in >= 0) s.cnt->overflow = 0;
 }
 __device__ __forceinline__ void sap_sorted(const SapView& s, uint32_t q, int i, float key) {
@@ -349,38 +350,46 @@ __device__ __forceinline__ int sap_test_unit(const SapView& s, uint32_t u, int q
     if (lane == 0) s.unit_hit[u] = hit;
     return (int)__popcll(hit);
 }
-// The candidate runs of SAP_BLOCK sorted bodies (the reference's sweep breaks at the first key above a body's
+// The candidate runs of a block's sorted bodies (the reference's sweep breaks at the first key above a body's
 // maximum) and their units, numbered from a common counter.  FUSED: the workgroup tests them itself, which
 // saves a launch while the longest run (of a ground: every body) stays short; else k_sap_test spreads
 // all units over the GPU (10 000 boxes at rest: with every workgroup testing its own, the ground's run alone
 // took 40 us).
 constexpr int SAP_FUSED_MAX = 2048;
 template <bool FUSED>
-static __global__ void __launch_bounds__(SAP_THREADS) k_sap_runs(SapView s) {
-    __shared__ uint32_t s_len[SAP_BLOCK], s_unit[SAP_BLOCK + 1], s_base;
+static __global__ void __launch_bounds__(sap_threads(FUSED)) k_sap_runs(SapView s) {
+    constexpr int BLOCK = sap_block(FUSED), THREADS = sap_threads(FUSED);
+    static_assert(BLOCK <= WAVE, "a lane per body");
+    __shared__ uint32_t s_len[BLOCK], s_unit[BLOCK + 1], s_base;
     __shared__ int s_pairs;
-    const int n = s.n, q0 = blockIdx.x * SAP_BLOCK, nq = min(SAP_BLOCK, n - q0);
+    const int n = s.n, q0 = blockIdx.x * BLOCK, nq = min(BLOCK, n - q0);
     const int tid = threadIdx.x, r = tid >> 4, q = q0 + r;
     const float m = r < nq ? s.srec[(size_t)q * 8 + 4 + s.ax()] : 0.0f;
     const int end = sap_search(s.skey, r < nq ? q + 1 : n, n, m);
     if ((tid & 15) == 0) s_len[r] = r < nq ? (uint32_t)(end - q - 1) : 0u;
     __syncthreads();
-    if (tid == 0) {
-        uint32_t run = 0, cand = 0;
-        for (int k = 0; k < SAP_BLOCK; k++) {
-            s_unit[k] = run;
-            run += (s_len[k] + SAP_UNIT - 1) / SAP_UNIT;
-            cand += s_len[k];
+    uint64_t cand = 0;
+    if (tid < WAVE) {
+        const uint32_t len = tid < BLOCK ? s_len[tid] : 0u, units = (len + SAP_UNIT - 1) / SAP_UNIT;
+        uint32_t incl = units;
+        cand = len;
+#pragma unroll
+        for (int o = 1; o < WAVE; o <<= 1) {
+            const uint32_t y = __shfl_up(incl, o, WAVE);
+            if (tid >= o) incl += y;
+            cand += (uint64_t)__shfl_xor((unsigned long long)cand, o, WAVE);
         }
-        s_unit[SAP_BLOCK] = run;
-        s_base = atomicAdd(&s.cnt->nunits, run);
-        atomicAdd((unsigned long long*)&s.cnt->ncand, (unsigned long long)cand);
-        s_pairs = 0;
+        if (tid < BLOCK) s_unit[tid] = incl - units;
+        if (tid == BLOCK - 1) {
+            s_unit[BLOCK] = incl;
+            s_base = atomicAdd(&s.cnt->nunits, incl);
+            s_pairs = 0;
+        }
     }
     __syncthreads();
     // the units beyond the workspace are dropped (an error that k_sap_emit reports)
     const uint32_t slots = (uint32_t)sap_units(s.chunk_cap, n), base = s_base;
-    const uint32_t units = base >= slots ? 0u : min(s_unit[SAP_BLOCK], slots - base);
+    const uint32_t units = base >= slots ? 0u : min(s_unit[BLOCK], slots - base);
     if (r < nq) {
         if ((tid & 15) == 0) {
             s.end[q] = (uint32_t)end;
@@ -391,14 +400,14 @@ static __global__ void __launch_bounds__(SAP_THREADS) k_sap_runs(SapView s) {
     }
     if (FUSED) {
         int pairs = 0, o = 0;   // o: the run of the wave's unit
-        for (uint32_t u = tid / WAVE; u < units; u += SAP_THREADS / WAVE) {
+        for (uint32_t u = tid / WAVE; u < units; u += THREADS / WAVE) {
             while (s_unit[o + 1] <= u) o++;
             pairs += sap_test_unit(s, base + u, q0 + o, (int)(u - s_unit[o]), q0 + o + 1 + (int)s_len[o]);
         }
         if ((tid & (WAVE - 1)) == 0 && pairs) atomicAdd(&s_pairs, pairs);
         __syncthreads();
     }
-    if (tid == 0) s.blk[blockIdx.x] = make_uint2(units, (uint32_t)s_pairs);
+    if (tid == 0) s.blk[blockIdx.x] = make_uint4(units, (uint32_t)s_pairs, (uint32_t)cand, (uint32_t)(cand >> 32));
 }
 static __global__ void __launch_bounds__(256) k_sap_test(SapView s) {
     const uint32_t units = min(s.cnt->nunits, (uint32_t)sap_units(s.chunk_cap, s.n));
@@ -406,29 +415,43 @@ static __global__ void __launch_bounds__(256) k_sap_test(SapView s) {
     for (uint32_t u = wave; u < units; u += nw) {
         const int q = (int)s.owner[u];
         const int pairs = sap_test_unit(s, u, q, (int)(u - s.first[q]), (int)s.end[q]);
-        if ((threadIdx.x & (WAVE - 1)) == 0 && pairs) atomicAdd(&s.blk[q / SAP_BLOCK].y, (uint32_t)pairs);
+        if ((threadIdx.x & (WAVE - 1)) == 0 && pairs) atomicAdd(&s.blk[q / sap_block(false)].y, (uint32_t)pairs);
     }
 }
 
-// The pairs of a workgroup's bodies after those of the workgroups before it; the last workgroup knows all of
-// them and sets the counts and the next axis from its nred partial sums.
-static __global__ void __launch_bounds__(SAP_THREADS) k_sap_emit(SapView s, int nred) {
-    __shared__ uint32_t s_unit[SAP_BLOCK];
-    __shared__ int wsum[SAP_THREADS / WAVE + 1];
-    const int tid = threadIdx.x, q0 = blockIdx.x * SAP_BLOCK, nq = min(SAP_BLOCK, s.n - q0);
-    const uint2 me = s.blk[blockIdx.x];
+// The pairs of a block's bodies after those of the blocks before it; the last workgroup knows all of them and sets
+// the counts and the next axis from its nred partial sums.
+template <bool FUSED>
+static __global__ void __launch_bounds__(SAP_EMIT_THREADS) k_sap_emit(SapView s, int nred) {
+    constexpr int BLOCK = sap_block(FUSED), THREADS = SAP_EMIT_THREADS;
+    __shared__ uint32_t s_unit[BLOCK];
+    __shared__ int wsum[THREADS / WAVE + 1];
+    __shared__ unsigned long long s_cand;
+    const int tid = threadIdx.x, q0 = blockIdx.x * BLOCK, nq = min(BLOCK, s.n - q0);
+    const bool last = blockIdx.x + 1 == gridDim.x;
+    const uint4 me = s.blk[blockIdx.x];
     const uint32_t base = s.first[q0];
     int before = 0;
-    for (int b = tid; b < (int)blockIdx.x; b += SAP_THREADS) before += (int)s.blk[b].y;
+    uint64_t cand = 0;
+    for (int b = tid; b < (int)blockIdx.x; b += THREADS) {
+        const uint4 o = s.blk[b];
+        before += (int)o.y;
+        cand += (uint64_t)o.w << 32 | o.z;
+    }
     if (tid < nq) s_unit[tid] = s.first[q0 + tid] - base;
+    if (tid == 0) s_cand = (uint64_t)me.w << 32 | me.z;
     int carry;
     block_exclusive_scan(before, wsum, &carry);
-    if (blockIdx.x + 1 == gridDim.x && tid < WAVE) {
+    if (last) {
+        if (cand) atomicAdd(&s_cand, (unsigned long long)cand);
+        __syncthreads();
+    }
+    if (last && tid < WAVE) {
         const int axis = sap_axis_final(s, nred);
         if (tid == 0) {
             const uint32_t total = (uint32_t)carry + me.y;
             int32_t ovf = 0;
-            if (s.cnt->ncand > (uint64_t)s.chunk_cap * SAP_CHUNK) ovf |= OVF_CHUNKS;
+            if (s_cand > (uint64_t)s.chunk_cap * SAP_CHUNK) ovf |= OVF_CHUNKS;
             if (total > (uint32_t)s.pcap) ovf |= OVF_PAIRS;
             ovf |= s.cnt->overflow;
             s.cnt->overflow = ovf;
@@ -444,7 +467,7 @@ static __global__ void __launch_bounds__(SAP_THREADS) k_sap_emit(SapView s, int 
         }
     }
     if (me.y == 0) return;
-    for (uint32_t u0 = 0; u0 < me.x; u0 += SAP_THREADS) {
+    for (uint32_t u0 = 0; u0 < me.x; u0 += THREADS) {
         const uint32_t u = u0 + tid;
         uint64_t hit = u < me.x ? s.unit_hit[base + u] : 0ull;
         int tot;
@@ -453,7 +476,7 @@ static __global__ void __launch_bounds__(SAP_THREADS) k_sap_emit(SapView s, int 
         if (hit == 0) continue;
         int r = 0;   // the last of the runs that start at or before this unit (empty runs share their starts)
 #pragma unroll
-        for (int k = 1; k < SAP_BLOCK; k++) r = k < nq && s_unit[k] <= u ? k : r;
+        for (int k = BLOCK / 2; k > 0; k >>= 1) r = r + k < nq && s_unit[r + k] <= u ? r + k : r;
         const int a = (int)s.vals[q0 + r], j0 = q0 + r + 1 + (int)(u - s_unit[r]) * SAP_UNIT;
         for (; hit; hit &= hit - 1, out++) {
             if ((int)out >= s.pcap) break;
@@ -486,12 +509,13 @@ inline void sap_launch(const SapView& s, hipStream_t st) {
         hipLaunchKernelGGL(k_sap_gather, dim3(nk), dim3(256), 0, st, s);
     }
     if (n <= SAP_FUSED_MAX) {
-        hipLaunchKernelGGL(k_sap_runs<true>, dim3(sap_blocks(n)), dim3(SAP_THREADS), 0, st, s);
+        hipLaunchKernelGGL(k_sap_runs<true>, dim3(sap_blocks(n, true)), dim3(sap_threads(true)), 0, st, s);
+        hipLaunchKernelGGL(k_sap_emit<true>, dim3(sap_blocks(n, true)), dim3(SAP_EMIT_THREADS), 0, st, s, nred);
     } else {
-        hipLaunchKernelGGL(k_sap_runs<false>, dim3(sap_blocks(n)), dim3(SAP_THREADS), 0, st, s);
+        hipLaunchKernelGGL(k_sap_runs<false>, dim3(sap_blocks(n, false)), dim3(sap_threads(false)), 0, st, s);
         hipLaunchKernelGGL(k_sap_test, dim3(2048), dim3(256), 0, st, s);
+        hipLaunchKernelGGL(k_sap_emit<false>, dim3(sap_blocks(n, false)), dim3(SAP_EMIT_THREADS), 0, st, s, nred);
     }
-    hipLaunchKernelGGL(k_sap_emit, dim3(sap_blocks(n)), dim3(SAP_THREADS), 0, st, s, nred);
 }
 
 }  // namespace pe

@@ -69,3 +69,9 @@ def test_sweep_equals_a_stable_sort_and_sweep(n, wide):
     few = min(few, len(a))
     assert np.array_equal(pa.numpy()[:few], a[:few])
     st.close()
+
+
+@pytest.mark.parametrize("n,wide", [(2111, 1), (2112, 0), (2113, 2), (60011, 1)])
+def test_sweep_in_blocks_of_64(n, wide):
+    """The sweep's blocks beyond 2048 bodies at their edges, and over more blocks than a workgroup has threads."""
+    test_sweep_equals_a_stable_sort_and_sweep(n, wide)
