@@ -7,7 +7,7 @@
 //                      reference's (i, j) order, next axis
 //   k_narrow           thread / pair: shape dispatch + 8-slot contact cache + depth sort
 //   k_setup            thread / pair: solver rows (FrictionContactConstraint::initSequentialImpulse)
-//   k_solve_small      worlds of up to 600 bodies: colouring and sweeps in one workgroup, on LDS; else
+//   k_solve_small      small worlds (pe_world::one_workgroup): colouring and sweeps in one workgroup, on LDS; else
 //   k_jp_*             the constraint graph: per body its pairs
 //   k_solve_flow       one launch over the whole GPU: colouring, then the Gauss-Seidel sweeps in
 //                      colour order as a data flow between the pairs, and the velocity sync
@@ -528,6 +528,9 @@ __global__ void k_jp_alloc(Dev d) {
         }
     }
 }
+
+// The list k_setup<false> adds to, emptied: k_solve_small leaves it so, a solve over the GPU does not.
+__global__ void k_no_pairs(Dev d) { d.cnt->nact = 0; }
 
 // BallJointConstraint / HingeJointConstraint / SliderJointConstraint::initSequentialImpulse, thread / joint
 // (after the contacts' rows, as setupSolver initialises them, sequential_impulse_solver.cpp:49-51).
@@ -1394,11 +1397,10 @@ __global__ void __launch_bounds__(FLOW_THREADS) k_solve_flow(Dev d, int claims, 
 }
 
 // ---- the solve of a small world in one workgroup
-// Up to SMALL_BODIES bodies the solve runs in one workgroup of an ordinary launch: the bodies' temp velocities in
-// LDS, a workgroup barrier between colours (0.1 us) where the flow over the GPU pays 0.9 us for a store to
-// be seen on another CU, and none of the cooperative launch's queue switches (about 25 us a step).  Four
-// lanes per pair as there (quad_solve_row): a colour of up to SMALL_THREADS / 4 pairs is one pass as long as
-// its longest pair's row chains; a larger one takes several, which is where the flow becomes faster.
+// The solve of a small world in one workgroup: the bodies' temp velocities in LDS, a workgroup barrier between
+// colours (0.1 us) where the flow over the GPU pays 0.9 us for a store to be seen on another CU, and three launches
+// less (4.5 us each).  Four lanes per pair as there (quad_solve_row): a colour of up to SMALL_THREADS / 4 pairs is one
+// pass as long as its longest pair's row chains; a larger one takes several, which is where the flow becomes faster.
 constexpr int SMALL_THREADS = FLOW_THREADS;
 constexpr int SMALL_LDS = 152 * 1024;
 constexpr int SMALL_COLORS = 128;   // colours counted in LDS (two 64-bit masks per body)
@@ -1677,11 +1679,12 @@ static int default_flow_blocks(int n, int max_blocks) { return std::min(max_bloc
 struct pe_world;
 namespace {
 // Turns at k_solve_flow between this process's worlds on one GPU.  As long as all of them fit on it at once
-// nothing is done; else each launch waits for the one before it, so that two of them never share the GPU with
-// neither complete.
+// nothing is done; else the worlds that can do without leave it (40 worlds of 500 bodies on their own streams: 3960 us
+// a step of all with turns, 2260 in a workgroup each), and if the others still do not fit each launch waits for the one
+// before it, so that two of them never share the GPU with neither complete.
 struct FlowTurns {
     std::mutex m;
-    int blocks = 0;              // workgroups of all live worlds
+    int blocks[2] = {0, 0};      // workgroups of all live worlds that can do without the flow, that cannot
     hipEvent_t last = nullptr;   // after the last launch (kept for the process)
 };
 // Those of a world's own device, whichever is current when it is changed or destroyed.
@@ -1700,10 +1703,18 @@ struct FlowTurn {
 };
 }  // namespace
 
-// Bodies up to which the solve runs in one workgroup (k_solve_small).  At rest, us per step in one workgroup /
-// over the GPU: boxes 250 bodies 248 / 322, 500 370 / 376, 750 440 / 396, 1 000 560 / 440; boxes and
-// spheres 250 230 / 290, 500 325 / 366, 750 390 / 372, 1 000 474 / 413.
-constexpr int SMALL_BODIES = 600;
+// Bodies up to which the solve runs in one workgroup (k_solve_small): the line lies where a colour's pairs come to fill
+// it more than once, about 800 contact points at rest.  us per step in one workgroup / over the GPU:
+//   bodies                  200        260        300        350        400        500        590
+//   boxes at rest           141 / 144  162 / 160  172 / 159  176 / 161  210 / 166  251 / 176  279 / 181
+//   boxes, spheres at rest  141 / 145  153 / 150  167 / 157  176 / 161  180 / 157  198 / 165  237 / 169
+//   a tower struck          158 / 186  221 / 236  235 / 241  255 / 246  310 / 263  375 / 280  415 / 293
+//   boxes, spheres falling  107 / 127  125 / 137  122 / 134  127 / 135  131 / 135  148 / 143  162 / 148
+//   joint chains             80 / 121  250 / 304  274 / 335  269 / 326  272 / 325  285 / 346  293 / 356
+// A joint's pass is as long as one joint in one workgroup, and its flow waits for two bodies a pass: worlds with at
+// least a joint for every two bodies stay in one workgroup up to SMALL_MAX bodies, others of that size while the
+// process's worlds crowd the GPU (FlowTurns).
+constexpr int SMALL_BODIES = 280, SMALL_MAX = 600;
 
 struct pe_world {
     Dev d{};
@@ -1714,14 +1725,30 @@ struct pe_world {
     int flow_max_blocks = 0;                 // and how many of them the GPU holds at once
     uint64_t flow_patience = 5000000;        // 50 ms
     int device = 0;
-    int flow_counted = 0;                    // workgroups entered in flow_turns(device)
-    void count_flow(int blocks) {
+    int flow_counted[2] = {0, 0};            // workgroups entered in flow_turns(device)
+    bool flowed = false;                     // the last solve was over the GPU: it leaves its pairs listed
+    int colouring = 0;                       // 0: by body count, 1: one workgroup's claims, 2: over the GPU
+    enum Route { ONE_WORKGROUP = -1, EITHER = 0, FLOW = 1 };
+    Route route() const {
+        if (colouring != 0 || n > SMALL_MAX) return FLOW;
+        return n <= SMALL_BODIES || 2 * (int64_t)joints.size() >= n ? ONE_WORKGROUP : EITHER;
+    }
+    bool one_workgroup() const {
+        if (route() != EITHER) return route() == ONE_WORKGROUP;
         FlowTurns& t = flow_turns(device);
         std::lock_guard<std::mutex> g(t.m);
-        t.blocks += blocks - flow_counted;
-        flow_counted = blocks;
+        return t.blocks[0] + t.blocks[1] > flow_max_blocks;
     }
-    int colouring = 0;                       // 0: by body count, 1: one workgroup's claims, 2: over the GPU
+    // Enters the world's workgroups for its route (leave: none).
+    void count_flow(bool leave = false) {
+        FlowTurns& t = flow_turns(device);
+        std::lock_guard<std::mutex> g(t.m);
+        for (int k = 0; k < 2; k++) {
+            const int b = !leave && (int)route() == k ? flow_blocks : 0;
+            t.blocks[k] += b - flow_counted[k];
+            flow_counted[k] = b;
+        }
+    }
     bool timing = false;
     hipEvent_t ev[5] = {};
     hipEvent_t order_ev[2] = {};   // orders work on a caller's stream with the world's own stream
@@ -1741,7 +1768,7 @@ struct pe_world {
 
     ~pe_world() {
         if (stream) hipStreamSynchronize(stream);
-        count_flow(0);
+        count_flow(true);
         for (void* p : allocs) hipFree(p);
         for (void* p : joint_mem) if (p) hipFree(p);
         if (ignore_mem) hipFree(ignore_mem);
@@ -1783,7 +1810,9 @@ struct pe_world {
         return PE_OK;
     }
     int launch_solve() {
-        if (colouring == 0 && n <= SMALL_BODIES) {
+        if (one_workgroup()) {
+            if (flowed) hipLaunchKernelGGL(k_no_pairs, dim3(1), dim3(1), 0, stream, d);
+            flowed = false;
             hipLaunchKernelGGL(k_setup<false>, dim3(grid(d.pcap, 128)), dim3(128), 0, stream, d);
             if (d.njoints > 0) hipLaunchKernelGGL(k_joint_setup, dim3(grid(d.njoints, 64)), dim3(64), 0, stream, d);
             hipLaunchKernelGGL(k_solve_small, dim3(1), dim3(SMALL_THREADS), SMALL_LDS, stream, d);
@@ -1795,6 +1824,7 @@ struct pe_world {
         hipLaunchKernelGGL(k_jp_alloc, dim3(grid(n, 256)), dim3(256), 0, stream, d);
         hipLaunchKernelGGL(k_jp_fill, dim3(grid(d.pcap, 256)), dim3(256), 0, stream, d);
         int claims = colouring == 1;
+        flowed = true;
         FlowTurn turn(*this);
         hipLaunchKernelGGL(k_solve_flow, dim3(flow_blocks), dim3(FLOW_THREADS), 0, stream, d, claims, flow_patience);
         return turn.done();
@@ -1824,7 +1854,7 @@ struct pe_world {
 };
 
 namespace {
-FlowTurn::FlowTurn(pe_world& w_) : w(w_), t(flow_turns(w_.device)), lock(t.m), crowded(t.blocks > w_.flow_max_blocks) {
+FlowTurn::FlowTurn(pe_world& w_) : w(w_), t(flow_turns(w_.device)), lock(t.m), crowded(t.blocks[1] > w_.flow_max_blocks) {
     if (crowded) {   // a stream under capture takes no part: what it waits for then is not this launch's time
         hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
         crowded = hipStreamIsCapturing(w.stream, &st) != hipSuccess || st == hipStreamCaptureStatusNone;
@@ -2026,7 +2056,7 @@ int pe_world_create(const pe_scene_desc* sc, const pe_world_params* prm, int32_t
         w->device = dev;
         w->flow_max_blocks = cus * per_cu;
         w->flow_blocks = default_flow_blocks(n, w->flow_max_blocks);
-        w->count_flow(n > SMALL_BODIES ? w->flow_blocks : 0);
+        w->count_flow();
         if (w->alloc(&d.jp_hist, (size_t)FLOW_BINS * w->flow_max_blocks) != PE_OK) return fail(PE_ERR_DEVICE);
     }
     if (hipStreamSynchronize(w->stream) != hipSuccess) { pe_set_error("init sync failed"); return fail(PE_ERR_DEVICE); }
@@ -2110,6 +2140,7 @@ int pe_world_add_joints(pe_world* w, int32_t n, const pe_joint_desc* jd) {
     w->d.jdeg = (const int32_t*)w->joint_mem[5];
     w->d.njoints = nj;
     w->d.njcol = ncol;
+    w->count_flow();
     return PE_OK;
 }
 
@@ -2519,7 +2550,7 @@ int pe_world_set_solver_blocks(pe_world* w, int32_t blocks) {
     if (int rc = check_world(w)) return rc;
     if (blocks < 0) { pe_set_error("blocks must be >= 0"); return PE_ERR_INVALID; }
     w->flow_blocks = blocks == 0 ? default_flow_blocks(w->n, w->flow_max_blocks) : std::min(blocks, w->flow_max_blocks);
-    w->count_flow(w->n > SMALL_BODIES || w->colouring != 0 ? w->flow_blocks : 0);
+    w->count_flow();
     return PE_OK;
 }
 
@@ -2530,8 +2561,7 @@ int pe_world_set_colouring(pe_world* w, int32_t mode) {
         return PE_ERR_INVALID;
     }
     w->colouring = mode;
-    w->count_flow(w->n > SMALL_BODIES || mode != 0 ? w->flow_blocks : 0);
-    PE_HIP(hipMemsetAsync(&w->d.cnt->nact, 0, sizeof(int32_t), w->stream));   // as the one-workgroup solve leaves it
+    w->count_flow();
     return PE_OK;
 }
 

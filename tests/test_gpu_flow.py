@@ -135,6 +135,64 @@ def test_one_workgroup_equals_the_flow(name):
     b.close()
 
 
+@pytest.mark.parametrize("name", ["mixed", "boxes", "limit", "beyond", "cluster", "chains"])
+def test_one_workgroup_up_to_its_limits(name):
+    """As test_one_workgroup_equals_the_flow, at the sizes to which one workgroup is the default: 280 bodies, 600
+    where most have joints; a cluster whose pairs outgrow its LDS."""
+    import pe_amd
+    from pe_amd import scenes
+    sc, steps = {"mixed": lambda: (scenes.grid_world(200, seed=5), 90),
+                 "boxes": lambda: (scenes.grid_world(275, seed=6, p_sphere=0.0), 100),
+                 "limit": lambda: (scenes.grid_world(279, seed=7, p_sphere=0.2), 80),
+                 "beyond": lambda: (scenes.grid_world(280, seed=7, p_sphere=0.2), 80),
+                 "cluster": lambda: (cluster_scene(279, 1.5), 1),
+                 "chains": lambda: (scenes.joint_chain_scene(66, 8, seed=3), 60)}[name]()
+    a, b = pe_amd.World(sc, max_pairs=200 * sc.n), pe_amd.World(sc, max_pairs=200 * sc.n)
+    b.set_colouring(2)
+    print(f"[one workgroup] {name}: {sc.n} bodies", flush=True)
+    for part in (steps, 2):
+        a.step(part)
+        b.step(part)
+        for x, y in zip(a.state(), b.state()):
+            assert np.array_equal(x.view(np.int32), y.view(np.int32))
+        assert np.array_equal(a.impulses(), b.impulses())
+        (oa, ca), (ob, cb) = a.solve_order(), b.solve_order()
+        assert np.array_equal(ca, cb)
+        for k in range(len(ca) - 1):
+            assert np.array_equal(np.sort(oa[ca[k]:ca[k + 1]]), np.sort(ob[ca[k]:ca[k + 1]]))
+        if len(oa):   # the flow counts its tries, one workgroup does not
+            assert (a.counts()["colour_rounds"] > 0) == (name == "beyond") and b.counts()["colour_rounds"] > 0
+        if name == "cluster" and part == steps:
+            assert len(oa) * 28 + sc.n * 56 > 152 * 1024   # beyond the LDS the kernel works in
+    a.close()
+    b.close()
+
+
+def test_joints_added_between_steps_change_the_route():
+    """A pile stepped over the GPU whose bodies then get joints (more than one for two bodies) goes on in one workgroup:
+    the same bits as over the GPU throughout."""
+    import pe_amd
+    from pe_amd import scenes
+    sc = scenes.joint_chain_scene(50, 8, seed=4)
+    joints, sc.joints = sc.joints, []
+    a, b = pe_amd.World(sc), pe_amd.World(sc)
+    b.set_colouring(2)
+    print(f"[route] {sc.n} bodies, {len(joints)} joints", flush=True)
+    for w in (a, b):
+        w.step(50)
+        w.sync()
+    assert a.counts()["colour_rounds"] > 0 and a.counts()["points"] > 0
+    for w in (a, b):
+        w.add_joints(joints)
+        w.step(10)
+        w.sync()
+    assert a.counts()["colour_rounds"] == 0
+    for x, y in zip(a.state(), b.state()):
+        assert np.array_equal(x.view(np.int32), y.view(np.int32))
+    a.close()
+    b.close()
+
+
 def heavy_scene(name):
     """Bodies in more than 32 pairs in contact beside each other: two plates on each other under spheres; a cluster
     whose bodies are all heavy; a plate in so many pairs that, beside the cluster, the colour sets outgrow
@@ -228,6 +286,38 @@ def test_worlds_on_their_own_streams_and_threads():
         for x, y in zip(w.state(), want):
             assert np.array_equal(x.view(np.int32), y.view(np.int32))
         w.close()
+    ref.close()
+
+
+def test_worlds_that_come_and_go_change_the_route():
+    """A world between the limits is solved over the GPU, in one workgroup while others crowd the GPU, and over it again
+    when they are gone: each step as a world stepped alone."""
+    import pe_amd
+    from pe_amd import scenes
+    sc = scenes.grid_world(400, seed=15, p_sphere=0.3)
+    ref, w = pe_amd.World(sc), pe_amd.World(sc)
+    big = scenes.grid_world(900, seed=5, p_sphere=0.3)
+    print("[crowd] 401 bodies", flush=True)
+    ref.step(60)
+    w.step(60)
+    others = []
+    for crowd in (False, True, False, True):
+        if crowd:
+            others = [pe_amd.World(big) for _ in range(2)]
+            for o in others:
+                o.set_solver_blocks(200)
+        else:
+            for o in others:
+                o.close()
+        w.step(3)
+        w.sync()
+        assert (w.counts()["colour_rounds"] > 0) == (not crowd)
+    for o in others:
+        o.close()
+    ref.step(12)
+    for x, y in zip(w.state(), ref.state()):
+        assert np.array_equal(x.view(np.int32), y.view(np.int32))
+    w.close()
     ref.close()
 
 
