@@ -287,19 +287,27 @@ int pe_world_set_axis(pe_world* w, int32_t axis);
 int pe_world_set_timing(pe_world* w, int32_t enable);
 int pe_world_get_stage_times(pe_world* w, double* ms /*4*/);
 /* Workgroups of the solve over the GPU (0 = the default: 8 to 256 by body count, about 16 pairs in contact
- * per wave; clamped to the co-resident limit).  No counterpart in the reference; results
- * do not depend on it. */
+ * per wave; clamped to the co-resident limit).  It has no effect on a solve in one workgroup, the default of
+ * small worlds (see pe_world_set_colouring).  No counterpart in the reference; results do not depend on it.
+ * The workgroups of a solve wait for each other.  The worlds of one process take turns where they would not
+ * fit the GPU together; where something else holds the GPU (another process, a long kernel of the caller) so
+ * that a solve's workgroups have not all started within 50 ms of the first, that solve is done by one
+ * workgroup: the same result, but for a large world many times later than a queued launch would give it. */
 int pe_world_set_solver_blocks(pe_world* w, int32_t blocks);
-/* How the solver's colouring runs (0 = the default; 1 = one workgroup's claims, at most 12 288 bodies;
- * 2 = over the GPU, unless a body is in more than 64 pairs in contact).  Both give the same colour
- * classes.  No counterpart in the reference; results do not depend on it. */
+/* How the solve runs.  0 = the default: worlds of up to 280 bodies, and of up to 600 where at least every second
+ * body has a joint or the process's worlds crowd the GPU, in one workgroup, others over the GPU.  1 and 2 =
+ * over the GPU whatever the size, coloured by one workgroup's claims (at most 12 288 bodies) or over the GPU.
+ * All give the same colour classes.  No counterpart in the reference; results do not depend on it. */
 int pe_world_set_colouring(pe_world* w, int32_t mode);
+/* How long the workgroups of a solve over the GPU wait for each other to start, in ticks of 10 ns (5 000 000 by
+ * default; with 0 every such solve is done by one workgroup).  For tests of that path. */
+int pe_internal_set_flow_patience(pe_world* w, int64_t ticks);
 /* The per-body records the stage entry points take (layouts under "stage entry points" below),
  * as the world's last integrate stage wrote them: AABB records [n][8], collision records [n][20],
  * solver records [n][24] (velocities after gravity, before the solve).  Any pointer may be NULL. */
 int pe_world_get_records(pe_world* w, float* aabb, float* body, float* solver);
-/* Counts of the last step: bodies, dynamic bodies, pairs, contact points, colours, rounds of the
- * colouring (0 when one workgroup coloured: see pe_world_set_colouring). */
+/* Counts of the last step: bodies, dynamic bodies, pairs, contact points, colours, and the most times a thread of
+ * the colouring over the GPU tried its pairs (0 when one workgroup coloured: see pe_world_set_colouring). */
 int pe_world_get_counts(pe_world* w, int64_t* counts /*6*/);
 
 /* ------------------------------------------------------------------ stage entry points
@@ -307,7 +315,8 @@ int pe_world_get_counts(pe_world* w, int64_t* counts /*6*/);
  * setConstraintSolver, src/intf/world.h:97-100).  These entry points run one stage each on the
  * caller's device buffers, enqueued on the caller's stream (a hipStream_t; NULL is the null
  * stream) without synchronising, so a host that keeps the reference's World can replace a stage
- * at a time (the C++ classes implementing the stage interfaces over them are in INTEGRATION.md).
+ * at a time (the C++ classes implementing the stage interfaces over them are in
+ * physics-engine_amd/integration).
  * All buffers are device memory.  A pe_stage holds the working memory; one host thread uses a
  * pe_stage at a time.  Record layouts (FP32, 16-byte aligned rows):
  *   AABB record      [8]  min x y z, kinematic (0 / 1), max x y z, collision flag (0: normal,

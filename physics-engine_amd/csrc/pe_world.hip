@@ -2565,7 +2565,6 @@ int pe_world_set_colouring(pe_world* w, int32_t mode) {
     return PE_OK;
 }
 
-// For the tests: how long (ticks of 10 ns) the workgroups of the solve over the GPU wait for each other to start.
 int pe_internal_set_flow_patience(pe_world* w, int64_t ticks) {
     if (int rc = check_world(w)) return rc;
     w->flow_patience = (uint64_t)std::max<int64_t>(ticks, 0);

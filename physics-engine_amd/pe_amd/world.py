@@ -265,8 +265,8 @@ class World:
         check(lib().pe_world_set_solver_blocks(self.h, ctypes.c_int32(blocks)))
 
     def set_colouring(self, mode: int):
-        """0: by body count, 1: one workgroup's claims (at most 12 288 bodies), 2: rounds over the GPU;
-        the colour classes are the same."""
+        """0: by body count (small worlds in one workgroup), 1 and 2: over the GPU, coloured by one workgroup's
+        claims (at most 12 288 bodies) or over the GPU; the colour classes are the same."""
         check(lib().pe_world_set_colouring(self.h, ctypes.c_int32(mode)))
 
     def records(self):
