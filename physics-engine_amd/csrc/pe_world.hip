@@ -22,6 +22,7 @@
 #include "../../include/pe_amd.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -1686,6 +1687,7 @@ struct FlowTurns {
     std::mutex m;
     int blocks[2] = {0, 0};      // workgroups of all live worlds that can do without the flow, that cannot
     hipEvent_t last = nullptr;   // after the last launch (kept for the process)
+    uint64_t last_order = 0;     // whose order it came in (pe_world::order)
 };
 // Those of a world's own device, whichever is current when it is changed or destroyed.
 FlowTurns& flow_turns(int device) {
@@ -1726,6 +1728,11 @@ struct pe_world {
     uint64_t flow_patience = 5000000;        // 50 ms
     int device = 0;
     int flow_counted[2] = {0, 0};            // workgroups entered in flow_turns(device)
+    hipStream_t own = nullptr;               // the world's own stream (stream: the one it is being stepped on)
+    uint64_t id = 0;                         // of this world, never used again
+    // Two launches of one order follow each other anyway, those on the world's own stream or on the null stream; 0: on
+    // another, whose handle may come to be another stream's.
+    uint64_t order() const { return stream == own ? id : stream == nullptr ? 1 : 0; }
     bool flowed = false;                     // the last solve was over the GPU: it leaves its pairs listed
     int colouring = 0;                       // 0: by body count, 1: one workgroup's claims, 2: over the GPU
     enum Route { ONE_WORKGROUP = -1, EITHER = 0, FLOW = 1 };
@@ -1864,10 +1871,13 @@ FlowTurn::FlowTurn(pe_world& w_) : w(w_), t(flow_turns(w_.device)), lock(t.m), c
         return;
     }
     if (!t.last) err = hipEventCreateWithFlags(&t.last, hipEventDisableTiming);
-    else err = hipStreamWaitEvent(w.stream, t.last, 0);
+    else if (w.order() == 0 || w.order() != t.last_order) err = hipStreamWaitEvent(w.stream, t.last, 0);
 }
 int FlowTurn::done() {
-    if (crowded && err == hipSuccess) err = hipEventRecord(t.last, w.stream);
+    if (crowded && err == hipSuccess) {
+        err = hipEventRecord(t.last, w.stream);
+        t.last_order = w.order();
+    }
     PE_HIP(err);
     return PE_OK;
 }
@@ -1918,6 +1928,9 @@ int pe_world_create(const pe_scene_desc* sc, const pe_world_params* prm, int32_t
     const int pcap = (int)want;
     auto fail = [&](int rc) { delete w; return rc; };
     if (hipStreamCreateWithFlags(&w->stream, hipStreamNonBlocking) != hipSuccess) { pe_set_error("stream create failed"); return fail(PE_ERR_DEVICE); }
+    static std::atomic<uint64_t> worlds{2};
+    w->id = worlds++;
+    w->own = w->stream;
     Dev& d = w->d;
     d.pcap = pcap;
     d.ps.cs = (size_t)pcap * 8;

@@ -357,3 +357,31 @@ def test_velocities_nothing_updates_are_solved_alike():
         for a, b in zip(states[0], other):
             for x, y in zip(a, b):
                 assert np.array_equal(x.view(np.int32), y.view(np.int32))
+
+
+def test_worlds_on_callers_streams_take_turns():
+    """Worlds that crowd the GPU, stepped on streams of the caller's that come and go (a new stream may have the handle
+    of a destroyed one): each as it is alone."""
+    import pe_amd
+    from pe_amd import scenes
+    from pe_amd.hip import Stream
+    sc = scenes.grid_world(900, seed=15, p_sphere=0.3)
+    ref = pe_amd.World(sc)
+    ref.step(60)
+    want = ref.state()
+    ws = [pe_amd.World(sc) for _ in range(4)]
+    for w in ws:
+        w.set_solver_blocks(256)
+    print("[streams] 4 worlds", flush=True)
+    for _ in range(6):
+        streams = [Stream() for _ in ws]
+        for w, st in zip(ws, streams):
+            w.step_async(10, st.handle.value)
+        for st in streams:
+            st.close()
+    for w in ws:
+        w.sync()
+        for x, y in zip(w.state(), want):
+            assert np.array_equal(x.view(np.int32), y.view(np.int32))
+        w.close()
+    ref.close()
