@@ -294,8 +294,8 @@ int pe_world_get_stage_times(pe_world* w, double* ms /*4*/);
  * that a solve's workgroups have not all started within 50 ms of the first, that solve is done by one
  * workgroup: the same result, but for a large world many times later than a queued launch would give it. */
 int pe_world_set_solver_blocks(pe_world* w, int32_t blocks);
-/* How the solve runs.  0 = the default: worlds of up to 280 bodies, and of up to 600 where at least every second
- * body has a joint or the process's worlds crowd the GPU, in one workgroup, others over the GPU.  1 and 2 =
+/* How the solve runs.  0 = the default: worlds of up to 280 bodies, and of up to 600 with few contact points (in a
+ * step before) or while the process's worlds crowd the GPU, in one workgroup, others over the GPU.  1 and 2 =
  * over the GPU whatever the size, coloured by one workgroup's claims (at most 12 288 bodies) or over the GPU.
  * All give the same colour classes.  No counterpart in the reference; results do not depend on it. */
 int pe_world_set_colouring(pe_world* w, int32_t mode);

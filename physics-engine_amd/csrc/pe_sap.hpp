@@ -32,6 +32,7 @@ struct DevCounts {          // device-side counters of one step
     int32_t nsat;           // ... of which these run the polyhedral separating-axis routine
     int32_t ncomp;          // ... and these involve a compound body
     int32_t nact;           // pairs the solve orders (contact points, not both bodies kinematic)
+    int32_t nrows;          // their contact points, where the host asks for them
     int32_t jp_ncol;        // colours the last sweep over the GPU counted
     uint32_t adj_total;     // colouring: adjacency entries
     uint32_t fl_arrive;     // solve over the GPU: workgroups that have started,

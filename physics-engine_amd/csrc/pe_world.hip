@@ -67,6 +67,7 @@ struct Dev {
     int32_t* color_start;   // [pcap+1]
     int32_t* claim;         // [n] claims of the colouring in one workgroup
     DevCounts* cnt;
+    int32_t* rows_out;      // host memory: contact points of the last solve (null: not asked for)
     int pcap;
     float dt;
     float g[3];
@@ -447,6 +448,7 @@ __global__ void k_solve_begin(Dev d) {
     for (int c = gtid; c < d.cnt->jp_ncol; c += gsz) d.jp_ccount[c] = 0;   // the colours the last solve counted
     if (gtid == 0) {
         d.cnt->nact = 0;
+        d.cnt->nrows = 0;
         d.cnt->adj_total = 0;
         d.cnt->jp_rounds = 0;
         d.cnt->jp_heavy = 0;
@@ -483,6 +485,10 @@ template <bool GRAPH> __global__ void k_setup(Dev d) {
         const int slot = wave_append(act, &d.cnt->nact);
         if (act) d.act[slot] = p;
     }
+}
+// Tells the host the solve's contact points (it reads them at some later launch: pe_world::one_workgroup).
+__device__ __forceinline__ void report_rows(const Dev& d, int rows) {
+    if (d.rows_out) __hip_atomic_store(d.rows_out, rows, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 // A body in more pairs than this is heavy: its pairs, which take different colours one after another, do not look at each
 // other but at the set of their colours (jp_colour_heavy).
@@ -1324,12 +1330,14 @@ __global__ void __launch_bounds__(FLOW_THREADS) k_solve_flow(Dev d, int claims, 
         const int q = cs(c) + d.jp_idx[p] + (!coloured && c < FLOW_BINS ? s_hist[c] : 0);
         const int a = d.ps.pa[p], b = d.ps.pb[p];
         const bool ka = d.b.iat(I_KIN, a) != 0, kb = d.b.iat(I_KIN, b) != 0;
+        if (d.rows_out) atomicAdd(&d.cnt->nrows, d.ps.npts[p]);
         d.order[q] = p;
         d.q_pair[q] = make_int4(p, ka ? a | 1 << 31 : a, kb ? b | 1 << 31 : b, d.ps.npts[p]);
         d.q_seq[q] = make_int4(ka ? 0 : jp_rank(d, a, p, c, sets), ka ? 0 : d.jp_deg[a] + (d.jdeg ? d.jdeg[a] : 0),
                                kb ? 0 : jp_rank(d, b, p, c, sets), kb ? 0 : d.jp_deg[b] + (d.jdeg ? d.jdeg[b] : 0));
     }
     grid_barrier(&d.cnt->bar_count, &d.cnt->bar_gen, gridDim.x);   // the order is complete
+    if (gtid == 0) report_rows(d, d.cnt->nrows);
 
     // consecutive items go to different workgroups, so a colour's pairs spread over the CUs; half of the
     // waves take the joints, if there are any
@@ -1572,7 +1580,10 @@ __global__ void __launch_bounds__(SMALL_THREADS) k_solve_small(Dev d) {
     }
     if (!small) {   // the same for every thread
         solve_alone<true>(d, nact, (int*)lds);
-        if (tid == 0) d.cnt->nact = 0;
+        if (tid == 0) {
+            d.cnt->nact = 0;
+            report_rows(d, 8 * nact);
+        }
         return;
     }
     if (tid == 0) {
@@ -1644,6 +1655,7 @@ __global__ void __launch_bounds__(SMALL_THREADS) k_solve_small(Dev d) {
         d.cnt->nordered = nact;
         d.cnt->jp_rounds = 0;
         d.cnt->nact = 0;   // counted from zero by the next step's set-up
+        report_rows(d, nrows);
     }
 }
 
@@ -1705,18 +1717,16 @@ struct FlowTurn {
 };
 }  // namespace
 
-// Bodies up to which the solve runs in one workgroup (k_solve_small): the line lies where a colour's pairs come to fill
-// it more than once, about 800 contact points at rest.  us per step in one workgroup / over the GPU:
-//   bodies                  200        260        300        350        400        500        590
-//   boxes at rest           141 / 144  162 / 160  172 / 159  176 / 161  210 / 166  251 / 176  279 / 181
-//   boxes, spheres at rest  141 / 145  153 / 150  167 / 157  176 / 161  180 / 157  198 / 165  237 / 169
-//   a tower struck          158 / 186  221 / 236  235 / 241  255 / 246  310 / 263  375 / 280  415 / 293
-//   boxes, spheres falling  107 / 127  125 / 137  122 / 134  127 / 135  131 / 135  148 / 143  162 / 148
-//   joint chains             80 / 121  250 / 304  274 / 335  269 / 326  272 / 325  285 / 346  293 / 356
-// A joint's pass is as long as one joint in one workgroup, and its flow waits for two bodies a pass: worlds with at
-// least a joint for every two bodies stay in one workgroup up to SMALL_MAX bodies, others of that size while the
-// process's worlds crowd the GPU (FlowTurns).
-constexpr int SMALL_BODIES = 280, SMALL_MAX = 600;
+// The solve runs in one workgroup (k_solve_small) up to SMALL_BODIES bodies, and up to SMALL_MAX while the last solve
+// the host knows of had at most SMALL_POINTS contact points or the process's worlds crowd the GPU (FlowTurns): a colour's
+// pairs then fill the workgroup about once.  us per step in one workgroup / over the GPU (contact points):
+//   bodies                  200              260               300               400                590
+//   boxes at rest           141 / 144 (716)  162 / 160 (958)   172 / 159 (1043)  210 / 166 (1429)   279 / 181 (2107)
+//   boxes, spheres at rest  141 / 145 (447)  153 / 150 (643)   167 / 157 (733)   180 / 157 (877)    237 / 169 (1322)
+//   a tower struck          158 / 186 (451)  221 / 236 (1004)  235 / 241 (1029)  310 / 263 (1667)   415 / 293 (2843)
+//   boxes, spheres falling  107 / 127 (279)  125 / 137 (362)   122 / 134 (389)   131 / 135 (472)    162 / 148 (748)
+//   joint chains             80 / 121 (0)    250 / 304 (0)     274 / 335 (3)     272 / 325 (5)      293 / 356 (8)
+constexpr int SMALL_BODIES = 280, SMALL_MAX = 600, SMALL_POINTS = 650;
 
 struct pe_world {
     Dev d{};
@@ -1735,13 +1745,19 @@ struct pe_world {
     uint64_t order() const { return stream == own ? id : stream == nullptr ? 1 : 0; }
     bool flowed = false;                     // the last solve was over the GPU: it leaves its pairs listed
     int colouring = 0;                       // 0: by body count, 1: one workgroup's claims, 2: over the GPU
-    enum Route { ONE_WORKGROUP = -1, EITHER = 0, FLOW = 1 };
-    Route route() const {
-        if (colouring != 0 || n > SMALL_MAX) return FLOW;
-        return n <= SMALL_BODIES || 2 * (int64_t)joints.size() >= n ? ONE_WORKGROUP : EITHER;
+    int32_t* rows = nullptr;                 // host memory: contact points of the last solve that has got that far,
+    int32_t* rows_dev = nullptr;             // and where a kernel finds it
+    int alloc_rows() {
+        PE_HIP(hipHostMalloc((void**)&rows, sizeof(int32_t), hipHostMallocMapped));
+        *rows = 0;
+        PE_HIP(hipHostGetDevicePointer((void**)&rows_dev, rows, 0));
+        return PE_OK;
     }
+    enum Route { ONE_WORKGROUP = -1, EITHER = 0, FLOW = 1 };
+    Route route() const { return colouring != 0 || n > SMALL_MAX ? FLOW : n <= SMALL_BODIES || !rows ? ONE_WORKGROUP : EITHER; }
     bool one_workgroup() const {
         if (route() != EITHER) return route() == ONE_WORKGROUP;
+        if (__atomic_load_n(rows, __ATOMIC_RELAXED) <= SMALL_POINTS) return true;
         FlowTurns& t = flow_turns(device);
         std::lock_guard<std::mutex> g(t.m);
         return t.blocks[0] + t.blocks[1] > flow_max_blocks;
@@ -1780,6 +1796,7 @@ struct pe_world {
         for (void* p : joint_mem) if (p) hipFree(p);
         if (ignore_mem) hipFree(ignore_mem);
         if (ray_mem) hipFree(ray_mem);
+        if (rows) hipHostFree(rows);
         meshes.release();
         for (auto& e : ev) if (e) hipEventDestroy(e);
         for (auto& e : order_ev) if (e) hipEventDestroy(e);
@@ -1817,6 +1834,7 @@ struct pe_world {
         return PE_OK;
     }
     int launch_solve() {
+        d.rows_out = route() == EITHER ? rows_dev : nullptr;
         if (one_workgroup()) {
             if (flowed) hipLaunchKernelGGL(k_no_pairs, dim3(1), dim3(1), 0, stream, d);
             flowed = false;
@@ -1931,6 +1949,7 @@ int pe_world_create(const pe_scene_desc* sc, const pe_world_params* prm, int32_t
     static std::atomic<uint64_t> worlds{2};
     w->id = worlds++;
     w->own = w->stream;
+    if (n > SMALL_BODIES && n <= SMALL_MAX && w->alloc_rows() != PE_OK) return fail(PE_ERR_DEVICE);
     Dev& d = w->d;
     d.pcap = pcap;
     d.ps.cs = (size_t)pcap * 8;
@@ -2153,7 +2172,6 @@ int pe_world_add_joints(pe_world* w, int32_t n, const pe_joint_desc* jd) {
     w->d.jdeg = (const int32_t*)w->joint_mem[5];
     w->d.njoints = nj;
     w->d.njcol = ncol;
-    w->count_flow();
     return PE_OK;
 }
 
@@ -2779,6 +2797,9 @@ int pe_stage_create(int32_t max_bodies, int32_t max_pairs, pe_stage** out) {
     pe_world_params prm{1.0 / 60.0, {0.0, 0.0, 0.0}, 10};
     auto* S = new pe_stage();
     if (int rc = pe_world_create(&sc, &prm, max_pairs, &S->w)) { delete S; return rc; }
+    if (max_bodies > SMALL_MAX) {   // it may be handed worlds of those sizes
+        if (int rc = S->w->alloc_rows()) { delete S; return rc; }
+    }
     S->w->has_shapes = true;
     S->max_bodies = max_bodies;
     S->max_pairs = max_pairs;

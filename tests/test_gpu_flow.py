@@ -1,7 +1,7 @@
 """The single world's solve: over the GPU (colouring and data-flow sweeps) where its paths change: more
 items than waves and an item per wave, bodies whose pairs exceed what a thread keeps (32), what a workgroup
 counts in LDS (64 colours) and the colour starts kept there (1024), joints beside contacts; in one
-workgroup (up to 600 bodies) with its rows in LDS, in memory, and where pairs or colours outgrow it.  Colour classes
+workgroup (small worlds) with its rows in LDS, in memory, and where pairs or colours outgrow it.  Colour classes
 equal the oracle's; velocities and impulses are the oracle's colour-order solve's within the 1e-5 the
 other solver tests use (both sides round the same operations; the contact points differ by an ulp of
 atan2f at most)."""
@@ -103,7 +103,8 @@ def cluster_scene(n, size, seed=9):
 
 @pytest.mark.parametrize("name", ["pair", "mixed", "boxes", "limit", "chains", "joint_demo", "cluster"])
 def test_one_workgroup_equals_the_flow(name):
-    """The solve of a small world in one workgroup and over the GPU: the same bits, the same colour classes."""
+    """The solve of a small world in one workgroup and over the GPU: the same bits, the same colour classes.  (Two
+    other worlds crowd the GPU, so that all of these up to 600 bodies are solved in one workgroup.)"""
     import pe_amd
     from pe_amd import scenes
     sc, steps = {"pair": lambda: (scenes.grid_world(1, seed=2), 70),
@@ -115,6 +116,9 @@ def test_one_workgroup_equals_the_flow(name):
                  "cluster": lambda: (cluster_scene(590, 2.6), 1)}[name]()
     a, b = pe_amd.World(sc, max_pairs=200 * sc.n), pe_amd.World(sc, max_pairs=200 * sc.n)
     b.set_colouring(2)
+    crowd = [pe_amd.World(scenes.grid_world(700, seed=1)) for _ in range(2)]
+    for w in crowd:
+        w.set_solver_blocks(200)
     print(f"[one workgroup] {name}: {sc.n} bodies", flush=True)
     for part in (steps, 2 if steps > 1 else 3):
         a.step(part)
@@ -129,30 +133,35 @@ def test_one_workgroup_equals_the_flow(name):
         for k in range(len(ca) - 1):
             assert np.array_equal(np.sort(oa[ca[k]:ca[k + 1]]), np.sort(ob[ca[k]:ca[k + 1]]))
         print(f"[one workgroup] {name}: {a.counts()}", flush=True)
+        assert a.counts()["colour_rounds"] == 0 and (len(oa) == 0 or b.counts()["colour_rounds"] > 0)
         if name == "cluster" and part == steps:
             assert len(oa) * 28 + sc.n * 56 > 152 * 1024   # beyond the LDS the kernel works in
+    for w in crowd:
+        w.close()
     a.close()
     b.close()
 
 
 @pytest.mark.parametrize("name", ["mixed", "boxes", "limit", "beyond", "cluster", "chains"])
 def test_one_workgroup_up_to_its_limits(name):
-    """As test_one_workgroup_equals_the_flow, at the sizes to which one workgroup is the default: 280 bodies, 600
-    where most have joints; a cluster whose pairs outgrow its LDS."""
+    """As test_one_workgroup_equals_the_flow, at the sizes to which one workgroup is the default: 280 bodies, 600 with
+    few contact points; a pile beyond; a cluster whose pairs outgrow its LDS."""
     import pe_amd
     from pe_amd import scenes
     sc, steps = {"mixed": lambda: (scenes.grid_world(200, seed=5), 90),
                  "boxes": lambda: (scenes.grid_world(275, seed=6, p_sphere=0.0), 100),
                  "limit": lambda: (scenes.grid_world(279, seed=7, p_sphere=0.2), 80),
-                 "beyond": lambda: (scenes.grid_world(280, seed=7, p_sphere=0.2), 80),
-                 "cluster": lambda: (cluster_scene(279, 1.5), 1),
+                 "beyond": lambda: (scenes.grid_world(330, seed=7, p_sphere=0.2), 110),
+                 "cluster": lambda: (cluster_scene(279, 0.9), 1),
                  "chains": lambda: (scenes.joint_chain_scene(66, 8, seed=3), 60)}[name]()
     a, b = pe_amd.World(sc, max_pairs=200 * sc.n), pe_amd.World(sc, max_pairs=200 * sc.n)
     b.set_colouring(2)
     print(f"[one workgroup] {name}: {sc.n} bodies", flush=True)
     for part in (steps, 2):
         a.step(part)
-        b.step(part)
+        a.sync()
+        a.step(1)   # by now the contact points of the steps before are known
+        b.step(part + 1)
         for x, y in zip(a.state(), b.state()):
             assert np.array_equal(x.view(np.int32), y.view(np.int32))
         assert np.array_equal(a.impulses(), b.impulses())
@@ -168,27 +177,32 @@ def test_one_workgroup_up_to_its_limits(name):
     b.close()
 
 
-def test_joints_added_between_steps_change_the_route():
-    """A pile stepped over the GPU whose bodies then get joints (more than one for two bodies) goes on in one workgroup:
-    the same bits as over the GPU throughout."""
+def test_a_pile_that_lands_changes_the_route():
+    """400 bodies: in one workgroup as they fall, over the GPU once they lie (by the contact points of a step before), and
+    again in one workgroup when they are set back into the air: the same bits as over the GPU throughout."""
     import pe_amd
     from pe_amd import scenes
-    sc = scenes.joint_chain_scene(50, 8, seed=4)
-    joints, sc.joints = sc.joints, []
+    sc = scenes.grid_world(400, seed=9, p_sphere=0.2)
     a, b = pe_amd.World(sc), pe_amd.World(sc)
     b.set_colouring(2)
-    print(f"[route] {sc.n} bodies, {len(joints)} joints", flush=True)
-    for w in (a, b):
-        w.step(50)
-        w.sync()
-    assert a.counts()["colour_rounds"] > 0 and a.counts()["points"] > 0
-    for w in (a, b):
-        w.add_joints(joints)
-        w.step(10)
-        w.sync()
-    assert a.counts()["colour_rounds"] == 0
-    for x, y in zip(a.state(), b.state()):
-        assert np.array_equal(x.view(np.int32), y.view(np.int32))
+    start = a.state()
+    routes = []
+    print(f"[route] {sc.n} bodies", flush=True)
+    for part in range(14):
+        if part == 12:
+            for w in (a, b):
+                w.set_state(*start)
+        for w in (a, b):
+            w.step(10)
+            w.sync()
+        points = a.counts()["points"]
+        if points:
+            routes.append((points, a.counts()["colour_rounds"] > 0))
+        for x, y in zip(a.state(), b.state()):
+            assert np.array_equal(x.view(np.int32), y.view(np.int32))
+    print(f"[route] {routes}", flush=True)
+    assert not routes[0][1]
+    assert any(r for _, r in routes) and not all(r for _, r in routes)
     a.close()
     b.close()
 
@@ -258,6 +272,8 @@ def test_launch_called_off_solves_the_same():
         for x, y in zip(a.state(), b.state()):
             assert np.array_equal(x.view(np.int32), y.view(np.int32))
         assert np.array_equal(a.impulses(), b.impulses())
+        # the solve over the GPU counts its tries, one workgroup does not
+        assert a.counts()["points"] > 0 and a.counts()["colour_rounds"] > 0 and b.counts()["colour_rounds"] == 0
         a.close()
         b.close()
 
@@ -298,8 +314,10 @@ def test_worlds_that_come_and_go_change_the_route():
     ref, w = pe_amd.World(sc), pe_amd.World(sc)
     big = scenes.grid_world(900, seed=5, p_sphere=0.3)
     print("[crowd] 401 bodies", flush=True)
-    ref.step(60)
-    w.step(60)
+    ref.step(120)
+    w.step(120)
+    w.sync()
+    assert w.counts()["points"] > 700
     others = []
     for crowd in (False, True, False, True):
         if crowd:
@@ -385,3 +403,30 @@ def test_worlds_on_callers_streams_take_turns():
             assert np.array_equal(x.view(np.int32), y.view(np.int32))
         w.close()
     ref.close()
+
+
+def test_more_than_1024_colours_with_joints():
+    """Colours beyond those whose starts a workgroup keeps, and joints after them: the same bits as coloured by claims in
+    one workgroup."""
+    import pe_amd
+    from pe_amd import scenes
+    sc = scenes.concat([plate_scene(1100), scenes.joint_chain_scene(6, 5, seed=2)], "plate_chains")
+    off = plate_scene(1100).n
+    sc.position[off:] += np.array([150.0, 0.0, 0.0])
+    joints = scenes.joint_chain_scene(6, 5, seed=2).joints
+    for j in joints:
+        j.body_a += off
+        j.body_b += off
+    a, b = pe_amd.World(sc, max_pairs=40 * sc.n), pe_amd.World(sc, max_pairs=40 * sc.n)
+    print(f"[colours] {sc.n} bodies, {len(joints)} joints", flush=True)
+    for w, mode in ((a, 2), (b, 1)):
+        w.add_joints(joints)
+        w.set_colouring(mode)
+        w.step(2)
+        w.sync()
+    assert a.counts()["colors"] > 1024
+    for x, y in zip(a.state(), b.state()):
+        assert np.array_equal(x.view(np.int32), y.view(np.int32))
+    assert np.array_equal(a.impulses(), b.impulses())
+    a.close()
+    b.close()
