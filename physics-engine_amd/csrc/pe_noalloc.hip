@@ -22,9 +22,9 @@ constexpr int NA_CHUNK_CAP = 1 << 20;   // 32 Mi candidate tests
 // Byte offsets of the working arrays inside the scratch array (each 256-byte aligned).  The units' owners, made
 // after the sort, take the place of the radix sort's other arrays.
 struct NoAllocLayout {
-    size_t keys, keys2, vals2, hist, owner, vals, skey, srec, end_, first, red, blk, unit_hit, cnt, end;
+    size_t keys, keys2, vals2, hist, owner, vals, skey, srec, end_, first, red, blk, sub, unit_hit, cnt, end;
     constexpr NoAllocLayout()
-        : keys(0), keys2(0), vals2(0), hist(0), owner(0), vals(0), skey(0), srec(0), end_(0), first(0), red(0), blk(0),
+        : keys(0), keys2(0), vals2(0), hist(0), owner(0), vals(0), skey(0), srec(0), end_(0), first(0), red(0), blk(0), sub(0),
           unit_hit(0), cnt(0), end(0) {
         size_t o = 0;
         auto take = [&o](size_t bytes) { const size_t at = o; o += (bytes + 255) & ~(size_t)255; return at; };
@@ -43,7 +43,8 @@ struct NoAllocLayout {
         end_ = take(4 * (size_t)NA_MAX_BODIES);
         first = take(4 * (size_t)NA_MAX_BODIES);
         red = take(8 * SAP_RED_VALUES * 256);
-        blk = take(sizeof(uint4) * (size_t)sap_blocks(NA_MAX_BODIES));
+        blk = take(4 * (size_t)sap_blocks(NA_MAX_BODIES));
+        sub = take(sizeof(uint2) * (size_t)sap_subs(NA_MAX_BODIES));
         unit_hit = take(8 * units);
         cnt = take(sizeof(DevCounts));
         end = o;
@@ -114,7 +115,8 @@ extern "C" int pe_stage_broadphase_noalloc(int32_t n, const float* aabb, int32_t
     s.hist = reinterpret_cast<uint32_t*>(base + NA_LAYOUT.hist);
     s.red = reinterpret_cast<double*>(base + NA_LAYOUT.red);
     s.srec = reinterpret_cast<float*>(base + NA_LAYOUT.srec);
-    s.blk = reinterpret_cast<uint4*>(base + NA_LAYOUT.blk);
+    s.blk = reinterpret_cast<uint32_t*>(base + NA_LAYOUT.blk);
+    s.sub = reinterpret_cast<uint2*>(base + NA_LAYOUT.sub);
     s.owner = reinterpret_cast<uint32_t*>(base + NA_LAYOUT.owner);
     s.unit_hit = reinterpret_cast<uint64_t*>(base + NA_LAYOUT.unit_hit);
     s.cnt = reinterpret_cast<DevCounts*>(base + NA_LAYOUT.cnt);

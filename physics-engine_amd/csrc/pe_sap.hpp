@@ -58,6 +58,9 @@ constexpr int OVF_STALL = 16;        // the solver gave up a wait (not a capacit
 constexpr int sap_block(bool fused) { return fused ? 16 : 64; }
 constexpr int sap_threads(bool fused) { return 16 * sap_block(fused); }
 constexpr int SAP_EMIT_THREADS = 256;
+// Sorted bodies per counter of pairs, which k_sap_test's waves add to (with one per 64 bodies it took 30 us for the 10 000
+// boxes at rest, with one per 16 22).
+constexpr int SAP_SUB = 16;
 constexpr int SAP_UNIT = 64;         // candidates per unit
 constexpr int SAP_CHUNK = 32;        // the workspace is sized in chunks of this many candidates
 // Units for at most `chunks` chunks of candidates over n bodies' runs.
@@ -83,7 +86,8 @@ struct SapView {
     float* srec;            // [n][8] the AABB records in sorted order
     uint32_t* end;          // [n] per sorted body: the end of its run
     uint32_t* first;        // [n] and its first unit
-    uint4* blk;             // [sap_blocks(n)] per block: units, pairs, candidates (low and high half)
+    uint32_t* blk;          // [sap_blocks(n)] per block its units
+    uint2* sub;             // [sap_subs(n)] per SAP_SUB sorted bodies: candidates, pairs
     uint32_t* owner;        // [sap_units(chunk_cap, n)] per unit its sorted body
     uint64_t* unit_hit;     // [sap_units(chunk_cap, n)] per unit, bit k: its candidate k is a pair
     uint32_t* hist;         // [256 * radix_blocks(n)] radix histograms
@@ -104,6 +108,7 @@ struct SapView {
 
 __host__ inline int sap_radix_blocks(int n) { return (n + RS_TILE - 1) / RS_TILE; }
 __host__ inline int sap_red_blocks(int n) { return n < 1 ? 1 : (n + SAP_RED_THREADS - 1) / SAP_RED_THREADS < 256 ? (n + SAP_RED_THREADS - 1) / SAP_RED_THREADS : 256; }
+__host__ __device__ constexpr int sap_subs(int n) { return (n + sap_block(false) - 1) / sap_block(false) * (sap_block(false) / SAP_SUB); }
 __host__ __device__ constexpr int sap_blocks(int n, bool fused = true) { return (n + sap_block(fused) - 1) / sap_block(fused); }
 
 // BroadPhaseBase::validateCollisionPair (broad_phase_base.cpp:5-19) on two AABB records: the
@@ -360,7 +365,7 @@ constexpr int SAP_FUSED_MAX = 2048;
 template <bool FUSED>
 static __global__ void __launch_bounds__(sap_threads(FUSED)) k_sap_runs(SapView s) {
     constexpr int BLOCK = sap_block(FUSED), THREADS = sap_threads(FUSED);
-    static_assert(BLOCK <= WAVE, "a lane per body");
+    static_assert(BLOCK == (FUSED ? SAP_SUB : WAVE), "a lane per body, and whole counters");
     __shared__ uint32_t s_len[BLOCK], s_unit[BLOCK + 1], s_base;
     __shared__ int s_pairs;
     const int n = s.n, q0 = blockIdx.x * BLOCK, nq = min(BLOCK, n - q0);
@@ -369,7 +374,7 @@ static __global__ void __launch_bounds__(sap_threads(FUSED)) k_sap_runs(SapView 
     const int end = sap_search(s.skey, r < nq ? q + 1 : n, n, m);
     if ((tid & 15) == 0) s_len[r] = r < nq ? (uint32_t)(end - q - 1) : 0u;
     __syncthreads();
-    uint64_t cand = 0;
+    uint32_t cand = 0;   // of the lane's SAP_SUB bodies
     if (tid < WAVE) {
         const uint32_t len = tid < BLOCK ? s_len[tid] : 0u, units = (len + SAP_UNIT - 1) / SAP_UNIT;
         uint32_t incl = units;
@@ -378,8 +383,9 @@ static __global__ void __launch_bounds__(sap_threads(FUSED)) k_sap_runs(SapView 
         for (int o = 1; o < WAVE; o <<= 1) {
             const uint32_t y = __shfl_up(incl, o, WAVE);
             if (tid >= o) incl += y;
-            cand += (uint64_t)__shfl_xor((unsigned long long)cand, o, WAVE);
+            if (o < SAP_SUB) cand += __shfl_xor(cand, o, WAVE);
         }
+        if (!FUSED && tid % SAP_SUB == 0) s.sub[blockIdx.x * (BLOCK / SAP_SUB) + tid / SAP_SUB] = make_uint2(cand, 0u);
         if (tid < BLOCK) s_unit[tid] = incl - units;
         if (tid == BLOCK - 1) {
             s_unit[BLOCK] = incl;
@@ -408,7 +414,10 @@ static __global__ void __launch_bounds__(sap_threads(FUSED)) k_sap_runs(SapView 
         if ((tid & (WAVE - 1)) == 0 && pairs) atomicAdd(&s_pairs, pairs);
         __syncthreads();
     }
-    if (tid == 0) s.blk[blockIdx.x] = make_uint4(units, (uint32_t)s_pairs, (uint32_t)cand, (uint32_t)(cand >> 32));
+    if (tid == 0) {
+        s.blk[blockIdx.x] = units;
+        if (FUSED) s.sub[blockIdx.x] = make_uint2(cand, (uint32_t)s_pairs);
+    }
 }
 static __global__ void __launch_bounds__(256) k_sap_test(SapView s) {
     const uint32_t units = min(s.cnt->nunits, (uint32_t)sap_units(s.chunk_cap, s.n));
@@ -416,7 +425,7 @@ static __global__ void __launch_bounds__(256) k_sap_test(SapView s) {
     for (uint32_t u = wave; u < units; u += nw) {
         const int q = (int)s.owner[u];
         const int pairs = sap_test_unit(s, u, q, (int)(u - s.first[q]), (int)s.end[q]);
-        if ((threadIdx.x & (WAVE - 1)) == 0 && pairs) atomicAdd(&s.blk[q / sap_block(false)].y, (uint32_t)pairs);
+        if ((threadIdx.x & (WAVE - 1)) == 0 && pairs) atomicAdd(&s.sub[q / SAP_SUB].y, (uint32_t)pairs);
     }
 }
 
@@ -424,23 +433,30 @@ static __global__ void __launch_bounds__(256) k_sap_test(SapView s) {
 // the counts and the next axis from its nred partial sums.
 template <bool FUSED>
 static __global__ void __launch_bounds__(SAP_EMIT_THREADS) k_sap_emit(SapView s, int nred) {
-    constexpr int BLOCK = sap_block(FUSED), THREADS = SAP_EMIT_THREADS;
+    constexpr int BLOCK = sap_block(FUSED), THREADS = SAP_EMIT_THREADS, SUBS = BLOCK / SAP_SUB;
     __shared__ uint32_t s_unit[BLOCK];
     __shared__ int wsum[THREADS / WAVE + 1];
     __shared__ unsigned long long s_cand;
     const int tid = threadIdx.x, q0 = blockIdx.x * BLOCK, nq = min(BLOCK, s.n - q0);
     const bool last = blockIdx.x + 1 == gridDim.x;
-    const uint4 me = s.blk[blockIdx.x];
-    const uint32_t base = s.first[q0];
+    const uint32_t units = s.blk[blockIdx.x], base = s.first[q0];
+    uint32_t own = 0;
+    uint64_t own_cand = 0;
+#pragma unroll
+    for (int g = 0; g < SUBS; g++) {
+        const uint2 o = s.sub[blockIdx.x * SUBS + g];
+        own += o.y;
+        own_cand += o.x;
+    }
     int before = 0;
     uint64_t cand = 0;
-    for (int b = tid; b < (int)blockIdx.x; b += THREADS) {
-        const uint4 o = s.blk[b];
+    for (int b = tid; b < (int)blockIdx.x * SUBS; b += THREADS) {
+        const uint2 o = s.sub[b];
         before += (int)o.y;
-        cand += (uint64_t)o.w << 32 | o.z;
+        cand += o.x;
     }
     if (tid < nq) s_unit[tid] = s.first[q0 + tid] - base;
-    if (tid == 0) s_cand = (uint64_t)me.w << 32 | me.z;
+    if (tid == 0) s_cand = own_cand;
     int carry;
     block_exclusive_scan(before, wsum, &carry);
     if (last) {
@@ -450,7 +466,7 @@ static __global__ void __launch_bounds__(SAP_EMIT_THREADS) k_sap_emit(SapView s,
     if (last && tid < WAVE) {
         const int axis = sap_axis_final(s, nred);
         if (tid == 0) {
-            const uint32_t total = (uint32_t)carry + me.y;
+            const uint32_t total = (uint32_t)carry + own;
             int32_t ovf = 0;
             if (s_cand > (uint64_t)s.chunk_cap * SAP_CHUNK) ovf |= OVF_CHUNKS;
             if (total > (uint32_t)s.pcap) ovf |= OVF_PAIRS;
@@ -467,10 +483,10 @@ static __global__ void __launch_bounds__(SAP_EMIT_THREADS) k_sap_emit(SapView s,
             }
         }
     }
-    if (me.y == 0) return;
-    for (uint32_t u0 = 0; u0 < me.x; u0 += THREADS) {
+    if (own == 0) return;
+    for (uint32_t u0 = 0; u0 < units; u0 += THREADS) {
         const uint32_t u = u0 + tid;
-        uint64_t hit = u < me.x ? s.unit_hit[base + u] : 0ull;
+        uint64_t hit = u < units ? s.unit_hit[base + u] : 0ull;
         int tot;
         uint32_t out = (uint32_t)(carry + block_exclusive_scan((int)__popcll(hit), wsum, &tot));
         carry += tot;

@@ -2020,6 +2020,7 @@ int pe_world_create(const pe_scene_desc* sc, const pe_world_params* prm, int32_t
     rc |= w->alloc(&sp.end, n);
     rc |= w->alloc(&sp.first, n);
     rc |= w->alloc(&sp.blk, sap_blocks(n));
+    rc |= w->alloc(&sp.sub, sap_subs(n));
     sp.axis_in = -1;
     rc |= w->alloc(&sp.hist, 256 * (size_t)sap_radix_blocks(n));
     rc |= w->alloc(&sp.red, SAP_RED_VALUES * (size_t)sap_red_blocks(n));
