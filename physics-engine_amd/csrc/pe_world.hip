@@ -1164,9 +1164,10 @@ __global__ void __launch_bounds__(FLOW_THREADS) k_solve_flow(Dev d, int claims, 
     }
     if (tid < FLOW_BINS) s_hist[tid] = 0;
     auto stalled = [&]() { atomicOr(&d.cnt->overflow, OVF_STALL); };
-    // the same for every workgroup: heavy bodies have their sets; the colouring is done by claims
+    // The same for every workgroup: heavy bodies have their sets; the colouring is done by claims.  Few worlds have any: said
+    // so, their code lies out of the way (else the sweeps of 10 000 boxes at rest take 359 us instead of 354).
     bool sets = !claims && d.cnt->jp_heavy > 0, coloured = claims;
-    if (sets) {
+    if (__builtin_expect(sets, 0)) {
         jp_set_alloc(d, gtid, gsz);
         grid_barrier(&d.cnt->bar_count, &d.cnt->bar_gen, gridDim.x);
         coloured = d.cnt->jp_fall != 0;
@@ -1179,7 +1180,7 @@ __global__ void __launch_bounds__(FLOW_THREADS) k_solve_flow(Dev d, int claims, 
         // the colours still missing, in flight together.
         int tries = 0;
         bool left = true;
-        if (sets) {
+        if (__builtin_expect(sets, 0)) {
             tries = jp_colour_heavy(d, nact, gtid, gsz, s_low[tid], FLOW_SPINS);
             left = tries < 0;
             tries = abs(tries);
