@@ -57,7 +57,8 @@ constexpr int OVF_STALL = 16;        // the solver gave up a wait (not a capacit
 // that, in blocks of 64: 16), and sums up the pairs of those before it.  16 lanes search a run.
 constexpr int sap_block(bool fused) { return fused ? 16 : 64; }
 constexpr int sap_threads(bool fused) { return 16 * sap_block(fused); }
-constexpr int SAP_EMIT_THREADS = 256;
+// Threads of k_sap_emit: 50 000 bodies whose pairs lie along the sort axis take it 67 / 48 / 45 us with 256 / 512 / 1024.
+constexpr int sap_emit_threads(bool fused) { return fused ? 256 : 512; }
 // Sorted bodies per counter of pairs, which k_sap_test's waves add to (with one per 64 bodies it took 30 us for the 10 000
 // boxes at rest, with one per 16 22).
 constexpr int SAP_SUB = 16;
@@ -239,9 +240,10 @@ __device__ __forceinline__ int sap_axis_final(const SapView& s, int nb) {
 
 // Stable sort by counting: a body's sorted position is the number of bodies with a smaller key, or an equal
 // one and a lower index.  SAP_RANK_BODIES bodies per workgroup, a lane each, the other keys split over its
-// waves: n^2 / 64 wave steps of about two instructions, spread over the whole GPU -- 10 000 bodies 9 us, in
-// one launch, where the radix sort's twelve take about 60 (each costs 4.5 us in a stream whatever it does).
-// Beyond SAP_RANK_MAX the square overtakes it.  The workgroups from nrank on make the axis's partial sums.
+// waves: n^2 / 64 wave steps of about two instructions, spread over the whole GPU -- 777 bodies 9 us, 10 000 30, in
+// one launch, where the radix sort's twelve cost 4.5 us each in a stream whatever they do.  The whole sweep with one / the
+// other: 2 000 bodies 27 / 68 us, 10 000 54 / 93, 16 000 79 / 105, 20 000 113 / 117, 30 000 169 / 152.
+// The workgroups from nrank on make the axis's partial sums.
 constexpr int SAP_RANK_MAX = 16384;
 constexpr int SAP_RANK_BODIES = WAVE, SAP_RANK_THREADS = 512, SAP_RANK_TILE = 2048;
 static __global__ void __launch_bounds__(SAP_RANK_THREADS) k_sap_rank(SapView s, int nrank) {
@@ -432,8 +434,8 @@ static __global__ void __launch_bounds__(256) k_sap_test(SapView s) {
 // The pairs of a block's bodies after those of the blocks before it; the last workgroup knows all of them and sets
 // the counts and the next axis from its nred partial sums.
 template <bool FUSED>
-static __global__ void __launch_bounds__(SAP_EMIT_THREADS) k_sap_emit(SapView s, int nred) {
-    constexpr int BLOCK = sap_block(FUSED), THREADS = SAP_EMIT_THREADS, SUBS = BLOCK / SAP_SUB;
+static __global__ void __launch_bounds__(sap_emit_threads(FUSED)) k_sap_emit(SapView s, int nred) {
+    constexpr int BLOCK = sap_block(FUSED), THREADS = sap_emit_threads(FUSED), SUBS = BLOCK / SAP_SUB;
     __shared__ uint32_t s_unit[BLOCK];
     __shared__ int wsum[THREADS / WAVE + 1];
     __shared__ unsigned long long s_cand;
@@ -453,13 +455,13 @@ static __global__ void __launch_bounds__(SAP_EMIT_THREADS) k_sap_emit(SapView s,
     for (int b = tid; b < (int)blockIdx.x * SUBS; b += THREADS) {
         const uint2 o = s.sub[b];
         before += (int)o.y;
-        cand += o.x;
+        if (!FUSED) cand += o.x;
     }
     if (tid < nq) s_unit[tid] = s.first[q0 + tid] - base;
-    if (tid == 0) s_cand = own_cand;
+    if (!FUSED && tid == 0) s_cand = own_cand;
     int carry;
     block_exclusive_scan(before, wsum, &carry);
-    if (last) {
+    if (!FUSED && last) {
         if (cand) atomicAdd(&s_cand, (unsigned long long)cand);
         __syncthreads();
     }
@@ -468,7 +470,8 @@ static __global__ void __launch_bounds__(SAP_EMIT_THREADS) k_sap_emit(SapView s,
         if (tid == 0) {
             const uint32_t total = (uint32_t)carry + own;
             int32_t ovf = 0;
-            if (s_cand > (uint64_t)s.chunk_cap * SAP_CHUNK) ovf |= OVF_CHUNKS;
+            // (SAP_FUSED_MAX bodies form fewer candidates than any workspace holds)
+            if (!FUSED && s_cand > (uint64_t)s.chunk_cap * SAP_CHUNK) ovf |= OVF_CHUNKS;
             if (total > (uint32_t)s.pcap) ovf |= OVF_PAIRS;
             ovf |= s.cnt->overflow;
             s.cnt->overflow = ovf;
@@ -527,11 +530,11 @@ inline void sap_launch(const SapView& s, hipStream_t st) {
     }
     if (n <= SAP_FUSED_MAX) {
         hipLaunchKernelGGL(k_sap_runs<true>, dim3(sap_blocks(n, true)), dim3(sap_threads(true)), 0, st, s);
-        hipLaunchKernelGGL(k_sap_emit<true>, dim3(sap_blocks(n, true)), dim3(SAP_EMIT_THREADS), 0, st, s, nred);
+        hipLaunchKernelGGL(k_sap_emit<true>, dim3(sap_blocks(n, true)), dim3(sap_emit_threads(true)), 0, st, s, nred);
     } else {
         hipLaunchKernelGGL(k_sap_runs<false>, dim3(sap_blocks(n, false)), dim3(sap_threads(false)), 0, st, s);
         hipLaunchKernelGGL(k_sap_test, dim3(2048), dim3(256), 0, st, s);
-        hipLaunchKernelGGL(k_sap_emit<false>, dim3(sap_blocks(n, false)), dim3(SAP_EMIT_THREADS), 0, st, s, nred);
+        hipLaunchKernelGGL(k_sap_emit<false>, dim3(sap_blocks(n, false)), dim3(sap_emit_threads(false)), 0, st, s, nred);
     }
 }
 
