@@ -67,7 +67,7 @@ struct Dev {
     int32_t* color_start;   // [pcap+1]
     int32_t* claim;         // [n] claims of the colouring in one workgroup
     DevCounts* cnt;
-    int32_t* rows_out;      // host memory: contact points of the last solve (null: not asked for)
+    int32_t* rows_out;      // host memory: how full the last solve would fill one workgroup (null: not asked for)
     int pcap;
     float dt;
     float g[3];
@@ -486,9 +486,11 @@ template <bool GRAPH> __global__ void k_setup(Dev d) {
         if (act) d.act[slot] = p;
     }
 }
-// Tells the host the solve's contact points (it reads them at some later launch: pe_world::one_workgroup).
-__device__ __forceinline__ void report_rows(const Dev& d, int rows) {
-    if (d.rows_out) __hip_atomic_store(d.rows_out, rows, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+// Tells the host what a solve's contact points come to beyond those that one workgroup takes a colour at a time (it reads
+// it at some later launch: pe_world::one_workgroup).
+constexpr int SMALL_COLOUR_POINTS = 160;
+__device__ __forceinline__ void report_rows(const Dev& d, int rows, int ncol) {
+    if (d.rows_out) __hip_atomic_store(d.rows_out, rows - SMALL_COLOUR_POINTS * ncol, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 // A body in more pairs than this is heavy: its pairs, which take different colours one after another, do not look at each
 // other but at the set of their colours (jp_colour_heavy).
@@ -1338,7 +1340,7 @@ __global__ void __launch_bounds__(FLOW_THREADS) k_solve_flow(Dev d, int claims, 
                                kb ? 0 : jp_rank(d, b, p, c, sets), kb ? 0 : d.jp_deg[b] + (d.jdeg ? d.jdeg[b] : 0));
     }
     grid_barrier(&d.cnt->bar_count, &d.cnt->bar_gen, gridDim.x);   // the order is complete
-    if (gtid == 0) report_rows(d, d.cnt->nrows);
+    if (gtid == 0) report_rows(d, d.cnt->nrows, ncol);
 
     // consecutive items go to different workgroups, so a colour's pairs spread over the CUs; half of the
     // waves take the joints, if there are any
@@ -1583,7 +1585,7 @@ __global__ void __launch_bounds__(SMALL_THREADS) k_solve_small(Dev d) {
         solve_alone<true>(d, nact, (int*)lds);
         if (tid == 0) {
             d.cnt->nact = 0;
-            report_rows(d, 8 * nact);
+            report_rows(d, 8 * nact, 0);
         }
         return;
     }
@@ -1656,7 +1658,7 @@ __global__ void __launch_bounds__(SMALL_THREADS) k_solve_small(Dev d) {
         d.cnt->nordered = nact;
         d.cnt->jp_rounds = 0;
         d.cnt->nact = 0;   // counted from zero by the next step's set-up
-        report_rows(d, nrows);
+        report_rows(d, nrows, ncol);
     }
 }
 
@@ -1719,15 +1721,20 @@ struct FlowTurn {
 }  // namespace
 
 // The solve runs in one workgroup (k_solve_small) up to SMALL_BODIES bodies, and up to SMALL_MAX while the last solve
-// the host knows of had at most SMALL_POINTS contact points or the process's worlds crowd the GPU (FlowTurns): a colour's
-// pairs then fill the workgroup about once.  us per step in one workgroup / over the GPU (contact points):
-//   bodies                  200              260               300               400                590
-//   boxes at rest           141 / 144 (716)  162 / 160 (958)   172 / 159 (1043)  210 / 166 (1429)   279 / 181 (2107)
-//   boxes, spheres at rest  141 / 145 (447)  153 / 150 (643)   167 / 157 (733)   180 / 157 (877)    237 / 169 (1322)
-//   a tower struck          158 / 186 (451)  221 / 236 (1004)  235 / 241 (1029)  310 / 263 (1667)   415 / 293 (2843)
-//   boxes, spheres falling  107 / 127 (279)  125 / 137 (362)   122 / 134 (389)   131 / 135 (472)    162 / 148 (748)
-//   joint chains             80 / 121 (0)    250 / 304 (0)     274 / 335 (3)     272 / 325 (5)      293 / 356 (8)
-constexpr int SMALL_BODIES = 280, SMALL_MAX = 600, SMALL_POINTS = 650;
+// the host knows of had no more contact points than SMALL_POINTS + SMALL_COLOUR_POINTS a colour, or the process's worlds
+// crowd the GPU (FlowTurns): more fill a colour's pass of the workgroup more than once, where the flow waits once a
+// colour whatever it holds.  us per step in one workgroup / over the GPU (contact points, colours):
+//   bodies                  200              260               300                400                590
+//   boxes at rest           141 / 144 (716)  162 / 160 (958)   172 / 159 (1043)   210 / 166 (1429)   279 / 181 (2107)
+//   boxes, spheres at rest  141 / 145 (447)  153 / 150 (643)   167 / 157 (733)    180 / 157 (877)    237 / 169 (1322)
+//   boxes, spheres falling  107 / 127 (279)  125 / 137 (362)   122 / 134 (389)    131 / 135 (472)    162 / 148 (748)
+//   joint chains             80 / 121 (0)    250 / 304 (0)     274 / 335 (3)      272 / 325 (5)      293 / 356 (8)
+//   bodies                  285                 330                 380                 440                 590
+//   a steeper pile, boxes   204 / 215 (994, 6)  214 / 219 (1142, 6) 236 / 228 (1339, 7) 268 / 237 (1539, 6) 328 / 267 (1981, 7)
+//   with spheres            181 / 186 (687, 5)  206 / 213 (789, 6)  211 / 212 (885, 6)  234 / 221 (1035, 6) 278 / 239 (1321, 6)
+//   a tower struck          233 / 248 (1188, 7) 263 / 263 (1232, 7) 281 / 258 (1240, 6) 305 / 271 (1932, 7) 429 / 306 (3281, 7)
+// (of these a line at 650 points gave up to 8 % away, this one up to 6 where it keeps one workgroup and 3 where not).
+constexpr int SMALL_BODIES = 280, SMALL_MAX = 600, SMALL_POINTS = 200;
 
 struct pe_world {
     Dev d{};
@@ -1746,7 +1753,7 @@ struct pe_world {
     uint64_t order() const { return stream == own ? id : stream == nullptr ? 1 : 0; }
     bool flowed = false;                     // the last solve was over the GPU: it leaves its pairs listed
     int colouring = 0;                       // 0: by body count, 1: one workgroup's claims, 2: over the GPU
-    int32_t* rows = nullptr;                 // host memory: contact points of the last solve that has got that far,
+    int32_t* rows = nullptr;                 // host memory: what report_rows left there last,
     int32_t* rows_dev = nullptr;             // and where a kernel finds it
     int alloc_rows() {
         PE_HIP(hipHostMalloc((void**)&rows, sizeof(int32_t), hipHostMallocMapped));

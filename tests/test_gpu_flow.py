@@ -178,8 +178,8 @@ def test_one_workgroup_up_to_its_limits(name):
 
 
 def test_a_pile_that_lands_changes_the_route():
-    """400 bodies: in one workgroup as they fall, over the GPU once they lie (by the contact points of a step before), and
-    again in one workgroup when they are set back into the air: the same bits as over the GPU throughout."""
+    """400 bodies: in one workgroup as they fall, over the GPU once they lie (by the contact points and colours of a step
+    before), and again in one workgroup when they are set back into the air: the same bits as over the GPU throughout."""
     import pe_amd
     from pe_amd import scenes
     sc = scenes.grid_world(400, seed=9, p_sphere=0.2)
