@@ -115,11 +115,12 @@ __global__ void k_integrate_status(Dev d) {
 // strictly nearer one), as a minimum over (distance key, index).
 // Bound by the passes over the bodies: every ray meets every body's record (72 bytes) and nearly all it meets
 // are far off.  So a body is read once for several rays, and a box is only tested (some 150 instructions, a dozen
-// divisions) for a ray that ray_may_hit_box lets through.  4096 rays against 10 000 boxes: 470 -> 247 us (the
-// tests left gathered in LDS and done 64 at a time: 314, by their second reads and the LDS they take from the waves).
+// divisions) for a ray that ray_may_hit_box lets through.  4096 rays against 10 000 boxes: 470 -> 152 us (with the mesh
+// walk's stacks in the same kernel 239; the tests left gathered in LDS and done 64 at a time were slower, by their second
+// reads and the LDS they take from the waves).
 // MESH: the world has meshes.  Their walks take a stack row per thread (bvh_stack_row), so a workgroup has no more
 // threads than there are rows; and the one thread that holds a terrain would walk it for each of its workgroup's rays
-// in turn, so it has one ray.
+// in turn, so it has one ray (4096 rays over a terrain: 3.0 ms).
 constexpr int RAY_IN = 7;    // start (3), direction (3), length
 constexpr int RAY_OUT = 12;  // hit, body (int bits), distance, point (3), normal (3), pad
 constexpr int RAYS_MAX = 4;

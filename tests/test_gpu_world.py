@@ -205,8 +205,8 @@ def test_reference_sample_scene_stages():
 
 @pytest.mark.parametrize("n,mode", [(13000, 0), (6000, 1), (6000, 2)])
 def test_large_world_colouring_matches_oracle(n, mode):
-    """The solver's colouring in one workgroup (claims in LDS) and in rounds over the GPU: a world
-    beyond the one-workgroup limit (12 288 bodies, rounds) and a smaller one both ways give colour
+    """The solver's colouring in one workgroup (claims) and over the GPU: a world
+    beyond the one-workgroup limit (12 288 bodies, over the GPU) and a smaller one both ways give colour
     classes equal to the oracle's (bit-exact), and the solved velocities stay within 1e-5, step after
     step in lock-step."""
     import pe_amd
